@@ -1138,8 +1138,28 @@ __global__ __launch_bounds__(256) void dkdv_group_sum_kernel(const float *part_k
   }
   T o8[8] = {from_float<T>(lo.x), from_float<T>(lo.y), from_float<T>(lo.z), from_float<T>(lo.w),
              from_float<T>(hi.x), from_float<T>(hi.y), from_float<T>(hi.z), from_float<T>(hi.w)};
-  *reinterpret_cast<uint4 *>((T *)out.ptr + b * out.sb + kvh * out.sh + (int64_t)key * out.st + ch * 8) =
-      *reinterpret_cast<const uint4 *>(o8);
+  uint4 *dst = reinterpret_cast<uint4 *>((T *)out.ptr + b * out.sb + kvh * out.sh + (int64_t)key * out.st + ch * 8);
+#pragma unroll
+  for (int i = 0; i < (int)sizeof(T) / 2; ++i) dst[i] = reinterpret_cast<const uint4 *>(o8)[i];
+}
+
+template <typename T>
+static int launch_group_sum_t(const BwdParams &p, const float *part_k, const float *part_v, hipStream_t stream) {
+  const int keys = p.seqs.max_k_len;
+  const int64_t total = (int64_t)p.seqs.batch * p.Hkv * keys * (p.D / 8);
+  DK_NOTE_KERNEL("dkdv_group_sum_kernel");
+  hipLaunchKernelGGL((dkdv_group_sum_kernel<T>), dim3((unsigned)cdiv64(total, 256), 2), dim3(256), 0, stream, part_k, part_v,
+                     p.dk, p.dv, p.seqs.batch, p.Hq, p.Hkv, keys, p.D);
+  DK_HIP_CHECK(hipGetLastError());
+  return DK_OK;
+}
+
+int launch_dkdv_group_sum(const BwdParams &p, int dtype, const float *part_k, const float *part_v, hipStream_t stream) {
+  switch (dtype) {
+    case DK_BF16: return launch_group_sum_t<bf16_t>(p, part_k, part_v, stream);
+    case DK_F16: return launch_group_sum_t<f16_t>(p, part_k, part_v, stream);
+    default: return launch_group_sum_t<float>(p, part_k, part_v, stream);
+  }
 }
 
 // Scratch for the head-split dK/dV pass: fp32 per-q-head partials of dK and dV (16-bit partials
@@ -1217,12 +1237,7 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
                               : "mfma_dkdv_kernel (one workgroup per q head)");
     hipLaunchKernelGGL((mfma_dkdv_kernel<T, D, PAD, SUB>), dim3(p.Hq, cblocks, s.batch), dim3(256), smem_dkdv, stream, pp, 1);
     DK_HIP_CHECK(hipGetLastError());
-    const int64_t total = (int64_t)s.batch * p.Hkv * keys * (p.D / 8);
-    DK_NOTE_KERNEL("dkdv_group_sum_kernel");
-    hipLaunchKernelGGL((dkdv_group_sum_kernel<T>), dim3((unsigned)cdiv64(total, 256), 2), dim3(256), 0, stream, part_k,
-                       part_v, p.dk, p.dv, s.batch, p.Hq, p.Hkv, (int)keys, p.D);
-    DK_HIP_CHECK(hipGetLastError());
-    return DK_OK;
+    return launch_group_sum_t<T>(p, part_k, part_v, stream);
   }
   DK_NOTE_KERNEL(po.csc.rot ? "mfma_dkdv_kernel, heads in rotation" : "mfma_dkdv_kernel");
   hipLaunchKernelGGL((mfma_dkdv_kernel<T, D, PAD, SUB>), dim3(p.Hkv, cblocks, s.batch), dim3(256), smem_dkdv, stream, po, 0);

@@ -1,7 +1,7 @@
-// fp32 inputs on the matrix cores of gfx950: v_mfma_f32_32x32x2_f32, head dims up to 64 (multiples
-// of 4, zero-padded to 64 on chip), 64 x 64 tiles with one int per table entry.  Forward (fixed,
-// padded, packed and single-token sequences, LSE) and backward (dQ over CSR rows, dK/dV over CSC
-// columns; delta = rowsum(O * dO) - dLSE by a small kernel ahead of them).  fp32 products with
+// fp32 inputs on the matrix cores of gfx950: v_mfma_f32_32x32x2_f32, head dims up to 128 (multiples
+// of 4, zero-padded on chip to 64, 96 or 128), 64 x 64 tiles with one int per table entry.  Forward
+// (fixed, padded, packed and single-token sequences, LSE) and backward (dQ over CSR rows, dK/dV over
+// CSC columns; delta = rowsum(O * dO) - dLSE by a small kernel ahead of them).  fp32 products with
 // fp32 accumulation: results agree with the generic fp32-FMA kernels to rounding.
 //
 //   D(32x32) += A(32x2) * B(2x32):  A operand, lane l: row l%32, k = l/32 (one float)
@@ -9,57 +9,93 @@
 //                                   accumulator, lane l, register r: col l%32, row 8(r/4) + 4(l/32) + r%4
 //
 // The contraction index of a product may be walked in any order as long as A and B agree, so:
-//  * products over head dims (S = K Q^T, dP = V dO^T, ...) give lane (x, g) the dims 32 g + s in
-//    step s: a lane's operands of 32 steps are 32 consecutive floats (16-byte reads);
+//  * products over head dims (S = K Q^T, dP = V dO^T, ...) give lane (x, g) the dims KD/2 g + s in
+//    step s: a lane's operands of KD/2 steps are consecutive floats (16-byte reads);
 //  * products over keys or q rows (O^T += V^T P^T, dQ^T += K^T dS^T, dV^T += dO^T P, dK^T += Q^T dS)
-//    take step (tile, r) = the pair of rows that accumulator register r of the two half-waves
-//    stands for, 8(r/4) + r%4 and 8(r/4) + 4 + r%4: the second operand is then the lane's own
-//    register r of the S / P / dS accumulator, with no exchange between lanes, and the first
-//    one a 4-byte LDS read per lane, 32 consecutive floats of one tile row per half-wave.
-// Tiles live in LDS as plain rows of 64 floats plus 4 floats of padding (16-byte row reads of 16
-// consecutive rows then touch every bank once).  One stage per workgroup: with up to five small
-// workgroups per CU, one loads while the others multiply.
+//    take step r = the pair of rows that accumulator register r of the two half-waves stands for,
+//    8(r/4) + r%4 and 8(r/4) + 4 + r%4: the second operand is then the lane's own register r of
+//    the S / P / dS accumulator, with no exchange between lanes, and the first one a 4-byte LDS read
+//    per lane, 32 consecutive floats of one tile row per half-wave.
+//
+// Work split: a workgroup of four waves takes one 64 x 64 block at a time and each wave one of its
+// 32 x 32 quadrants (row half x key half), so that a block's four products run on the four SIMDs at
+// once and the waves' partial results (over the key halves, or the q-row halves in the dK/dV pass)
+// are added through LDS once, at the end.  An instruction of this shape occupies the matrix pipe for
+// 64 cycles, so one wave per SIMD covers its own LDS reads, exponentials and bookkeeping; tiles are
+// copied HBM -> LDS asynchronously (LDS DMA) into two stages, the next block's while the current one
+// is multiplied.  Bound: fp32 MFMA (a large fp32 product of the vendor library: 153 TFLOP/s).  Measured
+// forward / backward, us: 1 x 8192 tokens, 32 heads of 64 dims, local 16, vert 8: 906 / 2765 = 101 / 82
+// TFLOP/s (two waves of 32 x 64 quadrants over a single stage: 1114 / 3836); 8 heads x 1024 tokens of 64
+// dims: 26 / 126 (52 / 262); 16 heads x 2000 tokens of 128 dims, local 8, vert 4: 122 / 505 (fp32-FMA
+// kernels of generic_*.hip: 474 / 3189), where the longest row and column, one workgroup each, set the
+// time.
+#include <type_traits>
+
 #include "common.h"
 #include "device_common.h"
 #include "mfma_common.h"
 
 namespace dk {
 
+size_t mfma_bwd_workspace_bytes(const BwdParams &p);
+int launch_dkdv_group_sum(const BwdParams &p, int dtype, const float *part_k, const float *part_v, hipStream_t stream);
+
 namespace f32 {
 
-constexpr int kD = 64;        // tile width (head dims, zero-padded)
-constexpr int kLd = kD + 4;   // floats per tile row in LDS
+constexpr int NT = 256;  // threads: four waves
 
 __device__ __forceinline__ floatx16 mma(float a, float b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-// 64 rows x 64 floats from memory (row r at base + r * stride, rows outside [lo, hi) and head
-// dims at or beyond d as zeros) into an LDS tile, by NT threads; 16-byte pieces, consecutive
-// threads along a row.
-template <int NT>
-__device__ __forceinline__ void load_tile(const float *base, int64_t stride, int lo, int hi, int d, float *tile, int tid) {
-#pragma unroll
-  for (int i = 0; i < 64 * 16 / NT; ++i) {
-    const int c = tid + i * NT, r = c >> 4, ch = c & 15;
-    float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (r >= lo && r < hi && ch * 4 < d) w = *reinterpret_cast<const float4 *>(base + (int64_t)r * stride + ch * 4);
-    *reinterpret_cast<float4 *>(tile + r * kLd + ch * 4) = w;
-  }
-}
+// KD: head dims multiplied (64, 96 or 128); tiles are 64 rows of W = 64 or 128 floats in the
+// swizzled layout of a 16-bit tile of twice the width (mfma_common.h).  PAD: the tensors hold fewer
+// head dims than KD (the others are zeros in LDS) or than W (never read).
+template <int KD, bool PAD>
+struct Shape {
+  static constexpr int W = KD <= 64 ? 64 : 128;
+  using TL = Tile<2 * W>;
+  using Loader = TileLoader<2 * W, NT, PAD>;
+  static constexpr int HD = KD / 2;   // head dims per lane of a product over head dims
+  static constexpr int DT = KD / 32;  // 32-dim tiles of a result
+  static constexpr int kTile = TL::kBytes;
+  static constexpr int kStage = 2 * kTile;  // two tiles: K and V, or Q and dO
+  static constexpr int kSmem = 2 * kStage;
+};
 
-// acc(32 x 32) += X Y^T over the 64 head dims: rows = the 32 rows of tile `xt` from row0, columns =
-// the lanes' own rows of Y.  Lane (x, g) multiplies dims 32 g + s in step s; yf[s] is dim 32 g + s
-// of the row of Y that is the lane's column.
-__device__ __forceinline__ floatx16 dot_dims(const float *xt, int row0, const float (&yf)[32], int lane, floatx16 acc) {
-  const float *src = xt + (row0 + (lane & 31)) * kLd + (lane >> 5) * 32;
+// acc(32 x 32) += X Y^T over the head dims: rows = rows row0 .. row0 + 31 of tile `xt` (row0 a
+// multiple of 32), columns = the lanes' own rows of Y, yf[s] = dim HD g + s of that row.
+template <int KD, bool PAD>
+__device__ __forceinline__ floatx16 dot_dims(const char *xt, int row0, const float (&yf)[KD / 2], int lane, floatx16 acc) {
+  using S = Shape<KD, PAD>;
+  constexpr int CH = S::HD / 4, B = 4;  // 16-byte chunks per lane, read in batches ahead of their multiplies
+  static_assert(CH % B == 0, "whole batches");
+  // (opaque: the read addresses - a few XORs per 64-cycle multiply - are computed here; hoisted out of
+  // the caller's loop they would occupy registers throughout)
+  asm volatile("" : "+v"(lane));
+  const int m = lane & 31, g = lane >> 5;
+  const char *row = xt + (row0 + m) * S::TL::kRowBytes;
+  const int swz = S::TL::swz(m);
+  float4 x[2][B];
 #pragma unroll
-  for (int s4 = 0; s4 < 8; ++s4) {
-    const float4 x = *reinterpret_cast<const float4 *>(src + s4 * 4);
-    acc = mma(x.x, yf[s4 * 4], acc);
-    acc = mma(x.y, yf[s4 * 4 + 1], acc);
-    acc = mma(x.z, yf[s4 * 4 + 2], acc);
-    acc = mma(x.w, yf[s4 * 4 + 3], acc);
+  for (int i = 0; i < B; ++i) x[0][i] = *reinterpret_cast<const float4 *>(row + (((g * CH + i) ^ swz) << 4));
+#pragma unroll
+  for (int b = 0; b < CH / B; ++b) {
+    if (b + 1 < CH / B) {
+#pragma unroll
+      for (int i = 0; i < B; ++i)
+        x[(b + 1) & 1][i] = *reinterpret_cast<const float4 *>(row + (((g * CH + (b + 1) * B + i) ^ swz) << 4));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      const float4 w = x[b & 1][i];
+      acc = mma(w.x, yf[(b * B + i) * 4], acc);
+      acc = mma(w.y, yf[(b * B + i) * 4 + 1], acc);
+      acc = mma(w.z, yf[(b * B + i) * 4 + 2], acc);
+      acc = mma(w.w, yf[(b * B + i) * 4 + 3], acc);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   return acc;
 }
@@ -67,145 +103,269 @@ __device__ __forceinline__ floatx16 dot_dims(const float *xt, int row0, const fl
 // acc[dt](32 dims x 32 columns) += T^T(dims x rows) * W(rows x columns) over the 32 rows row0 .. row0 + 31 of
 // tile `t`: step r takes rows 8(r/4) + r%4 (+4 in the upper half-wave), w[r] is the lane's own
 // accumulator register r of W^T's product (column = lane % 32).
-__device__ __forceinline__ void dot_rows(const float *t, int row0, const floatx16 &w, int lane, floatx16 (&acc)[2]) {
+template <int KD, bool PAD>
+__device__ __forceinline__ void dot_rows(const char *t, int row0, const floatx16 &w, int lane, floatx16 (&acc)[KD / 32]) {
+  using S = Shape<KD, PAD>;
+  constexpr int DT = S::DT, B = 2;  // steps per batch of operand reads
+  asm volatile("" : "+v"(lane));  // as in dot_dims
   const int g = lane >> 5, m = lane & 31;
+  const char *base = t + row0 * S::TL::kRowBytes + (m & 3) * 4;
+  auto read = [&](int r, int dt) {
+    const int row = (r >> 2) * 8 + g * 4 + (r & 3);
+    return *reinterpret_cast<const float *>(base + S::TL::off(row, dt * 8 + (m >> 2)));
+  };
+  float a[2][B][DT];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const float *row = t + (row0 + (r >> 2) * 8 + g * 4 + (r & 3)) * kLd + m;
-    acc[0] = mma(row[0], w[r], acc[0]);
-    acc[1] = mma(row[32], w[r], acc[1]);
+  for (int i = 0; i < B; ++i)
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) a[0][i][dt] = read(i, dt);
+#pragma unroll
+  for (int b = 0; b < 16 / B; ++b) {
+    if (b + 1 < 16 / B) {
+#pragma unroll
+      for (int i = 0; i < B; ++i)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) a[(b + 1) & 1][i][dt] = read((b + 1) * B + i, dt);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < B; ++i)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) acc[dt] = mma(a[b & 1][i][dt], w[b * B + i], acc[dt]);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// 32 consecutive floats of a row (dims 32 g ..) as one lane's operands; zeros when !ok or beyond d
-__device__ __forceinline__ void load_frag(const float *row, bool ok, int g, int d, float (&f)[32]) {
+// consecutive floats of a row (dims HD g ..) as one lane's operands; zeros when !ok or beyond d
+template <int HD>
+__device__ __forceinline__ void load_frag(const float *row, bool ok, int g, int d, float (&f)[HD]) {
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
+  for (int c = 0; c < HD / 4; ++c) {
     float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (ok && g * 32 + c * 4 < d) w = *reinterpret_cast<const float4 *>(row + g * 32 + c * 4);
+    if (ok && g * HD + c * 4 < d) w = *reinterpret_cast<const float4 *>(row + g * HD + c * 4);
     f[c * 4] = w.x, f[c * 4 + 1] = w.y, f[c * 4 + 2] = w.z, f[c * 4 + 3] = w.w;
   }
 }
 
-// the lane's 32 result values of a (dims x columns) accumulator pair: dims 32 dt + 8 r4 + 4 g + {0..3}
-__device__ __forceinline__ void store_frag(float *row, const floatx16 (&acc)[2], float scale, int g, int d) {
+// Addition of two waves' accumulators through LDS.  Each wave of a pair keeps half of the 32-dim
+// tiles (wave 0 the first half, wave 1 the second and the middle one of an odd count): it hands the
+// others over and adds the partner's share, scaled by `own` / `other`, to its own.  `buf`: DT * 4 KB
+// per pair.  Between give and take: a barrier.  (`second` is wave-uniform but not a compile-time
+// constant: accumulators are picked by selects between values in fixed registers - picked by a
+// branch they end up in scratch memory.)
+__device__ __forceinline__ void give_tile(const float (&v)[16], float *buf, int dt, int lane) {
 #pragma unroll
-  for (int dt = 0; dt < 2; ++dt)
+  for (int r4 = 0; r4 < 4; ++r4)
+    *reinterpret_cast<float4 *>(buf + ((dt * 4 + r4) * 64 + lane) * 4) =
+        make_float4(v[r4 * 4], v[r4 * 4 + 1], v[r4 * 4 + 2], v[r4 * 4 + 3]);
+}
+template <int DT>
+__device__ __forceinline__ void give_half(const floatx16 (&acc)[DT], bool second, float *buf, int lane) {
+  constexpr int N = DT / 2;
 #pragma unroll
-    for (int r4 = 0; r4 < 4; ++r4) {
-      const int d0 = dt * 32 + r4 * 8 + g * 4;
-      if (d0 < d)
-        *reinterpret_cast<float4 *>(row + d0) = make_float4(acc[dt][r4 * 4] * scale, acc[dt][r4 * 4 + 1] * scale,
-                                                            acc[dt][r4 * 4 + 2] * scale, acc[dt][r4 * 4 + 3] * scale);
-    }
+  for (int i = 0; i < N; ++i) {
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = second ? acc[i][r] : acc[DT - N + i][r];
+    give_tile(v, buf, second ? i : DT - N + i, lane);
+  }
+  if (DT % 2 && !second) {
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = acc[N][r];
+    give_tile(v, buf, N, lane);
+  }
+}
+// ... and the finished half of the row goes to memory (dims 32 dt + 8 r4 + 4 g + {0..3})
+__device__ __forceinline__ void take_tile(const float (&v)[16], const float *buf, int dt, int lane, float own, float other,
+                                          float *row, bool ok, int d) {
+#pragma unroll
+  for (int r4 = 0; r4 < 4; ++r4) {
+    const float4 p = *reinterpret_cast<const float4 *>(buf + ((dt * 4 + r4) * 64 + lane) * 4);
+    const int d0 = dt * 32 + r4 * 8 + (lane >> 5) * 4;
+    if (ok && d0 < d)
+      *reinterpret_cast<float4 *>(row + d0) = make_float4(v[r4 * 4] * own + p.x * other, v[r4 * 4 + 1] * own + p.y * other,
+                                                          v[r4 * 4 + 2] * own + p.z * other, v[r4 * 4 + 3] * own + p.w * other);
+  }
+}
+template <int DT>
+__device__ __forceinline__ void take_half_and_store(const floatx16 (&acc)[DT], bool second, const float *buf, int lane,
+                                                    float own, float other, float *row, bool ok, int d) {
+  constexpr int N = DT / 2;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = second ? acc[DT - N + i][r] : acc[i][r];
+    take_tile(v, buf, second ? DT - N + i : i, lane, own, other, row, ok, d);
+  }
+  if (DT % 2 && second) {
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = acc[N][r];
+    take_tile(v, buf, N, lane, own, other, row, ok, d);
+  }
 }
 
+template <int DT>
+__device__ __forceinline__ void clear(floatx16 (&acc)[DT]) {
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
+}
+
+template <int V>
+struct Stage {  // compile-time stage passed to a generic lambda
+  static constexpr int value = V;
+};
+
 // ---------------------------------------------------------------------------
-// forward: workgroup = 64 q rows of one head, 2 waves of 32 rows
+// forward: workgroup = 64 q rows of one head; wave = 32 rows x 32 keys of every block, with its own
+// running maximum and sum (the two key halves of a row are merged at the end)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(128) void fwd_kernel(const FwdParams p, int tiles_y) {
-  __shared__ __align__(16) float sK[64 * kLd];
-  __shared__ __align__(16) float sV[64 * kLd];
+template <int KD, bool PAD>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2 : 1, KD <= 64 ? 2 : 1))) void fwd_kernel(
+    const FwdParams p, int tiles_y) {
+  using S = Shape<KD, PAD>;
+  extern __shared__ __align__(16) char smem[];
   SeqInfo sq;
   int tile;
   bool has_rows;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (p.csr.order && !p.seqs.packed) {  // the table's own order, longest rows first (the grid covers every row of it)
     sq = load_seq(p.seqs, blockIdx.z, p.causal);
-    tile = p.csr.order[lut_head(p.csr, grid_head(p.csr), p.Hq, p.Hkv) * p.csr.order_sh + blockIdx.y] - sq.past / 64;
+    tile = scalar_load(p.csr.order + lut_head(p.csr, grid_head(p.csr), p.Hq, p.Hkv) * p.csr.order_sh + blockIdx.y) - sq.past / 64;
     has_rows = tile >= 0 && tile < seq_row_blocks(sq, 64);
   } else {
     has_rows = resolve_tile(p.seqs, p.causal, 64, 1, tiles_y - 1 - (int)blockIdx.y, blockIdx.z, sq, tile);
   }
   if (p.seqs.zero_outside)
-    zero_rows_outside<float>(p.seqs, sq, blockIdx.y, tiles_y, p.o, p.lse, grid_head(p.csr), 1, p.D, p.vec_ok, threadIdx.x, 128);
+    zero_rows_outside<float>(p.seqs, sq, blockIdx.y, tiles_y, p.o, p.lse, grid_head(p.csr), 1, p.D, p.vec_ok, tid, NT);
   if (!has_rows) return;
   const int rb = sq.past / 64 + tile;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int h = grid_head(p.csr), kvh = h / (p.Hq / p.Hkv);
+  const int rh = wave & 1, kh = wave >> 1;  // row half, key half
+  const int h = grid_head(p.csr), kvh = __builtin_amdgcn_readfirstlane(h / (p.Hq / p.Hkv));
   const int m = lane & 31, g = lane >> 5;
-  const int row0 = rb * 64 + wave * 32;
+  const int row0 = rb * 64 + rh * 32;
   const int pos = row0 + m, qi = pos - sq.past;
   const bool row_ok = qi >= 0 && qi < sq.q_len;
+  if constexpr (PAD) {  // the slots of the head dims beyond p.D stay zero for the whole kernel
+    zero_tiles<NT>(smem, S::kSmem, tid);
+    __syncthreads();
+  }
 
-  float qf[32];
-  load_frag((const float *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh + (int64_t)(sq.q_start + qi) * p.q.st, row_ok, g, p.D, qf);
   const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
   int e0 = 0, e1 = 0;
-  if (rb < p.csr.num_rows) e0 = p.csr.ptr[lh * p.csr.ptr_sh + rb], e1 = p.csr.ptr[lh * p.csr.ptr_sh + rb + 1];
+  if (rb < p.csr.num_rows)
+    scalar_load2(p.csr.ptr + lh * p.csr.ptr_sh + rb, p.csr.ptr + lh * p.csr.ptr_sh + rb + 1, e0, e1);
   const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
   const float *kbase = (const float *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh + (int64_t)sq.k_start * p.k.st;
   const float *vbase = (const float *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh + (int64_t)sq.k_start * p.v.st;
+  typename S::Loader kload, vload;
+  kload.init(tid, 2 * p.k.st, 2 * p.D);
+  vload.init(tid, 2 * p.v.st, 2 * p.D);
+  auto issue = [&](int col, int stage) {
+    const int key0 = col * 64, valid = col < 0 ? 0 : sq.k_len - key0;
+    kload.issue(reinterpret_cast<const char *>(kbase + (int64_t)key0 * p.k.st), 0, valid, smem + stage * S::kStage);
+    vload.issue(reinterpret_cast<const char *>(vbase + (int64_t)key0 * p.v.st), 0, valid, smem + stage * S::kStage + S::kTile);
+  };
+  int col_cur = 0, col_pending = 0;  // the block in work and (requested one block early) the one after it
+  if (e0 < e1) {
+    col_cur = scalar_load(cols + e0);
+    issue(col_cur, 0);
+    col_pending = e0 + 1 < e1 ? cols[e0 + 1] : 0;
+  }
+  float qf[S::HD];
+  load_frag<S::HD>((const float *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh + (int64_t)(sq.q_start + qi) * p.q.st, row_ok, g, p.D, qf);
 
-  floatx16 oacc[2];
-#pragma unroll
-  for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.f;
+  floatx16 oacc[S::DT];
+  clear(oacc);
   float m_run = -INFINITY, l_run = 0.f;  // running maximum (log2 domain) and this lane's share of the row sum
   const int lim = p.causal ? min(pos, sq.k_len - 1) : sq.k_len - 1;  // last visible key of this row
 
-  for (int e = e0; e < e1; ++e) {
-    const int col = cols[e];
-    const int key0 = col * 64;
-    if (col < 0 || key0 >= sq.k_len || (p.causal && key0 > rb * 64 + 63)) continue;  // (workgroup-uniform)
-    __syncthreads();  // every wave is done with the tiles of the block before
-    load_tile<128>(kbase + (int64_t)key0 * p.k.st, p.k.st, 0, sq.k_len - key0, p.D, sK, tid);
-    load_tile<128>(vbase + (int64_t)key0 * p.v.st, p.v.st, 0, sq.k_len - key0, p.D, sV, tid);
-    __syncthreads();
-    if (p.causal && key0 > row0 + 31) continue;  // nothing visible for this wave's rows (a barrier pair per block stays)
-    // S^T = K Q^T: lane = q row, registers = keys 32 nt + 8(r/4) + 4g + r%4
-    floatx16 s[2];
+  auto block_step = [&](int e, auto stage_tag) {
+    constexpr int stage = decltype(stage_tag)::value;
+    const int col = col_cur;
+    wait_tile_loads();
+    __syncthreads();  // the block's tiles are visible; every wave is done with the other stage
+    col_cur = __builtin_amdgcn_readfirstlane(col_pending);
+    if (e + 2 < e1) col_pending = cols[e + 2];
+    if (e + 1 < e1) issue(col_cur, stage ^ 1);
+    const int key0 = col * 64 + kh * 32;  // first key of this wave's half
+    if (col < 0 || key0 >= sq.k_len || (p.causal && key0 > row0 + 31)) return;  // nothing visible (wave-uniform)
+    const char *ks = smem + stage * S::kStage, *vs = ks + S::kTile;
+    // S^T = K Q^T: lane = q row, registers = keys 8(r/4) + 4g + r%4 of the half
+    floatx16 s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+    s = dot_dims<KD, PAD>(ks, kh * 32, qf, lane, s);
     float mx = -INFINITY;
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[nt][r] = 0.f;
-      s[nt] = dot_dims(sK, nt * 32, qf, lane, s[nt]);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = key0 + nt * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
-        s[nt][r] = key > lim || !row_ok ? -INFINITY : s[nt][r] * p.scale_log2;
-        mx = fmaxf(mx, s[nt][r]);
-      }
+    for (int r = 0; r < 16; ++r) {
+      const int key = key0 + (r >> 2) * 8 + g * 4 + (r & 3);
+      s[r] = key > lim || !row_ok ? -INFINITY : s[r] * p.scale_log2;
+      mx = fmaxf(mx, s[r]);
     }
-    mx = fmaxf(mx, xor32(mx));
+    mx = max_with_other_half(mx);
     const float m_new = fmaxf(m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = fast_exp2(m_run - m_use);  // exp2(-inf) = 0 before the first visible key
     float psum = 0.f;
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+    for (int r = 0; r < 16; ++r) {
+      s[r] = fast_exp2(s[r] - m_use);
+      psum += s[r];
+    }
+    if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {  // wave-uniform: some row's maximum has moved
+      const float alpha = fast_exp2(m_run - m_use);  // exp2(-inf) = 0 before the first visible key
+      l_run *= alpha;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        s[nt][r] = fast_exp2(s[nt][r] - m_use);
-        psum += s[nt][r];
-      }
-    l_run = l_run * alpha + psum;
-    m_run = m_new;
+      for (int dt = 0; dt < S::DT; ++dt)
 #pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-    // O^T += V^T P^T
-    dot_rows(sV, 0, s[0], lane, oacc);
-    dot_rows(sV, 32, s[1], lane, oacc);
+        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+      m_run = m_new;
+    }
+    l_run += psum;
+    dot_rows<KD, PAD>(vs, kh * 32, s, lane, oacc);  // O^T += V^T P^T
+  };
+  for (int e = e0; e < e1; e += 2) {
+    block_step(e, Stage<0>{});
+    if (e + 1 < e1) block_step(e + 1, Stage<1>{});
   }
   l_run += xor32(l_run);
-  if (!row_ok) return;
-  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  store_frag((float *)p.o.ptr + sq.b * p.o.sb + h * p.o.sh + (int64_t)(sq.q_start + qi) * p.o.st, oacc, inv, g, p.D);
-  if (p.lse.ptr && g == 0)
+
+  // ---- merge of the two key halves of a row: maxima and sums, then the accumulators by halves ----
+  __syncthreads();  // the tiles are free
+  float *ml = reinterpret_cast<float *>(smem + 2 * S::DT * 4096);  // behind the exchange areas of the two pairs
+  float *buf = reinterpret_cast<float *>(smem) + rh * S::DT * 1024;
+  if (g == 0) {
+    ml[(wave * 2) * 32 + m] = m_run;
+    ml[(wave * 2 + 1) * 32 + m] = l_run;
+  }
+  give_half<S::DT>(oacc, kh == 1, buf, lane);
+  __syncthreads();
+  const int mate = wave ^ 2;
+  const float m_o = ml[(mate * 2) * 32 + m], l_o = ml[(mate * 2 + 1) * 32 + m];
+  const float m_all = fmaxf(m_run, m_o), m_ref = m_all == -INFINITY ? 0.f : m_all;
+  const float a_own = fast_exp2(m_run - m_ref), a_other = fast_exp2(m_o - m_ref);
+  const float l_all = l_run * a_own + l_o * a_other;
+  const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
+  float *orow = (float *)p.o.ptr + sq.b * p.o.sb + h * p.o.sh + (int64_t)(sq.q_start + qi) * p.o.st;
+  take_half_and_store<S::DT>(oacc, kh == 1, buf, lane, a_own * inv, a_other * inv, orow, row_ok, p.D);
+  if (row_ok && p.lse.ptr && g == 0 && kh == 0)
     p.lse.ptr[sq.b * p.lse.sb + h * p.lse.sh + (int64_t)(sq.q_start + qi) * p.lse.st] =
-        l_run > 0.f ? (m_run + log2f(l_run)) * kLn2 : -INFINITY;
+        l_all > 0.f ? (m_all + log2f(l_all)) * kLn2 : -INFINITY;
 }
 
 // ---------------------------------------------------------------------------
 // backward
 // ---------------------------------------------------------------------------
-// delta = rowsum(O * dO) - dLSE: one thread per 16-byte piece of a row, 16 pieces per row
+// delta = rowsum(O * dO) - dLSE: one thread per 16-byte piece of a row, PIECES pieces per row
+template <int PIECES>
 __global__ __launch_bounds__(256) void delta_kernel(const BwdParams p) {
-  const int r = threadIdx.x >> 4, ch = threadIdx.x & 15;
-  const int qi = blockIdx.x * 16 + r, h = blockIdx.y, b = blockIdx.z;
+  const int r = threadIdx.x / PIECES, ch = threadIdx.x % PIECES;
+  const int qi = blockIdx.x * (256 / PIECES) + r, h = blockIdx.y, b = blockIdx.z;
   const bool ok = qi < p.seqs.max_q_len;
   float d = 0.f;
   if (ok && ch * 4 < p.D) {
@@ -214,172 +374,284 @@ __global__ __launch_bounds__(256) void delta_kernel(const BwdParams p) {
     d = o.x * g.x + o.y * g.y + o.z * g.z + o.w * g.w;
   }
 #pragma unroll
-  for (int off = 8; off > 0; off >>= 1) d += __shfl_xor(d, off);
+  for (int off = PIECES / 2; off > 0; off >>= 1) d += __shfl_xor(d, off);
   if (ok && ch == 0) {
     if (p.dlse.ptr) d -= p.dlse.ptr[b * p.dlse.sb + h * p.dlse.sh + (int64_t)qi * p.dlse.st];
     p.delta[((int64_t)b * p.Hq + h) * p.seqs.max_q_len + qi] = d;
   }
 }
 
-// dQ: workgroup = 64 q rows of one head, 2 waves of 32 rows; per listed block S^T = K Q^T,
+// dQ: workgroup = 64 q rows of one head; wave = 32 rows x 32 keys of every listed block: S^T = K Q^T,
 // dP^T = V dO^T (lane = q row: lse and delta are per-lane scalars), dS^T = P^T (dP^T - delta),
-// dQ^T += K^T dS^T.
-__global__ __launch_bounds__(128) void dq_kernel(const BwdParams p, int tiles_y) {
-  __shared__ __align__(16) float sK[64 * kLd];
-  __shared__ __align__(16) float sV[64 * kLd];
+// dQ^T += K^T dS^T; the two key halves are added at the end.
+template <int KD, bool PAD>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2 : 1, KD <= 64 ? 2 : 1))) void dq_kernel(
+    const BwdParams p, int tiles_y) {
+  using S = Shape<KD, PAD>;
+  extern __shared__ __align__(16) char smem[];
   const SeqInfo sq = load_seq(p.seqs, blockIdx.z, p.causal);
-  const int h = grid_head(p.csr), kvh = h / (p.Hq / p.Hkv);
+  const int h = grid_head(p.csr), kvh = __builtin_amdgcn_readfirstlane(h / (p.Hq / p.Hkv));
   int tile = tiles_y - 1 - (int)blockIdx.y;
-  if (p.csr.order) tile = p.csr.order[lut_head(p.csr, h, p.Hq, p.Hkv) * p.csr.order_sh + blockIdx.y] - sq.past / 64;
+  if (p.csr.order)
+    tile = scalar_load(p.csr.order + lut_head(p.csr, h, p.Hq, p.Hkv) * p.csr.order_sh + blockIdx.y) - sq.past / 64;
   if (tile < 0 || tile >= seq_row_blocks(sq, 64)) return;
   const int rb = sq.past / 64 + tile;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rh = wave & 1, kh = wave >> 1;
   const int m = lane & 31, g = lane >> 5;
-  const int row0 = rb * 64 + wave * 32;
+  const int row0 = rb * 64 + rh * 32;
   const int pos = row0 + m, qi = pos - sq.past;
   const bool row_ok = qi >= 0 && qi < sq.q_len;
+  if constexpr (PAD) {
+    zero_tiles<NT>(smem, S::kSmem, tid);
+    __syncthreads();
+  }
 
-  float qf[32], dof[32];
-  load_frag((const float *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh + (int64_t)qi * p.q.st, row_ok, g, p.D, qf);
-  load_frag((const float *)p.dout.ptr + sq.b * p.dout.sb + h * p.dout.sh + (int64_t)qi * p.dout.st, row_ok, g, p.D, dof);
+  const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
+  int e0 = 0, e1 = 0;
+  if (rb < p.csr.num_rows)
+    scalar_load2(p.csr.ptr + lh * p.csr.ptr_sh + rb, p.csr.ptr + lh * p.csr.ptr_sh + rb + 1, e0, e1);
+  const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
+  const float *kbase = (const float *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh;
+  const float *vbase = (const float *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh;
+  typename S::Loader kload, vload;
+  kload.init(tid, 2 * p.k.st, 2 * p.D);
+  vload.init(tid, 2 * p.v.st, 2 * p.D);
+  auto issue = [&](int col, int stage) {
+    const int key0 = col * 64, valid = col < 0 ? 0 : sq.k_len - key0;
+    kload.issue(reinterpret_cast<const char *>(kbase + (int64_t)key0 * p.k.st), 0, valid, smem + stage * S::kStage);
+    vload.issue(reinterpret_cast<const char *>(vbase + (int64_t)key0 * p.v.st), 0, valid, smem + stage * S::kStage + S::kTile);
+  };
+  int col_cur = 0, col_pending = 0;
+  if (e0 < e1) {
+    col_cur = scalar_load(cols + e0);
+    issue(col_cur, 0);
+    col_pending = e0 + 1 < e1 ? cols[e0 + 1] : 0;
+  }
+  float qf[S::HD], dof[S::HD];
+  load_frag<S::HD>((const float *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh + (int64_t)qi * p.q.st, row_ok, g, p.D, qf);
+  load_frag<S::HD>((const float *)p.dout.ptr + sq.b * p.dout.sb + h * p.dout.sh + (int64_t)qi * p.dout.st, row_ok, g, p.D, dof);
   float lse2 = INFINITY, delta = 0.f;  // a row outside the sequence: P = exp2(. - inf) = 0
   if (row_ok) {
     const float lse = p.lse.ptr[sq.b * p.lse.sb + h * p.lse.sh + (int64_t)qi * p.lse.st];
     lse2 = lse == -INFINITY ? INFINITY : lse * kLog2e;
     delta = p.delta[((int64_t)sq.b * p.Hq + h) * p.seqs.max_q_len + qi];
   }
-  const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
-  int e0 = 0, e1 = 0;
-  if (rb < p.csr.num_rows) e0 = p.csr.ptr[lh * p.csr.ptr_sh + rb], e1 = p.csr.ptr[lh * p.csr.ptr_sh + rb + 1];
-  const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
-  const float *kbase = (const float *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh;
-  const float *vbase = (const float *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh;
-  floatx16 acc[2];
-#pragma unroll
-  for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
+  floatx16 acc[S::DT];
+  clear(acc);
   const int lim = p.causal ? min(pos, sq.k_len - 1) : sq.k_len - 1;
 
-  for (int e = e0; e < e1; ++e) {
-    const int col = cols[e];
-    const int key0 = col * 64;
-    if (col < 0 || key0 >= sq.k_len || (p.causal && key0 > rb * 64 + 63)) continue;
+  auto block_step = [&](int e, auto stage_tag) {
+    constexpr int stage = decltype(stage_tag)::value;
+    const int col = col_cur;
+    wait_tile_loads();
     __syncthreads();
-    load_tile<128>(kbase + (int64_t)key0 * p.k.st, p.k.st, 0, sq.k_len - key0, p.D, sK, tid);
-    load_tile<128>(vbase + (int64_t)key0 * p.v.st, p.v.st, 0, sq.k_len - key0, p.D, sV, tid);
-    __syncthreads();
-    if (p.causal && key0 > row0 + 31) continue;
+    col_cur = __builtin_amdgcn_readfirstlane(col_pending);
+    if (e + 2 < e1) col_pending = cols[e + 2];
+    if (e + 1 < e1) issue(col_cur, stage ^ 1);
+    const int key0 = col * 64 + kh * 32;
+    if (col < 0 || key0 >= sq.k_len || (p.causal && key0 > row0 + 31)) return;
+    const char *ks = smem + stage * S::kStage, *vs = ks + S::kTile;
+    floatx16 s, dp;
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      floatx16 s, dp;
+    for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+    s = dot_dims<KD, PAD>(ks, kh * 32, qf, lane, s);
+    dp = dot_dims<KD, PAD>(vs, kh * 32, dof, lane, dp);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-      s = dot_dims(sK, nt * 32, qf, lane, s);
-      dp = dot_dims(sV, nt * 32, dof, lane, dp);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = key0 + nt * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
-        const float pr = key > lim ? 0.f : fast_exp2(fmaf(s[r], p.scale_log2, -lse2));
-        s[r] = pr * (dp[r] - delta);  // dS^T without sm_scale (applied once at the end)
-      }
-      dot_rows(sK, nt * 32, s, lane, acc);
+    for (int r = 0; r < 16; ++r) {
+      const int key = key0 + (r >> 2) * 8 + g * 4 + (r & 3);
+      const float pr = key > lim ? 0.f : fast_exp2(fmaf(s[r], p.scale_log2, -lse2));
+      s[r] = pr * (dp[r] - delta);  // dS^T without sm_scale (applied once at the end)
     }
+    dot_rows<KD, PAD>(ks, kh * 32, s, lane, acc);
+  };
+  for (int e = e0; e < e1; e += 2) {
+    block_step(e, Stage<0>{});
+    if (e + 1 < e1) block_step(e + 1, Stage<1>{});
   }
-  if (!row_ok) return;
-  store_frag((float *)p.dq.ptr + sq.b * p.dq.sb + h * p.dq.sh + (int64_t)qi * p.dq.st, acc, p.sm_scale, g, p.D);
+  __syncthreads();
+  float *buf = reinterpret_cast<float *>(smem) + rh * S::DT * 1024;
+  give_half<S::DT>(acc, kh == 1, buf, lane);
+  __syncthreads();
+  float *row = (float *)p.dq.ptr + sq.b * p.dq.sb + h * p.dq.sh + (int64_t)qi * p.dq.st;
+  take_half_and_store<S::DT>(acc, kh == 1, buf, lane, p.sm_scale, p.sm_scale, row, row_ok, p.D);
 }
 
-// dK / dV: workgroup = 64 keys of one kv head (the q heads of its group one after the other), 2
-// waves of 32 keys with their K and V rows in registers; per listed q block (64 rows in two halves)
-// S = Q K^T, dP = dO V^T (lane = key, registers = q rows), P = exp(S - lse), dS = P (dP - delta),
-// dV^T += dO^T P, dK^T += Q^T dS.  Every CSC entry is tested against the sequence length.
-__global__ __launch_bounds__(128) void dkdv_kernel(const BwdParams p) {
-  __shared__ __align__(16) float sQ[64 * kLd];
-  __shared__ __align__(16) float sDo[64 * kLd];
-  __shared__ float sLse[64], sDelta[64];
+// dK / dV: workgroup = 64 keys of one kv head (the q heads of its group one after the other) or of
+// one q head (head_split: p.dk / p.dv then describe per-q-head partial buffers); wave = 32 keys, with
+// their K and V rows in registers, x 32 q rows of every listed block: S = Q K^T, dP = dO V^T (lane =
+// key, registers = q rows), P = exp(S - lse), dS = P (dP - delta), dV^T += dO^T P, dK^T += Q^T dS; the
+// two q-row halves are added at the end.  Every CSC entry is tested against the sequence length.
+template <int KD, bool PAD>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2 : 1, KD <= 64 ? 2 : 1))) void dkdv_kernel(
+    const BwdParams p, int head_split) {
+  using S = Shape<KD, PAD>;
+  extern __shared__ __align__(16) char smem[];
+  float *const vecs = reinterpret_cast<float *>(smem + S::kSmem);  // per stage: lse[64] (log2 domain), delta[64]
   const SeqInfo sq = load_seq(p.seqs, blockIdx.z, p.causal);
-  const int kvh = grid_head(p.csc), ratio = p.Hq / p.Hkv;
+  const int ratio = __builtin_amdgcn_readfirstlane(p.Hq / p.Hkv);
+  const int out_head = grid_head(p.csc);
+  const int kvh = head_split ? __builtin_amdgcn_readfirstlane(out_head / ratio) : out_head;
+  const int gq_first = head_split ? out_head - kvh * ratio : 0, gq_end = head_split ? gq_first + 1 : ratio;
   int cb = blockIdx.y;  // longest columns first when the table gives the order (as in the 16-bit pass)
-  if (p.csc.order) cb = p.csc.order[lut_head(p.csc, kvh * ratio, p.Hq, p.Hkv) * p.csc.order_sh + blockIdx.y];
+  if (p.csc.order)
+    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv) * p.csc.order_sh + blockIdx.y);
   if (cb * 64 >= sq.k_len) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nh = wave & 1, qh = wave >> 1;  // key half, q-row half
   const int n = lane & 31, g = lane >> 5;
-  const int key = cb * 64 + wave * 32 + n;
+  const int key0 = cb * 64 + nh * 32, key = key0 + n;
   const bool key_ok = key < sq.k_len;
-  float kf[32], vf[32];
-  load_frag((const float *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh + (int64_t)key * p.k.st, key_ok, g, p.D, kf);
-  load_frag((const float *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh + (int64_t)key * p.v.st, key_ok, g, p.D, vf);
-  floatx16 dk[2], dv[2];
-#pragma unroll
-  for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) dk[dt][r] = dv[dt][r] = 0.f;
+  if constexpr (PAD) {
+    zero_tiles<NT>(smem, S::kSmem, tid);
+    __syncthreads();
+  }
+  float kf[S::HD], vf[S::HD];
+  load_frag<S::HD>((const float *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh + (int64_t)key * p.k.st, key_ok, g, p.D, kf);
+  load_frag<S::HD>((const float *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh + (int64_t)key * p.v.st, key_ok, g, p.D, vf);
+  floatx16 dk[S::DT], dv[S::DT];
+  clear(dk);
+  clear(dv);
+  typename S::Loader qload, doload;
+  qload.init(tid, 2 * p.q.st, 2 * p.D);
+  doload.init(tid, 2 * p.dout.st, 2 * p.D);
 
-  for (int gq = 0; gq < ratio; ++gq) {
+  for (int gq = gq_first; gq < gq_end; ++gq) {
     const int h = kvh * ratio + gq;
     const int lh = lut_head(p.csc, h, p.Hq, p.Hkv);
     int e0 = 0, e1 = 0;
-    if (cb < p.csc.num_rows) e0 = p.csc.ptr[lh * p.csc.ptr_sh + cb], e1 = p.csc.ptr[lh * p.csc.ptr_sh + cb + 1];
+    if (cb < p.csc.num_rows)
+      scalar_load2(p.csc.ptr + lh * p.csc.ptr_sh + cb, p.csc.ptr + lh * p.csc.ptr_sh + cb + 1, e0, e1);
     const int32_t *rows = p.csc.idx + lh * p.csc.idx_sh;
     const float *qbase = (const float *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh;
     const float *dobase = (const float *)p.dout.ptr + sq.b * p.dout.sb + h * p.dout.sh;
-    for (int e = e0; e < e1; ++e) {
-      const int rbq = rows[e];
+    const float *lsebase = p.lse.ptr + sq.b * p.lse.sb + h * p.lse.sh;
+    const float *deltabase = p.delta + ((int64_t)sq.b * p.Hq + h) * p.seqs.max_q_len;
+    float vec = 0.f;  // this thread's lse (threads 0..63) or delta (64..127) of the block that was requested last
+    auto issue = [&](int rbq, int stage) {
       const int qi0 = rbq * 64 - sq.past;  // query index of the block's first row
-      if (rbq < 0 || qi0 >= sq.q_len || qi0 + 64 <= 0) continue;
-      if (p.causal && cb * 64 > rbq * 64 + 63) continue;
-      __syncthreads();
-      load_tile<128>(qbase + (int64_t)qi0 * p.q.st, p.q.st, -qi0, sq.q_len - qi0, p.D, sQ, tid);
-      load_tile<128>(dobase + (int64_t)qi0 * p.dout.st, p.dout.st, -qi0, sq.q_len - qi0, p.D, sDo, tid);
-      if (tid < 64) {
-        const int qi = qi0 + tid;
-        const bool ok = qi >= 0 && qi < sq.q_len;
-        const float lse = ok ? p.lse.ptr[sq.b * p.lse.sb + h * p.lse.sh + (int64_t)qi * p.lse.st] : 0.f;
-        sLse[tid] = !ok || lse == -INFINITY ? INFINITY : lse * kLog2e;  // +inf: P = 0 for rows outside the sequence
-        sDelta[tid] = ok ? p.delta[((int64_t)sq.b * p.Hq + h) * p.seqs.max_q_len + qi] : 0.f;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {  // 32 q rows at a time
-        const int pos0 = rbq * 64 + qt * 32;
-        if (p.causal && cb * 64 + wave * 32 > pos0 + 31) continue;  // every key of this wave lies beyond these rows
-        floatx16 s, dp;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-        s = dot_dims(sQ, qt * 32, kf, lane, s);     // rows = q (tile), columns = keys (registers)
-        dp = dot_dims(sDo, qt * 32, vf, lane, dp);
-        floatx16 ds;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int ql = qt * 32 + (r >> 2) * 8 + g * 4 + (r & 3);  // row of the block
-          const bool vis = key_ok && (!p.causal || key <= rbq * 64 + ql);
-          const float pr = vis ? fast_exp2(fmaf(s[r], p.scale_log2, -sLse[ql])) : 0.f;
-          s[r] = pr;
-          ds[r] = pr * (dp[r] - sDelta[ql]);
-        }
-        dot_rows(sDo, qt * 32, s, lane, dv);
-        dot_rows(sQ, qt * 32, ds, lane, dk);
-      }
+      const int lo = rbq < 0 ? 64 : -qi0, hi = sq.q_len - qi0;
+      qload.issue(reinterpret_cast<const char *>(qbase + (int64_t)qi0 * p.q.st), lo, hi, smem + stage * S::kStage);
+      doload.issue(reinterpret_cast<const char *>(dobase + (int64_t)qi0 * p.dout.st), lo, hi, smem + stage * S::kStage + S::kTile);
+      const int r = tid & 63;
+      const bool ok = r >= lo && r < hi;
+      if (tid < 64)
+        vec = ok ? lsebase[(int64_t)(qi0 + r) * p.lse.st] : -INFINITY;
+      else if (tid < 128)
+        vec = ok ? deltabase[qi0 + r] : 0.f;
+    };
+    int rb_cur = 0, rb_pending = 0;
+    if (e0 < e1) {
+      rb_cur = scalar_load(rows + e0);
+      issue(rb_cur, 0);
+      rb_pending = e0 + 1 < e1 ? rows[e0 + 1] : 0;
     }
+    auto block_step = [&](int e, auto stage_tag) {
+      constexpr int stage = decltype(stage_tag)::value;
+      const int rbq = rb_cur;
+      wait_tile_loads();
+      // (+inf where there is no row or the row saw no key: P = 0)
+      if (tid < 64)
+        vecs[stage * 128 + tid] = vec == -INFINITY ? INFINITY : vec * kLog2e;
+      else if (tid < 128)
+        vecs[stage * 128 + tid] = vec;
+      __syncthreads();
+      rb_cur = __builtin_amdgcn_readfirstlane(rb_pending);
+      if (e + 2 < e1) rb_pending = rows[e + 2];
+      if (e + 1 < e1) issue(rb_cur, stage ^ 1);
+      const int pos0 = rbq * 64 + qh * 32;  // first q position of this wave's half
+      if (rbq < 0 || (p.causal && key0 > pos0 + 31)) return;  // nothing visible (wave-uniform)
+      const char *qs = smem + stage * S::kStage, *dos = qs + S::kTile;
+      const float *lse_s = vecs + stage * 128 + qh * 32, *delta_s = lse_s + 64;
+      floatx16 s, dp;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+      s = dot_dims<KD, PAD>(qs, qh * 32, kf, lane, s);  // rows = q (tile), columns = keys (registers)
+      dp = dot_dims<KD, PAD>(dos, qh * 32, vf, lane, dp);
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + r4 * 8 + g * 4);
+        const float4 d4 = *reinterpret_cast<const float4 *>(delta_s + r4 * 8 + g * 4);
+        const float lr[4] = {l4.x, l4.y, l4.z, l4.w}, dr[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = r4 * 4 + i;
+          const bool vis = key_ok && (!p.causal || key <= pos0 + r4 * 8 + g * 4 + i);
+          s[r] = vis ? fast_exp2(fmaf(s[r], p.scale_log2, -lr[i])) : 0.f;
+          dp[r] = s[r] * (dp[r] - dr[i]);  // dS without sm_scale (applied once at the end)
+        }
+      }
+      dot_rows<KD, PAD>(dos, qh * 32, s, lane, dv);
+      dot_rows<KD, PAD>(qs, qh * 32, dp, lane, dk);
+    };
+    for (int e = e0; e < e1; e += 2) {
+      block_step(e, Stage<0>{});
+      if (e + 1 < e1) block_step(e + 1, Stage<1>{});
+    }
+    __syncthreads();  // every wave is done with the tiles before the next head (or the sums below) reuses them
   }
-  if (!key_ok) return;
-  store_frag((float *)p.dk.ptr + sq.b * p.dk.sb + kvh * p.dk.sh + (int64_t)key * p.dk.st, dk, p.sm_scale, g, p.D);
-  store_frag((float *)p.dv.ptr + sq.b * p.dv.sb + kvh * p.dv.sh + (int64_t)key * p.dv.st, dv, 1.f, g, p.D);
+  // dK and dV one after the other through the same exchange areas
+  float *buf = reinterpret_cast<float *>(smem) + nh * S::DT * 1024;
+  float *buf2 = buf + 2 * S::DT * 1024;
+  give_half<S::DT>(dk, qh == 1, buf, lane);
+  give_half<S::DT>(dv, qh == 1, buf2, lane);
+  __syncthreads();
+  float *dkp = (float *)p.dk.ptr + sq.b * p.dk.sb + out_head * p.dk.sh + (int64_t)key * p.dk.st;
+  float *dvp = (float *)p.dv.ptr + sq.b * p.dv.sb + out_head * p.dv.sh + (int64_t)key * p.dv.st;
+  take_half_and_store<S::DT>(dk, qh == 1, buf, lane, p.sm_scale, p.sm_scale, dkp, key_ok, p.D);
+  take_half_and_store<S::DT>(dv, qh == 1, buf2, lane, 1.f, 1.f, dvp, key_ok, p.D);
 }
 
 static bool lut_ok(const LutView &l) {
   return l.block_rows == 64 && l.block_cols == 64 && l.entry_width == 1 && l.sub_block == 0;
 }
+static bool dims_ok(int d, bool wide) { return d % 4 == 0 && (wide ? d > 64 && d <= 128 : d >= 4 && d <= 64); }
+// the tile copies keep a tile's byte offsets in 32 bits
+static bool rows_ok(const TensorView &t) { return t.st >= 0 && t.st < (int64_t(1) << 23); }
+
+template <int KD, bool PAD>
+static int launch_fwd(const FwdParams &p, int tiles, hipStream_t stream) {
+  constexpr int smem = Shape<KD, PAD>::kSmem;
+  DK_ALLOW_DYNAMIC_LDS((fwd_kernel<KD, PAD>), smem);
+  hipLaunchKernelGGL((fwd_kernel<KD, PAD>), dim3(p.Hq, tiles, p.seqs.packed ? 1 : p.seqs.batch), dim3(NT), smem, stream, p, tiles);
+  DK_HIP_CHECK(hipGetLastError());
+  return DK_OK;
+}
+
+template <int KD, bool PAD>
+static int launch_dq(const BwdParams &p, int rows, hipStream_t stream) {
+  constexpr int smem = Shape<KD, PAD>::kSmem;
+  DK_ALLOW_DYNAMIC_LDS((dq_kernel<KD, PAD>), smem);
+  hipLaunchKernelGGL((dq_kernel<KD, PAD>), dim3(p.Hq, rows, p.seqs.batch), dim3(NT), smem, stream, p, rows);
+  DK_HIP_CHECK(hipGetLastError());
+  return DK_OK;
+}
+
+template <int KD, bool PAD>
+static int launch_dkdv(const BwdParams &p, int columns, int heads, hipStream_t stream) {
+  constexpr int smem = Shape<KD, PAD>::kSmem + 2 * 128 * (int)sizeof(float);
+  DK_ALLOW_DYNAMIC_LDS((dkdv_kernel<KD, PAD>), smem);
+  hipLaunchKernelGGL((dkdv_kernel<KD, PAD>), dim3(heads, columns, p.seqs.batch), dim3(NT), smem, stream, p, heads != p.Hkv);
+  DK_HIP_CHECK(hipGetLastError());
+  return DK_OK;
+}
+
+// head dims multiplied: the multiple of 32 from 64 on that holds the tensors' own
+#define DK_BY_HEAD_DIM(launch, D, ...)                                                                  \
+  ((D) == 64 ? launch<64, false>(__VA_ARGS__) : (D) < 64 ? launch<64, true>(__VA_ARGS__)                \
+   : (D) <= 96 ? launch<96, true>(__VA_ARGS__) : (D) < 128 ? launch<128, true>(__VA_ARGS__) : launch<128, false>(__VA_ARGS__))
 
 }  // namespace f32
 
-bool mfma_f32_fwd_supported(const FwdParams &p, int dtype) {
-  return dtype == DK_F32 && p.D >= 4 && p.D <= f32::kD && p.D % 4 == 0 && p.vec_ok && f32::lut_ok(p.csr);
+bool mfma_f32_fwd_supported(const FwdParams &p, int dtype, bool wide) {
+  return dtype == DK_F32 && f32::dims_ok(p.D, wide) && p.vec_ok && f32::lut_ok(p.csr) && f32::rows_ok(p.k) && f32::rows_ok(p.v);
 }
 
-bool mfma_f32_bwd_supported(const BwdParams &p, int dtype) {
-  return dtype == DK_F32 && p.D >= 4 && p.D <= f32::kD && p.D % 4 == 0 && p.vec_ok && f32::lut_ok(p.csr) && f32::lut_ok(p.csc);
+bool mfma_f32_bwd_supported(const BwdParams &p, int dtype, bool wide) {
+  return dtype == DK_F32 && f32::dims_ok(p.D, wide) && p.vec_ok && f32::lut_ok(p.csr) && f32::lut_ok(p.csc) &&
+         f32::rows_ok(p.q) && f32::rows_ok(p.k) && f32::rows_ok(p.v) && f32::rows_ok(p.dout);
 }
 
 int launch_mfma_f32_fwd(const FwdParams &p, hipStream_t stream) {
@@ -398,36 +670,52 @@ int launch_mfma_f32_fwd(const FwdParams &p, hipStream_t stream) {
   FwdParams pr = p;
   pr.csr.rot = head_rotation(p.csr, p.Hq, tiles);  // (uneven heads: dealt to the queues in rotation)
   DK_NOTE_KERNEL(pr.csr.rot ? "f32::fwd_kernel, heads in rotation" : "f32::fwd_kernel");
-  hipLaunchKernelGGL(f32::fwd_kernel, dim3(p.Hq, tiles, s.packed ? 1 : s.batch), dim3(128), 0, stream, pr, tiles);
-  DK_HIP_CHECK(hipGetLastError());
-  return DK_OK;
+  using namespace f32;
+  return DK_BY_HEAD_DIM(launch_fwd, p.D, pr, tiles, stream);
 }
 
-int launch_mfma_f32_bwd(const BwdParams &p, hipStream_t stream) {
+// Scratch of the dK/dV pass by q heads (wide head dims only: up to 64 the pass of a whole group is
+// short enough that the sum would cost what the balance gains)
+size_t mfma_f32_bwd_workspace_bytes(const BwdParams &p) { return p.D > 64 && p.D % 8 == 0 ? mfma_bwd_workspace_bytes(p) : 0; }
+
+int launch_mfma_f32_bwd(const BwdParams &p, void *workspace, size_t workspace_bytes, hipStream_t stream) {
   const SeqView &s = p.seqs;
   const int past = p.causal ? s.max_k_len - s.max_q_len : 0;
   const int tiles = (past + s.max_q_len - 1) / 64 - past / 64 + 1;
   const int cblocks = cdiv(s.max_k_len, 64);
   DK_REQUIRE(tiles <= 65535 && cblocks <= 65535, "sequence too long for one launch");
   DK_NOTE_KERNEL("f32::delta_kernel");
-  hipLaunchKernelGGL(f32::delta_kernel, dim3(cdiv(s.max_q_len, 16), p.Hq, s.batch), dim3(256), 0, stream, p);
+  if (p.D <= 64)
+    hipLaunchKernelGGL(f32::delta_kernel<16>, dim3(cdiv(s.max_q_len, 16), p.Hq, s.batch), dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL(f32::delta_kernel<32>, dim3(cdiv(s.max_q_len, 8), p.Hq, s.batch), dim3(256), 0, stream, p);
   DK_HIP_CHECK(hipGetLastError());
   DK_REQUIRE(!p.csr.order || p.csr.num_rows <= 65535, "sequence too long for one launch");
   const int rows = p.csr.order ? p.csr.num_rows : tiles;  // handed out in the table's order: all of them
   BwdParams pq = p;
   pq.csr.rot = head_rotation(p.csr, p.Hq, rows);
   DK_NOTE_KERNEL(pq.csr.rot ? "f32::dq_kernel, heads in rotation" : "f32::dq_kernel");
-  hipLaunchKernelGGL(f32::dq_kernel, dim3(p.Hq, rows, s.batch), dim3(128), 0, stream, pq, rows);
-  DK_HIP_CHECK(hipGetLastError());
+  using namespace f32;
+  if (int rc = DK_BY_HEAD_DIM(launch_dq, p.D, pq, rows, stream)) return rc;
+  // Several q heads per kv head: one workgroup per q head into fp32 partials of its own and a sum over
+  // each group, as in the 16-bit pass (one workgroup walking the whole group makes the longest column
+  // outlast the rest of the launch).
+  const bool per_q_head = workspace && mfma_f32_bwd_workspace_bytes(p) && workspace_bytes >= mfma_f32_bwd_workspace_bytes(p) &&
+                          ((uintptr_t)workspace % 16) == 0;
+  const int heads = per_q_head ? p.Hq : p.Hkv;
   BwdParams po = p;  // the order only where heads do not line up with the hardware's 32 workgroup queues
-  if (p.Hkv % 32 == 0) po.csc.order = nullptr;
+  if (heads % 32 == 0) po.csc.order = nullptr;
   DK_REQUIRE(p.csc.num_rows <= 65535, "sequence too long for one launch");
   const int columns = po.csc.order ? p.csc.num_rows : cblocks;
-  po.csc.rot = head_rotation(p.csc, p.Hkv, columns);
+  po.csc.rot = head_rotation(p.csc, heads, columns);
+  float *part_k = (float *)workspace, *part_v = part_k + (int64_t)s.batch * p.Hq * s.max_k_len * p.D;
+  if (per_q_head) {
+    po.dk = TensorView{part_k, (int64_t)p.Hq * s.max_k_len * p.D, (int64_t)s.max_k_len * p.D, p.D};
+    po.dv = TensorView{part_v, (int64_t)p.Hq * s.max_k_len * p.D, (int64_t)s.max_k_len * p.D, p.D};
+  }
   DK_NOTE_KERNEL(po.csc.rot ? "f32::dkdv_kernel, heads in rotation" : "f32::dkdv_kernel");
-  hipLaunchKernelGGL(f32::dkdv_kernel, dim3(p.Hkv, columns, s.batch), dim3(128), 0, stream, po);
-  DK_HIP_CHECK(hipGetLastError());
-  return DK_OK;
+  if (int rc = DK_BY_HEAD_DIM(launch_dkdv, p.D, po, columns, heads, stream)) return rc;
+  return per_q_head ? launch_dkdv_group_sum(p, DK_F32, part_k, part_v, stream) : DK_OK;
 }
 
 }  // namespace dk

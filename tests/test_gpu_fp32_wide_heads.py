@@ -1,0 +1,71 @@
+"""fp32 head dims above 64 on the matrix cores (multiplied as 96 or 128 dims): forward and backward
+against the fp32 oracle within 2e-4 (LSE 1e-4, the fp32 bar of the other fp32 tests), at the edges of
+the dims (68, 96, 100, 128), one block, ragged lengths, grouped heads with and without the scratch of
+the per-q-head dK/dV pass, more keys than queries, left padding."""
+import math
+
+import pytest
+import torch
+
+from dkernel_amd import LocalStrideSparseAttention, _lib, ops
+from helpers import F32_TOL, assert_close, expand_heads, make_qkv, oracle_fwd
+from oracle import attention as OA
+from oracle import layout as OL
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+New = LocalStrideSparseAttention.__wrapped__
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lk,D,causal,scratch", [
+    (1, 4, 4, 1000, 1000, 128, True, True),
+    (2, 8, 2, 500, 500, 128, True, True),    # grouped heads: per-q-head partials and their sum
+    (2, 8, 2, 500, 500, 128, True, False),   # ... and one workgroup per group
+    (1, 2, 2, 64, 64, 96, True, True),       # exactly one block
+    (2, 3, 3, 333, 333, 96, True, True),
+    (1, 2, 1, 200, 200, 68, True, True),
+    (1, 6, 2, 130, 430, 100, True, True),    # the queries are the last positions; 100: no partials
+    (1, 2, 2, 1, 1, 128, True, True),
+    (1, 2, 2, 384, 384, 104, False, True),
+])
+def test_forward_backward(monkeypatch, B, Hq, Hkv, Lq, Lk, D, causal, scratch):
+    print(f"case B={B} Hq={Hq} Hkv={Hkv} Lq={Lq} Lk={Lk} D={D} causal={causal} scratch={scratch}", flush=True)
+    monkeypatch.setattr(ops, "_bwd_workspace", scratch)
+    sm = 1 / math.sqrt(D)
+    q, k, v, do = make_qkv(B, Lq, Lk, Hq, Hkv, D, torch.float32, with_do=True)
+    Lr = (Lk + 63) // 64 * 64
+    bm = expand_heads(OL.block_mask(Hq, Lr, 64, 2, 3, num_kv_heads=Hkv, causal=causal), Hq)
+    dlse = torch.randn(B, Hq, Lq, generator=torch.Generator().manual_seed(3))
+    qo, ko, vo = (x.clone().requires_grad_() for x in (q, k, v))
+    ro, rl = oracle_fwd(qo, ko, vo, bm, 64, sm, causal=causal)
+    ((ro * do).sum() + (rl * dlse).sum()).backward()
+    mod = New(Hq, Lr, 64, 2, 3, num_kv_heads=Hkv, causal=causal).to(DEV)
+    qd, kd, vd = (x.to(DEV).requires_grad_() for x in (q, k, v))
+    out, lse = mod(qd, kd, vd, sm, return_lse=True)
+    assert _lib.lib().dk_last_kernels().startswith(b"f32::fwd_kernel")
+    ((out * do.to(DEV)).sum() + (lse * dlse.to(DEV)).sum()).backward()
+    summed = scratch and Hq > Hkv and D % 8 == 0
+    assert b"f32::dkdv_kernel" in ops.last_bwd_kernels and (b"group_sum" in ops.last_bwd_kernels) == summed
+    assert_close("O", out, ro, **F32_TOL)
+    assert_close("LSE", lse, rl, atol=1e-4, rtol=0)
+    assert_close("dQ", qd.grad, qo.grad, **F32_TOL)
+    assert_close("dK", kd.grad, ko.grad, **F32_TOL)
+    assert_close("dV", vd.grad, vo.grad, **F32_TOL)
+
+
+@pytest.mark.parametrize("D", [96, 128])
+def test_left_padded_prompts(D):
+    Hq, Hkv, Lmax, lens = 4, 2, 512, [512, 1, 130, 333]
+    print(f"case D={D}", flush=True)
+    sm = 1 / math.sqrt(D)
+    q, k, v = make_qkv(len(lens), Lmax, Lmax, Hq, Hkv, D, torch.float32)
+    bm = OL.block_mask(Hq, Lmax, 64, 2, 3, num_kv_heads=Hkv)
+    mod = New(Hq, Lmax, 64, 2, 3, num_kv_heads=Hkv).to(DEV)
+    left = torch.tensor([Lmax - x for x in lens])
+    out = mod(q.to(DEV), k.to(DEV), v.to(DEV), sm, left_paddings=left)
+    assert _lib.lib().dk_last_kernels().startswith(b"f32::fwd_kernel")
+    for i, n in enumerate(lens):
+        mask = OA.sequence_token_mask(bm, 64, n, n)
+        ro, _ = OA.dense_attention(*(x[i:i + 1, Lmax - n:] for x in (q, k, v)), torch.from_numpy(mask), sm)
+        assert_close(f"O[{i}]", out[i, Lmax - n:], ro[0], **F32_TOL)
+        assert (out[i, :Lmax - n] == 0).all()
