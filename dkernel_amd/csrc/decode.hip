@@ -6,28 +6,30 @@
 // exactly once, for all q heads of the group together), so the design goal is
 // bytes in flight, not FLOPs:
 //
-//   work unit = one wave = consecutive entries of the row of (sequence, kv
-//               head); the number of units of a row and the even split of its
-//               entries follow from its length on the device, so waves stream
+//   work unit = one wave = consecutive half blocks (32 keys) of the row of (sequence, kv
+//               head); the number of units of a row and the even split of its half
+//               blocks follow from its length on the device, so waves stream
 //               similar amounts of K/V whatever the sequence lengths are;
 //   workgroup = kDecodeWaves consecutive units of one row (workgroups beyond a
 //               row's unit count exit at once; a row that needs several
 //               workgroups is cut into a whole number of them, so that none
 //               holds LDS and wave slots for idle waves);
-//   wave      = per block: computes S^T = K Q^T (the q heads of the group are the MFMA
+//   wave      = per half block: computes S^T = K Q^T (the q heads of the group are the MFMA
 //               columns), softmax, O^T += V^T P^T with LDS transpose reads,
 //               keeping a running (max, sum, O) in registers;
-//   epilogue  = a row whose units all sit in one workgroup is merged there
-//               through LDS and written as O / LSE; otherwise one fp32
-//               partial (O unnormalised, max, sum) per (sequence, q head,
-//               unit) goes to the caller's workspace and decode_combine_kernel
-//               merges those rows.
+//   epilogue  = the waves of a workgroup merge their results through LDS.  A row
+//               whose units all sit in one workgroup is written as O / LSE;
+//               otherwise the workgroup leaves one fp32 partial (O unnormalised,
+//               max, sum) per q head in the caller's workspace, and the workgroup
+//               that arrives last merges the row's partials (arrive_last).
 // A wave works on half blocks (32 keys): 2 x 8.5 KB of private LDS tiles and
 // the next half block prefetched into registers, so 8 waves are resident per
 // CU (2 per SIMD, <= 256 VGPRs each): one wave's loads overlap the other's
 // multiplies on the same SIMD.  (Head dims above 128: 256-wide tiles, 2 x 33 KB per wave, one
 // workgroup of four waves per CU and one wave per SIMD.)
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <type_traits>
 
 #include "common.h"
@@ -44,27 +46,51 @@ static int decode_max_row_entries(const FwdParams &p) {
   return p.csr.max_row_entries > 0 ? p.csr.max_row_entries : p.csr.num_rows;
 }
 
-// Table entries per work unit (one wave).  With enough rows (sequences x kv heads) to fill the
+// Half blocks (32 keys) per work unit (one wave).  With enough rows (sequences x kv heads) to fill the
 // machine, a row is cut into as many units as a workgroup has waves, so that it is finished
-// inside one workgroup and the merge kernel is not launched at all; with few rows, into more
-// units (about 1024 waves in total).  At most 16 (the paged path keeps a unit's page numbers in
-// the lanes of one register).
-static int decode_unit_blocks(const FwdParams &p) {
+// inside one workgroup; with few rows, into more units (about 1024 waves in total, down to a half block
+// each: the reads of a wave then leave in one round).  At most 16 blocks (the paged path keeps a
+// unit's page numbers in the lanes of one register).  Measured: 1 sequence of 1000 keys (8 kv heads of
+// 16 blocks), 64 workgroups of half blocks, 8 us from the first workgroup's start to the last one's
+// end (4.3 us to the last key, 1 us merge inside the workgroups, 0.8 us to publish and count, 1.5 us last
+// merge), against 12 us + 4 us for units of two blocks and a merge kernel; 32 sequences (256 rows):
+// 1024 waves 38.6 us, 1536 42.1, 2048 41.2, 3072 45.5.
+static int decode_unit_halves(const FwdParams &p) {
   const int rows = p.seqs.batch * p.Hkv;
   const int units_per_row = std::max(kDecodeWaves, cdiv(1024, rows > 0 ? rows : 1));
-  return std::min(16, std::max(2, cdiv(decode_max_row_entries(p), units_per_row)));
+  return std::min(32, std::max(1, cdiv(2 * decode_max_row_entries(p), units_per_row)));
 }
 
-// Units a row of n table entries is cut into: as many as the unit size asks for, and at least
-// the waves of one workgroup (one entry each at worst), so that every wave of the workgroup that
+// Units a row of n half blocks is cut into: as many as the unit size asks for, and at least
+// the waves of one workgroup (one half block each at worst), so that every wave of the workgroup that
 // finishes a row streams a share of it.  A row that needs more than one workgroup gets a whole
 // number of them: a workgroup with a single busy wave would hold the LDS and the wave slots of
-// four.  Used by both kernels.
-__host__ __device__ inline int decode_row_units(int n, int unit_blocks, int waves) {
-  const int by_size = (n + unit_blocks - 1) / unit_blocks;
+// four.
+__host__ __device__ inline int decode_row_units(int n, int unit_halves, int waves) {
+  const int by_size = (n + unit_halves - 1) / unit_halves;
   const int by_waves = n < waves ? n : waves;
   const int units = by_size > by_waves ? by_size : by_waves;
   return units > waves ? (units + waves - 1) / waves * waves : units;
+}
+
+// Which workgroup of a row arrives last is counted in a slot of the caller's workspace that nobody has
+// cleared.  A slot in use holds (launch number, arrivals); every workgroup first makes sure of that
+// (open_slot: it replaces whatever else it read there, and if that fails another workgroup has done
+// so), long before it arrives.  Launch numbers are 56 bits from a random start, so what the memory
+// happens to hold is not taken for one; the workgroup that arrives last clears the slot, so that a
+// captured launch, whose number is the same on every replay, starts afresh each time.  Arriving is
+// then one atomic addition (as a compare-and-swap loop, eight workgroups took 3 - 6 us), and nobody
+// ever waits for another workgroup.
+using slot_t = unsigned long long;
+__device__ __forceinline__ void open_slot(slot_t *slot, slot_t seen, slot_t launch) {
+  if ((seen >> 8) != launch)
+    __hip_atomic_compare_exchange_strong(slot, &seen, launch << 8, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool arrive_last(slot_t *slot, int n) {
+  const slot_t before = __hip_atomic_fetch_add(slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((int)(before & 255) + 1 != n) return false;
+  __hip_atomic_store(slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
 }
 
 template <int D>
@@ -75,7 +101,8 @@ struct DecSmem {  // per wave: one 32-key half block of K and of V, plus q of th
   static int wave_bytes(int ratio) { return 2 * kHalf + ratio * D * 2; }
 };
 
-// workspace layout: [batch][Hq][max_units][D + 2] floats (O[D] unnormalised, max, sum)
+// workspace layout: [batch][Hq][max_groups + 1][D + 2] floats: a partial (O[D] unnormalised, max, sum)
+// per workgroup of the row; the last place of a kv group's first head holds the row's arrival slot
 // Eight OCP e4m3 bytes -> eight elements of T.  Exact (e4m3 has 3 mantissa bits), so bf16 is
 // the upper half of the fp32 value and fp16 needs no rounding mode: one convert and one pack per
 // two elements.
@@ -99,12 +126,10 @@ __device__ __forceinline__ uint4 fp8x8_to(uint2 w) {
 }
 
 // KV8 (with PAGED): the K/V pools hold fp8 bytes, converted to T on the way into LDS.
-// W waves per workgroup = W consecutive units of one row.  A row whose units all sit in one
-// workgroup is finished here (the waves exchange their partials through LDS and write O / LSE);
-// longer rows leave their partials in the workspace for decode_combine_kernel.
+// W waves per workgroup = W consecutive units of one row.
 template <typename T, int D, bool PAD, bool SUB, bool PAGED, bool KV8, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, D == 256 ? 1 : 2))) void decode_partial_kernel(
-    const FwdParams p, float *ws, int unit_blocks, int max_units) {
+    const FwdParams p, float *ws, int unit_halves, int max_groups, slot_t launch) {
   using M = Mma<T>;
   using vec8 = typename M::vec8;
   using S = DecSmem<D>;
@@ -129,19 +154,18 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
   int row0 = 0, row1 = 0;
   if (sq.k_len > 0 && rb < p.csr.num_rows)
     scalar_load2(p.csr.ptr + lh * p.csr.ptr_sh + rb, p.csr.ptr + lh * p.csr.ptr_sh + rb + 1, row0, row1);
-  // the row's entries are split evenly over as many units as the unit size asks for
-  const int n_ent = row1 - row0;
+  // the row's half blocks are split evenly over as many units as the unit size asks for
+  const int n_half = 2 * (row1 - row0);
   // never more than the host sized the grid and the workspace for: a row longer than the caller's
-  // max_row_entries hint said is still cut into max_units units, each with a larger share
-  const int u_cnt = min(decode_row_units(n_ent, unit_blocks, W), max_units);
+  // max_row_entries hint said is still cut into max_groups * W units, each with a larger share
+  const int u_cnt = min(decode_row_units(n_half, unit_halves, W), max_groups * W);
   if ((int)blockIdx.x * W >= u_cnt && blockIdx.x > 0) return;  // nothing for this workgroup
-  const bool merge_here = u_cnt <= W;  // (a row without entries is written here too: O = 0, LSE = -inf)
-  const int per = u_cnt > 0 ? (n_ent + u_cnt - 1) / u_cnt : 0;
+  const int groups = (u_cnt + W - 1) / W;  // workgroups of this row (a row without entries is written too: O = 0, LSE = -inf)
+  const int per = u_cnt > 0 ? (n_half + u_cnt - 1) / u_cnt : 0;
   const int unit = blockIdx.x * W + wave;
-  const bool active = unit < u_cnt;
-  if (!active && !merge_here) return;
-  const int e0 = row0 + unit * per;
-  const int e1 = active ? min(e0 + per, row1) : e0;
+  const int hb0 = min(unit * per, n_half), hb1 = min(hb0 + per, n_half);  // (units beyond u_cnt: empty)
+  const int e0 = row0 + (hb0 >> 1);  // table entry of the first half block
+  const int e1 = row0 + ((hb1 + 1) >> 1);
   const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
   // SUB: the query's row of pattern blocks inside its tile selects f of the entry's f x f mask
   // bits; half block hb & 1 holds key parts [hb & 1, hb & 1 + 1) * f / 2 of them
@@ -190,7 +214,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
   };
   if constexpr (PAGED) my_page = load_pages(0);
 
-  // half block hb of this unit = keys cols[e0 + hb/2] * 64 + 32 * (hb & 1) + [0, 32)
+  // half block hb, counted from the first half of entry e0: keys cols[e0 + hb/2] * 64 + 32 * (hb & 1) + [0, 32)
   constexpr int HCH = 32 * CPR / 64;  // 16-byte chunks per lane per half tile
   uint4 kreg[HCH], vreg[HCH];
   auto prefetch = [&](int hb, int col, int bits) {
@@ -250,13 +274,19 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
   };
   // the first K/V request goes out before anything else touches memory
   int col_cur = 0, bits_cur = 0;
-  if (e0 < e1) {  // (an even split can leave the last units of a row without entries: neutral partials)
+  const int first = hb0 & 1, nhalf = first + hb1 - hb0;
+  if (first < nhalf) {  // (an even split can leave the last units of a row without half blocks: neutral partials)
     if constexpr (SUB)
       scalar_load2(cols + e0 * EW, cols + e0 * EW + 1, col_cur, bits_cur);
     else
       col_cur = scalar_load(cols + e0);
-    prefetch(0, col_cur, bits_cur);
+    prefetch(first, col_cur, bits_cur);
   }
+
+  // behind it, for rows of several workgroups, the arrival slot
+  slot_t *const slot = reinterpret_cast<slot_t *>(ws + (((int64_t)b * p.Hq + h0 + 1) * (max_groups + 1) - 1) * (D + 2));
+  slot_t slot_seen = 0;
+  if (groups > 1 && threadIdx.x == 0) slot_seen = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   // q of the group's heads -> LDS (row min(m, ratio-1) feeds MFMA column m;
   // columns >= ratio are duplicates whose results are never stored)
@@ -270,6 +300,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
       *reinterpret_cast<uint4 *>(qs_ + h * D * 2 + ch * 16) = w;
     }
   }
+  if (groups > 1 && threadIdx.x == 0) open_slot(slot, slot_seen, launch);
   const int q_read = (m < ratio ? m : ratio - 1) * D * 2 + g * 16;
 
   floatx16 oacc[DT];
@@ -282,9 +313,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
   const int k_read = m * S::kStride + g * 16;
   const int i16 = lane & 15, dgrp = (lane >> 4) & 1;
   const int v_read = (4 * g + (i16 >> 2)) * S::kStride + (16 * dgrp + 4 * (i16 & 3)) * 2;
-  const int nhalf = 2 * (e1 - e0);
 
-  for (int hb = 0; hb < nhalf; ++hb) {
+  for (int hb = first; hb < nhalf; ++hb) {
     const int col = col_cur;
     const int hbits = SUB ? half_bits(bits_cur, hb) : 1;
     const int key0 = col * 64 + (hb & 1) * 32;
@@ -376,12 +406,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
     }
   }
 
-  // ---- partial result of this unit: lanes (m < ratio) hold head h0 + m ----
-  // rows [head][D + 2] floats (O unnormalised, max, sum): in the workspace, or, when the row is
-  // finished here, in this wave's own tile area (its tiles are dead by now)
+  // ---- result of this unit: lanes (m < ratio) hold head h0 + m ----
+  // rows [head][D + 2] floats (O unnormalised, max, sum) in this wave's own tile area (its tiles are
+  // dead by now)
   if (m < ratio) {
-    float *dst = merge_here ? reinterpret_cast<float *>(smem) + m * (D + 2)
-                            : ws + (((int64_t)b * p.Hq + h0 + m) * max_units + unit) * (D + 2);
+    float *dst = reinterpret_cast<float *>(smem) + m * (D + 2);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -393,114 +422,113 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
       dst[D + 1] = l_run;
     }
   }
-  {
-    if (!merge_here) return;
-    __syncthreads();  // every wave of the workgroup gets here (merge_here is workgroup-uniform)
-    // heads of the group are dealt to the waves; lane l owns dims l D/64 .. of its head
-    constexpr int PER = D / 64;
-    for (int h = wave; h < ratio; h += W) {
-      float mv[W], lv[W], ov[W][PER];
+  __syncthreads();
+  // heads of the group are dealt to the waves; lane l owns dims l D/64 .. of its head
+  constexpr int PER = D / 64;
+  auto store_row = [&](int h, const float (&o)[PER], float mmax, float l) {
+    const float inv = l > 0.f ? (p.paged.table ? p.paged.out_scale : 1.f) / l : 0.f;  // (includes the V scale)
+    T *op = (T *)p.o.ptr + sq.b * p.o.sb + (int64_t)(h0 + h) * p.o.sh + (int64_t)sq.q_start * p.o.st;
 #pragma unroll
-      for (int u = 0; u < W; ++u) {
-        const float *row = reinterpret_cast<const float *>(smem_all + u * wave_bytes) + h * (D + 2);
-        mv[u] = row[D];
-        lv[u] = row[D + 1];
+    for (int i = 0; i < PER; ++i)
+      if (!PAD || lane * PER + i < p.D) op[lane * PER + i] = from_float<T>(o[i] * inv);
+    if (p.lse.ptr && lane == 0)
+      p.lse.ptr[sq.b * p.lse.sb + (h0 + h) * p.lse.sh + (int64_t)sq.q_start * p.lse.st] =
+          l > 0.f ? (mmax + log2f(l)) * kLn2 : -INFINITY;
+  };
+  for (int h = wave; h < ratio; h += W) {
+    float mv[W], lv[W], ov[W][PER];
 #pragma unroll
-        for (int i = 0; i < PER; ++i) ov[u][i] = row[lane * PER + i];
-      }
-      float mmax = mv[0];
+    for (int u = 0; u < W; ++u) {
+      const float *row = reinterpret_cast<const float *>(smem_all + u * wave_bytes) + h * (D + 2);
+      mv[u] = row[D];
+      lv[u] = row[D + 1];
 #pragma unroll
-      for (int u = 1; u < W; ++u) mmax = fmaxf(mmax, mv[u]);
-      const float muse = mmax == -INFINITY ? 0.f : mmax;
-      float l = 0.f, o[PER];
-#pragma unroll
-      for (int i = 0; i < PER; ++i) o[i] = 0.f;
-#pragma unroll
-      for (int u = 0; u < W; ++u) {
-        const float sc = fast_exp2(mv[u] - muse);  // a wave without entries has max = -inf: weight 0
-        l += sc * lv[u];
-#pragma unroll
-        for (int i = 0; i < PER; ++i) o[i] += sc * ov[u][i];
-      }
-      const float inv = l > 0.f ? (p.paged.table ? p.paged.out_scale : 1.f) / l : 0.f;
-      T *op = (T *)p.o.ptr + sq.b * p.o.sb + (int64_t)(h0 + h) * p.o.sh + (int64_t)sq.q_start * p.o.st;
-#pragma unroll
-      for (int i = 0; i < PER; ++i)
-        if (!PAD || lane * PER + i < p.D) op[lane * PER + i] = from_float<T>(o[i] * inv);
-      if (p.lse.ptr && lane == 0)
-        p.lse.ptr[sq.b * p.lse.sb + (h0 + h) * p.lse.sh + (int64_t)sq.q_start * p.lse.st] =
-            l > 0.f ? (mmax + log2f(l)) * kLn2 : -INFINITY;
+      for (int i = 0; i < PER; ++i) ov[u][i] = row[lane * PER + i];
     }
+    float mmax = mv[0];
+#pragma unroll
+    for (int u = 1; u < W; ++u) mmax = fmaxf(mmax, mv[u]);
+    const float muse = mmax == -INFINITY ? 0.f : mmax;
+    float l = 0.f, o[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) o[i] = 0.f;
+#pragma unroll
+    for (int u = 0; u < W; ++u) {
+      const float sc = fast_exp2(mv[u] - muse);  // a wave without half blocks has max = -inf: weight 0
+      l += sc * lv[u];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) o[i] += sc * ov[u][i];
+    }
+    if (groups <= 1) {
+      store_row(h, o, mmax, l);
+    } else {  // write-through stores: the row's other workgroups may sit on another die
+      float *dst = ws + (((int64_t)b * p.Hq + h0 + h) * (max_groups + 1) + blockIdx.x) * (D + 2);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) __hip_atomic_store(dst + lane * PER + i, o[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (lane < 2) __hip_atomic_store(dst + D + lane, lane ? l : mmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (groups <= 1) return;
+  // the partial's write-through stores have reached memory (a release fence would write back the whole
+  // L2 for the sake of stores that are not in it: 2 us)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  int *flag = reinterpret_cast<int *>(smem_all + wave_bytes - ratio * D * 2);  // wave 0's q copy: dead as well
+  if (threadIdx.x == 0) *flag = arrive_last(slot, groups);
+  __syncthreads();
+  if (!*flag) return;
+  constexpr int MAXU = 8;  // partials merged per pass: their loads leave together
+  for (int h = wave; h < ratio; h += W) {
+    const float *src = ws + ((int64_t)b * p.Hq + h0 + h) * (max_groups + 1) * (D + 2);
+    float mmax = -INFINITY, l = 0.f, o[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) o[i] = 0.f;
+    for (int s0 = 0; s0 < groups; s0 += MAXU) {
+      float mv[MAXU], lv[MAXU], ov[MAXU][PER];
+#pragma unroll
+      for (int s = 0; s < MAXU; ++s) {
+        const float *row = src + min(s0 + s, groups - 1) * (D + 2);
+        mv[s] = __hip_atomic_load(row + D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lv[s] = __hip_atomic_load(row + D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < PER; ++i) ov[s][i] = __hip_atomic_load(row + lane * PER + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      float mnew = mmax;
+#pragma unroll
+      for (int s = 0; s < MAXU; ++s) mnew = fmaxf(mnew, mv[s]);
+      const float muse = mnew == -INFINITY ? 0.f : mnew;
+      const float alpha = fast_exp2(mmax - muse);  // exp2(-inf) = 0 on the first pass
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) o[i] *= alpha;
+#pragma unroll
+      for (int s = 0; s < MAXU; ++s) {
+        const float sc = s0 + s < groups ? fast_exp2(mv[s] - muse) : 0.f;
+        l += sc * lv[s];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) o[i] += sc * ov[s][i];
+      }
+      mmax = mnew;
+    }
+    store_row(h, o, mmax, l);
   }
 }
 
-// Merge of the unit partials: one wave per (sequence, q head), lane l owns
-// dims {2l, 2l+1} (D = 128) or dim l (D = 64).  All loads of a row are issued
-// before the first use (units are few, a dependent load chain per unit would
-// make this small kernel latency-bound).
-template <typename T, int D, bool PAD>
-__global__ __launch_bounds__(64) void decode_combine_kernel(const FwdParams p, const float *ws, int unit_blocks,
-                                                            int max_units, int merged_units) {
-  constexpr int PER = D / 64;  // dims per lane
-  constexpr int MAXU = 8;      // units merged per pass
-  const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
-  const SeqInfo sq = load_seq(p.seqs, b, p.causal);
-  if (sq.q_len <= 0) return;
-  int units = 0;
-  const int rb = sq.past / 64;
-  if (sq.k_len > 0 && rb < p.csr.num_rows) {
-    const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
-    const int n = scalar_load(p.csr.ptr + lh * p.csr.ptr_sh + rb + 1) - scalar_load(p.csr.ptr + lh * p.csr.ptr_sh + rb);
-    units = min(decode_row_units(n, unit_blocks, merged_units), max_units);  // as the partial kernel
-  }
-  // rows of at most merged_units units (the waves of a partial-kernel workgroup) were finished there
-  if (units <= merged_units) return;
-  const float *src = ws + ((int64_t)b * p.Hq + h) * max_units * (D + 2);
-  float mmax = -INFINITY, l = 0.f, o[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) o[i] = 0.f;
-  for (int s0 = 0; s0 < units; s0 += MAXU) {
-    float mv[MAXU], lv[MAXU], ov[MAXU][PER];
-#pragma unroll
-    for (int s = 0; s < MAXU; ++s) {
-      const bool ok = s0 + s < units;
-      const float *row = src + (s0 + (ok ? s : 0)) * (D + 2);
-      mv[s] = ok ? row[D] : -INFINITY;
-      lv[s] = ok ? row[D + 1] : 0.f;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) ov[s][i] = ok ? row[lane * PER + i] : 0.f;
-    }
-    float mnew = mmax;
-#pragma unroll
-    for (int s = 0; s < MAXU; ++s) mnew = fmaxf(mnew, mv[s]);
-    const float muse = mnew == -INFINITY ? 0.f : mnew;
-    const float alpha = fast_exp2(mmax - muse);  // exp2(-inf) = 0 on the first pass
-    l *= alpha;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) o[i] *= alpha;
-#pragma unroll
-    for (int s = 0; s < MAXU; ++s) {
-      const float sc = fast_exp2(mv[s] - muse);
-      l += sc * lv[s];
-#pragma unroll
-      for (int i = 0; i < PER; ++i) o[i] += sc * ov[s][i];
-    }
-    mmax = mnew;
-  }
-  const float inv = l > 0.f ? (p.paged.table ? p.paged.out_scale : 1.f) / l : 0.f;
-  T *op = (T *)p.o.ptr + sq.b * p.o.sb + h * p.o.sh + (int64_t)sq.q_start * p.o.st;
-#pragma unroll
-  for (int i = 0; i < PER; ++i)
-    if (!PAD || lane * PER + i < p.D) op[lane * PER + i] = from_float<T>(o[i] * inv);  // inv includes the V scale
-  if (p.lse.ptr && lane == 0)
-    p.lse.ptr[sq.b * p.lse.sb + h * p.lse.sh + (int64_t)sq.q_start * p.lse.st] =
-        l > 0.f ? (mmax + log2f(l)) * kLn2 : -INFINITY;
+// Workgroups of the longest row.  (At most 255: an arrival slot counts in eight bits; longer rows
+// are cut into larger units.)
+static int decode_max_groups(const FwdParams &p) {
+  return std::min(255, cdiv(decode_row_units(2 * decode_max_row_entries(p), decode_unit_halves(p), kDecodeWaves), kDecodeWaves));
 }
 
-// Unit slots per (sequence, q head) in the workspace: the longest row's units (rows that fit one
-// workgroup keep their partials in LDS).
-static int decode_max_units(const FwdParams &p) {
-  return decode_row_units(decode_max_row_entries(p), decode_unit_blocks(p), kDecodeWaves);
+// Numbers of the launches of this process (arrive_last): 56 bits, never 0.
+static slot_t next_launch_number() {
+  static std::atomic<slot_t> next{(uintptr_t)&next * 0x9E3779B97F4A7C15ull ^
+                                (slot_t)std::chrono::system_clock::now().time_since_epoch().count()};
+  slot_t n;
+  do {
+    n = (next.fetch_add(1, std::memory_order_relaxed) * 0xD1342543DE82EF95ull) >> 8;  // (an odd factor: 2^64 distinct products)
+  } while (n == 0);
+  return n;
 }
 
 bool decode_supported(const FwdParams &p, int dtype) {
@@ -517,26 +545,19 @@ bool decode_supported(const FwdParams &p, int dtype) {
 }
 
 size_t decode_workspace_bytes(const FwdParams &p) {
-  return (size_t)p.seqs.batch * p.Hq * decode_max_units(p) * (mfma_tile_width(p.D) + 2) * sizeof(float);
+  return (size_t)p.seqs.batch * p.Hq * (decode_max_groups(p) + 1) * (mfma_tile_width(p.D) + 2) * sizeof(float);
 }
 
 template <typename T, int D, bool PAD, bool SUB, bool PAGED, bool KV8 = false>
 static int launch_decode_td(const FwdParams &p, float *ws, hipStream_t stream) {
   constexpr int W = kDecodeWaves;
   const int smem = W * DecSmem<D>::wave_bytes(p.Hq / p.Hkv);
-  const int unit_blocks = decode_unit_blocks(p), max_units = decode_max_units(p);
-  const int groups = cdiv(max_units, W);
-  DK_REQUIRE(groups <= 65535, "too many decode units");
+  const int groups = std::max(1, decode_max_groups(p));
   DK_REQUIRE(smem <= 160 * 1024, "decode workgroup needs %d bytes of LDS", smem);
   DK_ALLOW_DYNAMIC_LDS((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W>), smem);
   DK_NOTE_KERNEL("decode_partial_kernel");
   hipLaunchKernelGGL((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W>), dim3(groups, p.Hkv, p.seqs.batch),
-                     dim3(64 * W), smem, stream, p, ws, unit_blocks, max_units);
-  DK_HIP_CHECK(hipGetLastError());
-  if (groups == 1) return DK_OK;  // every row was finished inside its workgroup
-  DK_NOTE_KERNEL("decode_combine_kernel");
-  hipLaunchKernelGGL((decode_combine_kernel<T, D, PAD>), dim3(p.Hq, p.seqs.batch), dim3(64), 0, stream, p, ws,
-                     unit_blocks, max_units, W);
+                     dim3(64 * W), smem, stream, p, ws, decode_unit_halves(p), groups, next_launch_number());
   DK_HIP_CHECK(hipGetLastError());
   return DK_OK;
 }
