@@ -33,15 +33,14 @@ class _NoGradContext:
 
 def _identical_head_run(pattern: Tensor) -> int:
     """Largest g dividing the number of pattern heads such that every run of g
-    consecutive heads holds one and the same pattern."""
+    consecutive heads holds one and the same pattern.  (Any g: groups of 3 or 16 q heads per kv
+    head decode on the split-KV kernels like groups of 2, 4 or 8.)"""
     H = pattern.size(0)
-    p = pattern.cpu()
-    for g in (8, 4, 2):
-        if H % g == 0 and H >= g:
-            grouped = p.reshape(H // g, g, *p.shape[1:])
-            if bool((grouped == grouped[:, :1]).all()):
-                return g
-    return 1
+    if pattern.stride(0) == 0:
+        return H
+    same = (pattern[1:] == pattern[:-1]).flatten(1).all(1).tolist()  # head i + 1 equals head i
+    starts = [i + 1 for i, x in enumerate(same) if not x]  # a new pattern starts at these heads
+    return max(g for g in range(1, H + 1) if H % g == 0 and all(s % g == 0 for s in starts))
 
 
 def _uneven_heads(pattern: Tensor) -> bool:

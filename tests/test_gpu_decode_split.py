@@ -49,6 +49,25 @@ def test_one_sequence_against_the_oracle(ctx, D, bs, local, vert, dtype):
         assert torch.equal(again[0], first[0]) and torch.equal(again[1], first[1])
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(6, 2), (16, 1), (12, 1)])
+def test_groups_that_are_no_power_of_two_or_large(Hq, Hkv):
+    """3, 12 and 16 q heads per kv head: the module finds runs of any length, so these groups decode on
+    the split-KV kernels (and may page their keys) too."""
+    print(f"case Hq={Hq} Hkv={Hkv}", flush=True)
+    B, ctx, D, Lmax = 2, 700, 128, 1024
+    sm = 1 / math.sqrt(D)
+    g = torch.Generator().manual_seed(Hq)
+    q = torch.randn(B, 1, Hq, D, generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(B, ctx, Hkv, D, generator=g).to(torch.bfloat16) for _ in range(2))
+    bm = OL.block_mask(Hq, Lmax, 64, 2, 4, num_kv_heads=Hkv)
+    ro, _ = OA.dense_attention(q, k, v, torch.from_numpy(OA.sequence_token_mask(bm, 64, 1, ctx)), sm)
+    mod = New(Hq, Lmax, 64, 2, 4, num_kv_heads=Hkv).to(DEV)
+    assert mod.lut_group % (Hq // Hkv) == 0
+    out = mod(q.to(DEV), k.to(DEV), v.to(DEV), sm)
+    assert _lib.lib().dk_last_kernels().startswith(b"decode_partial_kernel")
+    assert_close("O", out, ro, **TOL)
+
+
 @pytest.mark.parametrize("fill", [0x00, 0xff, 0x7f])
 def test_scratch_may_hold_anything(fill):
     B, Hq, Hkv, L, D = 2, 8, 2, 3000, 128
