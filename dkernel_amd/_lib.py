@@ -113,6 +113,24 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The C++ host path of the inference calls (dkernel_amd/_host.so, loaded on first use)."""
+    global _host
+    if _host is None:
+        path = os.path.join(_HERE, "_host.so")
+        if not os.path.exists(path):
+            raise ImportError(f"{path} is missing: build it with `make -C dkernel_amd/csrc`.")
+        from . import _host as module
+        handle = lib()
+        module.bind(*(C.cast(getattr(handle, name), vp).value
+                      for name in ("dk_fwd", "dk_fwd_workspace_bytes", "dk_fwd_paged")))
+        _host = module
+    return _host
+
+
 class DKernelError(RuntimeError):
     pass
 

@@ -40,7 +40,8 @@ static LutView view(const dk_lut &l) {
 }
 static SeqView view(const dk_seqs &s) {
   SeqView v{s.batch, s.max_q_len, s.max_k_len, s.packed & 3, s.q_starts, s.q_ends, s.k_starts, s.k_ends};
-  v.zero_outside = (s.packed & 4) && !(s.packed & 1) && s.q_starts ? 1 : 0;  // (without lengths every row holds a query)
+  v.any = s.k_ends ? s.k_ends : s.k_starts ? s.k_starts : s.q_ends ? s.q_ends : s.q_starts;
+  v.zero_outside = (s.packed & 4) && (s.q_starts || s.q_ends) ? 1 : 0;  // (without lengths every row holds a query)
   return v;
 }
 
@@ -72,10 +73,11 @@ static int check_common(const dk_seqs &s, int Hq, int Hkv, int D, int dtype, int
   DK_REQUIRE(dtype == DK_BF16 || dtype == DK_F16 || dtype == DK_F32, "unknown dtype %d", dtype);
   DK_REQUIRE(s.batch >= 0 && s.max_q_len >= 0 && s.max_k_len >= 0, "negative sizes");
   DK_REQUIRE(Hq <= 65535 && s.batch <= 65535, "too many heads or sequences for one launch");
-  const bool all = s.q_starts && s.q_ends && s.k_starts && s.k_ends;
   const bool none = !s.q_starts && !s.q_ends && !s.k_starts && !s.k_ends;
-  DK_REQUIRE(all || none, "q/k starts/ends must be given together");
-  DK_REQUIRE(!s.packed || all, "packed inputs need sequence offsets");
+  DK_REQUIRE((!s.q_starts || s.k_starts) && (!s.q_ends || s.k_ends), "q/k starts/ends must be given together");
+  DK_REQUIRE(!(s.packed & 1) || (s.k_starts && s.k_ends && (s.q_starts != nullptr) == (s.q_ends != nullptr) &&
+                                 (s.q_starts || (s.packed & 2))),
+             "packed inputs need sequence offsets");
   if (none && causal)
     DK_REQUIRE(s.max_k_len >= s.max_q_len, "causal attention needs k length (%d) >= q length (%d)", s.max_k_len,
                s.max_q_len);
@@ -118,7 +120,8 @@ static int make_bwd_params(const dk_bwd_args *a, BwdParams &p, bool &empty) {
   DK_REQUIRE(a != nullptr, "args is NULL");
   int rc = check_common(a->seqs, a->num_q_heads, a->num_kv_heads, a->head_dim, a->dtype, a->causal);
   if (rc) return rc;
-  DK_REQUIRE(!a->seqs.q_starts && !a->seqs.packed,
+  p.seqs = view(a->seqs);
+  DK_REQUIRE(!p.seqs.any && !a->seqs.packed,
              "Currently does not support paddings or variable length inputs in backward.");
   rc = check_lut(a->csr, "csr", a->num_q_heads, a->num_kv_heads);
   if (rc) return rc;
@@ -147,7 +150,6 @@ static int make_bwd_params(const dk_bwd_args *a, BwdParams &p, bool &empty) {
   p.delta = a->delta;
   p.csr = view(a->csr);
   p.csc = view(a->csc);
-  p.seqs = view(a->seqs);
   p.Hq = a->num_q_heads;
   p.Hkv = a->num_kv_heads;
   p.D = a->head_dim;
@@ -270,7 +272,7 @@ int dk_fwd_paged(const dk_fwd_args *a, const dk_paged_kv *pg) {
   int rc = make_fwd_params(a, p);
   if (rc) return rc;
   if (p.seqs.batch == 0 || p.seqs.max_q_len == 0) return DK_OK;
-  DK_REQUIRE(!p.seqs.packed && p.seqs.q_starts, "paged decode takes per-sequence lengths (dk_seqs arrays)");
+  DK_REQUIRE(!p.seqs.packed && p.seqs.k_ends, "paged decode takes per-sequence lengths (dk_seqs arrays)");
   DK_REQUIRE(pg->kv_dtype == DK_FP8_E4M3 || ((pg->page_stride_k * (int64_t)elem_size(a->dtype)) % 16 == 0 &&
                                               (pg->page_stride_v * (int64_t)elem_size(a->dtype)) % 16 == 0),
              "page strides must keep rows 16-byte aligned");

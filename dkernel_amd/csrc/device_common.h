@@ -84,11 +84,13 @@ __device__ __forceinline__ int grid_head(const LutView &l) {
 struct SeqView {
   int32_t batch, max_q_len, max_k_len, packed;
   const int32_t *q_starts, *q_ends, *k_starts, *k_ends;
+  const int32_t *any = nullptr;  // some array of the four above that is given; nullptr: none
   // packed inputs, optional: batch + 1 ints, entry b = work items (q tiles or pairs of q tiles) of
   // the sequences before b, written by a small kernel ahead of the one that reads it
   int32_t *item_offsets = nullptr;
   // padded inputs: the forward kernels also write the rows of o (zeros) and lse (-inf) that hold
-  // no query of their sequence, so that the caller need not clear the outputs first
+  // no query of their sequence, so that the caller need not clear the outputs first; packed inputs:
+  // the rows of lse before the first sequence and behind the last one (-inf)
   int32_t zero_outside = 0;
 };
 
@@ -142,13 +144,17 @@ struct SeqInfo {
 __device__ __forceinline__ SeqInfo load_seq_lane(const SeqView &s, int b, int causal) {
   SeqInfo r;
   r.b = b;
-  if (s.q_starts) {
+  if (s.any) {
+    // An array that is not given stands for starts of 0 / ends at the token dimension (packed: for
+    // one query token per sequence).  Its load goes to one that is, so that the four leave together.
+    const int qs = (s.q_starts ? s.q_starts : s.any)[b], qe = (s.q_ends ? s.q_ends : s.any)[b];
+    const int ks = (s.k_starts ? s.k_starts : s.any)[b], ke = (s.k_ends ? s.k_ends : s.any)[b];
     // ends beyond the token dimension are clamped, so a bad length can never
     // make a kernel read or write outside the tensors
-    r.q_start = max(s.q_starts[b], 0);
-    r.q_len = min(s.q_ends[b], s.max_q_len) - r.q_start;
-    r.k_start = max(s.k_starts[b], 0);
-    r.k_len = min(s.k_ends[b], s.max_k_len) - r.k_start;
+    r.q_start = s.q_starts ? max(qs, 0) : s.packed ? b : 0;
+    r.q_len = (s.q_ends ? min(qe, s.max_q_len) : s.packed ? min(b + 1, s.max_q_len) : s.max_q_len) - r.q_start;
+    r.k_start = s.k_starts ? max(ks, 0) : 0;
+    r.k_len = (s.k_ends ? min(ke, s.max_k_len) : s.max_k_len) - r.k_start;
   } else {
     r.q_start = r.k_start = 0;
     r.q_len = s.max_q_len;
@@ -333,6 +339,18 @@ __device__ __forceinline__ void zero_rows_outside(const SeqView &s, const SeqInf
       const int hh = idx % nh, i = lo + idx / nh;
       lse.ptr[sq.b * lse.sb + (h0 + hh) * lse.sh + (int64_t)token(i) * lse.st] = -INFINITY;
     }
+  }
+}
+
+// Packed inputs with SeqView::zero_outside: the log-sum-exps of the token rows that belong to no
+// sequence.  The workgroups of one work item per head (or head group) call it.
+__device__ __forceinline__ void lse_outside_packed(const SeqView &s, const RowView &lse, int h0, int nh, int tid, int nthreads) {
+  if (!lse.ptr || s.batch < 1 || !s.q_starts || !s.q_ends) return;
+  const int lo = min(max(s.q_starts[0], 0), s.max_q_len), hi = max(min(s.q_ends[s.batch - 1], s.max_q_len), lo);
+  const int outside = lo + s.max_q_len - hi;
+  for (int i = tid; i < outside * nh; i += nthreads) {
+    const int t = i / nh;
+    lse.ptr[(h0 + i % nh) * lse.sh + (int64_t)(t < lo ? t : t - lo + hi) * lse.st] = -INFINITY;
   }
 }
 

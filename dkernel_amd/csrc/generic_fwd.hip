@@ -29,7 +29,8 @@ __global__ __launch_bounds__(256) void generic_fwd_kernel(const FwdParams p) {
   SeqInfo sq;
   int tile;
   const bool has_rows = resolve_tile(p.seqs, p.causal, BM, tiles_per_block, blockIdx.x, blockIdx.z, sq, tile);
-  if (p.seqs.zero_outside)
+  if (p.seqs.packed && p.seqs.zero_outside && blockIdx.x == 0) lse_outside_packed(p.seqs, p.lse, blockIdx.y, 1, threadIdx.x, 256);
+  if (p.seqs.zero_outside && !p.seqs.packed)
     zero_rows_outside<T>(p.seqs, sq, blockIdx.x, gridDim.x, p.o, p.lse, blockIdx.y, 1, p.D, p.vec_ok, threadIdx.x, 256);
   if (!has_rows) return;
   const int h = blockIdx.y;
@@ -180,7 +181,7 @@ static int fwd_tiles_x(const FwdParams &p, int rows_per_wg) {
     // a sequence's queries touch at most ceil(q_len / BM) + 1 row blocks (they may start inside
     // one), and the ceilings add up to at most total / BM + batch
     blocks = cdiv(s.max_q_len, BM) + 2 * s.batch;
-  else if (s.q_starts)
+  else if (s.any)
     blocks = cdiv(s.max_q_len, BM) + 1;
   else {
     const int past = p.causal ? s.max_k_len - s.max_q_len : 0;

@@ -241,7 +241,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   } else {
     has_rows = resolve_tile(p.seqs, p.causal, 64, 1, tiles_y - 1 - (int)blockIdx.y, blockIdx.z, sq, tile);
   }
-  if (p.seqs.zero_outside)
+  if (p.seqs.packed && p.seqs.zero_outside && blockIdx.y == 0) lse_outside_packed(p.seqs, p.lse, grid_head(p.csr), 1, tid, NT);
+  if (p.seqs.zero_outside && !p.seqs.packed)
     zero_rows_outside<float>(p.seqs, sq, blockIdx.y, tiles_y, p.o, p.lse, grid_head(p.csr), 1, p.D, p.vec_ok, tid, NT);
   if (!has_rows) return;
   const int rb = sq.past / 64 + tile;
@@ -659,7 +660,7 @@ int launch_mfma_f32_fwd(const FwdParams &p, hipStream_t stream) {
   int tiles;
   if (s.packed)
     tiles = cdiv(s.max_q_len, 64) + 2 * s.batch;  // as for the 16-bit forward: an upper bound over all sequences
-  else if (s.q_starts)
+  else if (s.any)
     tiles = cdiv(s.max_q_len, 64) + 1;
   else {
     const int past = p.causal ? s.max_k_len - s.max_q_len : 0;

@@ -57,6 +57,8 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   SeqInfo sq;
   int tile;
   const int tid = threadIdx.x, lane = tid & 63;
+  if (p.seqs.packed && p.seqs.zero_outside && blockIdx.y == 0)
+    lse_outside_packed(p.seqs, p.lse, grid_head(p.csr) * (RP ? 1 : G), RP ? 1 : G, tid, NT);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: row tests and head indices follow it
   int rb;
   int first_rb = 0, last_rb = 0;  // RP: table rows that hold queries of this sequence
@@ -101,7 +103,7 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
       has_rows = resolve_tile(p.seqs, p.causal, 64, 1, ty, blockIdx.z, sq, tile);
     }
     if (!has_rows) {
-      if (p.seqs.zero_outside)  // (never with packed inputs, for which sq is not set here)
+      if (p.seqs.zero_outside && !p.seqs.packed)  // (with packed inputs sq is not set here)
         zero_rows_outside<T>(p.seqs, sq, blockIdx.y, tiles_y, p.o, p.lse, grid_head(p.csr) * G, G, p.D, p.vec_ok, tid, NT);
       return;
     }
@@ -411,7 +413,7 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   }
   // padded inputs: this workgroup's share of the rows that hold no query, behind its own work (at
   // the start the stores of every workgroup would go out together, ahead of all multiplies)
-  if (p.seqs.zero_outside)
+  if (p.seqs.zero_outside && !p.seqs.packed)
     zero_rows_outside<T>(p.seqs, sq, blockIdx.y, tiles_y, p.o, p.lse, RP ? hx : hx * G, RP ? 1 : G, p.D,
                          p.vec_ok, tid, NT);
   if (!row_ok) return;
@@ -537,7 +539,7 @@ static int launch_row_pairs(const FwdParams &p, hipStream_t stream) {
     // per sequence at most (ceil(q_len / 64) + 1) / 2 + 1 pairs; the ceilings add up to at most
     // total / 64 + batch
     pairs = (cdiv(s.max_q_len, 64) + s.batch) / 2 + 2 * s.batch;
-  } else if (s.q_starts) {
+  } else if (s.any) {
     pairs = (cdiv(s.max_q_len, 64) + 1) / 2 + 1;  // a sequence's rows start anywhere inside a pair
   } else {
     const int past = p.causal ? s.max_k_len - s.max_q_len : 0;
@@ -637,7 +639,7 @@ int launch_mfma_fwd(const FwdParams &p_in, int dtype, void *workspace, size_t wo
     // a sequence's queries touch at most ceil(q_len / 64) + 1 row blocks (they may start inside
     // one), and the ceilings add up to at most total / 64 + batch
     tiles = cdiv(s.max_q_len, 64) + 2 * s.batch;
-  else if (s.q_starts)
+  else if (s.any)
     tiles = cdiv(s.max_q_len, 64) + 1;
   else {
     const int past = p.causal ? s.max_k_len - s.max_q_len : 0;

@@ -244,6 +244,7 @@ class SparseAttention(torch.nn.Module):
                 self.register_buffer("exact_csc_row", exact_c[1].to(torch.int32), persistent=False)
 
         self.mask_tile = None
+        self.mask_lut_max_row = 0
         if mask_for_kernels:
             m_csr, m_csc = masked_tile_tables(block_size, kernel_pattern, _KERNEL_TILE)
             m_csr, m_csc = list(m_csr), list(m_csc)
@@ -257,6 +258,18 @@ class SparseAttention(torch.nn.Module):
             self.register_buffer("masked_csr_col", m_csr[1].to(torch.int32), persistent=False)
             self.register_buffer("masked_csc_ccol", m_csc[0].to(torch.int32), persistent=False)
             self.register_buffer("masked_csc_row", m_csc[1].to(torch.int32), persistent=False)
+
+        # names of the tables that the kernels read, with their tile sizes: (crow, col, rows, columns,
+        # masked crow, masked col, tile, pattern block size)
+        if self.kernel_tile is not None:
+            tables = ("kernel_csr_crow", "kernel_csr_col", self.kernel_tile, self.kernel_tile)
+        elif self.exact_tile is not None:
+            tables = ("exact_csr_crow", "exact_csr_col", self.exact_tile, self.exact_tile)
+        else:
+            tables = ("layout_csr_crow", "layout_csr_col", self.block_m, self.block_n)
+        masked = (None, None, 0, 0) if self.mask_tile is None else ("masked_csr_crow", "masked_csr_col", self.mask_tile,
+                                                                    self.block_size)
+        self._kernel_tables = tables + masked
 
     def forward(self,
                 q: Tensor,
@@ -282,6 +295,14 @@ class SparseAttention(torch.nn.Module):
         return_lse: also return the natural-log softmax normaliser, (batch,
             heads, seq) for 4-D inputs and (heads, total_tokens) for packed ones.
         """
+        if v is not None:
+            # inference on tensors that need no preparation: the same launch from C++ (None: not such a call)
+            res = _lib.host().forward(q, k, v, sm_scale, self._buffers, self._kernel_tables, self.mask_lut_max_row,
+                                      self.kwargs, self.seq_dim, cu_seqlen_k, cu_seqlen_q, left_paddings, seqlens,
+                                      return_lse, ops._impl, ops._fwd_workspace)
+            if res is not None:
+                output, lse, ops.last_fwd_workspace_bytes = res
+                return (output, lse) if return_lse else output
         inf_kwargs = {"cu_seqlen_k": cu_seqlen_k,
                       "cu_seqlen_q": cu_seqlen_q,
                       "left_paddings": left_paddings,
@@ -336,6 +357,12 @@ class SparseAttention(torch.nn.Module):
         of 8 up to 256).  No counterpart in the reference."""
         from .ops import paged_decode_attn
         assert self.kwargs.get('causal', True), "paged decode is causal"
+        if out is None:
+            res = _lib.host().paged(q, k_pool, v_pool, block_table, context_lens, sm_scale, self._buffers,
+                                    self._kernel_tables, self.mask_lut_max_row, self.lut_max_row, self.lut_group,
+                                    self.max_seqlen, return_lse, k_scale, v_scale, ops._impl)
+            if res is not None:
+                return res[:2] if return_lse else res[0]
         if self.kernel_tile is not None:
             layout = (self.kernel_csr_crow, self.kernel_csr_col, self.kernel_tile, self.kernel_tile)
             max_row = self.lut_max_row

@@ -358,7 +358,9 @@ def padded_sparse_attn(q: Tensor, k: Tensor, v: Tensor, sm_scale: float,
         k_starts = _const_i32(dev, batches, 0)
     if seqlens is not None:
         # ends beyond the padded length are clamped on the device
-        k_ends = k_starts + _as_i32(seqlens, dev)
+        k_ends = _as_i32(seqlens, dev)
+        if left_paddings is not None:
+            k_ends = k_starts + k_ends
     else:
         k_ends = _const_i32(dev, batches, k_len)
     if q_len == 1:
@@ -424,7 +426,7 @@ def paged_decode_attn(q: Tensor, k_pool: Tensor, v_pool: Tensor, block_table: Te
             f"block_table names pages outside the pools ({k_pool.size(0)} pages) inside a sequence: "
             f"first at (sequence, entry) {tuple(bad.nonzero()[0].tolist())}")
     o4 = (out[:, None] if out.dim() == 3 else out) if out is not None else q4.new_empty(q4.shape)
-    lse = torch.full((batches, num_heads, 1), float("-inf"), dtype=torch.float32, device=dev) if return_lse else None
+    lse = torch.empty((batches, num_heads, 1), dtype=torch.float32, device=dev) if return_lse else None
     k_ends = context_lens.to(dev, dtype=torch.int32).contiguous()
     zeros, ones = _const_i32(dev, batches, 0), _const_i32(dev, batches, 1)
 
@@ -497,14 +499,15 @@ def varlen_sparse_attn(q: Tensor, k: Tensor, v: Tensor,
     q, k, v = _unit_last(q), _unit_last(k), _unit_last(v)
     _check_out(out, q)
     out = out if out is not None else q.new_empty(q.shape)
-    lse = torch.full((num_heads, q.size(0)), float("-inf"), dtype=torch.float32, device=dev) if return_lse else None
+    # (the kernels write -inf where a token belongs to no sequence: bit 2 of dk_seqs.packed)
+    lse = torch.empty((num_heads, q.size(0)), dtype=torch.float32, device=dev) if return_lse else None
 
     args = _lib.FwdArgs()
     args.q, args.k, args.v, args.o = (_tensor3(x) for x in (q, k, v, out))
     args.lse = _rowvec(lse, (0, lse.stride(0), lse.stride(1))) if lse is not None else _rowvec(None)
     args.csr = _lut(sparse_layout, dev, lut_group, lut_max_row, uneven=uneven_heads and not single_query)
     isz = cu_q.element_size()
-    args.seqs = _lib.Seqs(batch_size, q.size(0), k.size(0), 3 if single_query else 1,
+    args.seqs = _lib.Seqs(batch_size, q.size(0), k.size(0), 3 if single_query else 5 if return_lse else 1,
                           cu_q.data_ptr(), cu_q.data_ptr() + isz, cu_k.data_ptr(), cu_k.data_ptr() + isz)
     args.num_q_heads, args.num_kv_heads, args.head_dim = num_heads, k.size(1), head_size
     args.dtype, args.causal, args.impl = _DTYPES[q.dtype], int(bool(causal)), _impl

@@ -155,7 +155,10 @@ typedef struct dk_lut {
  * q_len = max_q_len and k_len = max_k_len starting at token 0.  Otherwise the
  * arrays (device memory, int32, `batch` entries) give the first token and the
  * end (exclusive) of each sequence's queries and keys inside the token
- * dimension; query tokens are the LAST q_len positions of the sequence when
+ * dimension.  A single array may be left out: starts are then 0 and ends the
+ * token dimension's extent; an array for the queries needs the one for the
+ * keys, and packed inputs need all (with bit 1 of `packed` the queries' may be
+ * left out: query token b belongs to sequence b).  Query tokens are the LAST q_len positions of the sequence when
  * causal (past_len = k_len - q_len), positions counted from the first real
  * token.  Mirrors q/k_batch_starts/ends of
  * dkernel/ops/sparse_attn_inference.py:431-434,503-507. */
@@ -169,7 +172,9 @@ typedef struct dk_seqs {
                         bit 2 (without bit 0, with the arrays below): dk_fwd also writes the rows
                         of o (zeros) and lse (-inf) that hold no query of their sequence, so a
                         padded output need not be cleared first (the reference clears it with
-                        torch.zeros, dkernel/ops/sparse_attn_inference.py:67) */
+                        torch.zeros, dkernel/ops/sparse_attn_inference.py:67).  With bit 0: it
+                        writes lse (-inf) of the tokens before the first and behind the last
+                        sequence, which then follow each other without gaps */
   const int32_t *q_starts, *q_ends, *k_starts, *k_ends;
 } dk_seqs;
 

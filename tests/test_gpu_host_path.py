@@ -1,0 +1,128 @@
+"""The C++ host path of the inference calls (dkernel_amd/_host.so) against the Python launchers in
+ops.py: same kernels, so every output bit must agree; and what it leaves to them (None) still works.
+Also the tokens of packed inputs that belong to no sequence: their log-sum-exp reads -inf."""
+import math
+
+import pytest
+import torch
+
+from dkernel_amd import LocalStrideSparseAttention, SparseAttention, _lib, ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+New = LocalStrideSparseAttention.__wrapped__
+
+
+class _PythonOnly:
+    forward = paged = staticmethod(lambda *a: None)
+
+
+def both(monkeypatch, call):
+    """(result through _host, result through ops.py); asserts that _host took the call."""
+    real, taken = _lib.host(), []
+
+    class Spy:
+        @staticmethod
+        def forward(*a):
+            taken.append(real.forward(*a))
+            return taken[-1]
+
+        @staticmethod
+        def paged(*a):
+            taken.append(real.paged(*a))
+            return taken[-1]
+
+    monkeypatch.setattr(_lib, "host", lambda: Spy)
+    fast = call()
+    assert len(taken) == 1 and taken[0] is not None, "the C++ path did not take this call"
+    monkeypatch.setattr(_lib, "host", lambda: _PythonOnly)
+    slow = call()
+    monkeypatch.undo()
+    return fast, slow
+
+
+def same(a, b):
+    a, b = (x if isinstance(x, tuple) else (x,) for x in (a, b))
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        assert x.shape == y.shape and x.dtype == y.dtype and x.stride() == y.stride() and torch.equal(x, y)
+
+
+@pytest.mark.parametrize("dtype,D,bs,seq_dim,Hq,Hkv", [
+    (torch.bfloat16, 128, 64, 1, 8, 2), (torch.float16, 64, 32, 2, 4, 4), (torch.float32, 64, 64, 1, 4, 2),
+    (torch.bfloat16, 96, 128, 2, 6, 2), (torch.float32, 128, 32, 1, 2, 2)])
+def test_unpadded_padded_and_single_token(monkeypatch, dtype, D, bs, seq_dim, Hq, Hkv):
+    B, L = 3, 500
+    print(f"case {dtype} D={D} bs={bs} seq_dim={seq_dim}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    mod = New(Hq, 512, bs, 2, 3, num_kv_heads=Hkv, seq_dim=seq_dim).to(DEV)
+
+    def tensor(n, h):
+        return torch.randn((B, n, h, D) if seq_dim == 1 else (B, h, n, D), generator=g, device=DEV).to(dtype)
+    q, q1, k, v = tensor(L, Hq), tensor(1, Hq), tensor(L, Hkv), tensor(L, Hkv)
+    lens = torch.tensor([500, 1, 333], dtype=torch.int32, device=DEV)
+    for name, kw in (("plain", {}), ("left", dict(left_paddings=L - lens)), ("right", dict(seqlens=lens))):
+        for x in (q, q1):
+            for lse in (False, True):
+                print(name, x.shape, lse, flush=True)
+                same(*both(monkeypatch, lambda: mod(x, k, v, 0.1, return_lse=lse, **kw)))
+    # left to the Python path: both lengths at once, lengths of another type, gradients
+    for kw in (dict(left_paddings=L - lens, seqlens=lens), dict(seqlens=lens.long()), dict(left_paddings=(L - lens).cpu())):
+        assert _lib.host().forward(q, k, v, 0.1, mod._buffers, mod._kernel_tables, mod.mask_lut_max_row, mod.kwargs, mod.seq_dim,
+                                   None, None, kw.get("left_paddings"), kw.get("seqlens"), False, ops._impl, True) is None
+        assert torch.isfinite(mod(q, k, v, 0.1, **kw).float()).all()
+    out = mod(q.clone().requires_grad_(), k, v, 0.1)
+    assert out.requires_grad
+
+
+@pytest.mark.parametrize("Hq,Hkv,dtype,D", [(4, 2, torch.bfloat16, 128), (2, 2, torch.float32, 64), (3, 1, torch.float16, 40),
+                                            (2, 2, torch.bfloat16, 20)])
+def test_packed(monkeypatch, Hq, Hkv, dtype, D):
+    print(f"case Hq={Hq} Hkv={Hkv} {dtype} D={D}", flush=True)
+    lens, before, after = [70, 1, 200, 64], 5, 9
+    T = before + sum(lens) + after
+    g = torch.Generator(device=DEV).manual_seed(2)
+    q, k, v = (torch.randn(T, h, D, generator=g, device=DEV).to(dtype) for h in (Hq, Hkv, Hkv))
+    cu = torch.tensor([before] + [before + sum(lens[:i + 1]) for i in range(4)], dtype=torch.int32, device=DEV)
+    mod = New(Hq, 256, 64, 2, 3, num_kv_heads=Hkv).to(DEV)
+    fast, slow = both(monkeypatch, lambda: mod(q, k, v, 0.1, cu_seqlen_k=cu, return_lse=True))
+    inside = slice(before, T - after)
+    same((fast[0][inside], fast[1]), (slow[0][inside], slow[1]))
+    assert torch.isinf(fast[1][:, :before]).all() and torch.isinf(fast[1][:, T - after:]).all()
+    assert torch.isfinite(fast[1][:, inside]).all()
+    # one query token per sequence (no offsets for the queries), and chunked prefill
+    q1 = torch.randn(4, Hq, D, generator=g, device=DEV).to(dtype)
+    same(*both(monkeypatch, lambda: mod(q1, k, v, 0.1, cu_seqlen_k=cu, return_lse=True)))
+    cq = torch.tensor([0, 7, 8, 58, 60], dtype=torch.int32, device=DEV)
+    qc = torch.randn(60, Hq, D, generator=g, device=DEV).to(dtype)
+    same(*both(monkeypatch, lambda: mod(qc, k, v, 0.1, cu_seqlen_k=cu, cu_seqlen_q=cq, return_lse=True)))
+
+
+@pytest.mark.parametrize("bs,fp8,dims", [(64, False, 3), (32, False, 4), (64, True, 3), (128, False, 3)])
+def test_paged(monkeypatch, bs, fp8, dims):
+    print(f"case bs={bs} fp8={fp8} dims={dims}", flush=True)
+    B, Hq, Hkv, D, ps = 3, 8, 2, 128, 16
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q = torch.randn(B, Hq, D, generator=g, device=DEV).to(torch.bfloat16)
+    pools = [torch.randn(100, ps, Hkv, D, generator=g, device=DEV).to(torch.float8_e4m3fn if fp8 else torch.bfloat16) for _ in range(2)]
+    table = torch.randperm(96, generator=g, device=DEV).to(torch.int32).view(3, 32)
+    lens = torch.tensor([512, 1, 300], dtype=torch.int32, device=DEV)
+    mod = New(Hq, 512, bs, 2, 3, num_kv_heads=Hkv).to(DEV)
+    if dims == 4:
+        q = q[:, None]
+    for lse in (False, True):
+        same(*both(monkeypatch, lambda: mod.paged_decode(q, *pools, table, lens, 0.1, return_lse=lse, k_scale=0.5)))
+
+
+def test_user_pattern_and_errors():
+    pat = torch.eye(4, dtype=torch.bool)
+    mod = SparseAttention(64, pat).to(DEV)
+    q, k, v = (torch.randn(1, 256, 2, 64, device=DEV, dtype=torch.bfloat16) for _ in range(3))
+    assert mod(q, k, v).shape == q.shape
+    with pytest.raises(AssertionError):
+        mod(torch.cat([q, q], 1), torch.cat([k, k], 1), torch.cat([v, v], 1))  # longer than the pattern
+    with pytest.raises(RuntimeError, match="ROCm"):
+        mod(q.cpu(), k.cpu(), v.cpu())
+    with pytest.raises(TypeError):
+        mod(q.double(), k.double(), v.double())
+    assert math.isfinite(mod(q[:, :0 + 1], k[:, :1], v[:, :1]).float().sum().item())
