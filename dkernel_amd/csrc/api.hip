@@ -36,11 +36,15 @@ static LutView view(const dk_lut &l) {
             l.max_row_entries, l.sub_block};
   v.order = l.row_order, v.pair_order = l.pair_order, v.order_sh = l.row_order_stride_h;
   v.uneven = l.uneven_heads != 0;
+  v.fixed_walk = l.fixed_walk != 0;
   return v;
 }
 static SeqView view(const dk_seqs &s) {
   SeqView v{s.batch, s.max_q_len, s.max_k_len, s.packed & 3, s.q_starts, s.q_ends, s.k_starts, s.k_ends};
-  v.any = s.k_ends ? s.k_ends : s.k_starts ? s.k_starts : s.q_ends ? s.q_ends : s.q_starts;
+  v.given = (s.q_starts ? 1 : 0) | (s.q_ends ? 2 : 0) | (s.k_starts ? 4 : 0) | (s.k_ends ? 8 : 0);
+  const int32_t *some = s.k_ends ? s.k_ends : s.k_starts;  // (the queries' arrays come with the keys')
+  for (const int32_t **a : {&v.q_starts, &v.q_ends, &v.k_starts, &v.k_ends})
+    if (!*a) *a = some;
   v.zero_outside = (s.packed & 4) && (s.q_starts || s.q_ends) ? 1 : 0;  // (without lengths every row holds a query)
   return v;
 }
@@ -121,7 +125,7 @@ static int make_bwd_params(const dk_bwd_args *a, BwdParams &p, bool &empty) {
   int rc = check_common(a->seqs, a->num_q_heads, a->num_kv_heads, a->head_dim, a->dtype, a->causal);
   if (rc) return rc;
   p.seqs = view(a->seqs);
-  DK_REQUIRE(!p.seqs.any && !a->seqs.packed,
+  DK_REQUIRE(!p.seqs.given && !a->seqs.packed,
              "Currently does not support paddings or variable length inputs in backward.");
   rc = check_lut(a->csr, "csr", a->num_q_heads, a->num_kv_heads);
   if (rc) return rc;
@@ -272,7 +276,7 @@ int dk_fwd_paged(const dk_fwd_args *a, const dk_paged_kv *pg) {
   int rc = make_fwd_params(a, p);
   if (rc) return rc;
   if (p.seqs.batch == 0 || p.seqs.max_q_len == 0) return DK_OK;
-  DK_REQUIRE(!p.seqs.packed && p.seqs.k_ends, "paged decode takes per-sequence lengths (dk_seqs arrays)");
+  DK_REQUIRE(!p.seqs.packed && (p.seqs.given & 8), "paged decode takes per-sequence lengths (dk_seqs arrays)");
   DK_REQUIRE(pg->kv_dtype == DK_FP8_E4M3 || ((pg->page_stride_k * (int64_t)elem_size(a->dtype)) % 16 == 0 &&
                                               (pg->page_stride_v * (int64_t)elem_size(a->dtype)) % 16 == 0),
              "page strides must keep rows 16-byte aligned");

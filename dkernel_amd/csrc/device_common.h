@@ -55,6 +55,7 @@ struct LutView {
   const int32_t *pair_order = nullptr;  // optional: ... or the rows 2u, 2u + 1 with u = pair_order[h * order_sh + i]
   int64_t order_sh = 0;
   int32_t uneven = 0;  // the heads hold clearly different numbers of entries
+  int32_t fixed_walk = 0;  // a row's entries are taken in one order, whatever the size of the launch
   int32_t rot = 0;     // set per launch (head_rotation): 0, or 1 + shift of grid_head()
 };
 
@@ -83,8 +84,9 @@ __device__ __forceinline__ int grid_head(const LutView &l) {
 
 struct SeqView {
   int32_t batch, max_q_len, max_k_len, packed;
+  // all readable or (given == 0) none: an array that the caller left out is replaced by another one
   const int32_t *q_starts, *q_ends, *k_starts, *k_ends;
-  const int32_t *any = nullptr;  // some array of the four above that is given; nullptr: none
+  int32_t given = 0;  // bits 0..3: the arrays above that are the caller's
   // packed inputs, optional: batch + 1 ints, entry b = work items (q tiles or pairs of q tiles) of
   // the sequences before b, written by a small kernel ahead of the one that reads it
   int32_t *item_offsets = nullptr;
@@ -144,17 +146,16 @@ struct SeqInfo {
 __device__ __forceinline__ SeqInfo load_seq_lane(const SeqView &s, int b, int causal) {
   SeqInfo r;
   r.b = b;
-  if (s.any) {
-    // An array that is not given stands for starts of 0 / ends at the token dimension (packed: for
-    // one query token per sequence).  Its load goes to one that is, so that the four leave together.
-    const int qs = (s.q_starts ? s.q_starts : s.any)[b], qe = (s.q_ends ? s.q_ends : s.any)[b];
-    const int ks = (s.k_starts ? s.k_starts : s.any)[b], ke = (s.k_ends ? s.k_ends : s.any)[b];
+  if (s.given) {
+    // (an array that is not given stands for starts of 0 / ends at the token dimension, packed: for
+    // one query token per sequence; the four loads leave together all the same)
+    const int qs = s.q_starts[b], qe = s.q_ends[b], ks = s.k_starts[b], ke = s.k_ends[b];
     // ends beyond the token dimension are clamped, so a bad length can never
     // make a kernel read or write outside the tensors
-    r.q_start = s.q_starts ? max(qs, 0) : s.packed ? b : 0;
-    r.q_len = (s.q_ends ? min(qe, s.max_q_len) : s.packed ? min(b + 1, s.max_q_len) : s.max_q_len) - r.q_start;
-    r.k_start = s.k_starts ? max(ks, 0) : 0;
-    r.k_len = (s.k_ends ? min(ke, s.max_k_len) : s.max_k_len) - r.k_start;
+    r.q_start = s.given & 1 ? max(qs, 0) : s.packed ? b : 0;
+    r.q_len = (s.given & 2 ? min(qe, s.max_q_len) : s.packed ? min(b + 1, s.max_q_len) : s.max_q_len) - r.q_start;
+    r.k_start = s.given & 4 ? max(ks, 0) : 0;
+    r.k_len = (s.given & 8 ? min(ke, s.max_k_len) : s.max_k_len) - r.k_start;
   } else {
     r.q_start = r.k_start = 0;
     r.q_len = s.max_q_len;
@@ -345,7 +346,7 @@ __device__ __forceinline__ void zero_rows_outside(const SeqView &s, const SeqInf
 // Packed inputs with SeqView::zero_outside: the log-sum-exps of the token rows that belong to no
 // sequence.  The workgroups of one work item per head (or head group) call it.
 __device__ __forceinline__ void lse_outside_packed(const SeqView &s, const RowView &lse, int h0, int nh, int tid, int nthreads) {
-  if (!lse.ptr || s.batch < 1 || !s.q_starts || !s.q_ends) return;
+  if (!lse.ptr || s.batch < 1 || (s.given & 3) != 3) return;
   const int lo = min(max(s.q_starts[0], 0), s.max_q_len), hi = max(min(s.q_ends[s.batch - 1], s.max_q_len), lo);
   const int outside = lo + s.max_q_len - hi;
   for (int i = tid; i < outside * nh; i += nthreads) {

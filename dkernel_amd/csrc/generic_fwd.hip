@@ -181,7 +181,7 @@ static int fwd_tiles_x(const FwdParams &p, int rows_per_wg) {
     // a sequence's queries touch at most ceil(q_len / BM) + 1 row blocks (they may start inside
     // one), and the ceilings add up to at most total / BM + batch
     blocks = cdiv(s.max_q_len, BM) + 2 * s.batch;
-  else if (s.any)
+  else if (s.given)
     blocks = cdiv(s.max_q_len, BM) + 1;
   else {
     const int past = p.causal ? s.max_k_len - s.max_q_len : 0;

@@ -660,7 +660,7 @@ int launch_mfma_f32_fwd(const FwdParams &p, hipStream_t stream) {
   int tiles;
   if (s.packed)
     tiles = cdiv(s.max_q_len, 64) + 2 * s.batch;  // as for the 16-bit forward: an upper bound over all sequences
-  else if (s.any)
+  else if (s.given)
     tiles = cdiv(s.max_q_len, 64) + 1;
   else {
     const int past = p.causal ? s.max_k_len - s.max_q_len : 0;

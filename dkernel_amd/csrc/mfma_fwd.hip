@@ -21,6 +21,7 @@
 // y = q tile with the longest rows first, z = batch.
 #include "common.h"
 #include "device_common.h"
+#include "fwd_split.h"
 #include "mfma_common.h"
 
 namespace dk {
@@ -57,8 +58,6 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   SeqInfo sq;
   int tile;
   const int tid = threadIdx.x, lane = tid & 63;
-  if (p.seqs.packed && p.seqs.zero_outside && blockIdx.y == 0)
-    lse_outside_packed(p.seqs, p.lse, grid_head(p.csr) * (RP ? 1 : G), RP ? 1 : G, tid, NT);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // scalar: row tests and head indices follow it
   int rb;
   int first_rb = 0, last_rb = 0;  // RP: table rows that hold queries of this sequence
@@ -66,6 +65,7 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
     // workgroup = table rows 2u and 2u + 1 of one head (one per wave pair); tiles_y counts pairs
     int u;
     if (p.seqs.packed) {
+      if (p.seqs.zero_outside && blockIdx.y == 0) lse_outside_packed(p.seqs, p.lse, grid_head(p.csr), 1, tid, NT);
       // the sequences share one token dimension: row pairs are counted through all of them (last
       // pair first: within a sequence the longest rows start first, as for unpacked inputs)
       int idx;
@@ -100,6 +100,8 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
              sq.past / 64;
       has_rows = tile >= 0 && tile < seq_row_blocks(sq, 64);
     } else {
+      if (p.seqs.packed && p.seqs.zero_outside && blockIdx.y == 0)
+        lse_outside_packed(p.seqs, p.lse, grid_head(p.csr) * G, G, tid, NT);
       has_rows = resolve_tile(p.seqs, p.causal, 64, 1, ty, blockIdx.z, sq, tile);
     }
     if (!has_rows) {
@@ -512,10 +514,53 @@ static FwdParams for_grid(FwdParams p, int gx, int gy) {
   return p;
 }
 
+// q tiles of `rows` tokens along grid.y (packed inputs: through all sequences), an upper bound
+static int tile_count(const SeqView &s, int causal, int rows) {
+  if (s.packed)
+    // a sequence's queries touch at most ceil(q_len / rows) + 1 tiles (they may start inside
+    // one), and the ceilings add up to at most total / rows + batch
+    return cdiv(s.max_q_len, rows) + 2 * s.batch;
+  if (s.given) return cdiv(s.max_q_len, rows) + 1;
+  const int past = causal ? s.max_k_len - s.max_q_len : 0;
+  return (past + s.max_q_len - 1) / rows - past / rows + 1;
+}
+
+// Whether the launch is better split along the keys (fwd_split.h): as long as its workgroups are all
+// resident at once (256 compute units x 3, 2 or 1 of them by tile width).  Measured, us, main kernel /
+// split, bf16: 32 / 8 heads of 128: 64 tokens 7.5 / 5.4, 333 tokens 14.3 / 9.9, 500 tokens (512 workgroups)
+// 18.0 / 12.6, 750 (768) 23.7 / 22.2, 1000 (1024) 30.7 / 31.0; 8 heads of 128: 2000 tokens (504) 24.9 /
+// 18.6, 3000 (752) 29.9 / 33.3; 12 heads of 64: 2000 tokens (756) 19.2 / 14.7, 4 x 750 (1152) 15.0 / 16.2;
+// 16 heads of 256: 500 tokens (256) 26.9 / 19.4, 4 x 130 (320) 14.4 / 16.4.
+template <int D>
+static bool split_pays(const FwdParams &p) {
+  constexpr int kResident = 256 * (D == 64 ? 3 : D == 128 ? 2 : 1);
+  if (p.csr.fixed_walk) return false;  // (the split changes the order of a row's sums)
+  return (int64_t)tile_count(p.seqs, p.causal, 32) * p.Hq * (p.seqs.packed ? 1 : p.seqs.batch) <= kResident;
+}
+
+template <typename T, int D, bool PAD, bool SUB>
+static int launch_split(const FwdParams &p_in, hipStream_t stream) {
+  // (all workgroups are resident at once: the table's own order does not matter, and the sequences of a
+  // packed launch are few enough for a workgroup to scan their lengths)
+  const int tiles = tile_count(p_in.seqs, p_in.causal, 32);
+  FwdParams p = for_grid(p_in, p_in.Hq, tiles);
+  p.seqs.item_offsets = nullptr;
+  constexpr int smem = SplitSmem<D>::kBytes;
+  DK_ALLOW_DYNAMIC_LDS((mfma_fwd_split_kernel<T, D, PAD, SUB>), smem);
+  hipLaunchKernelGGL((mfma_fwd_split_kernel<T, D, PAD, SUB>), dim3(p.Hq, tiles, p.seqs.packed ? 1 : p.seqs.batch),
+                     dim3(64 * kSplitWaves), smem, stream, p, tiles);
+  DK_HIP_CHECK(hipGetLastError());
+  return DK_OK;
+}
+
 // Several q heads per workgroup (G = 2 or 4 heads that share a kv head and a table row).
 template <typename T, int D, int G, bool PAD>
 static int launch_tdg(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
   constexpr int smem = 2 * FwdSmem<D>::kStage;
+  if (split_pays<D>(p)) {
+    DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+    return launch_split<T, D, PAD, false>(p, stream);
+  }
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, G, PAD, false>), smem);
   grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
@@ -533,13 +578,17 @@ template <typename T, int D, bool PAD>
 static int launch_row_pairs(const FwdParams &p, hipStream_t stream) {
   const SeqView &s = p.seqs;
   constexpr int smem = 2 * FwdSmem<D>::kStage;
+  if (split_pays<D>(p)) {
+    DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+    return launch_split<T, D, PAD, false>(p, stream);
+  }
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, 2, PAD, true>), smem);
   int pairs;
   if (s.packed) {
     // per sequence at most (ceil(q_len / 64) + 1) / 2 + 1 pairs; the ceilings add up to at most
     // total / 64 + batch
     pairs = (cdiv(s.max_q_len, 64) + s.batch) / 2 + 2 * s.batch;
-  } else if (s.any) {
+  } else if (s.given) {
     pairs = (cdiv(s.max_q_len, 64) + 1) / 2 + 1;  // a sequence's rows start anywhere inside a pair
   } else {
     const int past = p.causal ? s.max_k_len - s.max_q_len : 0;
@@ -569,6 +618,10 @@ static int launch_tdp(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
 template <typename T, int D, int G, bool PAD>
 static int launch_sub_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
   constexpr int smem = 2 * FwdSmem<D>::kStage;
+  if (split_pays<D>(p)) {
+    DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+    return launch_split<T, D, PAD, true>(p, stream);
+  }
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, G, PAD, false, true>), smem);
   grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
@@ -595,6 +648,10 @@ static int launch_sub(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
 template <typename T, int G, bool SUB>
 static int launch_256_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
   constexpr int smem = 2 * FwdSmem<256>::kStage;
+  if (split_pays<256>(p)) {
+    DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+    return launch_split<T, 256, true, SUB>(p, stream);
+  }
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, 256, G, true, false, SUB>), smem);
   grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
@@ -634,17 +691,7 @@ int launch_mfma_fwd(const FwdParams &p_in, int dtype, void *workspace, size_t wo
   if (p.seqs.packed && workspace && workspace_bytes >= mfma_fwd_workspace_bytes(p) && ((uintptr_t)workspace % 4) == 0)
     p.seqs.item_offsets = (int32_t *)workspace;
   const SeqView &s = p.seqs;
-  int tiles;
-  if (s.packed)
-    // a sequence's queries touch at most ceil(q_len / 64) + 1 row blocks (they may start inside
-    // one), and the ceilings add up to at most total / 64 + batch
-    tiles = cdiv(s.max_q_len, 64) + 2 * s.batch;
-  else if (s.any)
-    tiles = cdiv(s.max_q_len, 64) + 1;
-  else {
-    const int past = p.causal ? s.max_k_len - s.max_q_len : 0;
-    tiles = (past + s.max_q_len - 1) / 64 - past / 64 + 1;
-  }
+  int tiles = tile_count(s, p.causal, 64);
   if (p.csr.order && !s.packed) tiles = p.csr.num_rows;  // handed out in the table's order: all of them
   DK_REQUIRE(tiles <= 65535, "too many q tiles for one launch (%d)", tiles);
   dim3 grid(1, tiles, s.packed ? 1 : s.batch);

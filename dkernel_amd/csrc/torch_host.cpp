@@ -26,7 +26,7 @@ int (*fwd_fn)(const dk_fwd_args *) = nullptr;
 size_t (*fwd_bytes_fn)(const dk_fwd_args *) = nullptr;
 int (*fwd_paged_fn)(const dk_fwd_args *, const dk_paged_kv *) = nullptr;
 
-PyObject *k_max_seqlen, *k_causal, *k_group, *k_max_row, *k_uneven, *k_unsorted, *k_out, *k_inference;
+PyObject *k_max_seqlen, *k_causal, *k_group, *k_max_row, *k_uneven, *k_unsorted, *k_fixed, *k_out, *k_inference;
 
 struct Unsupported {};  // thrown by the helpers below, turned into None
 
@@ -86,7 +86,7 @@ const int32_t *lengths(const at::Tensor *t, int64_t n, int dev) {
 }
 
 void fill_lut(dk_lut &l, const at::Tensor &ptr, const at::Tensor &idx, int dev, int64_t rows, int64_t cols, int64_t sub,
-              int64_t group, int64_t max_row, bool uneven) {
+              int64_t group, int64_t max_row, bool uneven, bool fixed_walk) {
   need(ptr.dim() == 2 && ptr.scalar_type() == at::kInt && idx.scalar_type() == at::kInt && ptr.is_cuda() &&
        idx.is_cuda() && ptr.get_device() == dev && idx.get_device() == dev && ptr.stride(1) == 1);
   l = dk_lut{};
@@ -103,13 +103,13 @@ void fill_lut(dk_lut &l, const at::Tensor &ptr, const at::Tensor &idx, int dev, 
   l.num_heads = (int32_t)ptr.size(0), l.num_rows = (int32_t)ptr.size(1) - 1;
   l.block_rows = (int32_t)rows, l.block_cols = (int32_t)cols;
   l.group = (int32_t)group, l.max_row_entries = (int32_t)max_row, l.sub_block = (int32_t)sub;
-  l.uneven_heads = uneven;
+  l.uneven_heads = uneven, l.fixed_walk = fixed_walk;
 }
 
 // The module's table for these tensors: tables = (crow name, col name, rows, cols, masked crow name or
 // None, masked col name, tile, sub_block), names of entries of `buffers`.
 void choose_lut(dk_lut &l, PyObject *buffers, PyObject *tables, int64_t masked_max_row, bool masked_ok, int dev, int64_t group,
-                int64_t max_row, bool uneven) {
+                int64_t max_row, bool uneven, bool fixed_walk) {
   need(PyDict_Check(buffers) && PyTuple_Check(tables) && PyTuple_GET_SIZE(tables) == 8);
   const bool masked = masked_ok && PyTuple_GET_ITEM(tables, 4) != Py_None;
   const int at = masked ? 4 : 0;
@@ -117,13 +117,13 @@ void choose_lut(dk_lut &l, PyObject *buffers, PyObject *tables, int64_t masked_m
   need(crow && col);
   const int64_t rows = integer(PyTuple_GET_ITEM(tables, at + 2)), last = integer(PyTuple_GET_ITEM(tables, at + 3));
   fill_lut(l, tensor(crow), tensor(col), dev, rows, masked ? rows : last, masked ? last : 0, group, masked ? masked_max_row : max_row,
-           uneven);
+           uneven, fixed_walk);
 }
 
 // What the module's kwargs say
 struct Options {
   int64_t max_seqlen, group, max_row;
-  bool causal, uneven, unsorted;
+  bool causal, uneven, unsorted, fixed_walk;
   explicit Options(PyObject *kw) {
     need(PyDict_Check(kw) && !item(kw, k_out) && !item(kw, k_inference));
     PyObject *len = item(kw, k_max_seqlen), *g = item(kw, k_group), *row = item(kw, k_max_row), *c = item(kw, k_causal);
@@ -132,6 +132,7 @@ struct Options {
     causal = truth(c);
     uneven = truth(item(kw, k_uneven));
     unsorted = truth(item(kw, k_unsorted));
+    fixed_walk = truth(item(kw, k_fixed));
   }
 };
 
@@ -211,7 +212,8 @@ PyObject *forward_impl(PyObject *const *args) {
     const int64_t B = q.size(0), Lq = q.size(s), Lk = k.size(s), Hq = q.size(h), Hkv = k.size(h);
     need(B > 0 && Lq > 0 && k.size(0) == B && Lk <= opt.max_seqlen && !(opt.unsorted && Lq > 1));
     const bool padded = left || right;
-    choose_lut(a.csr, args[4], args[5], integer(args[6]), masked_ok, dev, opt.group, opt.max_row, opt.uneven && !(padded && Lq == 1));
+    choose_lut(a.csr, args[4], args[5], integer(args[6]), masked_ok, dev, opt.group, opt.max_row, opt.uneven && !(padded && Lq == 1),
+               opt.fixed_walk);
     check_heads(a.csr, Hq, Hkv);
     a.seqs.batch = (int32_t)B, a.seqs.max_q_len = (int32_t)Lq, a.seqs.max_k_len = (int32_t)Lk;
     if (padded) {
@@ -242,7 +244,7 @@ PyObject *forward_impl(PyObject *const *args) {
       need(T == k.size(0));
       cq = ck;
     }
-    choose_lut(a.csr, args[4], args[5], integer(args[6]), masked_ok, dev, opt.group, opt.max_row, opt.uneven && !single);
+    choose_lut(a.csr, args[4], args[5], integer(args[6]), masked_ok, dev, opt.group, opt.max_row, opt.uneven && !single, opt.fixed_walk);
     check_heads(a.csr, Hq, Hkv);
     a.seqs = dk_seqs{(int32_t)B, (int32_t)T, (int32_t)k.size(0), single ? 3 : want_lse ? 5 : 1, cq, cq ? cq + 1 : nullptr, ck, ck + 1};
     out = at::empty(q.sizes(), q.options());
@@ -277,7 +279,7 @@ PyObject *paged_impl(PyObject *const *args) {
   a.sm_scale = (float)scale;
   a.causal = 1, a.impl = (int32_t)integer(args[15]), a.head_dim = (int32_t)D;
   // (paged decode runs on the matrix-core kernels only: always the masked table of a module that has one)
-  choose_lut(a.csr, args[6], args[7], integer(args[8]), true, dev, integer(args[10]), integer(args[9]), false);
+  choose_lut(a.csr, args[6], args[7], integer(args[8]), true, dev, integer(args[10]), integer(args[9]), false, false);
   check_heads(a.csr, Hq, Hkv);
   a.seqs = dk_seqs{(int32_t)B, 1, (int32_t)std::min(table.size(1) * page, integer(args[11])), 0, nullptr, nullptr, nullptr,
                    lengths(&lens, B, dev)};
@@ -310,6 +312,10 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
     PyErr_SetString(PyExc_TypeError, "wrong number of arguments, or bind() was not called");
     return nullptr;
   }
+  // training takes the Python path: told without the cost of an exception
+  if (at::GradMode::is_enabled())
+    for (int i = 0; i < 3; ++i)
+      if (THPVariable_Check(args[i]) && THPVariable_Unpack(args[i]).requires_grad()) Py_RETURN_NONE;
   try {
     return Impl(args);
   } catch (const Unsupported &) {
@@ -353,6 +359,7 @@ PyMODINIT_FUNC PyInit__host() {
   k_max_seqlen = PyUnicode_InternFromString("max_seqlen"), k_causal = PyUnicode_InternFromString("causal");
   k_group = PyUnicode_InternFromString("lut_group"), k_max_row = PyUnicode_InternFromString("lut_max_row");
   k_uneven = PyUnicode_InternFromString("uneven_heads"), k_unsorted = PyUnicode_InternFromString("unsorted_rows");
+  k_fixed = PyUnicode_InternFromString("fixed_walk");
   k_out = PyUnicode_InternFromString("out"), k_inference = PyUnicode_InternFromString("inference");
   return PyModule_Create(&module);
 }

@@ -148,6 +148,9 @@ class SparseAttention(torch.nn.Module):
         # - the longest of a causal pattern -, then take the rows in the table's own order, longest
         # first, instead of starting the long ones when the rest of the chip has run out of work
         self.kwargs['unsorted_rows'] = _unsorted_rows(sparse_pattern)
+        # ... and every launch of theirs, however small, takes a row's blocks in one order: results then do
+        # not depend on how sequences are batched, whichever way the rows are handed out
+        self.kwargs['fixed_walk'] = self.kwargs['unsorted_rows']
 
         if not causal:
             # merged q tiles are a causal-only optimisation
@@ -295,7 +298,9 @@ class SparseAttention(torch.nn.Module):
         return_lse: also return the natural-log softmax normaliser, (batch,
             heads, seq) for 4-D inputs and (heads, total_tokens) for packed ones.
         """
-        if v is not None:
+        needs_grad = torch.is_grad_enabled() and any(
+            x is not None and x.requires_grad for x in (q, k, v))
+        if v is not None and not needs_grad:
             # inference on tensors that need no preparation: the same launch from C++ (None: not such a call)
             res = _lib.host().forward(q, k, v, sm_scale, self._buffers, self._kernel_tables, self.mask_lut_max_row,
                                       self.kwargs, self.seq_dim, cu_seqlen_k, cu_seqlen_q, left_paddings, seqlens,
@@ -326,8 +331,6 @@ class SparseAttention(torch.nn.Module):
                                          self.mask_tile, self.block_size),
                                         (self.masked_csc_ccol, self.masked_csc_row, self.mask_tile,
                                          self.mask_tile, self.block_size), self.mask_lut_max_row)
-        needs_grad = torch.is_grad_enabled() and any(
-            x is not None and x.requires_grad for x in (q, k, v))
         if needs_grad:
             output, lse = _sparse_attention.apply(
                 q, k, v, sm_scale, layout_csr, layout_csc,

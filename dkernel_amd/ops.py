@@ -88,20 +88,20 @@ _LUT_CACHE = {}
 
 
 def _lut(layout: Tuple[Tensor, Tensor, int, int], device, group: int = 1, max_row: int = 0,
-         longest_first: bool = False, uneven: bool = False) -> _lib.Lut:
+         longest_first: bool = False, uneven: bool = False, fixed_walk: bool = False) -> _lib.Lut:
     """dk_lut of a layout tuple.  The descriptor of a module's tables never changes, so it is
     built (and checked) once per (tables, hints) and copied from then on (a decode step's host
     time counts).  An entry keeps its two tensors alive, so their addresses cannot be handed to
     other tensors while the entry exists; the caller gets a copy of its own."""
     key = (layout[0].data_ptr(), layout[1].data_ptr(), layout[0].dtype, layout[1].dtype, layout[0].shape,
            layout[1].shape, layout[0].stride(), layout[1].stride(), tuple(int(x) for x in layout[2:]), device, group,
-           max_row, longest_first, uneven)
+           max_row, longest_first, uneven, fixed_walk)
     hit = _LUT_CACHE.get(key)
     if hit is None:
         if len(_LUT_CACHE) > 256:
             _LUT_CACHE.clear()
         lut = _make_lut(layout, device, group, max_row)
-        lut.uneven_heads = int(bool(uneven))
+        lut.uneven_heads, lut.fixed_walk = int(bool(uneven)), int(bool(fixed_walk))
         order = None
         if longest_first:
             # rows of every head by descending length (stable: equal lengths stay in index order),
@@ -206,7 +206,8 @@ def _forward(ctx, q: Tensor, k: Tensor, v: Tensor, sm_scale: float,
              lut_group: int = 1,
              lut_max_row: int = 0,
              uneven_heads: bool = False,
-             unsorted_rows: bool = False) -> Tuple[Tensor, Optional[Tensor]]:
+             unsorted_rows: bool = False,
+             fixed_walk: bool = False) -> Tuple[Tensor, Optional[Tensor]]:
     """Unpadded 4-D forward (training, prefill, single-token decode).
     Reference: dkernel/ops/sparse_attn_fwd.py:383-567.  `d_splits` is accepted
     and ignored (a Triton shared-memory workaround)."""
@@ -234,7 +235,7 @@ def _forward(ctx, q: Tensor, k: Tensor, v: Tensor, sm_scale: float,
     args.q, args.k, args.v, args.o = (_tensor4(x, hdim, seq_dim) for x in (q, k, v, o))
     args.lse = _rowvec(lse)
     args.csr = _lut(layout_csr, q.device, lut_group, lut_max_row, uneven=uneven_heads,
-                    longest_first=unsorted_rows and qlen > 1)
+                    longest_first=unsorted_rows and qlen > 1, fixed_walk=fixed_walk)
     args.seqs = _lib.Seqs(q.size(0), qlen, klen, 0, None, None, None, None)
     args.num_q_heads, args.num_kv_heads, args.head_dim = num_heads, num_kv_heads, q.size(-1)
     args.dtype, args.causal, args.impl = _DTYPES[q.dtype], int(bool(causal)), _impl
@@ -321,7 +322,8 @@ def padded_sparse_attn(q: Tensor, k: Tensor, v: Tensor, sm_scale: float,
                        lut_group: int = 1,
                        lut_max_row: int = 0,
                        uneven_heads: bool = False,
-                       unsorted_rows: bool = False):
+                       unsorted_rows: bool = False,
+                       fixed_walk: bool = False):
     """4-D inputs with left paddings and / or explicit sequence lengths; q has
     either one token per sequence (decode) or the same padded length as k.
     Reference: dkernel/ops/sparse_attn_inference.py:10-147.  Padding rows of
@@ -376,7 +378,7 @@ def padded_sparse_attn(q: Tensor, k: Tensor, v: Tensor, sm_scale: float,
     args.q, args.k, args.v, args.o = (_tensor4(x, hdim, seq_dim) for x in (q, k, v, out))
     args.lse = _rowvec(lse)
     args.csr = _lut(sparse_layout, dev, lut_group, lut_max_row, uneven=uneven_heads and q_len > 1,
-                    longest_first=unsorted_rows and q_len > 1)
+                    longest_first=unsorted_rows and q_len > 1, fixed_walk=fixed_walk)
     args.seqs = _lib.Seqs(batches, q_len, k_len, 4 if clear_padding else 0, q_starts.data_ptr(), q_ends.data_ptr(),
                           k_starts.data_ptr(), k_ends.data_ptr())
     args.num_q_heads, args.num_kv_heads, args.head_dim = num_heads, num_kv_heads, head_size
@@ -467,7 +469,8 @@ def varlen_sparse_attn(q: Tensor, k: Tensor, v: Tensor,
                        return_lse: bool = False,
                        lut_group: int = 1,
                        lut_max_row: int = 0,
-                       uneven_heads: bool = False):
+                       uneven_heads: bool = False,
+                       fixed_walk: bool = False):
     """Packed variable-length inputs (total_tokens, heads, head_dim) with
     cumulative sequence lengths.  Reference:
     dkernel/ops/sparse_attn_inference.py:150-287.  The query tokens of a
@@ -505,7 +508,8 @@ def varlen_sparse_attn(q: Tensor, k: Tensor, v: Tensor,
     args = _lib.FwdArgs()
     args.q, args.k, args.v, args.o = (_tensor3(x) for x in (q, k, v, out))
     args.lse = _rowvec(lse, (0, lse.stride(0), lse.stride(1))) if lse is not None else _rowvec(None)
-    args.csr = _lut(sparse_layout, dev, lut_group, lut_max_row, uneven=uneven_heads and not single_query)
+    args.csr = _lut(sparse_layout, dev, lut_group, lut_max_row, uneven=uneven_heads and not single_query,
+                    fixed_walk=fixed_walk)
     isz = cu_q.element_size()
     args.seqs = _lib.Seqs(batch_size, q.size(0), k.size(0), 3 if single_query else 5 if return_lse else 1,
                           cu_q.data_ptr(), cu_q.data_ptr() + isz, cu_k.data_ptr(), cu_k.data_ptr() + isz)
@@ -588,7 +592,8 @@ class _sparse_attention(torch.autograd.Function):
             res = varlen_sparse_attn(q, k, v, inf_kwargs["cu_seqlen_k"], inf_kwargs.get("cu_seqlen_q", None),
                                      sm_scale, layout_csr, max_seqlen=max_seqlen, causal=causal,
                                      out=kwargs.get("out", None), return_lse=return_lse, lut_group=lut_group, lut_max_row=lut_max_row,
-                                     uneven_heads=kwargs.get("uneven_heads", False))
+                                     uneven_heads=kwargs.get("uneven_heads", False),
+                                     fixed_walk=kwargs.get("fixed_walk", False))
             output, lse = res if return_lse else (res, None)
         else:
             assert k.size(seq_dim) <= max_seqlen, \
@@ -604,14 +609,16 @@ class _sparse_attention(torch.autograd.Function):
                                          out=kwargs.get("out", None),
                                          causal=causal, return_lse=return_lse, lut_group=lut_group,
                                          lut_max_row=lut_max_row, uneven_heads=kwargs.get("uneven_heads", False),
-                                         unsorted_rows=kwargs.get("unsorted_rows", False))
+                                         unsorted_rows=kwargs.get("unsorted_rows", False),
+                                         fixed_walk=kwargs.get("fixed_walk", False))
                 output, lse = res if return_lse else (res, None)
             else:
                 ctx.support_backward = True
                 ctx.message = ""
                 fwd_kwargs = {k_: v_ for k_, v_ in kwargs.items()
                               if k_ in ("inference", "out", "d_splits", "max_seqlen", "return_lse",
-                                        "causal", "split_qkv", "lut_group", "uneven_heads", "unsorted_rows")}
+                                        "causal", "split_qkv", "lut_group", "uneven_heads", "unsorted_rows",
+                                        "fixed_walk")}
                 fwd_kwargs["lut_max_row"] = lut_max_row
                 output, lse = _forward(ctx, q, k, v, sm_scale, layout_csr, seq_dim=seq_dim, **fwd_kwargs)
         return output, lse

@@ -32,7 +32,8 @@ enum dk_impl { DK_IMPL_AUTO = 0, DK_IMPL_GENERIC = 1, DK_IMPL_MFMA = 2 };
 int dk_version(void);              /* 10000*major + 100*minor + patch */
 const char *dk_last_error(void);   /* thread-local, never NULL */
 /* Kernels that the latest dk_fwd / dk_fwd_paged / dk_fwd_noalloc / dk_bwd call on this thread
- * launched, "name [template arguments]; " each, in launch order (thread-local, never NULL).  No
+ * launched, "name [template arguments]; " each, in launch order (thread-local, never NULL).  (A
+ * small forward launch runs its kernel's form that is split along the keys under the same name.)  No
  * counterpart in the reference; tests and bench.py use it to tell which path a call took. */
 const char *dk_last_kernels(void);
 
@@ -138,7 +139,9 @@ typedef struct dk_lut {
                            of one head per queue, so that no part of the chip is left with the
                            dense heads alone; with even heads (0) a fixed head per queue shares more
                            tiles through the caches.  Results do not depend on it. */
-  int32_t reserved;     /* 0 */
+  int32_t fixed_walk;   /* nonzero: dk_fwd takes a row's entries in the same order and by the same waves in
+                           launches of every size, so that prefill results do not depend bit by bit on how
+                           sequences are batched; 0: small launches may split a row along the keys */
   const int32_t *pair_order; /* optional, with row_order on the row table of dk_fwd / dk_bwd (same head
                                 stride): pair_order[h * row_order_stride_h + i] is the pair u of table
                                 rows (2u, 2u + 1) that the i-th work item of head h takes in the kernels
