@@ -197,19 +197,56 @@ __device__ __forceinline__ int seq_row_pairs(const SeqInfo &s) {
 
 // Packed inputs: the sequences share one token dimension and work items (q tiles, pairs of q
 // tiles) are numbered through all of them, count(sequence) items each.  Finds the sequence that
-// holds `item` and the item's index inside it; returns -1 beyond the last item.  The search runs
+// holds `item` and the item's index inside it; false beyond the last item.  The search runs
 // on the device (no host copy of the lengths), a wave at a time with every lane active and the
 // same `item`: each lane adds up the counts of batch / 64 consecutive sequences, a prefix sum over
 // the lanes names the lane whose chunk holds the item, and its sequences are searched the same
-// way, 64 at a time -- a few dependent loads whatever the batch size.
+// way, 64 at a time -- a few dependent loads whatever the batch size.  `info` is the sequence's
+// geometry (unchanged when there is none).
+//
+// Up to kWaveSequences sequences (one per lane) the search is one round trip to the lengths and
+// some forty vector instructions, and the geometry comes out of the lane that holds it; the
+// launcher then leaves out the kernel that counts the items ahead (item_offsets), which takes
+// 5 us on one compute unit and whose counts are bisected in log2(batch) + 3 dependent reads per
+// workgroup.  Two forward calls and the merge of their results, 16 heads of 128: 8 sequences of
+// 512 - 4096 tokens 168 -> 160 us, 24 of 50 - 400 tokens (12 heads) 92 -> 51; at 65 sequences the bisection stands.
+constexpr int kWaveSequences = 64;
+
+// Inclusive sum over the lanes of a wave (all of them active), on the VALU.
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1 (rows of 16 lanes; 0 comes in)
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15, into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31, into rows 2 and 3
+  return v;
+}
+
 template <typename Count>
-__device__ __forceinline__ int find_packed_sequence(const SeqView &s, int causal, int item, Count count,
-                                                    int &index_in_seq) {
+__device__ __forceinline__ bool find_packed_sequence(const SeqView &s, int causal, int item, Count count, SeqInfo &info,
+                                                     int &index_in_seq) {
+  const int lane = threadIdx.x & 63;
+  if (s.batch <= kWaveSequences) {
+    const SeqInfo mine = load_seq_lane(s, min(lane, s.batch - 1), causal);
+    const int n = lane < s.batch ? count(mine) : 0;
+    const int upto = wave_inclusive_sum(n);
+    const unsigned long long holders = __ballot(item < upto);
+    if (holders == 0) return false;
+    const int owner = __ffsll(holders) - 1;
+    auto from_owner = [&](int v) { return __builtin_amdgcn_readfirstlane(__shfl(v, owner)); };
+    index_in_seq = item - from_owner(upto - n);
+    info.b = owner;
+    info.q_start = from_owner(mine.q_start), info.q_len = from_owner(mine.q_len);
+    info.k_start = from_owner(mine.k_start), info.k_len = from_owner(mine.k_len);
+    info.past = from_owner(mine.past);
+    return true;
+  }
   if (s.item_offsets) {
     // the running item counts are there: bisect (wave-uniform addresses; zero-item sequences
     // share their successor's offset and are never the answer)
     const int32_t *off = s.item_offsets;
-    if (item >= __builtin_amdgcn_readfirstlane(off[s.batch])) return -1;
+    if (item >= __builtin_amdgcn_readfirstlane(off[s.batch])) return false;
     int lo = 0, hi = s.batch;  // off[lo] <= item < off[hi]
     while (hi - lo > 1) {
       const int mid = (lo + hi) >> 1;
@@ -219,9 +256,9 @@ __device__ __forceinline__ int find_packed_sequence(const SeqView &s, int causal
         hi = mid;
     }
     index_in_seq = item - __builtin_amdgcn_readfirstlane(off[lo]);
-    return lo;
+    info = load_seq(s, lo, causal);
+    return true;
   }
-  const int lane = threadIdx.x & 63;
   const int per_lane = (s.batch + 63) / 64;
   int mine = 0;
   // (indices clamped instead of branched around, eight at a time: the loads of a group are
@@ -238,35 +275,25 @@ __device__ __forceinline__ int find_packed_sequence(const SeqView &s, int causal
 #pragma unroll
     for (int i = 0; i < 8; ++i) mine += n[i];
   }
-  auto prefix = [&](int v) {  // inclusive sum over the lanes
-    for (int off = 1; off < 64; off <<= 1) {
-      const int t = __shfl_up(v, off);
-      if (lane >= off) v += t;
-    }
-    return v;
-  };
-  const int upto = prefix(mine);
+  const int upto = wave_inclusive_sum(mine);
   const unsigned long long holders = __ballot(item < upto);
-  if (holders == 0) return -1;
+  if (holders == 0) return false;
   const int owner = __ffsll(holders) - 1;                     // first lane whose chunk reaches past the item
   int before = __shfl(upto - mine, owner);                    // items of the chunks before it
-  if (per_lane == 1) {
-    index_in_seq = __builtin_amdgcn_readfirstlane(item - before);
-    return __builtin_amdgcn_readfirstlane(owner);
-  }
   for (int j0 = 0; j0 < per_lane; j0 += 64) {
     const int j = j0 + lane, b = owner * per_lane + j;
     const int n = (j < per_lane && b < s.batch) ? count(load_seq_lane(s, b, causal)) : 0;
-    const int upto2 = prefix(n);
+    const int upto2 = wave_inclusive_sum(n);
     const unsigned long long hit = __ballot(item < before + upto2);
     if (hit != 0) {
       const int l2 = __ffsll(hit) - 1;
       index_in_seq = __builtin_amdgcn_readfirstlane(item - before - __shfl(upto2 - n, l2));
-      return __builtin_amdgcn_readfirstlane(owner * per_lane + j0 + l2);
+      info = load_seq(s, __builtin_amdgcn_readfirstlane(owner * per_lane + j0 + l2), causal);
+      return true;
     }
     before += __shfl(upto2, 63);
   }
-  return -1;  // not reached: the owner's chunk holds the item
+  return false;  // not reached: the owner's chunk holds the item
 }
 
 // Fills SeqView::item_offsets: one workgroup of 1024 threads; count(sequence) as in
@@ -366,12 +393,9 @@ __device__ __forceinline__ bool resolve_tile(const SeqView &s, int causal, int b
     tile_in_seq = tile_x;
     return tile_x < seq_row_blocks(info, block_rows) * tiles_per_block;
   }
-  const int b = find_packed_sequence(
-      s, causal, tile_x, [&](const SeqInfo &t) { return seq_row_blocks(t, block_rows) * tiles_per_block; },
+  return find_packed_sequence(
+      s, causal, tile_x, [&](const SeqInfo &t) { return seq_row_blocks(t, block_rows) * tiles_per_block; }, info,
       tile_in_seq);
-  if (b < 0) return false;
-  info = load_seq(s, b, causal);
-  return true;
 }
 
 }  // namespace dk

@@ -69,11 +69,9 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
       // the sequences share one token dimension: row pairs are counted through all of them (last
       // pair first: within a sequence the longest rows start first, as for unpacked inputs)
       int idx;
-      const int b = find_packed_sequence(
-          p.seqs, p.causal, tiles_y - 1 - (int)blockIdx.y,
-          [](const SeqInfo &t) { return seq_row_pairs(t); }, idx);
-      if (b < 0) return;
-      sq = load_seq(p.seqs, b, p.causal);
+      if (!find_packed_sequence(
+              p.seqs, p.causal, tiles_y - 1 - (int)blockIdx.y, [](const SeqInfo &t) { return seq_row_pairs(t); }, sq, idx))
+        return;
       first_rb = sq.past / 64, last_rb = (sq.past + sq.q_len - 1) / 64;
       u = (first_rb >> 1) + idx;
     } else {
@@ -473,9 +471,9 @@ static int fwd_group(const FwdParams &p) {
   return 1;
 }
 
-// Packed inputs: running work-item counts of the sequences (q tiles, or pairs of q tiles for the
-// row-pair kernel), so that a workgroup finds its sequence by bisection instead of adding up the
-// sequences before it.
+// Packed inputs of more than kWaveSequences sequences: running work-item counts of the sequences (q tiles, or
+// pairs of q tiles for the row-pair kernel), so that a workgroup finds its sequence by bisection instead of
+// adding up the sequences before it.
 __global__ __launch_bounds__(1024) void packed_item_offsets_kernel(const SeqView s, int causal, int pairs,
                                                                    int32_t *out) {
   if (pairs)
@@ -485,7 +483,7 @@ __global__ __launch_bounds__(1024) void packed_item_offsets_kernel(const SeqView
 }
 
 static int launch_item_offsets(const FwdParams &p, bool pairs, hipStream_t stream) {
-  if (!p.seqs.packed || !p.seqs.item_offsets) return DK_OK;
+  if (!p.seqs.packed || !p.seqs.item_offsets || p.seqs.batch <= kWaveSequences) return DK_OK;
   SeqView s = p.seqs;
   s.item_offsets = nullptr;
   DK_NOTE_KERNEL("packed_item_offsets_kernel");
@@ -495,7 +493,7 @@ static int launch_item_offsets(const FwdParams &p, bool pairs, hipStream_t strea
   return DK_OK;
 }
 
-// Scratch the forward can use: batch + 1 ints for packed inputs.
+// Scratch the forward can use: batch + 1 ints for packed inputs (only filled and read beyond kWaveSequences).
 size_t mfma_fwd_workspace_bytes(const FwdParams &p) {
   return p.seqs.packed ? (((size_t)p.seqs.batch + 1) * sizeof(int32_t) + 15) / 16 * 16 : 0;
 }
