@@ -137,6 +137,17 @@ __device__ __forceinline__ int lut_head(const LutView &l, int h, int Hq, int Hkv
   return __builtin_amdgcn_readfirstlane(h / (Hq / Hkv));  // integer division runs on the VALU
 }
 
+// Masked 64 x 64 tiles (LutView::sub_block 16 or 32; bit (row part) * f + (key part) of an entry's mask, f =
+// 64 / sub_block): the mask sorted by 32 x 32 quadrants.  Quadrant (row half rh, key half kh) is the four bits at
+// 8 rh + 4 kh, bit (row / 16) * 2 + key / 16 of it -- 0: nothing attended, 15: everything.  The kernels multiply
+// quadrant by quadrant and leave out those without a bit: a tile table over blocks of 32 with vertical columns
+// or scattered blocks holds mostly tiles of one or two quadrants.
+__device__ __forceinline__ int tile_quadrants(int bits, int sub_block) {
+  if (sub_block == 32) return ((bits & 1) | (bits & 2) << 3 | (bits & 4) << 6 | (bits & 8) << 9) * 15;
+  // rows of four bits -> (row 0, row 1) of key half 0, (row 0, row 1) of key half 1, and the same of rows 2, 3
+  return (bits & 0xc3c3) | (bits & 0x3030) >> 2 | (bits & 0x0c0c) << 2;
+}
+
 struct SeqInfo {
   int b;
   int q_start, q_len, k_start, k_len, past;

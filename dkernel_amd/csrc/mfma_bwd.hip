@@ -222,6 +222,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     col_cur = col_next;
     const int key0 = col * 64 + kh * 32;  // first key of this wave's half
     if (col < 0 || key0 >= sq.k_len || (p.causal && key0 > row0 + 31)) return;
+    const int quad = SUB ? tile_quadrants(bits, p.csr.sub_block) >> (8 * rh + 4 * kh) & 15 : 15;
+    if (SUB && quad == 0) return;  // nothing attended (wave-uniform)
     constexpr int ks_ = stage * STAGE, vs_ = ks_ + TL::kBytes;  // byte offsets of this stage's K and V tiles
 
     floatx16 s, dp;
@@ -264,17 +266,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       }
     }
     if constexpr (SUB) {
-      // pattern blocks of the tile that this row does not attend: bit (row part) * f + (key part)
-      const int lb = p.csr.sub_block == 16 ? 4 : 5, f = 64 >> lb;
-      const int full = f == 4 ? 0xffff : 0xf;
-      if ((bits & full) != full) {  // wave-uniform
-        const int row_bits = bits >> (((rh * 32 + m) >> lb) * f);
+      if (quad != 15) {  // wave-uniform: blocks of 16, the quadrant is not attended as a whole
+        const int row_bits = quad >> (2 * (m >> 4));
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          // key kh 32 + 8 (r / 4) + 4 g + r % 4: the last two terms stay inside a part of >= 16 keys
-          const int key_part = (kh * 32 + (r >> 2) * 8) >> lb;
-          s[r] = ((row_bits >> key_part) & 1) ? s[r] : 0.f;
-        }
+        for (int r = 0; r < 16; ++r) s[r] = ((row_bits >> (r >> 3)) & 1) ? s[r] : 0.f;
       }
     }
 #pragma unroll
@@ -577,6 +572,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
     for (int kh = 0; kh < 2; ++kh) {  // the two 32-key halves of the block
       const int key0 = col * 64 + kh * 32;
       if (key0 >= sq.k_len || (p.causal && key0 > row0 + 31)) continue;  // nothing visible (wave-uniform)
+      const int quad = SUB ? tile_quadrants(bits, p.csr.sub_block) >> (8 * rh + 4 * kh) & 15 : 15;
+      if (SUB && quad == 0) continue;  // nothing attended
       constexpr int kRow32 = 32 * TL::kRowBytes;
       floatx16 s, dp;
 #pragma unroll
@@ -618,17 +615,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
         }
       }
       if constexpr (SUB) {
-        // pattern blocks of the tile that this row does not attend: bit (row part) * f + (key part)
-        const int lb = p.csr.sub_block == 16 ? 4 : 5, f = 64 >> lb;
-        const int full = f == 4 ? 0xffff : 0xf;
-        if ((bits & full) != full) {  // wave-uniform
-          const int row_bits = bits >> (((rh * 32 + m) >> lb) * f);
+        if (quad != 15) {  // wave-uniform: blocks of 16, the quadrant is not attended as a whole
+          const int row_bits = quad >> (2 * (m >> 4));
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            // key kh 32 + 8 (r / 4) + 4 g + r % 4: the last two terms stay inside a part of >= 16 keys
-            const int key_part = (kh * 32 + (r >> 2) * 8) >> lb;
-            s[r] = ((row_bits >> key_part) & 1) ? s[r] : 0.f;
-          }
+          for (int r = 0; r < 16; ++r) s[r] = ((row_bits >> (r >> 3)) & 1) ? s[r] : 0.f;
         }
       }
 #pragma unroll
@@ -704,6 +694,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   constexpr int KS = D / 16, DT = D / 32;
   using Loader = TileLoader<D, NT, PAD, S::kRows>;
   constexpr int LPT = 2 * Loader::kChunks + 1;  // load instructions per wave per step
+  // SUB: steps without an attended block are left out, and a pair of waves without a bit in its quadrant sits the
+  // step out (not at the 256-wide tile and the padded 128-wide one: slower, and one register too many).  Blocks of
+  // 32, local 16, vertical 8, 16 heads x 8000 tokens, forward and backward: 555 -> 473 us with the two other kernels.
+  constexpr bool kIdle = SUB && (D == 64 || (D == 128 && !PAD));
   // SUB: table entries are (row block, bit mask over the pattern blocks inside the 64 x 64 tile)
   constexpr int EW = SUB ? 2 : 1;  // ints per table entry
   extern __shared__ __align__(16) char smem[];
@@ -876,9 +870,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     constexpr bool kDp = decltype(role_tag)::value;
     int issued = 0, iq = 0, ido = 0;  // next step to request and its ring positions
     bool exact = true;                // every wave has issued exactly LPT load instructions per outstanding step
-    static_assert(S::kAhead == 2, "the first block's two steps are requested together");
+    static_assert(S::kAhead == 2, "two steps in flight ahead of the one that is worked on");
     int rb_next = 0;                  // q block of the next step to request (steps 2k and 2k + 1 share block k)
-    if (nstep > 0) {
+    // SUB: the steps are the 32-row halves of the listed tiles that attend anything.  ent: next entry to
+    // read; left: halves of block rb_next still to come; s0, s1: the steps that the loop works on next,
+    // each as 32-row tile << 8 | the masks of its two quadrants, 4 bits each.
+    int ent = 0, left = 0, bits_next = 0, s0 = 0, s1 = 0;
+    auto request_next = [&](int &s) -> bool {  // SUB: requests the next such step; false behind the last one
+      while (left == 0 && ent < e1 - e0) {
+        scalar_load2(rows + ent * EW, rows + ent * EW + 1, rb_next, bits_next);
+        ++ent;
+        bits_next = tile_quadrants(bits_next, p.csc.sub_block);
+        left = ((bits_next & 255) != 0 ? 1 : 0) | ((bits_next >> 8) != 0 ? 2 : 0);
+      }
+      if (left == 0) return false;
+      const int half = left & 1 ? 0 : 1;
+      left &= left - 1;
+      s = (rb_next * 2 + half) << 8 | (bits_next >> (8 * half) & 255);
+      exact = issue(rb_next, half, iq, ido) && exact;
+      iq = iq + 1 == S::kQStages ? 0 : iq + 1;
+      ido = ido + 1 == S::kDoStages ? 0 : ido + 1;
+      ++issued;
+      return true;
+    };
+    if constexpr (SUB) {
+      if (request_next(s0)) request_next(s1);
+    } else if (nstep > 0) {
       rb_next = scalar_load(rows);
       for (int i = 0; i < S::kAhead; ++i, ++issued) {
         exact = issue(rb_next, i, iq, ido) && exact;
@@ -900,12 +917,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     }
     floatx16 dp_prev;
     int cq = 0, cdo = 0, pq = 0;  // ring positions of step t (Q, dO) and of step t - 1 (Q)
-    int rbq = 0, bits = 0;        // S wave: q block (and its mask) of the current step
-    for (int t = 0; t < nstep; ++t) {
+    int rbq = 0;                  // S wave: q block (SUB: 32-row tile) of the current step
+    int quad = 15, quad_prev = 15;  // SUB: masks of this wave's quadrant of steps t and t - 1 (0: both waves of the pair idle)
+    for (int t = 0; SUB ? t < issued : t < nstep; ++t) {
       const int half = t & 1;
       wait_tiles_ahead<LPT>(exact ? issued - t - 1 : 0);
       __syncthreads();  // step t is visible, so is P of step t - 1; the stages of step t - 2 are free
-      if (issued < nstep) {
+      if constexpr (SUB) {
+        rbq = s0 >> 8;
+        quad = (s0 >> (4 * nh)) & 15;
+        s0 = s1;
+        request_next(s1);
+      } else if (issued < nstep) {
         if ((issued & 1) == 0) rb_next = scalar_load(rows + (issued >> 1) * EW);
         exact = issue(rb_next, issued & 1, iq, ido) && exact;
         iq = iq + 1 == S::kQStages ? 0 : iq + 1;
@@ -914,92 +937,84 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       }
       const char *qs_ = smem + S::kQ + cq * S::kTile, *dos_ = smem + S::kDo + cdo * S::kTile;
       if constexpr (!kDp) {
-        if (half == 0) {
-          if constexpr (SUB)
-            scalar_load2(rows + (t >> 1) * EW, rows + (t >> 1) * EW + 1, rbq, bits);
-          else
-            rbq = scalar_load(rows + (t >> 1));
+        if constexpr (!SUB) {
+          if (half == 0) rbq = scalar_load(rows + (t >> 1));
         }
-        const int pos0 = rbq * 64 + half * 32;  // first q position of this step
-        const float *lse_s = reinterpret_cast<const float *>(smem + S::kVec + cq * 256);
-        // S = Q K^T : rows = 32 q positions, cols = 32 keys
-        floatx16 sc;
+        if (!kIdle || quad != 0) {
+          const int pos0 = SUB ? rbq * 32 : rbq * 64 + half * 32;  // first q position of this step
+          const float *lse_s = reinterpret_cast<const float *>(smem + S::kVec + cq * 256);
+          // S = Q K^T : rows = 32 q positions, cols = 32 keys
+          floatx16 sc;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[r] = 0.f;
-        {
-          vec8 qa[KS];
+          for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+          {
+            vec8 qa[KS];
 #pragma unroll
-          for (int ks = 0; ks < KS; ++ks) qa[ks] = lds_read8<vec8>(qs_ + rd[ks]);
+            for (int ks = 0; ks < KS; ++ks) qa[ks] = lds_read8<vec8>(qs_ + rd[ks]);
 #pragma unroll
-          for (int ks = 0; ks < KS; ++ks) sc = M::mma(qa[ks], kvf[ks], sc);
-        }
-        // first dO^T operands do not depend on P
-        vec8 dot[DT];
+            for (int ks = 0; ks < KS; ++ks) sc = M::mma(qa[ks], kvf[ks], sc);
+          }
+          // first dO^T operands do not depend on P
+          vec8 dot[DT];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) dot[dt] = lds_read_tr8<vec8>(dos_ + tr[dt][0], dos_ + tr[dt][1]);
-        // P = exp2(S scale - lse log2e).  Rows outside the sequence arrive with lse = +inf
-        // (P = 0).  A row that saw no key has lse = -inf, but then every one of its entries
-        // here is masked by causality and the select below discards the infinite value, so no
-        // conversion is needed.  Masks are applied only in steps that need them (the diagonal
-        // block and the last, partial column block): wave-uniform choice between two loops.
-        const bool edge = (p.causal && (cb * 64 + nh * 32 + 31 > pos0)) || cb * 64 + 63 >= sq.k_len;
-        // last visible q-row offset test: key is visible to row pos iff key <= pos
-        const int kcmp = key_ok ? (p.causal ? key - pos0 : INT_MIN) : INT_MAX;  // masked iff kcmp > row offset
-        float *x = xbuf + (t & 1) * 1024;
+          for (int dt = 0; dt < DT; ++dt) dot[dt] = lds_read_tr8<vec8>(dos_ + tr[dt][0], dos_ + tr[dt][1]);
+          // P = exp2(S scale - lse log2e).  Rows outside the sequence arrive with lse = +inf
+          // (P = 0).  A row that saw no key has lse = -inf, but then every one of its entries
+          // here is masked by causality and the select below discards the infinite value, so no
+          // conversion is needed.  Masks are applied only in steps that need them (the diagonal
+          // block and the last, partial column block): wave-uniform choice between two loops.
+          const bool edge = (p.causal && (cb * 64 + nh * 32 + 31 > pos0)) || cb * 64 + 63 >= sq.k_len;
+          // last visible q-row offset test: key is visible to row pos iff key <= pos
+          const int kcmp = key_ok ? (p.causal ? key - pos0 : INT_MIN) : INT_MAX;  // masked iff kcmp > row offset
+          float *x = xbuf + (t & 1) * 1024;
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-          // registers 4*r4 .. +3 are q rows 8*r4 + 4g + {0..3} of the step
-          const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + r4 * 8 + g * 4);
-          const float lr[4] = {l4.x, l4.y, l4.z, l4.w};
+          for (int r4 = 0; r4 < 4; ++r4) {
+            // registers 4*r4 .. +3 are q rows 8*r4 + 4g + {0..3} of the step
+            const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + r4 * 8 + g * 4);
+            const float lr[4] = {l4.x, l4.y, l4.z, l4.w};
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            sc[r4 * 4 + i] = fast_exp2(fmaf(sc[r4 * 4 + i], p.scale_log2, -lr[i] * kLog2e));
-        }
-        if (edge) {
+            for (int i = 0; i < 4; ++i)
+              sc[r4 * 4 + i] = fast_exp2(fmaf(sc[r4 * 4 + i], p.scale_log2, -lr[i] * kLog2e));
+          }
+          if (edge) {
 #pragma unroll
-          for (int r = 0; r < 16; ++r) sc[r] = kcmp > (r >> 2) * 8 + g * 4 + (r & 3) ? 0.f : sc[r];
-        }
-        if constexpr (SUB) {
-          // pattern blocks of the tile that are not attended: bit (row part) * f + (key part); this
-          // lane's key is nh 32 + n, register r is q row half 32 + 8 (r / 4) + 4 g + r % 4
-          const int lb = p.csc.sub_block == 16 ? 4 : 5, f = 64 >> lb;
-          const int full = f == 4 ? 0xffff : 0xf;
-          if ((bits & full) != full) {  // wave-uniform
-            const int key_bits = bits >> ((nh * 32 + n) >> lb);
+            for (int r = 0; r < 16; ++r) sc[r] = kcmp > (r >> 2) * 8 + g * 4 + (r & 3) ? 0.f : sc[r];
+          }
+          if constexpr (SUB) {
+            if (quad != 15) {  // wave-uniform: blocks of 16, the quadrant is not attended as a whole
+              const int key_bits = quad >> (n >> 4);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int row_part = (half * 32 + (r >> 2) * 8) >> lb;
-              sc[r] = ((key_bits >> (row_part * f)) & 1) ? sc[r] : 0.f;
+              for (int r = 0; r < 16; ++r) sc[r] = ((key_bits >> (2 * (r >> 3))) & 1) ? sc[r] : 0.f;
             }
           }
-        }
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4)
-          *reinterpret_cast<float4 *>(x + (r4 * 64 + lane) * 4) =
-              make_float4(sc[r4 * 4], sc[r4 * 4 + 1], sc[r4 * 4 + 2], sc[r4 * 4 + 3]);
-        // dV^T += dO^T P
+          for (int r4 = 0; r4 < 4; ++r4)
+            *reinterpret_cast<float4 *>(x + (r4 * 64 + lane) * 4) =
+                make_float4(sc[r4 * 4], sc[r4 * 4 + 1], sc[r4 * 4 + 2], sc[r4 * 4 + 3]);
+          // dV^T += dO^T P
 #pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) {
-          float pf[8];
+          for (int t2 = 0; t2 < 2; ++t2) {
+            float pf[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) pf[i] = sc[t2 * 8 + i];
-          const vec8 pb = M::pack(pf);
+            for (int i = 0; i < 8; ++i) pf[i] = sc[t2 * 8 + i];
+            const vec8 pb = M::pack(pf);
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt) {
-            acc[dt] = M::mma(dot[dt], pb, acc[dt]);
-            if (t2 == 0) {
-              const int rowoff = 16 * TL::kRowBytes;
-              dot[dt] = lds_read_tr8<vec8>(dos_ + rowoff + tr[dt][0], dos_ + rowoff + tr[dt][1]);
+            for (int dt = 0; dt < DT; ++dt) {
+              acc[dt] = M::mma(dot[dt], pb, acc[dt]);
+              if (t2 == 0) {
+                const int rowoff = 16 * TL::kRowBytes;
+                dot[dt] = lds_read_tr8<vec8>(dos_ + rowoff + tr[dt][0], dos_ + rowoff + tr[dt][1]);
+              }
             }
           }
         }
       } else {
         // second half of step t - 1 first: it frees dp_prev for this step's dP
-        if (t > 0) finish_dk(t - 1, pq, dp_prev);
+        if (t > 0 && (!kIdle || quad_prev != 0)) finish_dk(t - 1, pq, dp_prev);
         // dP = dO V^T
 #pragma unroll
         for (int r = 0; r < 16; ++r) dp_prev[r] = 0.f;
-        {
+        if (!kIdle || quad != 0) {
           vec8 da[KS];
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) da[ks] = lds_read8<vec8>(dos_ + rd[ks]);
@@ -1007,13 +1022,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
           for (int ks = 0; ks < KS; ++ks) dp_prev = M::mma(da[ks], kvf[ks], dp_prev);
         }
       }
+      if constexpr (SUB) quad_prev = quad;
       pq = cq;
       cq = cq + 1 == S::kQStages ? 0 : cq + 1;
       cdo = cdo + 1 == S::kDoStages ? 0 : cdo + 1;
     }
     __syncthreads();  // P of the last step is visible
     if constexpr (kDp) {
-      if (nstep > 0) finish_dk(nstep - 1, pq, dp_prev);
+      if constexpr (SUB) {
+        if (issued > 0 && (!kIdle || quad_prev != 0)) finish_dk(issued - 1, pq, dp_prev);
+      } else {
+        if (nstep > 0) finish_dk(nstep - 1, pq, dp_prev);
+      }
     }
     };
     if (dp_wave)

@@ -53,7 +53,6 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
 
   static_assert(!RP || G == 2, "row pairs: two wave pairs, one q tile each");
   // SUB: table entries are (column, bit mask over the pattern blocks inside the 64 x 64 tile)
-  static_assert(!SUB || !RP, "sub-block masks: one q tile per workgroup");
   constexpr int EW = SUB ? 2 : 1;  // ints per table entry
   SeqInfo sq;
   int tile;
@@ -209,11 +208,20 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   int col_cur = 0, col_pending = 0;
   int bits_cur = 0, bits_pending = 0;  // SUB: the entry's mask, carried like the column
   int a_pos = e0, b_pos = emid, head_a = kEnd, head_b = kEnd, pend_a = 0, pend_b = 0, flg_cur = 0;
+  int hbits_a = 0, hbits_b = 0, pbits_a = 0, pbits_b = 0;  // RP with SUB: the masks of those entries
+  const bool second_row = RP && (wave >> 1) != 0;          // RP: this wave's table row is 2u + 1
   if constexpr (RP) {
-    if (a_pos < emid) head_a = scalar_load(cols + a_pos);
-    if (b_pos < e1) head_b = scalar_load(cols + b_pos);
-    if (a_pos + 1 < emid) pend_a = cols[a_pos + 1];
-    if (b_pos + 1 < e1) pend_b = cols[b_pos + 1];
+    if (a_pos < emid) head_a = scalar_load(cols + a_pos * EW);
+    if (b_pos < e1) head_b = scalar_load(cols + b_pos * EW);
+    if (a_pos + 1 < emid) pend_a = cols[(a_pos + 1) * EW];
+    if (b_pos + 1 < e1) pend_b = cols[(b_pos + 1) * EW];
+    if constexpr (SUB) {
+      if (a_pos < emid) hbits_a = scalar_load(cols + a_pos * EW + 1);
+      if (b_pos < e1) hbits_b = scalar_load(cols + b_pos * EW + 1);
+      if (a_pos + 1 < emid) pbits_a = cols[(a_pos + 1) * EW + 1];
+      if (b_pos + 1 < e1) pbits_b = cols[(b_pos + 1) * EW + 1];
+      bits_cur = second_row ? hbits_b : hbits_a;
+    }
     col_cur = min(head_a, head_b);
     flg_cur = (head_a == col_cur ? 1 : 0) | (head_b == col_cur ? 2 : 0);
     if (col_cur != kEnd) issue(col_cur, 0);
@@ -226,7 +234,7 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
     }
     if (e0 < e1) issue(col_cur, 0);
   }
-  auto block_step = [&](int e, auto stage_tag) {
+  auto block_step = [&](int e, auto stage_tag) __attribute__((always_inline)) {
     constexpr int stage = decltype(stage_tag)::value;
     const int col = col_cur;
     const int bits = bits_cur;
@@ -237,15 +245,24 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
       if (flg & 1) {
         ++a_pos;
         head_a = a_pos < emid ? __builtin_amdgcn_readfirstlane(pend_a) : kEnd;
-        if (a_pos + 1 < emid) pend_a = cols[a_pos + 1];
+        if (a_pos + 1 < emid) pend_a = cols[(a_pos + 1) * EW];
+        if constexpr (SUB) {
+          hbits_a = __builtin_amdgcn_readfirstlane(pbits_a);
+          if (a_pos + 1 < emid) pbits_a = cols[(a_pos + 1) * EW + 1];
+        }
       }
       if (flg & 2) {
         ++b_pos;
         head_b = b_pos < e1 ? __builtin_amdgcn_readfirstlane(pend_b) : kEnd;
-        if (b_pos + 1 < e1) pend_b = cols[b_pos + 1];
+        if (b_pos + 1 < e1) pend_b = cols[(b_pos + 1) * EW];
+        if constexpr (SUB) {
+          hbits_b = __builtin_amdgcn_readfirstlane(pbits_b);
+          if (b_pos + 1 < e1) pbits_b = cols[(b_pos + 1) * EW + 1];
+        }
       }
       const int col_next = min(head_a, head_b);
       flg_cur = (head_a == col_next ? 1 : 0) | (head_b == col_next ? 2 : 0);
+      if constexpr (SUB) bits_cur = second_row ? hbits_b : hbits_a;
       if (col_next != kEnd) issue(col_next, stage ^ 1);
       col_cur = col_next;
       if (!((flg >> __builtin_amdgcn_readfirstlane(wave >> 1)) & 1)) return;  // not in this wave pair's row
@@ -263,127 +280,151 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
     if (col < 0 || key0 >= sq.k_len || (p.causal && key0 > row0 + 31)) return;  // nothing visible (wave-uniform)
     constexpr int ks_ = stage * S::kStage, vs_ = ks_ + TL::kBytes;  // byte offsets of this stage's K and V tiles
 
-    // S^T = K Q^T : two 32-key tiles.  Operand reads run one tile ahead of the
-    // multiplies so that LDS latency is hidden behind the MFMA pipe.
-    floatx16 sacc[2];
+    // The 32-key tiles [N0, N1) of the block (SUB: q0, q1 are the masks of this wave's quadrants; without SUB always
+    // both tiles)
+    auto multiply = [&](auto first, auto end, int q0, int q1) __attribute__((always_inline)) {
+      constexpr int N0 = decltype(first)::value, N1 = decltype(end)::value;
+      // S^T = K Q^T : 32-key tiles.  Operand reads run one tile ahead of the
+      // multiplies so that LDS latency is hidden behind the MFMA pipe.
+      floatx16 sacc[2];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+      for (int nt = N0; nt < N1; ++nt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) sacc[nt][r] = 0.f;
-    // The scheduler barriers pin the order "issue a batch of LDS reads, then
-    // multiply the previous batch": left alone, the compiler sinks every read
-    // next to its MFMA and each multiply then waits out the LDS latency.
-    vec8 va[2][DT];
-    if constexpr (D == 256) {
-      // 256-wide tiles: the K operands of a 32-key tile are fetched in two batches of eight, so
-      // that they fit the register file next to the 128 accumulator registers
+        for (int r = 0; r < 16; ++r) sacc[nt][r] = 0.f;
+      // The scheduler barriers pin the order "issue a batch of LDS reads, then
+      // multiply the previous batch": left alone, the compiler sinks every read
+      // next to its MFMA and each multiply then waits out the LDS latency.
+      vec8 va[2][DT];
+      constexpr int vs0 = vs_ + N0 * 32 * TL::kRowBytes;
+      if constexpr (D == 256) {
+        // 256-wide tiles: the K operands of a 32-key tile are fetched in two batches of eight, so
+        // that they fit the register file next to the 128 accumulator registers
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
+        for (int nt = N0; nt < N1; ++nt)
 #pragma unroll
-        for (int kb = 0; kb < KS; kb += 8) {
-          vec8 ka[8];
+          for (int kb = 0; kb < KS; kb += 8) {
+            vec8 ka[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) ka[i] = lds_operand<vec8>(rd[kb + i] + ks_ + nt * 32 * TL::kRowBytes);
-          __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < 8; ++i) ka[i] = lds_operand<vec8>(rd[kb + i] + ks_ + nt * 32 * TL::kRowBytes);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int i = 0; i < 8; ++i) sacc[nt] = M::mma(ka[i], qf[kb + i], sacc[nt]);
+            for (int i = 0; i < 8; ++i) sacc[nt] = M::mma(ka[i], qf[kb + i], sacc[nt]);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) va[0][dt] = lds_operand_tr<vec8>(tr[dt][0] + vs0, tr[dt][1] + vs0);
+      } else {
+        vec8 ka[2][KS];
+#pragma unroll
+        for (int nt = N0; nt < N1; ++nt)
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) ka[nt][ks] = lds_operand<vec8>(rd[ks] + ks_ + nt * 32 * TL::kRowBytes);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) sacc[N0] = M::mma(ka[N0][ks], qf[ks], sacc[N0]);
+        // first V^T operands do not depend on the softmax: fetch them behind the multiplies
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) va[0][dt] = lds_operand_tr<vec8>(tr[dt][0] + vs0, tr[dt][1] + vs0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (N1 - N0 == 2) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) sacc[1] = M::mma(ka[1][ks], qf[ks], sacc[1]);
           __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) va[0][dt] = lds_operand_tr<vec8>(tr[dt][0] + vs_, tr[dt][1] + vs_);
-    } else {
-      vec8 ka[2][KS];
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) ka[0][ks] = lds_operand<vec8>(rd[ks] + ks_);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) ka[1][ks] = lds_operand<vec8>(rd[ks] + ks_ + 32 * TL::kRowBytes);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) sacc[0] = M::mma(ka[0][ks], qf[ks], sacc[0]);
-      // first V^T operands do not depend on the softmax: fetch them behind the multiplies
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) va[0][dt] = lds_operand_tr<vec8>(tr[dt][0] + vs_, tr[dt][1] + vs_);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) sacc[1] = M::mma(ka[1][ks], qf[ks], sacc[1]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+      }
 
-    // online softmax in the log2 domain.  Register r of tile nt is key
-    // 32nt + 8(r/4) + 4g + r%4.  m_run is a reference maximum that is only
-    // raised when a row's maximum grows by more than 2^8 (the accumulator
-    // and the row sum stay consistent with it, so the result is exact).
-    if constexpr (SUB) {
-      // pattern blocks of the tile that this row does not attend: bit (row part) * f + (key part)
-      const int lb = p.csr.sub_block == 16 ? 4 : 5, f = 64 >> lb;
-      const int full = f == 4 ? 0xffff : 0xf;
-      if ((bits & full) != full) {  // wave-uniform
-        const int row_part = ((wave & 1) * 32 + m) >> lb;
-        const int row_bits = bits >> (row_part * f);
+      // online softmax in the log2 domain.  Register r of tile nt is key
+      // 32nt + 8(r/4) + 4g + r%4.  m_run is a reference maximum that is only
+      // raised when a row's maximum grows by more than 2^8 (the accumulator
+      // and the row sum stay consistent with it, so the result is exact).
+      if constexpr (SUB) {
+        // blocks of 16: this row's share of a quadrant that is not attended as a whole
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
+        for (int nt = N0; nt < N1; ++nt) {
+          const int quad = nt == 0 ? q0 : q1;
+          if (quad == 15) continue;  // (wave-uniform; always so with blocks of 32)
+          const int row_bits = quad >> (2 * (m >> 4));
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sacc[nt][r] = ((row_bits >> (r >> 3)) & 1) ? sacc[nt][r] : -INFINITY;
+        }
+      }
+      const bool need_mask = (key0 + 63 >= sq.k_len) || (p.causal && key0 + 63 > row0);
+      if (need_mask) {
+        const int lim = p.causal ? min(pos, sq.k_len - 1) : sq.k_len - 1;  // last visible key of this row
+#pragma unroll
+        for (int nt = N0; nt < N1; ++nt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            // key 32 nt + 8 (r / 4) + 4 g + r % 4: the last two terms stay inside a part of >= 16 keys
-            const int key_part = (nt * 32 + (r >> 2) * 8) >> lb;
-            sacc[nt][r] = ((row_bits >> key_part) & 1) ? sacc[nt][r] : -INFINITY;
+            const int key = key0 + nt * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
+            sacc[nt][r] = key > lim ? -INFINITY : sacc[nt][r];
           }
       }
-    }
-    const bool need_mask = (key0 + 63 >= sq.k_len) || (p.causal && key0 + 63 > row0);
-    if (need_mask) {
-      const int lim = p.causal ? min(pos, sq.k_len - 1) : sq.k_len - 1;  // last visible key of this row
+      float mx;
+      if constexpr (N1 - N0 == 2) {
+        mx = max2(sacc[0][0], sacc[1][0]);
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
+        for (int r = 1; r < 16; ++r) mx = max3(mx, sacc[0][r], sacc[1][r]);
+      } else {
+        mx = max2(sacc[N0][0], sacc[N0][1]);
+#pragma unroll
+        for (int r = 2; r < 16; r += 2) mx = max3(mx, sacc[N0][r], sacc[N0][r + 1]);
+      }
+      mx = max_with_other_half(mx) * p.scale_log2;  // scale > 0: max commutes with it
+      if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {  // wave-uniform: some row needs a new reference
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = fast_exp2(m_run - (m_new == -INFINITY ? 0.f : m_new));
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+        m_run = m_new;
+      }
+      const float m_use = m_run == -INFINITY ? 0.f : m_run;
+      float psum = 0.f;
+#pragma unroll
+      for (int nt = N0; nt < N1; ++nt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int key = key0 + nt * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
-          sacc[nt][r] = key > lim ? -INFINITY : sacc[nt][r];
+          const float pv = fast_exp2(fmaf(sacc[nt][r], p.scale_log2, -m_use));
+          sacc[nt][r] = pv;
+          psum += pv;
         }
-    }
-    float mx = max2(sacc[0][0], sacc[1][0]);
-#pragma unroll
-    for (int r = 1; r < 16; ++r) mx = max3(mx, sacc[0][r], sacc[1][r]);
-    mx = max_with_other_half(mx) * p.scale_log2;  // scale > 0: max commutes with it
-    if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {  // wave-uniform: some row needs a new reference
-      const float m_new = fmaxf(m_run, mx);
-      const float alpha = fast_exp2(m_run - (m_new == -INFINITY ? 0.f : m_new));
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-      m_run = m_new;
-    }
-    const float m_use = m_run == -INFINITY ? 0.f : m_run;
-    float psum = 0.f;
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float pv = fast_exp2(fmaf(sacc[nt][r], p.scale_log2, -m_use));
-        sacc[nt][r] = pv;
-        psum += pv;
-      }
-    // fp32 sum of the unrounded probabilities (the LSE has to hold 1e-3); per-lane partial,
-    // the two half-waves are added once in the epilogue
-    l_run += psum;
+      // fp32 sum of the unrounded probabilities (the LSE has to hold 1e-3); per-lane partial,
+      // the two half-waves are added once in the epilogue
+      l_run += psum;
 
-    // O^T += V^T P^T : k-step (nt, t) covers keys 32nt + 16t + {4g..4g+3, 8+4g..8+4g+3}
+      // O^T += V^T P^T : k-step (nt, t) covers keys 32nt + 16t + {4g..4g+3, 8+4g..8+4g+3}
 #pragma unroll
-    for (int step = 0; step < 4; ++step) {
-      const int nt = step >> 1, t = step & 1;
-      float pf[8];
+      for (int step = 2 * N0; step < 2 * N1; ++step) {
+        const int nt = step >> 1, t = step & 1;
+        float pf[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) pf[i] = sacc[nt][t * 8 + i];
-      const vec8 pb = M::pack(pf);
-      if (step < 3) {
-        const int vrow = vs_ + ((step + 1) * 16) * TL::kRowBytes;
+        for (int i = 0; i < 8; ++i) pf[i] = sacc[nt][t * 8 + i];
+        const vec8 pb = M::pack(pf);
+        if (step + 1 < 2 * N1) {
+          const int vrow = vs_ + ((step + 1) * 16) * TL::kRowBytes;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) va[(step + 1) & 1][dt] = lds_operand_tr<vec8>(tr[dt][0] + vrow, tr[dt][1] + vrow);
+          for (int dt = 0; dt < DT; ++dt) va[(step + 1) & 1][dt] = lds_operand_tr<vec8>(tr[dt][0] + vrow, tr[dt][1] + vrow);
+        }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) oacc[dt] = M::mma(va[step & 1][dt], pb, oacc[dt]);
       }
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) oacc[dt] = M::mma(va[step & 1][dt], pb, oacc[dt]);
+    };
+    if constexpr (SUB) {
+      const int quads = tile_quadrants(bits, p.csr.sub_block) >> (8 * (wave & 1)), q0 = quads & 15, q1 = quads >> 4 & 15;
+      if constexpr (D == 256) {  // (one more copy of the block step spills)
+        if (q0 != 0 || q1 != 0) multiply(Const<0>{}, Const<2>{}, q0, q1);
+        return;
+      }
+      if (q0 != 0 && q1 != 0)
+        multiply(Const<0>{}, Const<2>{}, q0, q1);
+      else if (q0 != 0)
+        multiply(Const<0>{}, Const<1>{}, q0, q1);
+      else if (q1 != 0)
+        multiply(Const<1>{}, Const<2>{}, q0, q1);
+    } else {
+      multiply(Const<0>{}, Const<2>{}, 0, 0);
     }
   };
   if constexpr (RP) {
@@ -431,6 +472,7 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   template __global__ void mfma_fwd_kernel<T, D, 4, PAD, false>(const FwdParams, int);
 #define DK_INSTANTIATE_FWD_SUB(T, D, PAD)                                                    \
   template __global__ void mfma_fwd_kernel<T, D, 1, PAD, false, true>(const FwdParams, int); \
+  template __global__ void mfma_fwd_kernel<T, D, 2, PAD, true, true>(const FwdParams, int);  \
   template __global__ void mfma_fwd_kernel<T, D, 2, PAD, false, true>(const FwdParams, int); \
   template __global__ void mfma_fwd_kernel<T, D, 4, PAD, false, true>(const FwdParams, int);
 DK_INSTANTIATE_FWD_SUB(bf16_t, 128, false)
@@ -446,7 +488,8 @@ DK_INSTANTIATE_FWD_SUB(f16_t, 64, true)
 #define DK_INSTANTIATE_FWD_256(T)                                                            \
   template __global__ void mfma_fwd_kernel<T, 256, 2, true, false, false>(const FwdParams, int); \
   template __global__ void mfma_fwd_kernel<T, 256, 2, true, true, false>(const FwdParams, int);  \
-  template __global__ void mfma_fwd_kernel<T, 256, 1, true, false, true>(const FwdParams, int);
+  template __global__ void mfma_fwd_kernel<T, 256, 2, true, true, true>(const FwdParams, int);  \
+  template __global__ void mfma_fwd_kernel<T, 256, 2, true, false, true>(const FwdParams, int);
 DK_INSTANTIATE_FWD_256(bf16_t)
 DK_INSTANTIATE_FWD_256(f16_t)
 #undef DK_INSTANTIATE_FWD_256
@@ -572,15 +615,15 @@ static int launch_tdg(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
 
 // One head per workgroup: two adjacent q tiles of a head share a workgroup (and the K/V tiles
 // their rows have in common), which gives the two waves per SIMD that a single 64-row tile cannot.
-template <typename T, int D, bool PAD>
+template <typename T, int D, bool PAD, bool SUB = false>
 static int launch_row_pairs(const FwdParams &p, hipStream_t stream) {
   const SeqView &s = p.seqs;
   constexpr int smem = 2 * FwdSmem<D>::kStage;
   if (split_pays<D>(p)) {
     DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
-    return launch_split<T, D, PAD, false>(p, stream);
+    return launch_split<T, D, PAD, SUB>(p, stream);
   }
-  DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, 2, PAD, true>), smem);
+  DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, 2, PAD, true, SUB>), smem);
   int pairs;
   if (s.packed) {
     // per sequence at most (ceil(q_len / 64) + 1) / 2 + 1 pairs; the ceilings add up to at most
@@ -597,7 +640,7 @@ static int launch_row_pairs(const FwdParams &p, hipStream_t stream) {
   if (int rc = launch_item_offsets(p, true, stream)) return rc;
   const FwdParams pr = for_grid(p, p.Hq, pairs);
   DK_NOTE_KERNEL(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
-  hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 2, PAD, true>), dim3(p.Hq, pairs, s.packed ? 1 : s.batch), dim3(256), smem,
+  hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 2, PAD, true, SUB>), dim3(p.Hq, pairs, s.packed ? 1 : s.batch), dim3(256), smem,
                      stream, pr, pairs);
   DK_HIP_CHECK(hipGetLastError());
   return DK_OK;
@@ -612,7 +655,9 @@ static int launch_tdp(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
 }
 
 // Tables whose entries carry a bit mask over the pattern's 16- or 32-token blocks inside each
-// 64 x 64 tile: the plain kernel with the mask applied to S (no row pairs).
+// 64 x 64 tile: the same kernels, each wave multiplying its attended quadrants only.  Blocks of 32, local 16,
+// vertical 8, 8000 tokens: 32 / 8 heads of 128 191 -> 166 us, 16 heads in row pairs 150 -> 102 (whole tiles, one
+// row per workgroup before).
 template <typename T, int D, int G, bool PAD>
 static int launch_sub_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
   constexpr int smem = 2 * FwdSmem<D>::kStage;
@@ -637,7 +682,10 @@ static int launch_sub(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
   switch (group) {
     case 4: return launch_sub_g<T, D, 4, PAD>(p, grid, tiles_y, stream);
     case 2: return launch_sub_g<T, D, 2, PAD>(p, grid, tiles_y, stream);
-    default: return launch_sub_g<T, D, 1, PAD>(p, grid, tiles_y, stream);
+    // (global rows: the longest row is the run time, and shorter alone than in a pair: 12 heads of 64, 4 x 3000
+    // tokens 86 us against 101; a causal pattern, 16 heads of 128, 8000 tokens: 150 against 102)
+    default:
+      return p.csr.pair_order ? launch_sub_g<T, D, 1, PAD>(p, grid, tiles_y, stream) : launch_row_pairs<T, D, PAD, true>(p, stream);
   }
 }
 
@@ -663,11 +711,10 @@ static int launch_256_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t 
 
 template <typename T>
 static int launch_256(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
-  if (p.csr.sub_block)  // (with the mask registers two heads per workgroup would spill)
-    return launch_256_g<T, 1, true>(p, grid, tiles_y, stream);
-  // one head per workgroup: two adjacent q tiles share the workgroup and their K/V tiles
-  if (fwd_group(p) < 2) return launch_row_pairs<T, 256, true>(p, stream);
-  return launch_256_g<T, 2, false>(p, grid, tiles_y, stream);
+  // one head per workgroup: two adjacent q tiles share the workgroup and their K/V tiles (masked tiles too: one
+  // row of one head per workgroup spilled 700 bytes, 8 heads x 4000 tokens of blocks of 32 453 us, now 69)
+  if (fwd_group(p) < 2) return p.csr.sub_block ? launch_row_pairs<T, 256, true, true>(p, stream) : launch_row_pairs<T, 256, true>(p, stream);
+  return p.csr.sub_block ? launch_256_g<T, 2, true>(p, grid, tiles_y, stream) : launch_256_g<T, 2, false>(p, grid, tiles_y, stream);
 }
 
 // head dims below the tile width (64 or 128) run the zero-padded instantiation
