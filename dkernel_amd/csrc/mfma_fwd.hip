@@ -615,12 +615,13 @@ static int launch_tdg(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
 
 // One head per workgroup: two adjacent q tiles of a head share a workgroup (and the K/V tiles
 // their rows have in common), which gives the two waves per SIMD that a single 64-row tile cannot.
-template <typename T, int D, bool PAD, bool SUB = false>
-static int launch_row_pairs(const FwdParams &p, hipStream_t stream) {
+// (signature: the caller's, which names the kernel's instantiation in dk_last_kernels())
+template <typename T, int D, bool PAD, bool SUB>
+static int launch_row_pairs_as(const FwdParams &p, hipStream_t stream, const char *signature) {
   const SeqView &s = p.seqs;
   constexpr int smem = 2 * FwdSmem<D>::kStage;
   if (split_pays<D>(p)) {
-    DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+    note_kernel(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel", signature);
     return launch_split<T, D, PAD, SUB>(p, stream);
   }
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, 2, PAD, true, SUB>), smem);
@@ -639,11 +640,21 @@ static int launch_row_pairs(const FwdParams &p, hipStream_t stream) {
   DK_REQUIRE(pairs <= 65535, "too many q tiles for one launch (%d)", pairs);
   if (int rc = launch_item_offsets(p, true, stream)) return rc;
   const FwdParams pr = for_grid(p, p.Hq, pairs);
-  DK_NOTE_KERNEL(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+  note_kernel(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel", signature);
   hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 2, PAD, true, SUB>), dim3(p.Hq, pairs, s.packed ? 1 : s.batch), dim3(256), smem,
                      stream, pr, pairs);
   DK_HIP_CHECK(hipGetLastError());
   return DK_OK;
+}
+
+template <typename T, int D, bool PAD>
+static int launch_row_pairs(const FwdParams &p, hipStream_t stream) {
+  return launch_row_pairs_as<T, D, PAD, false>(p, stream, __PRETTY_FUNCTION__);
+}
+
+template <typename T, int D, bool PAD, bool SUB>
+static int launch_masked_row_pairs(const FwdParams &p, hipStream_t stream) {
+  return launch_row_pairs_as<T, D, PAD, SUB>(p, stream, __PRETTY_FUNCTION__);
 }
 
 template <typename T, int D, bool PAD>
@@ -685,7 +696,8 @@ static int launch_sub(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
     // (global rows: the longest row is the run time, and shorter alone than in a pair: 12 heads of 64, 4 x 3000
     // tokens 86 us against 101; a causal pattern, 16 heads of 128, 8000 tokens: 150 against 102)
     default:
-      return p.csr.pair_order ? launch_sub_g<T, D, 1, PAD>(p, grid, tiles_y, stream) : launch_row_pairs<T, D, PAD, true>(p, stream);
+      return p.csr.pair_order ? launch_sub_g<T, D, 1, PAD>(p, grid, tiles_y, stream)
+                              : launch_masked_row_pairs<T, D, PAD, true>(p, stream);
   }
 }
 
@@ -713,7 +725,8 @@ template <typename T>
 static int launch_256(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
   // one head per workgroup: two adjacent q tiles share the workgroup and their K/V tiles (masked tiles too: one
   // row of one head per workgroup spilled 700 bytes, 8 heads x 4000 tokens of blocks of 32 453 us, now 69)
-  if (fwd_group(p) < 2) return p.csr.sub_block ? launch_row_pairs<T, 256, true, true>(p, stream) : launch_row_pairs<T, 256, true>(p, stream);
+  if (fwd_group(p) < 2)
+    return p.csr.sub_block ? launch_masked_row_pairs<T, 256, true, true>(p, stream) : launch_row_pairs<T, 256, true>(p, stream);
   return p.csr.sub_block ? launch_256_g<T, 2, true>(p, grid, tiles_y, stream) : launch_256_g<T, 2, false>(p, grid, tiles_y, stream);
 }
 
