@@ -413,7 +413,10 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
     };
     if constexpr (SUB) {
       const int quads = tile_quadrants(bits, p.csr.sub_block) >> (8 * (wave & 1)), q0 = quads & 15, q1 = quads >> 4 & 15;
-      if constexpr (D == 256) {  // (one more copy of the block step spills)
+      // Whole tiles at the 256-wide tile (one more copy of the block step spills) and for single rows at the 64-wide
+      // one: those are the tables whose longest rows, nearly all whole tiles, are the run time (12 heads of 64,
+      // 4 x 3000 tokens with global blocks: 81 us by quadrants, 75.5 whole; 16 heads of 128: 144 and 151).
+      if constexpr (D == 256 || (D == 64 && G == 1)) {
         if (q0 != 0 || q1 != 0) multiply(Const<0>{}, Const<2>{}, q0, q1);
         return;
       }
@@ -693,11 +696,19 @@ static int launch_sub(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
   switch (group) {
     case 4: return launch_sub_g<T, D, 4, PAD>(p, grid, tiles_y, stream);
     case 2: return launch_sub_g<T, D, 2, PAD>(p, grid, tiles_y, stream);
-    // (global rows: the longest row is the run time, and shorter alone than in a pair: 12 heads of 64, 4 x 3000
-    // tokens 86 us against 101; a causal pattern, 16 heads of 128, 8000 tokens: 150 against 102)
-    default:
-      return p.csr.pair_order ? launch_sub_g<T, D, 1, PAD>(p, grid, tiles_y, stream)
-                              : launch_masked_row_pairs<T, D, PAD, true>(p, stream);
+    // Global rows: the longest row is the run time, and shorter alone than in a pair (12 heads of 64, 4 x 3000
+    // tokens: 75.5 us against 101).  Otherwise pairs (16 heads of 128, 8000 tokens: 98 us against 150), unless
+    // so few that compute units are left empty or with one pair and no second one to overlap it with:
+    // single rows / pairs, us, blocks of 32, 128-wide tile: 8 heads x 2500 tokens (160 pairs) 25.2 / 31.7, 12 x 2600
+    // (252) 27.1 / 35.9, 8 x 4800 (304) 36.1 / 44.4, 8 x 6000 (376) 47.5 / 55.0, 12 x 4000 (384) 40.7 / 45.0, 32 x
+    // 1500 (384) 31.6 / 30.9; 96 of 128 dims: 16 x 2300 (288) 29.5 / 34.8, 16 x 2800 (352) 42.3 / 38.8.  The 64-wide
+    // tile holds three waves per SIMD either way: 12 heads x 2500 tokens (240) 25.8 / 24.1.
+    default: {
+      const int64_t pairs = (int64_t)tile_count(p.seqs, p.causal, 128) * p.Hq * (p.seqs.packed ? 1 : p.seqs.batch);
+      return p.csr.pair_order || (D == 128 && pairs <= (PAD ? 320 : 384))
+                 ? launch_sub_g<T, D, 1, PAD>(p, grid, tiles_y, stream)
+                 : launch_masked_row_pairs<T, D, PAD, true>(p, stream);
+    }
   }
 }
 

@@ -23,8 +23,14 @@ pytestmark = pytest.mark.gpu
     (1, 2, 2, 330, 200, 16, torch.bfloat16, True, 0.04),
     (1, 3, 3, 575, 96, 32, torch.bfloat16, False, 0.05),
     (1, 4, 4, 2600, 120, 32, torch.float16, True, 0.03),   # (too large for the kernel of small launches)
+    (1, 8, 8, 2100, 128, 32, torch.bfloat16, True, 0.03),  # (single rows)
+    (4, 32, 32, 400, 128, 16, torch.bfloat16, False, 0.05),  # (row pairs)
+    (1, 2, 2, 650, 64, 32, torch.float16, "global", 0.05),   # (single rows, whole tiles)
+    (2, 2, 2, 450, 40, 16, torch.bfloat16, "global", 0.03),
+    (1, 2, 2, 650, 128, 32, torch.bfloat16, "global", 0.05),
 ])
 def test_sparse_tiles(B, Hq, Hkv, L, D, bs, dtype, causal, density):
+    long_rows, causal = causal == "global", causal is True
     print(f"case B={B} Hq={Hq} Hkv={Hkv} L={L} D={D} bs={bs} causal={causal} density={density}", flush=True)
     nb = -(-L // 64) * 64 // bs
     rng = np.random.default_rng(L)
@@ -32,6 +38,8 @@ def test_sparse_tiles(B, Hq, Hkv, L, D, bs, dtype, causal, density):
     pat |= np.eye(nb, dtype=bool)[None]
     if causal:
         pat = np.tril(pat)
+    if long_rows:
+        pat[:, :64 // bs] = True
     sm = 1 / math.sqrt(D)
     q, k, v, do = make_qkv(B, L, L, Hq, Hkv, D, dtype, with_do=True)
     qo, ko, vo = (x.float().requires_grad_() for x in (q, k, v))
