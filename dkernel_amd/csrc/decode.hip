@@ -81,13 +81,19 @@ __host__ __device__ inline int decode_row_units(int n, int unit_halves, int wave
 // captured launch, whose number is the same on every replay, starts afresh each time.  Arriving is
 // then one atomic addition (as a compare-and-swap loop, eight workgroups took 3 - 6 us), and nobody
 // ever waits for another workgroup.
+//
+// The addition releases the workgroup's partial (which its waves have written and waited for ahead of
+// a barrier) and acquires those of the workgroups that arrived before: the chain of additions orders
+// every partial before the reads of the last one, on whichever die it sits.  A step over one sequence
+// of 1000 keys: 7.9 us, 7.8 without the ordering; 8.6 with one more acquire in each of the last
+// workgroup's waves, which the barrier behind the addition makes redundant.
 using slot_t = unsigned long long;
 __device__ __forceinline__ void open_slot(slot_t *slot, slot_t seen, slot_t launch) {
   if ((seen >> 8) != launch)
     __hip_atomic_compare_exchange_strong(slot, &seen, launch << 8, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ bool arrive_last(slot_t *slot, int n) {
-  const slot_t before = __hip_atomic_fetch_add(slot, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const slot_t before = __hip_atomic_fetch_add(slot, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
   if ((int)(before & 255) + 1 != n) return false;
   __hip_atomic_store(slot, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return true;
@@ -469,8 +475,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
     }
   }
   if (groups <= 1) return;
-  // the partial's write-through stores have reached memory (a release fence would write back the whole
-  // L2 for the sake of stores that are not in it: 2 us)
+  // each wave's part of the partial has reached memory before the barrier (a barrier orders the waves'
+  // stores for their own compute unit; the addition behind it publishes them to the other dies)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   int *flag = reinterpret_cast<int *>(smem_all + wave_bytes - ratio * D * 2);  // wave 0's q copy: dead as well
