@@ -107,8 +107,10 @@ struct DecSmem {  // per wave: one 32-key half block of K and of V, plus q of th
   static int wave_bytes(int ratio) { return 2 * kHalf + ratio * D * 2; }
 };
 
-// workspace layout: [batch][Hq][max_groups + 1][D + 2] floats: a partial (O[D] unnormalised, max, sum)
-// per workgroup of the row; the last place of a kv group's first head holds the row's arrival slot
+// workspace layout, where rows are cut over several workgroups: [batch][Hq][max_groups + 1][D + 2] floats,
+// a partial (O[D] unnormalised, max, sum) per workgroup of the row; the last place of a kv group's first
+// head holds the row's arrival slot
+
 // Eight OCP e4m3 bytes -> eight elements of T.  Exact (e4m3 has 3 mantissa bits), so bf16 is
 // the upper half of the fp32 value and fp16 needs no rounding mode: one convert and one pack per
 // two elements.
@@ -550,8 +552,12 @@ bool decode_supported(const FwdParams &p, int dtype) {
          !p.seqs.zero_outside;  // (rows without a query are cleared by the prefill kernels only)
 }
 
+// Rows of one workgroup each use none of it; one place per q head then stands for "these arguments run the
+// decode kernels" (dk_fwd_workspace_bytes).  With two, steps over many rows of a single block no longer
+// fitted the fixed scratch of dk_fwd_noalloc (tests/test_decode_scratch.py).
 size_t decode_workspace_bytes(const FwdParams &p) {
-  return (size_t)p.seqs.batch * p.Hq * (decode_max_groups(p) + 1) * (mfma_tile_width(p.D) + 2) * sizeof(float);
+  const int groups = decode_max_groups(p), places = groups > 1 ? groups + 1 : 1;
+  return (size_t)p.seqs.batch * p.Hq * places * (mfma_tile_width(p.D) + 2) * sizeof(float);
 }
 
 template <typename T, int D, bool PAD, bool SUB, bool PAGED, bool KV8 = false>
