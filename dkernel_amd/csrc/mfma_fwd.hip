@@ -591,6 +591,7 @@ static int launch_split(const FwdParams &p_in, hipStream_t stream) {
   p.seqs.item_offsets = nullptr;
   constexpr int smem = SplitSmem<D>::kBytes;
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_split_kernel<T, D, PAD, SUB>), smem);
+  DK_NOTE_KERNEL(p.csr.rot ? "mfma_fwd_split_kernel, heads in rotation" : "mfma_fwd_split_kernel");
   hipLaunchKernelGGL((mfma_fwd_split_kernel<T, D, PAD, SUB>), dim3(p.Hq, tiles, p.seqs.packed ? 1 : p.seqs.batch),
                      dim3(64 * kSplitWaves), smem, stream, p, tiles);
   DK_HIP_CHECK(hipGetLastError());
@@ -601,10 +602,7 @@ static int launch_split(const FwdParams &p_in, hipStream_t stream) {
 template <typename T, int D, int G, bool PAD>
 static int launch_tdg(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
   constexpr int smem = 2 * FwdSmem<D>::kStage;
-  if (split_pays<D>(p)) {
-    DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
-    return launch_split<T, D, PAD, false>(p, stream);
-  }
+  if (split_pays<D>(p)) return launch_split<T, D, PAD, false>(p, stream);
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, G, PAD, false>), smem);
   grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
@@ -623,10 +621,7 @@ template <typename T, int D, bool PAD, bool SUB>
 static int launch_row_pairs_as(const FwdParams &p, hipStream_t stream, const char *signature) {
   const SeqView &s = p.seqs;
   constexpr int smem = 2 * FwdSmem<D>::kStage;
-  if (split_pays<D>(p)) {
-    note_kernel(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel", signature);
-    return launch_split<T, D, PAD, SUB>(p, stream);
-  }
+  if (split_pays<D>(p)) return launch_split<T, D, PAD, SUB>(p, stream);
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, 2, PAD, true, SUB>), smem);
   int pairs;
   if (s.packed) {
@@ -675,10 +670,7 @@ static int launch_tdp(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
 template <typename T, int D, int G, bool PAD>
 static int launch_sub_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
   constexpr int smem = 2 * FwdSmem<D>::kStage;
-  if (split_pays<D>(p)) {
-    DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
-    return launch_split<T, D, PAD, true>(p, stream);
-  }
+  if (split_pays<D>(p)) return launch_split<T, D, PAD, true>(p, stream);
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, G, PAD, false, true>), smem);
   grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
@@ -717,10 +709,7 @@ static int launch_sub(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
 template <typename T, int G, bool SUB>
 static int launch_256_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t stream) {
   constexpr int smem = 2 * FwdSmem<256>::kStage;
-  if (split_pays<256>(p)) {
-    DK_NOTE_KERNEL(p.csr.uneven && p.Hq > 1 ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
-    return launch_split<T, 256, true, SUB>(p, stream);
-  }
+  if (split_pays<256>(p)) return launch_split<T, 256, true, SUB>(p, stream);
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, 256, G, true, false, SUB>), smem);
   grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;

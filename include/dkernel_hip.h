@@ -32,8 +32,7 @@ enum dk_impl { DK_IMPL_AUTO = 0, DK_IMPL_GENERIC = 1, DK_IMPL_MFMA = 2 };
 int dk_version(void);              /* 10000*major + 100*minor + patch */
 const char *dk_last_error(void);   /* thread-local, never NULL */
 /* Kernels that the latest dk_fwd / dk_fwd_paged / dk_fwd_noalloc / dk_bwd call on this thread
- * launched, "name [template arguments]; " each, in launch order (thread-local, never NULL).  (A
- * small forward launch runs its kernel's form that is split along the keys under the same name.)  No
+ * launched, "name [template arguments]; " each, in launch order (thread-local, never NULL).  No
  * counterpart in the reference; tests and bench.py use it to tell which path a call took. */
 const char *dk_last_kernels(void);
 

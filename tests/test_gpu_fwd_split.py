@@ -8,7 +8,7 @@ import math
 import pytest
 import torch
 
-from dkernel_amd import LocalStrideSparseAttention
+from dkernel_amd import LocalStrideSparseAttention, _lib
 from helpers import LSE_TOL, TOL, assert_close, expand_heads, make_qkv, oracle_fwd
 from oracle import attention as OA
 from oracle import layout as OL
@@ -16,6 +16,10 @@ from oracle import layout as OL
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 New = LocalStrideSparseAttention.__wrapped__
+
+
+def _split_ran():
+    return _lib.lib().dk_last_kernels().startswith(b"mfma_fwd_split_kernel")
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,Lq,Lk,D,bs,dtype,causal", [
@@ -44,6 +48,7 @@ def test_against_the_oracle(B, Hq, Hkv, Lq, Lk, D, bs, dtype, causal):
     ro, rl = oracle_fwd(q.float(), k.float(), v.float(), bm, bs, sm, causal=causal)
     mod = New(Hq, Lr, bs, 2, 3, num_kv_heads=Hkv, causal=causal).to(DEV)
     out, lse = mod(q.to(DEV), k.to(DEV), v.to(DEV), sm, return_lse=True)
+    assert _split_ran() == (Lq <= 2048), _lib.lib().dk_last_kernels()
     assert_close("O", out, ro, **TOL)
     assert_close("LSE", lse, rl, atol=LSE_TOL, rtol=0)
 
@@ -58,9 +63,12 @@ def test_padded_and_packed(D, bs):
     mod = New(Hq, Lmax, bs, 2, 3, num_kv_heads=Hkv).to(DEV)
     dev = [x.to(DEV) for x in (q, k, v)]
     left = mod(*dev, sm, left_paddings=torch.tensor([Lmax - n for n in lens], dtype=torch.int32, device=DEV))
+    assert _split_ran()
     right, lse = mod(*dev, sm, seqlens=torch.tensor(lens, dtype=torch.int32, device=DEV), return_lse=True)
+    assert _split_ran()
     cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
     packed = mod(*(torch.cat([x[i, :n] for i, n in enumerate(lens)]) for x in dev), sm, cu_seqlen_k=cu)
+    assert _split_ran()
     for i, n in enumerate(lens):
         mask = torch.from_numpy(OA.sequence_token_mask(bm, bs, n, n))
         ro, rl = OA.dense_attention(*(x[i:i + 1, :n].float() for x in (q, k, v)), mask, sm)

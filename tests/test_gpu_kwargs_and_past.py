@@ -233,12 +233,17 @@ def test_last_kernels_names_the_path_taken():
     L, D = 256, 128
     sm = 1 / math.sqrt(D)
     try:
-        for Hq, Hkv, impl, want in ((8, 2, "auto", "mfma_fwd_kernel [T = dk::bf16_t, D = 128, G = 4, PAD = false]; "),
-                                    (2, 2, "auto", "mfma_fwd_kernel [T = dk::bf16_t, D = 128, PAD = false]; "),
-                                    (2, 2, "generic", "generic_fwd_kernel<128> [T = dk::bf16_t]; ")):
+        # (launches of up to 512 workgroups of 32 rows are split along the keys; two sequences of 1100 tokens
+        # with 8 q heads are 560)
+        main, split = "mfma_fwd_kernel [T = dk::bf16_t, D = 128, ", "mfma_fwd_split_kernel [T = dk::bf16_t, D = 128, "
+        for B, n, Hq, Hkv, impl, want in ((1, L, 8, 2, "auto", split + "PAD = false, SUB = false]; "),
+                                          (1, L, 2, 2, "auto", split + "PAD = false, SUB = false]; "),
+                                          (2, 1100, 8, 2, "auto", main + "G = 4, PAD = false]; "),
+                                          (2, 1100, 8, 8, "auto", main + "PAD = false]; "),
+                                          (1, L, 2, 2, "generic", "generic_fwd_kernel<128> [T = dk::bf16_t]; ")):
             ops.set_impl(impl)
-            q, k, v = (x.to(DEV) for x in make_qkv(1, L, L, Hq, Hkv, D, torch.bfloat16))
-            New(Hq, L, 64, 2, 3, num_kv_heads=Hkv).to(DEV)(q, k, v, sm)
+            q, k, v = (x.to(DEV) for x in make_qkv(B, n, n, Hq, Hkv, D, torch.bfloat16))
+            New(Hq, n, 64, 2, 3, num_kv_heads=Hkv).to(DEV)(q, k, v, sm)
             assert lib.dk_last_kernels().decode() == want
         q.requires_grad_()
         New(2, L, 64, 2, 3).to(DEV)(q, k, v, sm).sum().backward()
