@@ -504,6 +504,8 @@ def varlen_sparse_attn(q: Tensor, k: Tensor, v: Tensor,
     out = out if out is not None else q.new_empty(q.shape)
     # (the kernels write -inf where a token belongs to no sequence: bit 2 of dk_seqs.packed)
     lse = torch.empty((num_heads, q.size(0)), dtype=torch.float32, device=dev) if return_lse else None
+    if lse is not None and batch_size == 0:
+        lse.fill_(float("-inf"))  # no sequence, so no kernel either
 
     args = _lib.FwdArgs()
     args.q, args.k, args.v, args.o = (_tensor3(x) for x in (q, k, v, out))

@@ -98,6 +98,22 @@ def test_packed(monkeypatch, Hq, Hkv, dtype, D):
     same(*both(monkeypatch, lambda: mod(qc, k, v, 0.1, cu_seqlen_k=cu, cu_seqlen_q=cq, return_lse=True)))
 
 
+def test_packed_tokens_without_any_sequence(monkeypatch):
+    """Offsets of no sequence at all launch nothing; the log-sum-exps still read -inf, whatever the
+    memory held before."""
+    T, H, D = 300, 2, 64
+    q, k, v = (torch.randn(T, H, D, device=DEV, dtype=torch.bfloat16) for _ in range(3))
+    mod, cu = New(H, 512, 64, 2, 3).to(DEV), torch.zeros(1, dtype=torch.int32, device=DEV)
+    empty = torch.empty
+
+    def poisoned(*a, **kw):
+        x = empty(*a, **kw)
+        return x.fill_(float("nan")) if x.is_floating_point() else x
+    monkeypatch.setattr(torch, "empty", poisoned)
+    lse = mod(q, k, v, cu_seqlen_k=cu, return_lse=True)[1]
+    assert lse.shape == (H, T) and torch.isneginf(lse).all()
+
+
 @pytest.mark.parametrize("bs,fp8,dims", [(64, False, 3), (32, False, 4), (64, True, 3), (128, False, 3)])
 def test_paged(monkeypatch, bs, fp8, dims):
     print(f"case bs={bs} fp8={fp8} dims={dims}", flush=True)
