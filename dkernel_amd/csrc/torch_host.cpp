@@ -8,6 +8,11 @@
 // type, gradients, tables in an order of their own, wrong arguments of any kind): the caller then takes
 // the path in ops.py, which handles it or raises.  The C ABI is reached through the addresses that
 // bind() gets from the library that ops.py has loaded.
+//
+// Everything that comes from Python objects is read first; allocations and the launch run without the
+// interpreter lock (Unlocked), as they do through torch's own bindings and ctypes: threads that serve on
+// several streams do not wait for each other's launches, nor a launch into a full queue for a host callback
+// that needs the lock.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -17,6 +22,7 @@
 
 #include <cmath>
 #include <cstdlib>
+#include <optional>
 
 #include "../../include/dkernel_hip.h"
 
@@ -29,6 +35,13 @@ int (*fwd_paged_fn)(const dk_fwd_args *, const dk_paged_kv *) = nullptr;
 PyObject *k_max_seqlen, *k_causal, *k_group, *k_max_row, *k_uneven, *k_unsorted, *k_fixed, *k_out, *k_inference;
 
 struct Unsupported {};  // thrown by the helpers below, turned into None
+
+struct Unlocked {  // the interpreter lock is released while this lives
+  PyThreadState *state = PyEval_SaveThread();
+  Unlocked() = default;
+  Unlocked(const Unlocked &) = delete;
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
 
 const at::Tensor &tensor(PyObject *o) {
   if (!THPVariable_CheckExact(o)) throw Unsupported{};
@@ -106,9 +119,14 @@ void fill_lut(dk_lut &l, const at::Tensor &ptr, const at::Tensor &idx, int dev, 
   l.uneven_heads = uneven, l.fixed_walk = fixed_walk;
 }
 
+// A table's tensors, held across the launch: another thread may give the module other ones meanwhile.
+struct Table {
+  at::Tensor ptr, idx;
+};
+
 // The module's table for these tensors: tables = (crow name, col name, rows, cols, masked crow name or
 // None, masked col name, tile, sub_block), names of entries of `buffers`.
-void choose_lut(dk_lut &l, PyObject *buffers, PyObject *tables, int64_t masked_max_row, bool masked_ok, int dev, int64_t group,
+Table choose_lut(dk_lut &l, PyObject *buffers, PyObject *tables, int64_t masked_max_row, bool masked_ok, int dev, int64_t group,
                 int64_t max_row, bool uneven, bool fixed_walk) {
   need(PyDict_Check(buffers) && PyTuple_Check(tables) && PyTuple_GET_SIZE(tables) == 8);
   const bool masked = masked_ok && PyTuple_GET_ITEM(tables, 4) != Py_None;
@@ -116,8 +134,10 @@ void choose_lut(dk_lut &l, PyObject *buffers, PyObject *tables, int64_t masked_m
   PyObject *crow = item(buffers, PyTuple_GET_ITEM(tables, at)), *col = item(buffers, PyTuple_GET_ITEM(tables, at + 1));
   need(crow && col);
   const int64_t rows = integer(PyTuple_GET_ITEM(tables, at + 2)), last = integer(PyTuple_GET_ITEM(tables, at + 3));
-  fill_lut(l, tensor(crow), tensor(col), dev, rows, masked ? rows : last, masked ? last : 0, group, masked ? masked_max_row : max_row,
-           uneven, fixed_walk);
+  Table t{tensor(crow), tensor(col)};
+  fill_lut(l, t.ptr, t.idx, dev, rows, masked ? rows : last, masked ? last : 0, group, masked ? masked_max_row : max_row, uneven,
+           fixed_walk);
+  return t;
 }
 
 // What the module's kwargs say
@@ -190,7 +210,7 @@ PyObject *forward_impl(PyObject *const *args) {
   const Options opt(args[7]);
   const at::Tensor *cu_k = optional_tensor(args[9]), *cu_q = optional_tensor(args[10]);
   const at::Tensor *left = optional_tensor(args[11]), *right = optional_tensor(args[12]);
-  const bool want_lse = truth(args[13]);
+  const bool want_lse = truth(args[13]), use_workspace = truth(args[15]);
   const int64_t impl = integer(args[14]);
   const int dev = q.get_device();
   const int64_t D = q.size(-1);
@@ -203,6 +223,8 @@ PyObject *forward_impl(PyObject *const *args) {
   const bool masked_ok = scale > 0 && impl != DK_IMPL_GENERIC && a.dtype != DK_F32 && D % 8 == 0 && D <= 256 &&
                          rows_aligned(q) && rows_aligned(k) && rows_aligned(v);
   at::Tensor out, lse;
+  Table table;
+  std::optional<Unlocked> unlocked;
 
   if (q.dim() == 4) {
     need(!cu_k && !cu_q);
@@ -212,8 +234,8 @@ PyObject *forward_impl(PyObject *const *args) {
     const int64_t B = q.size(0), Lq = q.size(s), Lk = k.size(s), Hq = q.size(h), Hkv = k.size(h);
     need(B > 0 && Lq > 0 && k.size(0) == B && Lk <= opt.max_seqlen && !(opt.unsorted && Lq > 1));
     const bool padded = left || right;
-    choose_lut(a.csr, args[4], args[5], integer(args[6]), masked_ok, dev, opt.group, opt.max_row, opt.uneven && !(padded && Lq == 1),
-               opt.fixed_walk);
+    table = choose_lut(a.csr, args[4], args[5], integer(args[6]), masked_ok, dev, opt.group, opt.max_row,
+                       opt.uneven && !(padded && Lq == 1), opt.fixed_walk);
     check_heads(a.csr, Hq, Hkv);
     a.seqs.batch = (int32_t)B, a.seqs.max_q_len = (int32_t)Lq, a.seqs.max_k_len = (int32_t)Lk;
     if (padded) {
@@ -225,6 +247,7 @@ PyObject *forward_impl(PyObject *const *args) {
         a.seqs.packed = 4;  // the kernels clear the padding rows
       }
     }
+    unlocked.emplace();
     out = at::empty(q.sizes(), q.options());
     if (want_lse) lse = at::empty({B, Hq, Lq}, q.options().dtype(at::kFloat));
     a.q = view(q, 0, h, s), a.k = view(k, 0, h, s), a.v = view(v, 0, h, s), a.o = view(out, 0, h, s);
@@ -244,16 +267,19 @@ PyObject *forward_impl(PyObject *const *args) {
       need(T == k.size(0));
       cq = ck;
     }
-    choose_lut(a.csr, args[4], args[5], integer(args[6]), masked_ok, dev, opt.group, opt.max_row, opt.uneven && !single, opt.fixed_walk);
+    table = choose_lut(a.csr, args[4], args[5], integer(args[6]), masked_ok, dev, opt.group, opt.max_row, opt.uneven && !single,
+                       opt.fixed_walk);
     check_heads(a.csr, Hq, Hkv);
     a.seqs = dk_seqs{(int32_t)B, (int32_t)T, (int32_t)k.size(0), single ? 3 : want_lse ? 5 : 1, cq, cq ? cq + 1 : nullptr, ck, ck + 1};
+    unlocked.emplace();
     out = at::empty(q.sizes(), q.options());
     if (want_lse) lse = at::empty({Hq, T}, q.options().dtype(at::kFloat));
     a.q = view(q, -1, 1, 0), a.k = view(k, -1, 1, 0), a.v = view(v, -1, 1, 0), a.o = view(out, -1, 1, 0);
     if (want_lse) a.lse = dk_rowvec{static_cast<float *>(lse.data_ptr()), 0, T, 1};
     a.num_q_heads = (int32_t)Hq, a.num_kv_heads = (int32_t)Hkv;
   }
-  const size_t bytes = launch(a, q, truth(args[15]));
+  const size_t bytes = launch(a, q, use_workspace);
+  unlocked.reset();
   return result(out, lse, bytes);
 }
 
@@ -279,12 +305,21 @@ PyObject *paged_impl(PyObject *const *args) {
   a.sm_scale = (float)scale;
   a.causal = 1, a.impl = (int32_t)integer(args[15]), a.head_dim = (int32_t)D;
   // (paged decode runs on the matrix-core kernels only: always the masked table of a module that has one)
-  choose_lut(a.csr, args[6], args[7], integer(args[8]), true, dev, integer(args[10]), integer(args[9]), false, false);
+  const Table lut_tensors = choose_lut(a.csr, args[6], args[7], integer(args[8]), true, dev, integer(args[10]), integer(args[9]),
+                                       false, false);
   check_heads(a.csr, Hq, Hkv);
   a.seqs = dk_seqs{(int32_t)B, 1, (int32_t)std::min(table.size(1) * page, integer(args[11])), 0, nullptr, nullptr, nullptr,
                    lengths(&lens, B, dev)};
+  const bool want_lse = truth(args[12]);
+  const double ks = PyFloat_AsDouble(args[13]), vs = PyFloat_AsDouble(args[14]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    throw Unsupported{};
+  }
+  std::optional<Unlocked> unlocked;
+  unlocked.emplace();
   at::Tensor out = at::empty(q.sizes(), q.options()), lse;
-  if (truth(args[12])) {
+  if (want_lse) {
     lse = at::empty({B, Hq, 1}, q.options().dtype(at::kFloat));
     a.lse = dk_rowvec{static_cast<float *>(lse.data_ptr()), Hq, 1, 1};
   }
@@ -292,17 +327,13 @@ PyObject *paged_impl(PyObject *const *args) {
   a.k = dk_tensor{k.data_ptr(), 0, k.stride(2), k.stride(1)}, a.v = dk_tensor{v.data_ptr(), 0, v.stride(2), v.stride(1)};
   a.num_q_heads = (int32_t)Hq, a.num_kv_heads = (int32_t)Hkv;
   a.stream = current_stream();
-  const double ks = PyFloat_AsDouble(args[13]), vs = PyFloat_AsDouble(args[14]);
-  if (PyErr_Occurred()) {
-    PyErr_Clear();
-    throw Unsupported{};
-  }
   const dk_paged_kv pg{static_cast<const int32_t *>(table.data_ptr()), table.stride(0), k.stride(0), v.stride(0), (int32_t)page,
                        fp8 ? DK_FP8_E4M3 : a.dtype, (float)ks, (float)vs};
   const size_t bytes = fwd_bytes_fn(&a);
   at::Tensor ws = at::empty({(int64_t)std::max<size_t>(bytes, 16)}, q.options().dtype(at::kByte));
   a.workspace = ws.data_ptr(), a.workspace_bytes = bytes;
   need(fwd_paged_fn(&a, &pg) == DK_OK);
+  unlocked.reset();
   return result(out, lse, bytes);
 }
 

@@ -1,6 +1,7 @@
 """The C++ host path of the inference calls (dkernel_amd/_host.so) against the Python launchers in
 ops.py: same kernels, so every output bit must agree; and what it leaves to them (None) still works.
 Also the tokens of packed inputs that belong to no sequence: their log-sum-exp reads -inf."""
+import ctypes as C
 import math
 
 import pytest
@@ -128,6 +129,27 @@ def test_paged(monkeypatch, bs, fp8, dims):
         q = q[:, None]
     for lse in (False, True):
         same(*both(monkeypatch, lambda: mod.paged_decode(q, *pools, table, lens, 0.1, return_lse=lse, k_scale=0.5)))
+
+
+def test_launches_run_without_the_interpreter_lock():
+    """PyGILState_Check in the place of dk_fwd and dk_fwd_paged: its 0 for a thread that does not hold the
+    lock reads as DK_OK, its 1 as a refusal, for which the C++ path returns None.  (Nothing is launched.)"""
+    def address(f):
+        return C.cast(f, C.c_void_p).value
+    host, lib, check = _lib.host(), _lib.lib(), address(C.pythonapi.PyGILState_Check)
+    mod = New(4, 256, 64, 2, 3, num_kv_heads=2).to(DEV)
+    q, k, v = (torch.zeros(1, 256, h, 64, device=DEV, dtype=torch.bfloat16) for h in (4, 2, 2))
+    n = torch.tensor([0, 256], dtype=torch.int32, device=DEV)
+    tail = (mod._buffers, mod._kernel_tables, mod.mask_lut_max_row)
+    try:
+        host.bind(check, address(lib.dk_fwd_workspace_bytes), check)
+        res = [host.forward(q, k, v, 0.1, *tail, mod.kwargs, 1, None, None, None, None, True, ops._impl, True),
+               host.forward(q[0], k[0], v[0], 0.1, *tail, mod.kwargs, 1, n, None, None, None, True, ops._impl, True),
+               host.paged(q[:, 0], k.view(4, 64, 2, 64), v.view(4, 64, 2, 64), torch.arange(4, dtype=torch.int32, device=DEV)[None],
+                          n[1:], 0.1, *tail, mod.lut_max_row, mod.lut_group, 256, True, 1.0, 1.0, ops._impl)]
+    finally:
+        host.bind(*(address(f) for f in (lib.dk_fwd, lib.dk_fwd_workspace_bytes, lib.dk_fwd_paged)))
+    assert all(r is not None for r in res)
 
 
 def test_user_pattern_and_errors():
