@@ -262,8 +262,11 @@ class SparseAttention(torch.nn.Module):
             self.register_buffer("masked_csc_ccol", m_csc[0].to(torch.int32), persistent=False)
             self.register_buffer("masked_csc_row", m_csc[1].to(torch.int32), persistent=False)
 
-        # names of the tables that the kernels read, with their tile sizes: (crow, col, rows, columns,
-        # masked crow, masked col, tile, pattern block size)
+        self._kernel_tables = self._table_names()
+
+    def _table_names(self) -> Tuple:
+        """Names of the tables that the kernels read, with their tile sizes: (crow, col, rows, columns,
+        masked crow, masked col, tile, pattern block size)."""
         if self.kernel_tile is not None:
             tables = ("kernel_csr_crow", "kernel_csr_col", self.kernel_tile, self.kernel_tile)
         elif self.exact_tile is not None:
@@ -272,7 +275,14 @@ class SparseAttention(torch.nn.Module):
             tables = ("layout_csr_crow", "layout_csr_col", self.block_m, self.block_n)
         masked = (None, None, 0, 0) if self.mask_tile is None else ("masked_csr_crow", "masked_csr_col", self.mask_tile,
                                                                     self.block_size)
-        self._kernel_tables = tables + masked
+        return tables + masked
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        # modules saved whole (torch.save, pickle) by versions whose forward() did not read these
+        self.__dict__.setdefault("mask_lut_max_row", 0)
+        self.__dict__.setdefault("_kernel_tables", self._table_names())
+        self.kwargs.setdefault("fixed_walk", self.kwargs.get("unsorted_rows", False))
 
     def forward(self,
                 q: Tensor,

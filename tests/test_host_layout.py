@@ -464,3 +464,20 @@ def test_which_patterns_count_as_uneven():
     assert _uneven_heads(mask(num_dense_heads=1))
     assert _uneven_heads(mask(num_dense_heads=4))
     assert not _uneven_heads(mask(num_dense_heads=8))  # every head dense: even again
+
+
+@pytest.mark.parametrize("bs", [32, 64, 128])
+def test_modules_saved_whole_by_earlier_versions_load(bs):
+    """A pickled module without the attributes that forward() has come to read since gets them on loading."""
+    import pickle
+    from dkernel_amd import SparseAttention
+    pattern = torch.tril(torch.ones(8, 8, dtype=torch.uint8))
+    pattern[0] = 1  # (a global row: the rows are not sorted by length)
+    mod = SparseAttention(bs, pattern, causal=False)
+    old = SparseAttention(bs, pattern, causal=False)
+    del old._kernel_tables, old.kwargs["fixed_walk"]
+    if old.mask_tile is None:
+        del old.mask_lut_max_row
+    new = pickle.loads(pickle.dumps(old))
+    assert new._kernel_tables == mod._kernel_tables and new.mask_lut_max_row == mod.mask_lut_max_row
+    assert new.kwargs == mod.kwargs
