@@ -85,7 +85,12 @@ class SparseAttention(torch.nn.Module):
         merged table lets the earlier rows attend it too), those tables are
         built from the widened pattern: the result is that of the merged table.
     kwargs: "out" (output tensor), "d_splits" (accepted, unused), "inference"
-        (skip saving the log-sum-exp for backward; default: no input needs grad).
+        (skip saving the log-sum-exp for backward; default: no input needs grad),
+        "fixed_walk" (True: the prefill of a sequence gives the same bits alone, in a padded or packed
+        batch and in a batch of any size; costs small launches up to a third of their speed.  False: small
+        launches round differently, within the precision of the data type.  Default: False, but True for
+        patterns with rows clearly longer than all rows after them, such as global rows).  Results of
+        single-token decode steps depend on the batch in their last bits either way.
 
     forward(q, k, v, sm_scale=None, *, cu_seqlen_k, cu_seqlen_q, left_paddings,
             seqlens, return_lse, split_qkv): see the method.
@@ -148,9 +153,10 @@ class SparseAttention(torch.nn.Module):
         # - the longest of a causal pattern -, then take the rows in the table's own order, longest
         # first, instead of starting the long ones when the rest of the chip has run out of work
         self.kwargs['unsorted_rows'] = _unsorted_rows(sparse_pattern)
-        # ... and every launch of theirs, however small, takes a row's blocks in one order: results then do
-        # not depend on how sequences are batched, whichever way the rows are handed out
-        self.kwargs['fixed_walk'] = self.kwargs['unsorted_rows']
+        # Small forward launches split a row's blocks over the waves of a workgroup, which rounds
+        # differently from the walk of larger ones.  Patterns whose rows are handed out in two possible
+        # orders stay bit-identical under both, so they keep the one walk unless told otherwise.
+        self.kwargs.setdefault('fixed_walk', self.kwargs['unsorted_rows'])
 
         if not causal:
             # merged q tiles are a causal-only optimisation
