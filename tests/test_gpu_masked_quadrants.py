@@ -1,7 +1,8 @@
 """Masked 64 x 64 tiles (pattern blocks of 16 and 32): the kernels multiply 32 x 32 quadrants and leave out those
 that hold no attended block.  Sparse random patterns, in which most tiles hold one or two quadrants and single
-16-token blocks inside them, at every tile width, with rows in pairs and in head groups, forward and backward,
-against the fp32 oracle at the 16-bit bar."""
+16-token blocks inside them, at every tile width, forward and backward, against the fp32 oracle at the 16-bit bar.
+(The first six forwards are split along the keys, the others run single rows; row pairs and head groups:
+test_gpu_large_launch_kernels.py.)"""
 import math
 
 import numpy as np
@@ -22,10 +23,10 @@ pytestmark = pytest.mark.gpu
     (1, 2, 1, 450, 256, 32, torch.bfloat16, True, 0.08),
     (1, 2, 2, 330, 200, 16, torch.bfloat16, True, 0.04),
     (1, 3, 3, 575, 96, 32, torch.bfloat16, False, 0.05),
-    (1, 4, 4, 2600, 120, 32, torch.float16, True, 0.03),   # (too large for the kernel of small launches)
-    (1, 8, 8, 2100, 128, 32, torch.bfloat16, True, 0.03),  # (single rows)
-    (4, 32, 32, 400, 128, 16, torch.bfloat16, False, 0.05),  # (row pairs)
-    (1, 2, 2, 650, 64, 32, torch.float16, "global", 0.05),   # (single rows, whole tiles)
+    (1, 4, 4, 2600, 120, 32, torch.float16, True, 0.03),   # (single rows, and so are the cases below)
+    (1, 8, 8, 2100, 128, 32, torch.bfloat16, True, 0.03),
+    (4, 32, 32, 400, 128, 16, torch.bfloat16, False, 0.05),
+    (1, 2, 2, 650, 64, 32, torch.float16, "global", 0.05),   # (whole tiles)
     (2, 2, 2, 450, 40, 16, torch.bfloat16, "global", 0.03),
     (1, 2, 2, 650, 128, 32, torch.bfloat16, "global", 0.05),
 ])

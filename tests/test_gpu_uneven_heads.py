@@ -23,6 +23,8 @@ def _last_fwd() -> bytes:
     return _lib.lib().dk_last_kernels()
 
 
+# (The 16-bit forwards below 512 workgroups of 32 rows are split along the keys here; the kernels named below run
+# them in test_gpu_large_launch_kernels.py.)
 # (q heads, kv heads, dense heads, tokens, head dim, dtype): 32 and 16 heads sit on fixed queues
 # without the rotation; 2 heads over 16 row pairs move on every second / fourth step; a GQA group
 # per workgroup; head dims of the padded and of the 256-wide kernels; fp32 on the matrix cores
