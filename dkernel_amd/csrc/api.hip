@@ -1,7 +1,7 @@
 // C-ABI entry points for the device side: argument checks (the reference's
 // Python asserts, done before any launch so that a bad shape can never reach a
-// kernel), parameter-block construction and dispatch between the MFMA kernels
-// (bf16 / fp16, head_dim 128 or 64, 64x64 blocks) and the generic kernels.
+// kernel), parameter-block construction and dispatch between the decode kernels, the MFMA
+// kernels (64 x 64 tiles; 16-bit floats of head dims up to 256, fp32 up to 128) and the generic kernels.
 #include <hip/hip_runtime.h>
 
 #include "common.h"

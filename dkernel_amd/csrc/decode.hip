@@ -205,8 +205,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
   // page table beyond the sequence's last token are never read; a negative entry inside the
   // sequence (a caller's mistake: such slots mark unused pages) is read as page 0 rather than
   // as an address before the pool.
-  // A unit of more than 16 entries (only when the caller's max_row_entries hint understated the
-  // row) reloads the register every 16 entries.
+  // A unit of more than 16 entries (one of 16 whole blocks that starts at a second half, or any when the
+  // caller's max_row_entries hint understated the row) reloads the register every 16 entries.
   int my_page = 0;
   auto load_pages = [&](int j0) {  // pages of entries e0 + j0 .. e0 + j0 + 15
     int pg = 0;
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
   auto prefetch = [&](int hb, int col, int bits) {
     const int key0 = col * 64 + (hb & 1) * 32;
     if constexpr (PAGED)
-      if (hb > 0 && (hb & 31) == 0) my_page = load_pages(hb >> 1);  // (never with the default unit sizes)
+      if (hb > 0 && (hb & 31) == 0) my_page = load_pages(hb >> 1);
     if (SUB && half_bits(bits, hb) == 0) return;  // no attended key in this half: neither read nor used
     // element offset of row r of the half block from kbase / vbase
     int pg_lo = 0, pg_hi = 0, in_page0 = 0;

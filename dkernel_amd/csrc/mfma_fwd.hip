@@ -690,7 +690,8 @@ static int launch_sub(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
     case 2: return launch_sub_g<T, D, 2, PAD>(p, grid, tiles_y, stream);
     // Global rows: the longest row is the run time, and shorter alone than in a pair (12 heads of 64, 4 x 3000
     // tokens: 75.5 us against 101).  Otherwise pairs (16 heads of 128, 8000 tokens: 98 us against 150), unless
-    // so few that compute units are left empty or with one pair and no second one to overlap it with:
+    // so few that compute units are left empty or with one pair and no second one to overlap it with (the line lies
+    // between the sizes measured: at 384 pairs few long rows prefer single rows, many short ones are equal):
     // single rows / pairs, us, blocks of 32, 128-wide tile: 8 heads x 2500 tokens (160 pairs) 25.2 / 31.7, 12 x 2600
     // (252) 27.1 / 35.9, 8 x 4800 (304) 36.1 / 44.4, 8 x 6000 (376) 47.5 / 55.0, 12 x 4000 (384) 40.7 / 45.0, 32 x
     // 1500 (384) 31.6 / 30.9; 96 of 128 dims: 16 x 2300 (288) 29.5 / 34.8, 16 x 2800 (352) 42.3 / 38.8.  The 64-wide

@@ -27,6 +27,9 @@ extern "C" {
 
 enum dk_dtype { DK_BF16 = 0, DK_F16 = 1, DK_F32 = 2,
                 DK_FP8_E4M3 = 3 /* OCP e4m3 bytes; K/V pools of dk_fwd_paged only */ };
+/* Kernel family: AUTO takes the matrix-core kernels where one serves the call and the generic ones
+ * otherwise; MFMA fails with DK_ERR_UNSUPPORTED instead.  fp32 head dims 68 - 128 run their matrix-core
+ * kernels under AUTO only: MFMA refuses them, as it did before those kernels existed. */
 enum dk_impl { DK_IMPL_AUTO = 0, DK_IMPL_GENERIC = 1, DK_IMPL_MFMA = 2 };
 
 int dk_version(void);              /* 10000*major + 100*minor + patch */
