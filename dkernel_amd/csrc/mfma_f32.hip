@@ -26,7 +26,7 @@
 // is multiplied.  Bound: fp32 MFMA (a large fp32 product of the vendor library: 153 TFLOP/s).  Measured
 // forward / backward, us: 1 x 8192 tokens, 32 heads of 64 dims, local 16, vert 8: 906 / 2765 = 101 / 82
 // TFLOP/s (two waves of 32 x 64 quadrants over a single stage: 1114 / 3836); 8 heads x 1024 tokens of 64
-// dims: 26 / 126 (52 / 262); 16 heads x 2000 tokens of 128 dims, local 8, vert 4: 122 / 505 (fp32-FMA
+// dims: 26 / 126 (52 / 262); 16 heads x 2000 tokens of 128 dims, local 8, vert 4: 128 / 491 (fp32-FMA
 // kernels of generic_*.hip: 474 / 3189), where the longest row and column, one workgroup each, set the
 // time.
 #include <type_traits>
@@ -63,13 +63,33 @@ struct Shape {
   static constexpr int kSmem = 2 * kStage;
 };
 
-// acc(32 x 32) += X Y^T over the head dims: rows = rows row0 .. row0 + 31 of tile `xt` (row0 a
-// multiple of 32), columns = the lanes' own rows of Y, yf[s] = dim HD g + s of that row.
+// Result of dot_dims: above 64 dims the last chain is left to be added where the sum is read, so that
+// nobody waits for the matrix core in between.
+template <int KD>
+struct DimSum {
+  floatx16 sum, last;
+  __device__ __forceinline__ float operator[](int r) const { return sum[r] + last[r]; }
+};
+template <>
+struct DimSum<64> {
+  floatx16 sum;
+  __device__ __forceinline__ float operator[](int r) const { return sum[r]; }
+};
+
+// X Y^T (32 x 32) over the head dims: rows = rows row0 .. row0 + 31 of tile `xt` (row0 a multiple of
+// 32), columns = the lanes' own rows of Y, yf[s] = dim HD g + s of that row.
+//
+// Above 64 dims the sum is built from chains of 32 dims (one batch of operand reads each), added on the
+// vector unit while the matrix core multiplies the next one.  Relative error of the output against 64
+// bits, 300 tokens of 128 dims: one chain of 128 roundings 3.1e-7, chains of 32 1.7e-7, the fp32-FMA
+// kernels (four chains of 32) 2.0e-7; dQ 4.6e-7, 3.5e-7, 3.6e-7.  Price: 16 heads x 2000 tokens
+// of 128 dims, forward 126 -> 128 us, forward and backward 608 -> 621.
 template <int KD, bool PAD>
-__device__ __forceinline__ floatx16 dot_dims(const char *xt, int row0, const float (&yf)[KD / 2], int lane, floatx16 acc) {
+__device__ __forceinline__ DimSum<KD> dot_dims(const char *xt, int row0, const float (&yf)[KD / 2], int lane) {
   using S = Shape<KD, PAD>;
   constexpr int CH = S::HD / 4, B = 4;  // 16-byte chunks per lane, read in batches ahead of their multiplies
   static_assert(CH % B == 0, "whole batches");
+  constexpr int RUN = KD <= 64 ? CH / B : 1;  // batches per chain
   // (opaque: the read addresses - a few XORs per 64-cycle multiply - are computed here; hoisted out of
   // the caller's loop they would occupy registers throughout)
   asm volatile("" : "+v"(lane));
@@ -79,6 +99,7 @@ __device__ __forceinline__ floatx16 dot_dims(const char *xt, int row0, const flo
   float4 x[2][B];
 #pragma unroll
   for (int i = 0; i < B; ++i) x[0][i] = *reinterpret_cast<const float4 *>(row + (((g * CH + i) ^ swz) << 4));
+  floatx16 chain[2], sum;  // the chain in work and the finished one before it; their sum
 #pragma unroll
   for (int b = 0; b < CH / B; ++b) {
     if (b + 1 < CH / B) {
@@ -87,6 +108,11 @@ __device__ __forceinline__ floatx16 dot_dims(const char *xt, int row0, const flo
         x[(b + 1) & 1][i] = *reinterpret_cast<const float4 *>(row + (((g * CH + (b + 1) * B + i) ^ swz) << 4));
     }
     __builtin_amdgcn_sched_barrier(0);
+    floatx16 &acc = chain[(b / RUN) & 1];
+    if (b % RUN == 0) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    }
 #pragma unroll
     for (int i = 0; i < B; ++i) {
       const float4 w = x[b & 1][i];
@@ -94,10 +120,20 @@ __device__ __forceinline__ floatx16 dot_dims(const char *xt, int row0, const flo
       acc = mma(w.y, yf[(b * B + i) * 4 + 1], acc);
       acc = mma(w.z, yf[(b * B + i) * 4 + 2], acc);
       acc = mma(w.w, yf[(b * B + i) * 4 + 3], acc);
+      if (RUN == 1 && b > 0 && i == 0) {  // (the chain before has long left the matrix core)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[r] = b == 1 ? chain[0][r] : sum[r] + chain[(b - 1) & 1][r];
+        asm volatile("" : "+v"(sum));  // (here, not sunk behind the last chain with all of them alive)
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  return acc;
+  if constexpr (RUN > 1)
+    return {chain[0]};
+  else
+    return {sum, chain[(CH / B - 1) & 1]};
 }
 
 // acc[dt](32 dims x 32 columns) += T^T(dims x rows) * W(rows x columns) over the 32 rows row0 .. row0 + 31 of
@@ -298,15 +334,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
     if (col < 0 || key0 >= sq.k_len || (p.causal && key0 > row0 + 31)) return;  // nothing visible (wave-uniform)
     const char *ks = smem + stage * S::kStage, *vs = ks + S::kTile;
     // S^T = K Q^T: lane = q row, registers = keys 8(r/4) + 4g + r%4 of the half
+    const DimSum<KD> dots = dot_dims<KD, PAD>(ks, kh * 32, qf, lane);
     floatx16 s;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.f;
-    s = dot_dims<KD, PAD>(ks, kh * 32, qf, lane, s);
     float mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = key0 + (r >> 2) * 8 + g * 4 + (r & 3);
-      s[r] = key > lim || !row_ok ? -INFINITY : s[r] * p.scale_log2;
+      s[r] = key > lim || !row_ok ? -INFINITY : dots[r] * p.scale_log2;
       mx = fmaxf(mx, s[r]);
     }
     mx = max_with_other_half(mx);
@@ -454,15 +488,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
     const int key0 = col * 64 + kh * 32;
     if (col < 0 || key0 >= sq.k_len || (p.causal && key0 > row0 + 31)) return;
     const char *ks = smem + stage * S::kStage, *vs = ks + S::kTile;
-    floatx16 s, dp;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-    s = dot_dims<KD, PAD>(ks, kh * 32, qf, lane, s);
-    dp = dot_dims<KD, PAD>(vs, kh * 32, dof, lane, dp);
+    const DimSum<KD> dots = dot_dims<KD, PAD>(ks, kh * 32, qf, lane), dp = dot_dims<KD, PAD>(vs, kh * 32, dof, lane);
+    floatx16 s;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = key0 + (r >> 2) * 8 + g * 4 + (r & 3);
-      const float pr = key > lim ? 0.f : fast_exp2(fmaf(s[r], p.scale_log2, -lse2));
+      const float pr = key > lim ? 0.f : fast_exp2(fmaf(dots[r], p.scale_log2, -lse2));
       s[r] = pr * (dp[r] - delta);  // dS^T without sm_scale (applied once at the end)
     }
     dot_rows<KD, PAD>(ks, kh * 32, s, lane, acc);
@@ -566,11 +597,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
       if (rbq < 0 || (p.causal && key0 > pos0 + 31)) return;  // nothing visible (wave-uniform)
       const char *qs = smem + stage * S::kStage, *dos = qs + S::kTile;
       const float *lse_s = vecs + stage * 128 + qh * 32, *delta_s = lse_s + 64;
-      floatx16 s, dp;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-      s = dot_dims<KD, PAD>(qs, qh * 32, kf, lane, s);  // rows = q (tile), columns = keys (registers)
-      dp = dot_dims<KD, PAD>(dos, qh * 32, vf, lane, dp);
+      // rows = q (tile), columns = keys (registers)
+      const DimSum<KD> dots = dot_dims<KD, PAD>(qs, qh * 32, kf, lane), dps = dot_dims<KD, PAD>(dos, qh * 32, vf, lane);
+      floatx16 s, ds;
 #pragma unroll
       for (int r4 = 0; r4 < 4; ++r4) {
         const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + r4 * 8 + g * 4);
@@ -580,12 +609,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
         for (int i = 0; i < 4; ++i) {
           const int r = r4 * 4 + i;
           const bool vis = key_ok && (!p.causal || key <= pos0 + r4 * 8 + g * 4 + i);
-          s[r] = vis ? fast_exp2(fmaf(s[r], p.scale_log2, -lr[i])) : 0.f;
-          dp[r] = s[r] * (dp[r] - dr[i]);  // dS without sm_scale (applied once at the end)
+          s[r] = vis ? fast_exp2(fmaf(dots[r], p.scale_log2, -lr[i])) : 0.f;
+          ds[r] = s[r] * (dps[r] - dr[i]);  // dS without sm_scale (applied once at the end)
         }
       }
       dot_rows<KD, PAD>(dos, qh * 32, s, lane, dv);
-      dot_rows<KD, PAD>(qs, qh * 32, dp, lane, dk);
+      dot_rows<KD, PAD>(qs, qh * 32, ds, lane, dk);
     };
     for (int e = e0; e < e1; e += 2) {
       block_step(e, Stage<0>{});
