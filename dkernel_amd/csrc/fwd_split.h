@@ -30,14 +30,14 @@ struct SplitSmem {  // per wave
   static constexpr int kBytes = kSplitWaves * kWave;
 };
 
-template <typename T, int D, bool PAD, bool SUB>
+template <typename T, int D, bool PAD, bool SUB, int KD = D>
 __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, D == 64 ? 3 : D == 256 ? 1 : 2))) void mfma_fwd_split_kernel(
     const FwdParams p, int tiles_y) {
   using M = Mma<T>;
   using vec8 = typename M::vec8;
   using S = SplitSmem<D>;
   constexpr int W = kSplitWaves, NT = 64 * W;
-  constexpr int KS = D / 16, DT = D / 32, CPR = D / 8;
+  constexpr int KS = KD / 16, DT = KD / 32, CPR = D / 8;
   constexpr int EW = SUB ? 2 : 1;  // ints per table entry
   extern __shared__ __align__(16) char smem_all[];
 

@@ -2,6 +2,7 @@
 // CSR / CSC look-up tables with -1 padding, kernel-tile merge / split, and the
 // KV-cache-efficiency check.  Integer work on the CPU, one pass per table; it
 // replaces the per-head Python loops of dkernel/utils.py.
+#include <cstdlib>
 #include <cstring>
 #include <vector>
 
@@ -27,7 +28,16 @@ void note_kernel(const char *kernel, const char *launcher_signature) {
   // "... launcher(args) [T = dk::bf16_t, D = 128, ...]" -> "kernel [T = dk::bf16_t, D = 128, ...]; "
   const char *args = launcher_signature ? strrchr(launcher_signature, '[') : nullptr;
   const size_t used = strlen(g_kernels);
-  snprintf(g_kernels + used, sizeof(g_kernels) - used, "%s%s%s; ", kernel, args ? " " : "", args ? args : "");
+  // the head dims that are multiplied, where they are fewer than the tiles': "...], 96 dims; "
+  const char *d = args ? strstr(args, " D = ") : nullptr, *kd = args ? strstr(args, ", KD = ") : nullptr;
+  const int dims = d && kd && atoi(d + 5) != atoi(kd + 7) ? atoi(kd + 7) : 0;
+  snprintf(g_kernels + used, sizeof(g_kernels) - used, "%s%s%.*s%s", kernel, args ? " " : "",
+           kd ? (int)(kd - args) : args ? (int)strlen(args) : 0, args ? args : "", kd ? kd + 7 + strcspn(kd + 7, ",]") : "");
+  const size_t now = strlen(g_kernels);
+  if (dims)
+    snprintf(g_kernels + now, sizeof(g_kernels) - now, ", %d dims; ", dims);
+  else
+    snprintf(g_kernels + now, sizeof(g_kernels) - now, "; ");
 }
 
 }  // namespace dk

@@ -362,14 +362,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 // the L2 into LDS (what the one-tile kernel spent a quarter of its time on) is halved; a wave
 // skips the blocks its own row does not hold.  Every wave owns the finished dQ of its rows:
 // nothing is summed across waves at the end.
-template <typename T, int D, bool PAD, bool SUB>
+template <typename T, int D, bool PAD, bool SUB, int KD = D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 ? 3 : 2))) void mfma_dq_pair_kernel(const BwdParams p,
                                                                                                       int pairs_y) {
   using M = Mma<T>;
   using vec8 = typename M::vec8;
   using TL = Tile<D>;
   constexpr int NT = 256;
-  constexpr int KS = D / 16, DT = D / 32;
+  constexpr int KS = KD / 16, DT = KD / 32;
   constexpr int STAGE = 2 * TL::kBytes;
   constexpr int EW = SUB ? 2 : 1;  // ints per table entry
   extern __shared__ __align__(16) char smem[];
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   const int pos = row0 + m;
   const int qi = pos - sq.past;
   const bool row_ok = qi >= 0 && qi < sq.q_len;  // (a table row without queries of this sequence: false everywhere)
-  if constexpr (PAD) {  // the slots of the head dims beyond p.D stay zero for the whole kernel
+  if (PAD && p.D < KD) {  // the slots of the head dims beyond p.D stay zero for the whole kernel
     zero_tiles<NT>(smem, 2 * STAGE, tid);
     __syncthreads();
   }
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   for (int j = 0; j < OCH; ++j) {
     const int r = tid / CPR + j * (NT / CPR), ch = tid % CPR;
     const uint4 dow = *reinterpret_cast<const uint4 *>(smem + (r >> 6) * STAGE + TL::kBytes + TL::off(r & 63, ch));
-    float d = dot8<T>(oreg[j], dow, 0.f);
+    float d = !PAD || ch * 8 < p.D ? dot8<T>(oreg[j], dow, 0.f) : 0.f;  // (those slots may hold anything)
 #pragma unroll
     for (int off = CPR / 2; off > 0; off >>= 1) d += __shfl_xor(d, off);
     if (ch == 0) delta_rows[r] = d;
@@ -684,20 +684,20 @@ struct DkdvSmem {
   static constexpr int kBytes = kX + 2 * 2 * 4096;
 };
 
-template <typename T, int D, bool PAD, bool SUB>
+template <typename T, int D, bool PAD, bool SUB, int KD = D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, D == 256 ? 1 : 2))) void mfma_dkdv_kernel(const BwdParams p, int head_split) {
   using M = Mma<T>;
   using vec8 = typename M::vec8;
   using TL = Tile<D>;
   using S = DkdvSmem<D>;
   constexpr int NT = 256;
-  constexpr int KS = D / 16, DT = D / 32;
+  constexpr int KS = KD / 16, DT = KD / 32;
   using Loader = TileLoader<D, NT, PAD, S::kRows>;
   constexpr int LPT = 2 * Loader::kChunks + 1;  // load instructions per wave per step
   // SUB: steps without an attended block are left out, and a pair of waves without a bit in its quadrant sits the
-  // step out (not at the 256-wide tile and the padded 128-wide one: slower, and one register too many).  Blocks of
+  // step out (not at the 256-wide tile and the zero-padded 128 dims: slower, and one register too many).  Blocks of
   // 32, local 16, vertical 8, 16 heads x 8000 tokens, forward and backward: 555 -> 473 us with the two other kernels.
-  constexpr bool kIdle = SUB && (D == 64 || (D == 128 && !PAD));
+  constexpr bool kIdle = SUB && (D == 64 || (D == 128 && (!PAD || KD < D)));
   // SUB: table entries are (row block, bit mask over the pattern blocks inside the 64 x 64 tile)
   constexpr int EW = SUB ? 2 : 1;  // ints per table entry
   extern __shared__ __align__(16) char smem[];
@@ -728,7 +728,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   Loader qload, doload;
   qload.init(tid, p.q.st, p.D);
   doload.init(tid, p.dout.st, p.D);
-  if constexpr (PAD) {  // the slots of the head dims beyond p.D stay zero in every stage
+  if (PAD && p.D < KD) {  // the slots of the head dims beyond p.D stay zero in every stage
     zero_tiles<NT>(smem, S::kBytes, tid);
     __syncthreads();
   }
@@ -1099,32 +1099,40 @@ template __global__ void mfma_dkdv_kernel<f16_t, 256, true, false>(const BwdPara
 template __global__ void mfma_dkdv_kernel<f16_t, 256, true, true>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<bf16_t, 128, false, false>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, false, 96>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<bf16_t, 128, false, true>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, true, 96>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<bf16_t, 64, false, false>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<bf16_t, 64, true, false>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<bf16_t, 64, false, true>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<bf16_t, 64, true, true>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<f16_t, 128, false, false>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, false, 96>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<f16_t, 128, false, true>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, true, 96>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<f16_t, 64, false, false>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<f16_t, 64, true, false>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<f16_t, 64, false, true>(const BwdParams, int);
 template __global__ void mfma_dq_pair_kernel<f16_t, 64, true, true>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 128, false, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 128, true, false>(const BwdParams, int);
+template __global__ void mfma_dkdv_kernel<bf16_t, 128, true, false, 96>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 128, false, true>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 128, true, true>(const BwdParams, int);
+template __global__ void mfma_dkdv_kernel<bf16_t, 128, true, true, 96>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 64, false, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 64, true, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 64, false, true>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 64, true, true>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 128, false, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 128, true, false>(const BwdParams, int);
+template __global__ void mfma_dkdv_kernel<f16_t, 128, true, false, 96>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 128, false, true>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 128, true, true>(const BwdParams, int);
+template __global__ void mfma_dkdv_kernel<f16_t, 128, true, true, 96>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 64, false, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 64, true, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 64, false, true>(const BwdParams, int);
@@ -1202,12 +1210,12 @@ bool mfma_bwd_supported(const BwdParams &p, int dtype) {
          mfma_row_bytes_ok(p.dout);
 }
 
-template <typename T, int D, bool PAD, bool SUB>
+template <typename T, int D, bool PAD, bool SUB, int KD = D>
 static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_bytes, hipStream_t stream) {
   const SeqView &s = p.seqs;
   constexpr int smem_dq = 2 * 2 * Tile<D>::kBytes;
   constexpr int smem_dkdv = DkdvSmem<D>::kBytes;
-  DK_ALLOW_DYNAMIC_LDS((mfma_dkdv_kernel<T, D, PAD, SUB>), smem_dkdv);
+  DK_ALLOW_DYNAMIC_LDS((mfma_dkdv_kernel<T, D, PAD, SUB, KD>), smem_dkdv);
   const int past = p.causal ? s.max_k_len - s.max_q_len : 0;
   const int tiles = (past + s.max_q_len - 1) / 64 - past / 64 + 1;
   DK_REQUIRE(tiles <= 65535 && cdiv(s.max_k_len, 64) <= 65535 && p.csc.num_rows <= 65535 &&
@@ -1216,12 +1224,12 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
   // dQ first: it also writes delta, which the dK/dV pass reads
   if constexpr (D <= 128) {  // two table rows per workgroup
     int pairs = (((past + s.max_q_len - 1) / 64) >> 1) - ((past / 64) >> 1) + 1;
-    DK_ALLOW_DYNAMIC_LDS((mfma_dq_pair_kernel<T, D, PAD, SUB>), smem_dq);
+    DK_ALLOW_DYNAMIC_LDS((mfma_dq_pair_kernel<T, D, PAD, SUB, KD>), smem_dq);
     if (p.csr.pair_order) pairs = (p.csr.num_rows + 1) / 2;  // handed out in the table's order: all of them
     BwdParams pq = p;
     pq.csr.rot = head_rotation(p.csr, p.Hq, pairs);  // (uneven heads: dealt to the queues in rotation)
     DK_NOTE_KERNEL(pq.csr.rot ? "mfma_dq_pair_kernel, heads in rotation" : "mfma_dq_pair_kernel");
-    hipLaunchKernelGGL((mfma_dq_pair_kernel<T, D, PAD, SUB>), dim3(p.Hq, pairs, s.batch), dim3(256), smem_dq, stream, pq, pairs);
+    hipLaunchKernelGGL((mfma_dq_pair_kernel<T, D, PAD, SUB, KD>), dim3(p.Hq, pairs, s.batch), dim3(256), smem_dq, stream, pq, pairs);
   } else {
     DK_ALLOW_DYNAMIC_LDS((mfma_dq_kernel<T, D, PAD, SUB>), smem_dq);
     const int rows = p.csr.order ? p.csr.num_rows : tiles;  // handed out in the table's order: all of them
@@ -1255,17 +1263,18 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
     pp.dv = TensorView{part_v, p.Hq * keys * p.D, keys * p.D, p.D};
     DK_NOTE_KERNEL(pp.csc.rot ? "mfma_dkdv_kernel (one workgroup per q head), heads in rotation"
                               : "mfma_dkdv_kernel (one workgroup per q head)");
-    hipLaunchKernelGGL((mfma_dkdv_kernel<T, D, PAD, SUB>), dim3(p.Hq, cblocks, s.batch), dim3(256), smem_dkdv, stream, pp, 1);
+    hipLaunchKernelGGL((mfma_dkdv_kernel<T, D, PAD, SUB, KD>), dim3(p.Hq, cblocks, s.batch), dim3(256), smem_dkdv, stream, pp, 1);
     DK_HIP_CHECK(hipGetLastError());
     return launch_group_sum_t<T>(p, part_k, part_v, stream);
   }
   DK_NOTE_KERNEL(po.csc.rot ? "mfma_dkdv_kernel, heads in rotation" : "mfma_dkdv_kernel");
-  hipLaunchKernelGGL((mfma_dkdv_kernel<T, D, PAD, SUB>), dim3(p.Hkv, cblocks, s.batch), dim3(256), smem_dkdv, stream, po, 0);
+  hipLaunchKernelGGL((mfma_dkdv_kernel<T, D, PAD, SUB, KD>), dim3(p.Hkv, cblocks, s.batch), dim3(256), smem_dkdv, stream, po, 0);
   DK_HIP_CHECK(hipGetLastError());
   return DK_OK;
 }
 
-// head dims below the tile width (64 or 128) run the zero-padded instantiation
+// head dims below the tile width (64 or 128) run the zero-padded instantiation, those of 72 - 96 with 96 of the 128
+// dims multiplied (as in the forward; training, 96 dims, 2 x 3000 tokens, 32 / 8 heads: 516 -> 460 us)
 template <typename T>
 static int launch_bwd_t(const BwdParams &p, void *ws, size_t ws_bytes, hipStream_t stream) {
   if (p.D > 128)  // 256-wide tiles, one wave per SIMD
@@ -1274,11 +1283,13 @@ static int launch_bwd_t(const BwdParams &p, void *ws, size_t ws_bytes, hipStream
   if (p.csr.sub_block) {  // entries carry a bit mask over the pattern's 16- or 32-token blocks
     if (p.D == 128) return launch_bwd_td<T, 128, false, true>(p, ws, ws_bytes, stream);
     if (p.D == 64) return launch_bwd_td<T, 64, false, true>(p, ws, ws_bytes, stream);
+    if (p.D > 64 && p.D <= 96) return launch_bwd_td<T, 128, true, true, 96>(p, ws, ws_bytes, stream);
     return p.D > 64 ? launch_bwd_td<T, 128, true, true>(p, ws, ws_bytes, stream)
                     : launch_bwd_td<T, 64, true, true>(p, ws, ws_bytes, stream);
   }
   if (p.D == 128) return launch_bwd_td<T, 128, false, false>(p, ws, ws_bytes, stream);
   if (p.D == 64) return launch_bwd_td<T, 64, false, false>(p, ws, ws_bytes, stream);
+  if (p.D > 64 && p.D <= 96) return launch_bwd_td<T, 128, true, false, 96>(p, ws, ws_bytes, stream);
   return p.D > 64 ? launch_bwd_td<T, 128, true, false>(p, ws, ws_bytes, stream)
                   : launch_bwd_td<T, 64, true, false>(p, ws, ws_bytes, stream);
 }

@@ -202,12 +202,12 @@ struct Tile {
 // arithmetic is left in the inner loops (the row0 part becomes an immediate).
 // The lane (d = 32*dt + lane%32, k-group g) receives rows
 // row0 + {4g..4g+3, 8+4g..8+4g+3} of column d.
-template <int D>
-__device__ __forceinline__ void transposed_offsets(int lane, int (&off)[D / 32][2]) {
+template <int D, int DT>
+__device__ __forceinline__ void transposed_offsets(int lane, int (&off)[DT][2]) {
   const int i16 = lane & 15, dgrp = (lane >> 4) & 1, g = lane >> 5;
   const int r0 = 4 * g + (i16 >> 2);
 #pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt) {
+  for (int dt = 0; dt < DT; ++dt) {
     const int chunk = 4 * dt + 2 * dgrp + ((i16 & 3) >> 1);
     off[dt][0] = Tile<D>::off(r0, chunk) + (i16 & 1) * 8;
     off[dt][1] = Tile<D>::off(r0 + 8, chunk) + (i16 & 1) * 8;
@@ -392,11 +392,10 @@ __device__ __forceinline__ void store_staged_rows(const char *stage, T *g_row0, 
   }
 }
 
-template <typename T, int D, bool PAD>
-__device__ __forceinline__ void store_tile_rows(char *stage, const floatx16 (&acc)[D / 32], float row_scale, T *g_row0,
+template <typename T, int D, bool PAD, int DT>
+__device__ __forceinline__ void store_tile_rows(char *stage, const floatx16 (&acc)[DT], float row_scale, T *g_row0,
                                                 int64_t row_stride, int lane, int row_lo, int row_hi, int real_d) {
   using TL = Tile<D>;
-  constexpr int DT = D / 32;
   asm volatile("" : "+v"(lane));  // as in store_staged_rows
   const int m = lane & 31, g = lane >> 5;
 #pragma unroll
