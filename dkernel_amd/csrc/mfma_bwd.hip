@@ -684,8 +684,12 @@ struct DkdvSmem {
   static constexpr int kBytes = kX + 2 * 2 * 4096;
 };
 
+// At the 64-wide tile a step is eight multiplies per wave against the same barrier, waits and scalar work as at the
+// 128-wide one, so a third workgroup per CU (45 KB of LDS and 166 registers each) fills what two leave idle: training,
+// 64 dims, two / three workgroups, us: 32 heads x 8192 tokens 558 / 523, 4 x 3000 tokens of 12 heads with global blocks of
+// 32 334 / 310.
 template <typename T, int D, bool PAD, bool SUB, int KD = D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, D == 256 ? 1 : 2))) void mfma_dkdv_kernel(const BwdParams p, int head_split) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, D == 64 ? 3 : D == 256 ? 1 : 2))) void mfma_dkdv_kernel(const BwdParams p, int head_split) {
   using M = Mma<T>;
   using vec8 = typename M::vec8;
   using TL = Tile<D>;
