@@ -59,6 +59,10 @@ class BwdArgs(C.Structure):
                 ("workspace", vp), ("workspace_bytes", C.c_size_t), ("stream", vp)]
 
 
+class RowLengths(C.Structure):
+    _fields_ = [("csr_rows", vp), ("csr_pairs", vp), ("csc_rows", vp)]
+
+
 class PagedKV(C.Structure):
     _fields_ = [("block_table", vp), ("table_stride_b", i64), ("page_stride_k", i64), ("page_stride_v", i64),
                 ("page_size", i32), ("kv_dtype", i32), ("k_scale", f32), ("v_scale", f32)]
@@ -90,6 +94,8 @@ SYMBOLS = {
     "dk_fwd_paged": (C.c_int, [C.POINTER(FwdArgs), C.POINTER(PagedKV)]),
     "dk_bwd": (C.c_int, [C.POINTER(BwdArgs)]),
     "dk_bwd_workspace_bytes": (C.c_size_t, [C.POINTER(BwdArgs)]),
+    "dk_bwd_balanced": (C.c_int, [C.POINTER(BwdArgs), C.POINTER(RowLengths)]),
+    "dk_bwd_balanced_workspace_bytes": (C.c_size_t, [C.POINTER(BwdArgs), C.POINTER(RowLengths)]),
     "dk_combine": (C.c_int, [C.POINTER(CombineArgs)]),
     "dk_combine_bwd": (C.c_int, [C.POINTER(CombineArgs)]),
 }

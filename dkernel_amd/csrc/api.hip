@@ -119,7 +119,7 @@ static int make_fwd_params(const dk_fwd_args *a, FwdParams &p) {
 
 // Checks the backward arguments and fills the kernel parameter block.  `empty` is set when
 // there is nothing to compute (no pointers are looked at then).
-static int make_bwd_params(const dk_bwd_args *a, BwdParams &p, bool &empty) {
+static int make_bwd_params(const dk_bwd_args *a, const dk_row_lengths *lengths, BwdParams &p, bool &empty) {
   empty = false;
   DK_REQUIRE(a != nullptr, "args is NULL");
   int rc = check_common(a->seqs, a->num_q_heads, a->num_kv_heads, a->head_dim, a->dtype, a->causal);
@@ -154,6 +154,11 @@ static int make_bwd_params(const dk_bwd_args *a, BwdParams &p, bool &empty) {
   p.delta = a->delta;
   p.csr = view(a->csr);
   p.csc = view(a->csc);
+  if (lengths) {
+    if (p.csr.order) p.csr.row_lengths = lengths->csr_rows;
+    if (p.csr.pair_order) p.csr.pair_lengths = lengths->csr_pairs;
+    if (p.csc.order) p.csc.row_lengths = lengths->csc_rows;
+  }
   p.Hq = a->num_q_heads;
   p.Hkv = a->num_kv_heads;
   p.D = a->head_dim;
@@ -257,12 +262,16 @@ int dk_fwd(const dk_fwd_args *a) {
   return launch_generic_fwd(p, a->dtype, stream);
 }
 
-size_t dk_bwd_workspace_bytes(const dk_bwd_args *a) {
+size_t dk_bwd_workspace_bytes(const dk_bwd_args *a) { return dk_bwd_balanced_workspace_bytes(a, nullptr); }
+
+size_t dk_bwd_balanced_workspace_bytes(const dk_bwd_args *a, const dk_row_lengths *lengths) {
   BwdParams p;
   bool empty;
-  if (make_bwd_params(a, p, empty) != DK_OK || empty) return 0;
+  if (make_bwd_params(a, lengths, p, empty) != DK_OK || empty) return 0;
   if (a->impl != DK_IMPL_GENERIC && mfma_bwd_supported(p, a->dtype)) return mfma_bwd_workspace_bytes(p);
-  if (a->impl == DK_IMPL_AUTO && mfma_f32_bwd_supported(p, a->dtype, true)) return mfma_f32_bwd_workspace_bytes(p);
+  if ((a->impl != DK_IMPL_GENERIC && mfma_f32_bwd_supported(p, a->dtype, false)) ||
+      (a->impl == DK_IMPL_AUTO && mfma_f32_bwd_supported(p, a->dtype, true)))
+    return mfma_f32_bwd_workspace_bytes(p);
   return 0;
 }
 
@@ -301,12 +310,14 @@ int dk_fwd_paged(const dk_fwd_args *a, const dk_paged_kv *pg) {
   return launch_decode(p, a->dtype, a->workspace, a->workspace_bytes, (hipStream_t)a->stream);
 }
 
-int dk_bwd(const dk_bwd_args *a) {
+int dk_bwd(const dk_bwd_args *a) { return dk_bwd_balanced(a, nullptr); }
+
+int dk_bwd_balanced(const dk_bwd_args *a, const dk_row_lengths *lengths) {
   clear_error();
   clear_kernels();
   BwdParams p;
   bool empty;
-  const int rc = make_bwd_params(a, p, empty);
+  const int rc = make_bwd_params(a, lengths, p, empty);
   if (rc || empty) return rc;
   hipStream_t stream = (hipStream_t)a->stream;
   if (a->impl != DK_IMPL_GENERIC) {

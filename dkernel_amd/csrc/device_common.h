@@ -57,6 +57,21 @@ struct LutView {
   int32_t uneven = 0;  // the heads hold clearly different numbers of entries
   int32_t fixed_walk = 0;  // a row's entries are taken in one order, whatever the size of the launch
   int32_t rot = 0;     // set per launch (head_rotation): 0, or 1 + shift of grid_head()
+  // optional, host memory: entries of the i-th row (pair of rows) of the order, the most in any head
+  const int32_t *row_lengths = nullptr, *pair_lengths = nullptr;
+};
+
+// Rows (or columns, or pairs of rows) of a backward launch that are cut into segments of their own
+// workgroups: each leaves an fp32 partial sum in memory and a second kernel adds a row's partials in order
+// (segment_sum_kernel, mfma_bwd.hip).  Work item y of the launch is segment 1 of the first n[1] rows of the
+// table's order, then segment 2 of the first n[2], ..., at last segment 0 of all of them: the order is by
+// descending length, so the rows that have a segment s come first in it.
+constexpr int kMaxSegments = 16;
+struct SegView {
+  int32_t entries = 0;  // entries per segment, 0: no row is cut
+  int32_t n[kMaxSegments] = {};  // rows that have a segment s in any head (n[0]: unused)
+  float *partial = nullptr;  // [batch][heads][slots] partial sums, slot = segment * n[1] + place in the order
+  int32_t slots = 0;
 };
 
 // Workgroups reach the chip's 32 queues (8 dies x 4 shader engines) by their linear id, in order.
@@ -80,6 +95,61 @@ __device__ __forceinline__ int grid_head(const LutView &l) {
   unsigned x = blockIdx.x;
   if (l.rot) x = (x + (blockIdx.y >> (l.rot - 1))) % gridDim.x;
   return __builtin_amdgcn_readfirstlane((int)x);
+}
+
+// Segments of a row of `len` entries: len / entries, rounded.
+__host__ __device__ inline int row_segments(int len, int entries) {
+  const int n = (2 * len + entries) / (2 * entries);
+  return n < 1 ? 1 : n;
+}
+// Whether and how a launch cuts its long rows.  lengths: entries of the rows in the table's order, `per_step` of them a
+// step (two for pairs of rows, which mostly list the same columns); copies: heads x batch; slots: workgroups that the
+// chip holds at once.  A workgroup costs its steps and kStart more.  Rows are cut when the longest one takes more than
+// `limit` times what every slot has to do on average (below that the hand-out by descending length evens it out), into
+// segments of `share` times the average and of at least eight steps: shorter ones cost more in start-up and
+// partial sums than they even out.  Below kWorth steps the kernel that adds the sums takes what the cut gains.
+inline SegView plan_segments(const int32_t *lengths, int rows, int per_step, int64_t copies, int slots, double limit, double share) {
+  constexpr int kStart = 5, kLeast = 8, kWorth = 20;
+  SegView s;
+  if (!lengths || rows < 1) return s;
+  auto steps = [&](int i) { return (lengths[i] + per_step - 1) / per_step; };
+  int64_t total = 0;
+  for (int i = 0; i < rows; ++i) total += steps(i) + kStart;
+  const double average = (double)total * (double)copies / slots;
+  const int longest = steps(0);
+  if (longest < kWorth || longest + kStart <= limit * average) return s;
+  int entries = average * share > kLeast ? (int)(average * share) : kLeast;
+  const int least = (longest + kMaxSegments - 2) / (kMaxSegments - 1);
+  if (entries < least) entries = least;
+  const int most = row_segments(longest, entries);
+  if (most < 2) return s;
+  s.entries = entries;
+  for (int i = 0; i < rows; ++i)
+    for (int j = row_segments(steps(i), entries) - 1; j > 0; --j)
+      if (j < kMaxSegments) ++s.n[j];
+  s.slots = most * s.n[1];
+  return s;
+}
+
+// ... of the row at `place` of the order; never more than the launch has work items for
+__device__ __forceinline__ int planned_segments(const SegView &s, int place, int len) {
+  int have = 1;
+#pragma unroll
+  for (int i = 1; i < kMaxSegments; ++i) have += place < s.n[i] ? 1 : 0;
+  return min(__builtin_amdgcn_readfirstlane(row_segments(len, s.entries)), have);  // (integer division runs on the VALU)
+}
+// (place in the order, segment) of work item y
+__device__ __forceinline__ void find_segment(const SegView &s, int y, int &place, int &seg) {
+  place = y, seg = 0;
+  if (s.entries == 0) return;
+  bool found = false;
+#pragma unroll
+  for (int i = 1; i < kMaxSegments; ++i) {
+    const bool here = !found && place < s.n[i];
+    seg = here ? i : seg;
+    found |= here;
+    place -= found ? 0 : s.n[i];
+  }
 }
 
 struct SeqView {
@@ -128,6 +198,8 @@ struct BwdParams {
   int32_t Hq, Hkv, D, causal;
   float sm_scale, scale_log2;
   int32_t vec_ok;
+  SegView seg;       // set per launch
+  int32_t trim = 0;  // the column table lists rows beyond the queries (it was built for longer sequences)
 };
 
 // Which LUT head serves q head h (h is the same for every lane of a wave).

@@ -25,6 +25,7 @@
 // into rings of stages, in the swizzled row-major layout of mfma_common.h.
 #include <climits>
 
+#include "bwd_scratch.h"
 #include "common.h"
 #include "device_common.h"
 #include "mfma_common.h"
@@ -379,8 +380,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   const int first_rb = sq.past / 64, last_rb = (sq.past + sq.q_len - 1) / 64;
   const int h = grid_head(p.csr);
   int u = (first_rb >> 1) + pairs_y - 1 - (int)blockIdx.y;  // longest rows first (of a causal pattern)
+  int place, seg;  // (long pairs cut into segments: with the table's own order only)
+  find_segment(p.seg, blockIdx.y, place, seg);
   if (p.csr.pair_order)  // the table's own order, longest pairs first (the grid then covers every pair of it)
-    u = scalar_load(p.csr.pair_order + lut_head(p.csr, h, p.Hq, p.Hkv) * p.csr.order_sh + blockIdx.y);
+    u = scalar_load(p.csr.pair_order + lut_head(p.csr, h, p.Hq, p.Hkv) * p.csr.order_sh + place);
   if (u > (last_rb >> 1) || u < (first_rb >> 1)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -392,6 +395,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   const int pos = row0 + m;
   const int qi = pos - sq.past;
   const bool row_ok = qi >= 0 && qi < sq.q_len;  // (a table row without queries of this sequence: false everywhere)
+  // the two table rows: entries [e0, emid) are row 2u, [emid, e1) row 2u + 1 (consecutive rows
+  // follow each other in the table); a row without queries of this sequence contributes nothing
+  const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
+  int e0 = 0, emid = 0, e1 = 0;
+  {
+    const int32_t *rp = p.csr.ptr + lh * p.csr.ptr_sh;
+    if (ra < p.csr.num_rows) scalar_load2(rp + ra, rp + ra + 1, e0, emid);
+    e1 = emid;
+    if (ra + 1 < p.csr.num_rows) e1 = scalar_load(rp + ra + 2);
+    if (ra < first_rb) e0 = emid;
+    if (ra + 1 > last_rb) e1 = emid;
+  }
+  const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
+  // this workgroup's entries of the two rows, and the place of its partial sum (-1: it takes both rows whole); kept
+  // in LDS until they are used (every wave writes and reads the same values)
+  __shared__ int part[5];
+  part[0] = e0, part[1] = emid, part[2] = emid, part[3] = e1, part[4] = -1;
+  if (p.seg.entries && place < p.seg.n[1]) {
+    const int segments = planned_segments(p.seg, place, (e1 - e0 + 1) / 2);
+    if (seg >= segments) return;
+    if (segments > 1) {
+      part[4] = seg * p.seg.n[1] + place;
+      // columns [lo, hi): an even share of the longer row's entries, and what the other row lists between them
+      const bool first_longer = emid - e0 >= e1 - emid;
+      const int l0 = first_longer ? e0 : emid, len = first_longer ? emid - e0 : e1 - emid;
+      const int s0 = __builtin_amdgcn_readfirstlane(len * seg / segments), s1 = __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
+      const int o0 = first_longer ? emid : e0, o1 = first_longer ? e1 : emid;
+      int p0 = o0, p1 = o1;
+      if (seg > 0) p0 = entry_lower_bound<EW>(cols, o0, o1, scalar_load(cols + (l0 + s0) * EW));
+      if (seg + 1 < segments) p1 = entry_lower_bound<EW>(cols, p0, o1, scalar_load(cols + (l0 + s1) * EW));
+      part[0] = first_longer ? l0 + s0 : p0, part[1] = first_longer ? l0 + s1 : p1;
+      part[2] = first_longer ? p0 : l0 + s0, part[3] = first_longer ? p1 : l0 + s1;
+    }
+  }
+
   if (PAD && p.D < KD) {  // the slots of the head dims beyond p.D stay zero for the whole kernel
     zero_tiles<NT>(smem, 2 * STAGE, tid);
     __syncthreads();
@@ -433,19 +471,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
     }
   }
 
-  // the two table rows: entries [e0, emid) are row 2u, [emid, e1) row 2u + 1 (consecutive rows
-  // follow each other in the table); a row without queries of this sequence contributes nothing
-  const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
-  int e0 = 0, emid = 0, e1 = 0;
-  {
-    const int32_t *rp = p.csr.ptr + lh * p.csr.ptr_sh;
-    if (ra < p.csr.num_rows) scalar_load2(rp + ra, rp + ra + 1, e0, emid);
-    e1 = emid;
-    if (ra + 1 < p.csr.num_rows) e1 = scalar_load(rp + ra + 2);
-    if (ra < first_rb) e0 = emid;
-    if (ra + 1 > last_rb) e1 = emid;
-  }
-  const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
   const T *kbase = (const T *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh;
   const T *vbase = (const T *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh;
 
@@ -490,17 +515,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   // (scalar), pend_a / pend_b the entries after them (vector loads, first used behind a tile
   // wait, so that no table read stalls the loop); flg_cur says which rows hold the current column.
   constexpr int kEnd = 0x7fffffff;
-  int a_pos = e0, b_pos = emid, head_a = kEnd, head_b = kEnd, pend_a = 0, pend_b = 0;
+  int a_pos = __builtin_amdgcn_readfirstlane(part[0]), b_pos = __builtin_amdgcn_readfirstlane(part[2]);
+  const int a_end = __builtin_amdgcn_readfirstlane(part[1]), b_end = __builtin_amdgcn_readfirstlane(part[3]);
+  int head_a = kEnd, head_b = kEnd, pend_a = 0, pend_b = 0;
   int hbits_a = 0, hbits_b = 0, pbits_a = 0, pbits_b = 0;  // SUB: the entries' masks, carried like the columns
-  if (a_pos < emid) head_a = scalar_load(cols + a_pos * EW);
-  if (b_pos < e1) head_b = scalar_load(cols + b_pos * EW);
-  if (a_pos + 1 < emid) pend_a = cols[(a_pos + 1) * EW];
-  if (b_pos + 1 < e1) pend_b = cols[(b_pos + 1) * EW];
+  if (a_pos < a_end) head_a = scalar_load(cols + a_pos * EW);
+  if (b_pos < b_end) head_b = scalar_load(cols + b_pos * EW);
+  if (a_pos + 1 < a_end) pend_a = cols[(a_pos + 1) * EW];
+  if (b_pos + 1 < b_end) pend_b = cols[(b_pos + 1) * EW];
   if constexpr (SUB) {
-    if (a_pos < emid) hbits_a = scalar_load(cols + a_pos * EW + 1);
-    if (b_pos < e1) hbits_b = scalar_load(cols + b_pos * EW + 1);
-    if (a_pos + 1 < emid) pbits_a = cols[(a_pos + 1) * EW + 1];
-    if (b_pos + 1 < e1) pbits_b = cols[(b_pos + 1) * EW + 1];
+    if (a_pos < a_end) hbits_a = scalar_load(cols + a_pos * EW + 1);
+    if (b_pos < b_end) hbits_b = scalar_load(cols + b_pos * EW + 1);
+    if (a_pos + 1 < a_end) pbits_a = cols[(a_pos + 1) * EW + 1];
+    if (b_pos + 1 < b_end) pbits_b = cols[(b_pos + 1) * EW + 1];
   }
   int col_cur = min(head_a, head_b);
   int flg_cur = (head_a == col_cur ? 1 : 0) | (head_b == col_cur ? 2 : 0);
@@ -531,7 +558,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   if (row_ok) {
     lse2 = lse_raw == -INFINITY ? INFINITY : lse_raw * kLog2e;
     delta = delta_rows[ts * 64 + rh * 32 + m] - dlse_raw;
-    if (g == 0) p.delta[((int64_t)sq.b * p.Hq + h) * p.seqs.max_q_len + qi] = delta;
+    if (g == 0 && part[4] < p.seg.n[1]) p.delta[((int64_t)sq.b * p.Hq + h) * p.seqs.max_q_len + qi] = delta;
   }
 
   auto block_step = [&](auto stage_tag) {
@@ -543,20 +570,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
     __syncthreads();  // the tile is visible; every wave is done with the other stage
     if (flg & 1) {
       ++a_pos;
-      head_a = a_pos < emid ? __builtin_amdgcn_readfirstlane(pend_a) : kEnd;
-      if (a_pos + 1 < emid) pend_a = cols[(a_pos + 1) * EW];
+      head_a = a_pos < a_end ? __builtin_amdgcn_readfirstlane(pend_a) : kEnd;
+      if (a_pos + 1 < a_end) pend_a = cols[(a_pos + 1) * EW];
       if constexpr (SUB) {
         hbits_a = __builtin_amdgcn_readfirstlane(pbits_a);
-        if (a_pos + 1 < emid) pbits_a = cols[(a_pos + 1) * EW + 1];
+        if (a_pos + 1 < a_end) pbits_a = cols[(a_pos + 1) * EW + 1];
       }
     }
     if (flg & 2) {
       ++b_pos;
-      head_b = b_pos < e1 ? __builtin_amdgcn_readfirstlane(pend_b) : kEnd;
-      if (b_pos + 1 < e1) pend_b = cols[(b_pos + 1) * EW];
+      head_b = b_pos < b_end ? __builtin_amdgcn_readfirstlane(pend_b) : kEnd;
+      if (b_pos + 1 < b_end) pend_b = cols[(b_pos + 1) * EW];
       if constexpr (SUB) {
         hbits_b = __builtin_amdgcn_readfirstlane(pbits_b);
-        if (b_pos + 1 < e1) pbits_b = cols[(b_pos + 1) * EW + 1];
+        if (b_pos + 1 < b_end) pbits_b = cols[(b_pos + 1) * EW + 1];
       }
     }
     const int col_next = min(head_a, head_b);
@@ -645,6 +672,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
     block_step(IntConst<1>{});
   }
 
+  const int slot_end = p.seg.entries ? __builtin_amdgcn_readfirstlane(part[4]) : -1;
+  if (slot_end >= 0) {  // fp32 partial sum, unscaled
+    int late = lane;  // (opaque: the addresses are computed here, not kept through the loop)
+    asm volatile("" : "+v"(late));
+    float *outp = p.seg.partial + ((((int64_t)sq.b * p.Hq + h) * p.seg.slots + slot_end) * 128 + wave * 32 + (late & 31)) * p.D + (late >> 5) * 4;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4)
+        if (!PAD || dt * 32 + r4 * 8 + (late >> 5) * 4 < p.D)
+          *reinterpret_cast<float4 *>(outp + dt * 32 + r4 * 8) =
+              make_float4(acc[dt][r4 * 4], acc[dt][r4 * 4 + 1], acc[dt][r4 * 4 + 2], acc[dt][r4 * 4 + 3]);
+    return;
+  }
   // every wave holds the finished dQ^T of its 32 rows
   __syncthreads();  // the K / V stages are free: each wave stages its tile in 32 rows of them
   {
@@ -717,10 +758,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // Columns are handed out longest first when the table says in which order: the hardware deals
   // workgroups to its shader engines round-robin and in order, so long columns that recur with a
   // period pile up on a few engines otherwise.
-  int cb = blockIdx.y;
+  int place, seg;  // (long columns are cut into segments in that order, where a workgroup takes one q head)
+  find_segment(p.seg, blockIdx.y, place, seg);
+  int cb = place;
   if (p.csc.order)  // (the grid then covers every column of the table)
-    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv) * p.csc.order_sh + blockIdx.y);
+    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv) * p.csc.order_sh + place);
   if (cb * 64 >= sq.k_len) return;
+  __shared__ int part[3];  // of a cut column: this workgroup's entries and the place of its sums (-1: not cut)
+  if (p.seg.entries) {
+    int e0, e1;
+    const int segments = column_part<EW>(p, lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv), cb, place, seg, sq, e0, e1);
+    if (seg >= segments) return;
+    part[0] = e0, part[1] = e1, part[2] = segments > 1 ? seg * p.seg.n[1] + place : -1;
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nh = wave & 1;  // key half; also the index of the (S wave, dP wave) pair
@@ -794,6 +844,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     int e0 = 0, e1 = 0;
     if (cb < p.csc.num_rows)
       scalar_load2(p.csc.ptr + lh * p.csc.ptr_sh + cb, p.csc.ptr + lh * p.csc.ptr_sh + cb + 1, e0, e1);
+    if (p.seg.entries)  // (every wave has written the same values)
+      e0 = __builtin_amdgcn_readfirstlane(part[0]), e1 = __builtin_amdgcn_readfirstlane(part[1]);
+    else if (p.trim)
+      e1 = entry_lower_bound<EW>(p.csc.idx + lh * p.csc.idx_sh, e0, e1, (sq.past + sq.q_len + 63) / 64);
     const int nstep = 2 * (e1 - e0);  // two steps of 32 q rows per listed block
     const int32_t *rows = p.csc.idx + lh * p.csc.idx_sh + e0 * EW;
     const T *qbase = (const T *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh;
@@ -1052,9 +1106,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // every wave holds the finished dV^T (S wave) or dK^T (dP wave) of its 32 keys
   const float out_scale = dp_wave ? p.sm_scale : 1.f;
   const TensorView &outv = dp_wave ? p.dk : p.dv;
-  if (head_split) {  // fp32 partial of this q head
+  const int slot = p.seg.entries ? __builtin_amdgcn_readfirstlane(part[2]) : -1;
+  if (head_split || slot >= 0) {  // fp32 partial of this q head, or of this segment
     if (!key_ok) return;
-    float *outp = (float *)outv.ptr + sq.b * outv.sb + out_head * outv.sh + (int64_t)key * outv.st;
+    float *outp;
+    if (slot >= 0)
+      outp = p.seg.partial + ((((int64_t)sq.b * gridDim.x + out_head) * p.seg.slots + slot) * 128 + (dp_wave ? 0 : 64) + nh * 32 + n) * p.D;
+    else
+      outp = (float *)outv.ptr + sq.b * outv.sb + out_head * outv.sh + (int64_t)key * outv.st;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -1175,6 +1234,94 @@ __global__ __launch_bounds__(256) void dkdv_group_sum_kernel(const float *part_k
   for (int i = 0; i < (int)sizeof(T) / 2; ++i) dst[i] = reinterpret_cast<const uint4 *>(o8)[i];
 }
 
+// Sums of the segments of long rows and columns: eight workgroups per (place in the order, head, batch) add the partial sums
+// of a row's segments in their order.  A slot has room for 128 rows of D floats: 128 q rows (dQ of a pair of rows), 64 q
+// rows (dQ of a row), or 64 keys of dK and the same 64 of dV.  Bound: latency of a launch over few bytes (64 KB per
+// segment at 128 dims).
+constexpr int kSumParts = 8;  // workgroups per row: one or two 16-byte pieces of every segment per thread
+template <typename TO>
+__global__ __launch_bounds__(256) void segment_sum_kernel(const LutView lut, const SegView seg, SegRows what, TensorView a, TensorView b,
+                                                          int Hq, int Hkv, int ratio, int D, float scale, int tokens,
+                                                          int past, int trim_rows, int entry_width) {
+  const int place = blockIdx.x / kSumParts, share = blockIdx.x % kSumParts, head = blockIdx.y;
+  const int h = head * ratio;  // a q head that the table head of this row serves
+  const int lh = lut_head(lut, h, Hq, Hkv);
+  const bool pairs = what == SegRows::kQueryPairs, queries = what != SegRows::kKeys;
+  const int row = (pairs ? lut.pair_order : lut.order)[lh * lut.order_sh + place];
+  const int32_t *ptr = lut.ptr + lh * lut.ptr_sh;
+  int len;
+  if (pairs) {
+    // (as the dQ kernel counts: a row without queries contributes nothing)
+    const int first_rb = past / 64, last_rb = (past + tokens - 1) / 64, ra = 2 * row;
+    if (row > (last_rb >> 1) || row < (first_rb >> 1)) return;
+    int e0 = ptr[ra], mid = ptr[ra + 1], e1 = mid;
+    if (ra + 1 < lut.num_rows) e1 = ptr[ra + 2];
+    if (ra < first_rb) e0 = mid;
+    if (ra + 1 > last_rb) e1 = mid;
+    len = (e1 - e0 + 1) / 2;
+  } else {
+    if (row * 64 >= tokens + (queries ? past : 0)) return;
+    int e0 = ptr[row], e1 = ptr[row + 1];
+    if (trim_rows > 0) {
+      const int32_t *idx = lut.idx + lh * lut.idx_sh;
+      int lo = e0, hi = e1;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (idx[mid * entry_width] < trim_rows)
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
+      e1 = lo;
+    }
+    len = e1 - e0;
+  }
+  const int segments = planned_segments(seg, place, len);
+  if (segments < 2) return;
+  const float *src = seg.partial + (((int64_t)blockIdx.z * gridDim.y + head) * seg.slots + place) * 128 * D;
+  const int64_t step = (int64_t)seg.n[1] * 128 * D;
+  const int pieces = D / 4, rows = (what == SegRows::kQueries ? 64 : 128) / kSumParts;
+  for (int j = threadIdx.x; j < rows * pieces; j += 256) {
+    const int i = share * rows * pieces + j, r = i / pieces, c = i % pieces;
+    const int t = pairs ? row * 128 + r - past : queries ? row * 64 + r - past : row * 64 + (r & 63);
+    if (t < 0 || t >= tokens) continue;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < segments; s0 += 4) {
+      float4 w[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) w[k] = *reinterpret_cast<const float4 *>(src + min(s0 + k, segments - 1) * step + (int64_t)i * 4);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (s0 + k < segments) v.x += w[k].x, v.y += w[k].y, v.z += w[k].z, v.w += w[k].w;
+    }
+    const TensorView &out = queries || r < 64 ? a : b;
+    TO *dst = (TO *)out.ptr + blockIdx.z * out.sb + head * out.sh + (int64_t)t * out.st + c * 4;
+    if constexpr (sizeof(TO) == 4)
+      *reinterpret_cast<float4 *>(dst) = make_float4(v.x * scale, v.y * scale, v.z * scale, v.w * scale);
+    else
+      *reinterpret_cast<uint2 *>(dst) = pack4<TO>(v.x * scale, v.y * scale, v.z * scale, v.w * scale);
+  }
+}
+
+template <typename TO>
+static int launch_segment_sum_t(const LutView &lut, const SegView &seg, SegRows what, const TensorView &a, const TensorView &b, int heads,
+                                const BwdParams &p, float scale, int tokens, int past, hipStream_t stream) {
+  DK_NOTE_KERNEL("segment_sum_kernel");
+  hipLaunchKernelGGL((segment_sum_kernel<TO>), dim3(seg.n[1] * kSumParts, heads, p.seqs.batch), dim3(256), 0, stream, lut, seg, what, a, b,
+                     p.Hq, p.Hkv, p.Hq / heads, p.D, scale, tokens, past, p.trim ? (past + p.seqs.max_q_len + 63) / 64 : 0,
+                     lut.entry_width);
+  DK_HIP_CHECK(hipGetLastError());
+  return DK_OK;
+}
+int launch_segment_sum(const LutView &lut, const SegView &seg, SegRows what, const TensorView &a, const TensorView &b, int dtype, int heads,
+                       const BwdParams &p, float scale, int tokens, int past, hipStream_t stream) {
+  switch (dtype) {
+    case DK_BF16: return launch_segment_sum_t<bf16_t>(lut, seg, what, a, b, heads, p, scale, tokens, past, stream);
+    case DK_F16: return launch_segment_sum_t<f16_t>(lut, seg, what, a, b, heads, p, scale, tokens, past, stream);
+    default: return launch_segment_sum_t<float>(lut, seg, what, a, b, heads, p, scale, tokens, past, stream);
+  }
+}
+
 template <typename T>
 static int launch_group_sum_t(const BwdParams &p, const float *part_k, const float *part_v, hipStream_t stream) {
   const int keys = p.seqs.max_k_len;
@@ -1197,13 +1344,19 @@ int launch_dkdv_group_sum(const BwdParams &p, int dtype, const float *part_k, co
 // Scratch for the head-split dK/dV pass: fp32 per-q-head partials of dK and dV (16-bit partials
 // would round each head's share before the sum).  Zero when the pass would not be split (one
 // q head per kv head).
-size_t mfma_bwd_workspace_bytes(const BwdParams &p) {
+size_t bwd_group_bytes(const BwdParams &p) {
   if (p.Hq == p.Hkv) return 0;
   const size_t need = 2 * (size_t)p.seqs.batch * p.Hq * p.seqs.max_k_len * p.D * sizeof(float);
   // beyond 4 GiB of partials (large batches) the pass keeps its in-workgroup loop over the group:
   // there are enough columns to balance then, and the scratch would rival the tensors themselves
   return need <= ((size_t)4 << 30) ? need : 0;
 }
+
+static BwdScratch mfma_bwd_scratch(const BwdParams &p) {
+  const int width = mfma_tile_width(p.D), per_cu = width == 64 ? 3 : width == 128 ? 2 : 1;
+  return plan_bwd_scratch(p, bwd_group_bytes(p), width == 256 ? 0 : 256 * per_cu, true, 256 * per_cu);
+}
+size_t mfma_bwd_workspace_bytes(const BwdParams &p) { return mfma_bwd_scratch(p).bytes; }
 
 bool mfma_bwd_supported(const BwdParams &p, int dtype) {
   return (dtype == DK_BF16 || dtype == DK_F16) && mfma_head_dim_ok(p.D) && p.csr.block_rows == 64 &&
@@ -1225,15 +1378,23 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
   DK_REQUIRE(tiles <= 65535 && cdiv(s.max_k_len, 64) <= 65535 && p.csc.num_rows <= 65535 &&
                  (!(p.csr.order || p.csr.pair_order) || p.csr.num_rows <= 65535),
              "sequence too long for one launch");
+  const BwdScratch scratch = usable_bwd_scratch(mfma_bwd_scratch(p), workspace, workspace_bytes);
   // dQ first: it also writes delta, which the dK/dV pass reads
   if constexpr (D <= 128) {  // two table rows per workgroup
     int pairs = (((past + s.max_q_len - 1) / 64) >> 1) - ((past / 64) >> 1) + 1;
     DK_ALLOW_DYNAMIC_LDS((mfma_dq_pair_kernel<T, D, PAD, SUB, KD>), smem_dq);
     if (p.csr.pair_order) pairs = (p.csr.num_rows + 1) / 2;  // handed out in the table's order: all of them
     BwdParams pq = p;
-    pq.csr.rot = head_rotation(p.csr, p.Hq, pairs);  // (uneven heads: dealt to the queues in rotation)
+    if (p.csr.pair_order && segment_items(scratch.dq, pairs) <= 65535) pq.seg = scratch.dq;
+    const int items = (int)segment_items(pq.seg, pairs);
+    pq.csr.rot = head_rotation(p.csr, p.Hq, items);  // (uneven heads: dealt to the queues in rotation)
     DK_NOTE_KERNEL(pq.csr.rot ? "mfma_dq_pair_kernel, heads in rotation" : "mfma_dq_pair_kernel");
-    hipLaunchKernelGGL((mfma_dq_pair_kernel<T, D, PAD, SUB, KD>), dim3(p.Hq, pairs, s.batch), dim3(256), smem_dq, stream, pq, pairs);
+    hipLaunchKernelGGL((mfma_dq_pair_kernel<T, D, PAD, SUB, KD>), dim3(p.Hq, items, s.batch), dim3(256), smem_dq, stream, pq, pairs);
+    DK_HIP_CHECK(hipGetLastError());
+    if (pq.seg.entries) {
+      const int dtype = std::is_same<T, bf16_t>::value ? DK_BF16 : DK_F16;
+      if (int rc = launch_segment_sum(p.csr, pq.seg, SegRows::kQueryPairs, p.dq, p.dq, dtype, p.Hq, p, p.sm_scale, s.max_q_len, past, stream)) return rc;
+    }
   } else {
     DK_ALLOW_DYNAMIC_LDS((mfma_dq_kernel<T, D, PAD, SUB>), smem_dq);
     const int rows = p.csr.order ? p.csr.num_rows : tiles;  // handed out in the table's order: all of them
@@ -1247,17 +1408,18 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
   // column (a vertical one near the start: every later q block, times the group size) alone
   // outlasts the average CU's share of the whole pass.  Given scratch, the pass runs one
   // workgroup per q head into per-head partials and a bandwidth-bound kernel sums each group.
-  const size_t need = mfma_bwd_workspace_bytes(p);
-  const bool per_q_head = need > 0 && workspace && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0;
+  const bool per_q_head = scratch.group > 0;
   // The table's longest-first order is taken unless the heads along grid.x are a multiple of the
   // 32 (XCD, shader engine) queues that the hardware deals workgroups to in turn: then every queue
   // serves whole heads, long columns and short ones alike, and the ascending order keeps
   // neighbouring columns - which share most of their Q / dO tiles - together in time (1.7 %
   // faster on the 32-head benchmark; with 8 or 16 heads the order is worth 20 - 40 %).
   BwdParams po = p;
-  if (((per_q_head ? p.Hq : p.Hkv) % 32) == 0) po.csc.order = nullptr;
+  po.trim = p.csr.num_rows > tiles + past / 64;
+  if (p.csc.order && segment_items(scratch.kv, p.csc.num_rows) <= 65535) po.seg = scratch.kv;
+  if (((per_q_head ? p.Hq : p.Hkv) % 32) == 0 && !po.seg.entries) po.csc.order = nullptr;
   // with a hand-out order the grid covers every column of the table (those beyond the keys exit at once)
-  const int cblocks = po.csc.order ? p.csc.num_rows : cdiv(s.max_k_len, 64);
+  const int cblocks = po.csc.order ? (int)segment_items(po.seg, p.csc.num_rows) : cdiv(s.max_k_len, 64);
   po.csc.rot = head_rotation(p.csc, per_q_head ? p.Hq : p.Hkv, cblocks);
   if (per_q_head) {
     BwdParams pp = po;
@@ -1269,11 +1431,17 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
                               : "mfma_dkdv_kernel (one workgroup per q head)");
     hipLaunchKernelGGL((mfma_dkdv_kernel<T, D, PAD, SUB, KD>), dim3(p.Hq, cblocks, s.batch), dim3(256), smem_dkdv, stream, pp, 1);
     DK_HIP_CHECK(hipGetLastError());
+    if (pp.seg.entries)
+      if (int rc = launch_segment_sum(p.csc, pp.seg, SegRows::kKeys, pp.dk, pp.dv, DK_F32, p.Hq, po, 1.f, s.max_k_len, past, stream)) return rc;
     return launch_group_sum_t<T>(p, part_k, part_v, stream);
   }
   DK_NOTE_KERNEL(po.csc.rot ? "mfma_dkdv_kernel, heads in rotation" : "mfma_dkdv_kernel");
   hipLaunchKernelGGL((mfma_dkdv_kernel<T, D, PAD, SUB, KD>), dim3(p.Hkv, cblocks, s.batch), dim3(256), smem_dkdv, stream, po, 0);
   DK_HIP_CHECK(hipGetLastError());
+  if (po.seg.entries) {
+    const int dtype = std::is_same<T, bf16_t>::value ? DK_BF16 : DK_F16;
+    return launch_segment_sum(p.csc, po.seg, SegRows::kKeys, p.dk, p.dv, dtype, p.Hkv, po, 1.f, s.max_k_len, past, stream);
+  }
   return DK_OK;
 }
 

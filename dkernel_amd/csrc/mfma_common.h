@@ -256,6 +256,31 @@ __device__ __forceinline__ void scalar_load2(const int32_t *p0, const int32_t *p
                : "s"(uniform_address(p0)), "s"(uniform_address(p1))
                : "memory");
 }
+// First of the sorted table entries [e0, e1) whose row / column is not below `limit` (wave-uniform).
+template <int EW>
+__device__ __forceinline__ int entry_lower_bound(const int32_t *idx, int e0, int e1, int limit) {
+  while (e0 < e1) {
+    const int mid = (e0 + e1) >> 1;
+    if (scalar_load(idx + mid * EW) < limit)
+      e0 = mid + 1;
+    else
+      e1 = mid;
+  }
+  return e0;
+}
+// dK/dV pass with columns cut into segments: the entries [e0, e1) of segment `seg` of column cb and how many
+// segments the column has.
+template <int EW>
+__device__ __forceinline__ int column_part(const BwdParams &p, int lh, int cb, int place, int seg, const SeqInfo &sq, int &e0, int &e1) {
+  e0 = e1 = 0;
+  if (cb < p.csc.num_rows)
+    scalar_load2(p.csc.ptr + lh * p.csc.ptr_sh + cb, p.csc.ptr + lh * p.csc.ptr_sh + cb + 1, e0, e1);
+  if (p.trim) e1 = entry_lower_bound<EW>(p.csc.idx + lh * p.csc.idx_sh, e0, e1, (sq.past + sq.q_len + 63) / 64);
+  const int len = e1 - e0, segments = planned_segments(p.seg, place, len);
+  e1 = e0 + __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
+  e0 += __builtin_amdgcn_readfirstlane(len * seg / segments);
+  return segments;
+}
 // base + rows * row_bytes for a wave-uniform, non-negative row count: one 32 x 32 -> 64 bit
 // unsigned multiply (two scalar instructions) where `base + (int64_t)rows * stride` takes a
 // signed 64 x 64 bit one (six).

@@ -26,18 +26,20 @@
 // is multiplied.  Bound: fp32 MFMA (a large fp32 product of the vendor library: 153 TFLOP/s).  Measured
 // forward / backward, us: 1 x 8192 tokens, 32 heads of 64 dims, local 16, vert 8: 906 / 2765 = 101 / 82
 // TFLOP/s (two waves of 32 x 64 quadrants over a single stage: 1114 / 3836); 8 heads x 1024 tokens of 64
-// dims: 26 / 126 (52 / 262); 16 heads x 2000 tokens of 128 dims, local 8, vert 4: 128 / 491 (fp32-FMA
-// kernels of generic_*.hip: 474 / 3189), where the longest row and column, one workgroup each, set the
-// time.
+// dims: 26 / 126 (52 / 262); 16 heads x 2000 tokens of 128 dims, local 8, vert 4: 128 / 430 (fp32-FMA
+// kernels of generic_*.hip: 474 / 3189; backward with every column whole: 491, the longest one's time).
 #include <type_traits>
 
+#include "bwd_scratch.h"
 #include "common.h"
 #include "device_common.h"
 #include "mfma_common.h"
 
 namespace dk {
 
-size_t mfma_bwd_workspace_bytes(const BwdParams &p);
+size_t bwd_group_bytes(const BwdParams &p);
+int launch_segment_sum(const LutView &lut, const SegView &seg, SegRows what, const TensorView &a, const TensorView &b, int dtype, int heads,
+                       const BwdParams &p, float scale, int tokens, int past, hipStream_t stream);
 int launch_dkdv_group_sum(const BwdParams &p, int dtype, const float *part_k, const float *part_v, hipStream_t stream);
 
 namespace f32 {
@@ -427,10 +429,23 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   const SeqInfo sq = load_seq(p.seqs, blockIdx.z, p.causal);
   const int h = grid_head(p.csr), kvh = __builtin_amdgcn_readfirstlane(h / (p.Hq / p.Hkv));
   int tile = tiles_y - 1 - (int)blockIdx.y;
+  int place, seg, segments = 1;  // (long rows are cut into segments: with the table's own order only)
+  find_segment(p.seg, blockIdx.y, place, seg);
   if (p.csr.order)
-    tile = scalar_load(p.csr.order + lut_head(p.csr, h, p.Hq, p.Hkv) * p.csr.order_sh + blockIdx.y) - sq.past / 64;
+    tile = scalar_load(p.csr.order + lut_head(p.csr, h, p.Hq, p.Hkv) * p.csr.order_sh + place) - sq.past / 64;
   if (tile < 0 || tile >= seq_row_blocks(sq, 64)) return;
   const int rb = sq.past / 64 + tile;
+  const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
+  int e0 = 0, e1 = 0;
+  if (rb < p.csr.num_rows)
+    scalar_load2(p.csr.ptr + lh * p.csr.ptr_sh + rb, p.csr.ptr + lh * p.csr.ptr_sh + rb + 1, e0, e1);
+  if (p.seg.entries && place < p.seg.n[1]) {
+    const int len = e1 - e0;
+    segments = planned_segments(p.seg, place, len);
+    if (seg >= segments) return;
+    e1 = e0 + __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
+    e0 += __builtin_amdgcn_readfirstlane(len * seg / segments);
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rh = wave & 1, kh = wave >> 1;
@@ -443,10 +458,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
     __syncthreads();
   }
 
-  const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
-  int e0 = 0, e1 = 0;
-  if (rb < p.csr.num_rows)
-    scalar_load2(p.csr.ptr + lh * p.csr.ptr_sh + rb, p.csr.ptr + lh * p.csr.ptr_sh + rb + 1, e0, e1);
   const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
   const float *kbase = (const float *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh;
   const float *vbase = (const float *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh;
@@ -507,7 +518,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   give_half<S::DT>(acc, kh == 1, buf, lane);
   __syncthreads();
   float *row = (float *)p.dq.ptr + sq.b * p.dq.sb + h * p.dq.sh + (int64_t)qi * p.dq.st;
-  take_half_and_store<S::DT>(acc, kh == 1, buf, lane, p.sm_scale, p.sm_scale, row, row_ok, p.D);
+  if (segments > 1)
+    row = p.seg.partial + ((((int64_t)sq.b * p.Hq + h) * p.seg.slots + seg * p.seg.n[1] + place) * 128 + rh * 32 + m) * p.D;
+  const float scale = segments > 1 ? 1.f : p.sm_scale;
+  take_half_and_store<S::DT>(acc, kh == 1, buf, lane, scale, scale, row, row_ok, p.D);
 }
 
 // dK / dV: workgroup = 64 keys of one kv head (the q heads of its group one after the other) or of
@@ -526,10 +540,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   const int out_head = grid_head(p.csc);
   const int kvh = head_split ? __builtin_amdgcn_readfirstlane(out_head / ratio) : out_head;
   const int gq_first = head_split ? out_head - kvh * ratio : 0, gq_end = head_split ? gq_first + 1 : ratio;
-  int cb = blockIdx.y;  // longest columns first when the table gives the order (as in the 16-bit pass)
+  // longest columns first when the table gives the order, long ones in segments (as in the 16-bit pass)
+  int place, seg;
+  find_segment(p.seg, blockIdx.y, place, seg);
+  int cb = place;
   if (p.csc.order)
-    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv) * p.csc.order_sh + blockIdx.y);
+    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv) * p.csc.order_sh + place);
   if (cb * 64 >= sq.k_len) return;
+  __shared__ int part[3];  // of a cut column: this workgroup's entries and the place of its sums (-1: not cut)
+  if (p.seg.entries) {
+    int e0, e1;
+    const int segments = column_part<1>(p, lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv), cb, place, seg, sq, e0, e1);
+    if (seg >= segments) return;
+    part[0] = e0, part[1] = e1, part[2] = segments > 1 ? seg * p.seg.n[1] + place : -1;
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nh = wave & 1, qh = wave >> 1;  // key half, q-row half
@@ -557,6 +581,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
     if (cb < p.csc.num_rows)
       scalar_load2(p.csc.ptr + lh * p.csc.ptr_sh + cb, p.csc.ptr + lh * p.csc.ptr_sh + cb + 1, e0, e1);
     const int32_t *rows = p.csc.idx + lh * p.csc.idx_sh;
+    if (p.seg.entries)  // (every wave has written the same values)
+      e0 = __builtin_amdgcn_readfirstlane(part[0]), e1 = __builtin_amdgcn_readfirstlane(part[1]);
     const float *qbase = (const float *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh;
     const float *dobase = (const float *)p.dout.ptr + sq.b * p.dout.sb + h * p.dout.sh;
     const float *lsebase = p.lse.ptr + sq.b * p.lse.sb + h * p.lse.sh;
@@ -630,6 +656,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   __syncthreads();
   float *dkp = (float *)p.dk.ptr + sq.b * p.dk.sb + out_head * p.dk.sh + (int64_t)key * p.dk.st;
   float *dvp = (float *)p.dv.ptr + sq.b * p.dv.sb + out_head * p.dv.sh + (int64_t)key * p.dv.st;
+  const int slot = p.seg.entries ? __builtin_amdgcn_readfirstlane(part[2]) : -1;
+  if (slot >= 0) {
+    dkp = p.seg.partial + ((((int64_t)sq.b * gridDim.x + out_head) * p.seg.slots + slot) * 128 + nh * 32 + n) * p.D;
+    dvp = dkp + 64 * p.D;
+  }
   take_half_and_store<S::DT>(dk, qh == 1, buf, lane, p.sm_scale, p.sm_scale, dkp, key_ok, p.D);
   take_half_and_store<S::DT>(dv, qh == 1, buf2, lane, 1.f, 1.f, dvp, key_ok, p.D);
 }
@@ -706,7 +737,11 @@ int launch_mfma_f32_fwd(const FwdParams &p, hipStream_t stream) {
 
 // Scratch of the dK/dV pass by q heads (wide head dims only: up to 64 the pass of a whole group is
 // short enough that the sum would cost what the balance gains)
-size_t mfma_f32_bwd_workspace_bytes(const BwdParams &p) { return p.D > 64 && p.D % 8 == 0 ? mfma_bwd_workspace_bytes(p) : 0; }
+static BwdScratch mfma_f32_bwd_scratch(const BwdParams &p) {
+  const int slots = 256 * (p.D <= 64 ? 2 : 1);
+  return plan_bwd_scratch(p, p.D > 64 && p.D % 8 == 0 ? bwd_group_bytes(p) : 0, slots, false, slots);
+}
+size_t mfma_f32_bwd_workspace_bytes(const BwdParams &p) { return mfma_f32_bwd_scratch(p).bytes; }
 
 int launch_mfma_f32_bwd(const BwdParams &p, void *workspace, size_t workspace_bytes, hipStream_t stream) {
   const SeqView &s = p.seqs;
@@ -721,22 +756,28 @@ int launch_mfma_f32_bwd(const BwdParams &p, void *workspace, size_t workspace_by
     hipLaunchKernelGGL(f32::delta_kernel<32>, dim3(cdiv(s.max_q_len, 8), p.Hq, s.batch), dim3(256), 0, stream, p);
   DK_HIP_CHECK(hipGetLastError());
   DK_REQUIRE(!p.csr.order || p.csr.num_rows <= 65535, "sequence too long for one launch");
-  const int rows = p.csr.order ? p.csr.num_rows : tiles;  // handed out in the table's order: all of them
+  const BwdScratch scratch = usable_bwd_scratch(mfma_f32_bwd_scratch(p), workspace, workspace_bytes);
   BwdParams pq = p;
+  if (p.csr.order && segment_items(scratch.dq, p.csr.num_rows) <= 65535) pq.seg = scratch.dq;
+  // handed out in the table's order: all of them
+  const int rows = p.csr.order ? (int)segment_items(pq.seg, p.csr.num_rows) : tiles;
   pq.csr.rot = head_rotation(p.csr, p.Hq, rows);
   DK_NOTE_KERNEL(pq.csr.rot ? "f32::dq_kernel, heads in rotation" : "f32::dq_kernel");
   using namespace f32;
   if (int rc = DK_BY_HEAD_DIM(launch_dq, p.D, pq, rows, stream)) return rc;
+  if (pq.seg.entries)
+    if (int rc = launch_segment_sum(p.csr, pq.seg, SegRows::kQueries, p.dq, p.dq, DK_F32, p.Hq, p, p.sm_scale, s.max_q_len, past, stream)) return rc;
   // Several q heads per kv head: one workgroup per q head into fp32 partials of its own and a sum over
   // each group, as in the 16-bit pass (one workgroup walking the whole group makes the longest column
   // outlast the rest of the launch).
-  const bool per_q_head = workspace && mfma_f32_bwd_workspace_bytes(p) && workspace_bytes >= mfma_f32_bwd_workspace_bytes(p) &&
-                          ((uintptr_t)workspace % 16) == 0;
+  const bool per_q_head = scratch.group > 0;
   const int heads = per_q_head ? p.Hq : p.Hkv;
   BwdParams po = p;  // the order only where heads do not line up with the hardware's 32 workgroup queues
-  if (heads % 32 == 0) po.csc.order = nullptr;
+  po.trim = p.csr.num_rows > tiles + past / 64;
+  if (p.csc.order && segment_items(scratch.kv, p.csc.num_rows) <= 65535) po.seg = scratch.kv;
+  if (heads % 32 == 0 && !po.seg.entries) po.csc.order = nullptr;
   DK_REQUIRE(p.csc.num_rows <= 65535, "sequence too long for one launch");
-  const int columns = po.csc.order ? p.csc.num_rows : cblocks;
+  const int columns = po.csc.order ? (int)segment_items(po.seg, p.csc.num_rows) : cblocks;
   po.csc.rot = head_rotation(p.csc, heads, columns);
   float *part_k = (float *)workspace, *part_v = part_k + (int64_t)s.batch * p.Hq * s.max_k_len * p.D;
   if (per_q_head) {
@@ -745,6 +786,8 @@ int launch_mfma_f32_bwd(const BwdParams &p, void *workspace, size_t workspace_by
   }
   DK_NOTE_KERNEL(po.csc.rot ? "f32::dkdv_kernel, heads in rotation" : "f32::dkdv_kernel");
   if (int rc = DK_BY_HEAD_DIM(launch_dkdv, p.D, po, columns, heads, stream)) return rc;
+  if (po.seg.entries)
+    if (int rc = launch_segment_sum(p.csc, po.seg, SegRows::kKeys, po.dk, po.dv, DK_F32, heads, po, 1.f, s.max_k_len, past, stream)) return rc;
   return per_q_head ? launch_dkdv_group_sum(p, DK_F32, part_k, part_v, stream) : DK_OK;
 }
 

@@ -5,6 +5,7 @@ that a model written against `dkernel` runs unchanged.
 """
 from __future__ import annotations
 
+import array
 import copy
 import math
 import warnings
@@ -61,6 +62,17 @@ def _unsorted_rows(pattern: Tensor) -> bool:
         return False
     later = torch.flip(torch.cummax(torch.flip(lens, (1,)), dim=1).values, (1,))[:, 1:]  # longest later row
     return bool((4 * lens[:, :-1] > 5 * later + 8).any())
+
+
+def _row_lengths(ptr: Tensor) -> array.array:
+    """Entries of a table's rows by descending length, the most over the heads at every place, followed by
+    those of the pairs of rows (2u, 2u + 1): what the backward's launches are planned by (host memory)."""
+    ptr = ptr if ptr.dim() == 2 else ptr[None]
+    if ptr.stride(0) == 0:
+        ptr = ptr[:1]
+    lens = (ptr[:, 1:] - ptr[:, :-1]).to("cpu", torch.int32)
+    pairs = torch.nn.functional.pad(lens, (0, lens.size(1) % 2)).view(lens.size(0), -1, 2).sum(2, dtype=torch.int32)
+    return array.array("i", torch.cat([torch.sort(x, dim=1, descending=True).values.amax(0) for x in (lens, pairs)]).tolist())
 
 
 class SparseAttention(torch.nn.Module):
@@ -269,6 +281,17 @@ class SparseAttention(torch.nn.Module):
             self.register_buffer("masked_csc_row", m_csc[1].to(torch.int32), persistent=False)
 
         self._kernel_tables = self._table_names()
+        # lengths of the rows and columns of the tables that the backward reads
+        csr, csc = self._backward_tables()
+        self.kwargs["row_lengths"] = tuple(
+            tuple(_row_lengths(getattr(self, name)) for name in names)
+            for names in [(csr, csc)] + ([("masked_csr_crow", "masked_csc_ccol")] if self.mask_tile is not None else []))
+
+    def _backward_tables(self) -> Tuple[str, str]:
+        if self.kernel_tile is not None:
+            return "kernel_csr_crow", "kernel_csc_ccol"
+        return ("layout_csr_crow" if self.exact_tile is None else "exact_csr_crow",
+                "exact_csc_ccol" if self.exact_tile is not None and self.exact_csc else "layout_csc_ccol")
 
     def _table_names(self) -> Tuple:
         """Names of the tables that the kernels read, with their tile sizes: (crow, col, rows, columns,

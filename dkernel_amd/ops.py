@@ -207,7 +207,8 @@ def _forward(ctx, q: Tensor, k: Tensor, v: Tensor, sm_scale: float,
              lut_max_row: int = 0,
              uneven_heads: bool = False,
              unsorted_rows: bool = False,
-             fixed_walk: bool = False) -> Tuple[Tensor, Optional[Tensor]]:
+             fixed_walk: bool = False,
+             row_lengths=()) -> Tuple[Tensor, Optional[Tensor]]:
     """Unpadded 4-D forward (training, prefill, single-token decode).
     Reference: dkernel/ops/sparse_attn_fwd.py:383-567.  `d_splits` is accepted
     and ignored (a Triton shared-memory workaround)."""
@@ -251,6 +252,7 @@ def _forward(ctx, q: Tensor, k: Tensor, v: Tensor, sm_scale: float,
     ctx.lut_group = lut_group
     ctx.uneven_heads = uneven_heads
     ctx.unsorted_rows = unsorted_rows
+    ctx.row_lengths = row_lengths
     return o, (lse if return_lse else None)
 
 
@@ -288,6 +290,9 @@ def _backward(ctx, do: Tensor, dlse: Optional[Tensor],
     masked = getattr(ctx, "masked_layouts", None)
     if masked is not None and _matrix_core_applies(q, k, v, o, do, dq, dk, dv):
         layout_csr, layout_csc = masked[0], masked[1]
+        lengths = ctx.row_lengths[1:]
+    else:
+        lengths = ctx.row_lengths[:1]
     uneven = getattr(ctx, "uneven_heads", False)
     args.csr = _lut(layout_csr, q.device, ctx.lut_group, uneven=uneven,
                     longest_first=getattr(ctx, "unsorted_rows", False))
@@ -297,12 +302,18 @@ def _backward(ctx, do: Tensor, dlse: Optional[Tensor],
     args.dtype, args.causal, args.impl = _DTYPES[q.dtype], int(bool(ctx.causal)), _impl
     args.sm_scale = float(ctx.sm_scale)
     args.stream = _stream()
+    rows = _lib.RowLengths()
+    for (csr_lengths, csc_lengths) in lengths:
+        n, m = args.csr.num_rows, args.csc.num_rows
+        assert len(csr_lengths) == n + (n + 1) // 2 and len(csc_lengths) == m + (m + 1) // 2
+        csr, csc = csr_lengths.buffer_info()[0], csc_lengths.buffer_info()[0]
+        rows = _lib.RowLengths(csr, csr + 4 * n, csc)
     lib = _lib.lib()
-    need = lib.dk_bwd_workspace_bytes(C.byref(args)) if _bwd_workspace else 0
-    if need:  # per-q-head dK/dV partials of the head-split pass (several q heads per kv head)
+    need = lib.dk_bwd_balanced_workspace_bytes(C.byref(args), C.byref(rows)) if _bwd_workspace else 0
+    if need:  # dK/dV partials per q head (several q heads per kv head), partial sums of long rows and columns
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
         args.workspace, args.workspace_bytes = ws.data_ptr(), need
-    _lib.check(lib.dk_bwd(C.byref(args)))
+    _lib.check(lib.dk_bwd_balanced(C.byref(args), C.byref(rows)))
     global last_bwd_kernels
     last_bwd_kernels = lib.dk_last_kernels()  # (backward runs on an autograd thread; the list is per thread)
     return dq, dk, dv
@@ -620,7 +631,7 @@ class _sparse_attention(torch.autograd.Function):
                 fwd_kwargs = {k_: v_ for k_, v_ in kwargs.items()
                               if k_ in ("inference", "out", "d_splits", "max_seqlen", "return_lse",
                                         "causal", "split_qkv", "lut_group", "uneven_heads", "unsorted_rows",
-                                        "fixed_walk")}
+                                        "fixed_walk", "row_lengths")}
                 fwd_kwargs["lut_max_row"] = lut_max_row
                 output, lse = _forward(ctx, q, k, v, sm_scale, layout_csr, seq_dim=seq_dim, **fwd_kwargs)
         return output, lse

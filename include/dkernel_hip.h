@@ -282,6 +282,20 @@ int dk_bwd(const dk_bwd_args *args);
 /* Scratch that dk_bwd can use for these arguments (0 = none useful; never more than 4 GiB). */
 size_t dk_bwd_workspace_bytes(const dk_bwd_args *args);
 
+/* Lengths of a backward call's tables in HOST memory, read during the call only: entries of the i-th row in the
+ * table's row_order (csr_rows, csc_rows: num_rows values) or of the i-th pair in its pair_order (csr_pairs:
+ * (num_rows + 1) / 2 values), the most over the heads.  Any may be NULL, and those of a table without that
+ * order are not read.  Wrong lengths cost time, never correctness. */
+typedef struct dk_row_lengths {
+  const int32_t *csr_rows, *csr_pairs, *csc_rows;
+} dk_row_lengths;
+
+/* dk_bwd that knows how long the rows of its tables are: rows and columns that would outlast the rest of the launch
+ * (global rows, vertical columns with few heads) are cut into segments of their own workgroups, whose fp32 sums
+ * lie in the workspace until a small kernel adds them.  Results differ from dk_bwd's by the order of those sums. */
+int dk_bwd_balanced(const dk_bwd_args *args, const dk_row_lengths *lengths);
+size_t dk_bwd_balanced_workspace_bytes(const dk_bwd_args *args, const dk_row_lengths *lengths);
+
 /* Merge of attention results computed over disjoint K/V partitions, per row:
  *     out = sum_p softmax_p(lse_p) * out_p
  * in fp32, rounded once to the outputs' type.  A partition in which a row saw no key
