@@ -8,20 +8,38 @@
 
 namespace dk {
 
+
 enum class SegRows { kKeys, kQueries, kQueryPairs };  // what the rows of a launch's segments are
 
 struct BwdScratch {
-  size_t group = 0;  // bytes of the per-q-head partials, 0: the pass works per kv head
+  size_t group = 0;  // bytes of the per-q-head partials of dK / dV, 0: the pass works per kv head
   SegView dq, kv;    // the two passes run one after the other and use the same bytes behind them
   size_t bytes = 0;  // all of it
 };
 
-// dq_slots, kv_slots: workgroups of the two passes that the chip holds at once (0: its rows are not cut);
-// dq_pairs: the dQ pass takes pairs of rows.
-inline BwdScratch plan_bwd_scratch(const BwdParams &p, size_t group, int dq_slots, bool dq_pairs, int kv_slots) {
+// Several q heads per kv head: whether a workgroup of the dK/dV pass walks a column for all of them, long columns cut into
+// segments, instead of one workgroup per q head into fp32 partials that are summed.  The walk saves those partials (twice
+// their bytes of traffic), but its pieces are longer by the group's size: below some hundred steps per resident workgroup
+// it needs so many segments to even them out that their sums cost as much.  Per q head / walk, us, training, 32 / 8 heads of
+// 128: 4000 tokens (68 steps) 394 / 418, 2 x 3000 of 96 dims (92) 474 / 496, 9000 of 16 / 4 heads (101) 600 / 619, 4 x 2048
+// (110) 661 / 610, 3 x 3000 (138) 808 / 742, 8000 (171) 937 / 872, 10000 (236) 1261 / 1186, 10000, local 8, vertical 16 (128)
+// 773 / 684; blocks of 32, 3 x 3000 (110) 675 / 614; 24 / 8 heads of 64, 6 x 2000 (85) 444 / 416.
+constexpr double kWalkFrom = 105;
+inline bool walk_groups(const BwdParams &p, size_t group, int kv_slots, double from) {
+  const int ratio = p.Hq / p.Hkv;
+  const bool one_table = p.csc.num_heads != p.Hq || p.csc.group % ratio == 0;  // for all q heads of a kv head
+  if (ratio == 1 || !one_table || !p.csc.row_lengths || !kv_slots) return false;
+  return group == 0 || average_steps(p.csc.row_lengths, p.csc.num_rows, 1, (int64_t)p.seqs.batch * p.Hkv, kv_slots, ratio) >= from;
+}
+
+// group: bytes of the per-q-head partials if the pass uses them; dq_slots, kv_slots: workgroups of the two passes that the
+// chip holds at once (0: its rows are not cut); dq_pairs: the dQ pass takes pairs of rows; walk_from: steps per resident
+// workgroup from which on the dK/dV pass walks whole groups although it could use partials (< 0: it does not walk them).
+inline BwdScratch plan_bwd_scratch(const BwdParams &p, size_t group, int dq_slots, bool dq_pairs, int kv_slots, double walk_from) {
   constexpr size_t kMost = (size_t)4 << 30;
+  const bool walk = walk_from >= 0 && walk_groups(p, group, kv_slots, walk_from);
   BwdScratch s;
-  s.group = s.bytes = group <= kMost ? group : 0;
+  s.group = s.bytes = !walk && group <= kMost ? group : 0;
   const int64_t copies = (int64_t)p.seqs.batch * p.Hq;
   // limit: longest row : average per slot from which on rows are cut; share: segment : average.  Both lower with masked
   // tiles, whose average is overestimated (long rows are mostly whole tiles, short ones mostly parts of them): 12 heads
@@ -35,16 +53,26 @@ inline BwdScratch plan_bwd_scratch(const BwdParams &p, size_t group, int dq_slot
   if (dq_slots)
     dq = dq_pairs ? plan_segments(p.csr.pair_lengths, (p.csr.num_rows + 1) / 2, 2, copies, dq_slots, limit, share)
                   : plan_segments(p.csr.row_lengths, p.csr.num_rows, 1, copies, dq_slots, limit, share);
-  // (columns only where a workgroup serves one q head)
-  if (kv_slots && (p.Hq == p.Hkv || s.group)) kv = plan_segments(p.csc.row_lengths, p.csc.num_rows, 1, copies, kv_slots, kv_limit, share);
+  // (walks: columns of one length that is a good part of the average are the rule, so they are cut finer: 3 x 4000 tokens, 24
+  // / 8 heads, share 0.6 / 0.5 / 0.4 884 / 854 / 822, 4 x 2048, 32 / 8 625 / - / 610)
+  if (walk)
+    kv = plan_segments(p.csc.row_lengths, p.csc.num_rows, 1, (int64_t)p.seqs.batch * p.Hkv, kv_slots, limit, 0.4, p.Hq / p.Hkv);
+  else if (kv_slots && (p.Hq == p.Hkv || s.group))
+    kv = plan_segments(p.csc.row_lengths, p.csc.num_rows, 1, copies, kv_slots, kv_limit, share);
   const size_t at = (s.group + 255) / 256 * 256;
-  const size_t need = at + (size_t)std::max(dq.slots, kv.slots) * copies * 128 * p.D * sizeof(float);
+  const int64_t dq_slots_all = dq.slots * copies, kv_slots_all = kv.slots * (walk ? copies / (p.Hq / p.Hkv) : copies);
+  const size_t need = at + (size_t)std::max(dq_slots_all, kv_slots_all) * 128 * p.D * sizeof(float);
+  if (walk && need > kMost && group) return plan_bwd_scratch(p, group, dq_slots, dq_pairs, kv_slots, -1);
   if (need > at && need <= kMost && p.D % 4 == 0) s.dq = dq, s.kv = kv, s.bytes = need;
   return s;
 }
 
-// The scratch as the caller's workspace allows it: all of it, the per-q-head partials only, or none.
-inline BwdScratch usable_bwd_scratch(BwdScratch s, void *workspace, size_t bytes) {
+// The scratch as the caller's workspace allows it: all of it, the per-q-head partials only, or none.  plan(walk) plans it,
+// with or without walks of whole groups.
+template <typename Plan>
+inline BwdScratch usable_bwd_scratch(Plan plan, void *workspace, size_t bytes) {
+  BwdScratch s = plan(true);
+  if (bytes < s.bytes) s = plan(false);
   const bool ok = workspace && ((uintptr_t)workspace % 16) == 0;
   if (!ok || bytes < s.group) return BwdScratch{};
   if (bytes < s.bytes) s.dq = s.kv = SegView{}, s.bytes = s.group;

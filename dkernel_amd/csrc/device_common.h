@@ -102,22 +102,29 @@ __host__ __device__ inline int row_segments(int len, int entries) {
   const int n = (2 * len + entries) / (2 * entries);
   return n < 1 ? 1 : n;
 }
+// Steps that every slot of a launch has to do on average (arguments as below); a workgroup costs its steps and kStartSteps more.
+constexpr int kStartSteps = 5;
+inline double average_steps(const int32_t *lengths, int rows, int per_step, int64_t copies, int slots, int heads) {
+  int64_t total = 0;
+  for (int i = 0; i < rows; ++i) total += (lengths[i] + per_step - 1) / per_step * heads + kStartSteps;
+  return (double)total * (double)copies / slots;
+}
 // Whether and how a launch cuts its long rows.  lengths: entries of the rows in the table's order, `per_step` of them a
-// step (two for pairs of rows, which mostly list the same columns); copies: heads x batch; slots: workgroups that the
-// chip holds at once.  A workgroup costs its steps and kStart more.  Rows are cut when the longest one takes more than
+// step (two for pairs of rows, which mostly list the same columns); heads: q heads that a workgroup walks for one row;
+// copies: workgroups per row (heads x batch); slots: workgroups that the chip holds at once.   Rows are cut when the longest one takes more than
 // `limit` times what every slot has to do on average (below that the hand-out by descending length evens it out), into
 // segments of `share` times the average and of at least eight steps: shorter ones cost more in start-up and
 // partial sums than they even out.  Below kWorth steps the kernel that adds the sums takes what the cut gains.
-inline SegView plan_segments(const int32_t *lengths, int rows, int per_step, int64_t copies, int slots, double limit, double share) {
-  constexpr int kStart = 5, kLeast = 8, kWorth = 20;
+inline SegView plan_segments(const int32_t *lengths, int rows, int per_step, int64_t copies, int slots, double limit, double share,
+                             int heads = 1) {
+  constexpr int kLeast = 8;
+  const int kWorth = heads > 1 ? 40 : 20;
   SegView s;
   if (!lengths || rows < 1) return s;
-  auto steps = [&](int i) { return (lengths[i] + per_step - 1) / per_step; };
-  int64_t total = 0;
-  for (int i = 0; i < rows; ++i) total += steps(i) + kStart;
-  const double average = (double)total * (double)copies / slots;
+  auto steps = [&](int i) { return (lengths[i] + per_step - 1) / per_step * heads; };
+  const double average = average_steps(lengths, rows, per_step, copies, slots, heads);
   const int longest = steps(0);
-  if (longest < kWorth || longest + kStart <= limit * average) return s;
+  if (longest < kWorth || longest + kStartSteps <= limit * average) return s;
   int entries = average * share > kLeast ? (int)(average * share) : kLeast;
   const int least = (longest + kMaxSegments - 2) / (kMaxSegments - 1);
   if (entries < least) entries = least;

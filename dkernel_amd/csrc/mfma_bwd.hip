@@ -726,7 +726,7 @@ struct DkdvSmem {
 };
 
 // At the 64-wide tile a step is eight multiplies per wave against the same barrier, waits and scalar work as at the
-// 128-wide one, so a third workgroup per CU (45 KB of LDS and 166 registers each) fills what two leave idle: training,
+// 128-wide one, so a third workgroup per CU (45 KB of LDS and 142 registers each) fills what two leave idle: training,
 // 64 dims, two / three workgroups, us: 32 heads x 8192 tokens 558 / 523, 4 x 3000 tokens of 12 heads with global blocks of
 // 32 334 / 310.
 template <typename T, int D, bool PAD, bool SUB, int KD = D>
@@ -753,8 +753,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   const int ratio = __builtin_amdgcn_readfirstlane(p.Hq / p.Hkv);  // integer division runs on the VALU
   const int out_head = grid_head(p.csc);
   const int kvh = head_split ? __builtin_amdgcn_readfirstlane(out_head / ratio) : out_head;
-  const int gq_first = head_split ? out_head - kvh * ratio : 0;
-  const int gq_end = head_split ? gq_first + 1 : ratio;
+  const int gq_base = head_split ? out_head - kvh * ratio : 0, heads = head_split ? 1 : ratio;
   // Columns are handed out longest first when the table says in which order: the hardware deals
   // workgroups to its shader engines round-robin and in order, so long columns that recur with a
   // period pile up on a few engines otherwise.
@@ -762,14 +761,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   find_segment(p.seg, blockIdx.y, place, seg);
   int cb = place;
   if (p.csc.order)  // (the grid then covers every column of the table)
-    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv) * p.csc.order_sh + place);
+    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_base, p.Hq, p.Hkv) * p.csc.order_sh + place);
   if (cb * 64 >= sq.k_len) return;
-  __shared__ int part[3];  // of a cut column: this workgroup's entries and the place of its sums (-1: not cut)
+  // of a cut column: the entries of each q head, the part of all heads' entries that is this workgroup's, and the
+  // place of its sums (-1: not cut)
+  __shared__ int part[5];
+  int gq_first = gq_base, gq_end = gq_base + heads;
   if (p.seg.entries) {
-    int e0, e1;
-    const int segments = column_part<EW>(p, lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv), cb, place, seg, sq, e0, e1);
+    int e0, len, lo, hi;
+    const int segments = column_part<EW>(p, lut_head(p.csc, kvh * ratio + gq_base, p.Hq, p.Hkv), cb, place, seg, heads, sq, e0, len, lo, hi);
     if (seg >= segments) return;
-    part[0] = e0, part[1] = e1, part[2] = segments > 1 ? seg * p.seg.n[1] + place : -1;
+    part[0] = e0, part[1] = len, part[2] = lo, part[3] = hi, part[4] = segments > 1 ? seg * p.seg.n[1] + place : -1;
+    if (segments > 1 && heads > 1)  // (then len > 0)
+      gq_first = __builtin_amdgcn_readfirstlane(lo / len), gq_end = __builtin_amdgcn_readfirstlane((hi + len - 1) / len);
   }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -836,282 +840,279 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // tiles whose first query index lies in [0, full_span) hold 32 queries
   const uint32_t full_span = sq.q_len >= S::kRows ? (uint32_t)(sq.q_len - S::kRows) + 1u : 0u;
   const uint32_t q_row_bytes = (uint32_t)p.q.st * 2u, do_row_bytes = (uint32_t)p.dout.st * 2u;
-  // (the body is instantiated twice: the first head also takes the K / V fragments out of LDS,
-  // unconditionally - guarded by a run-time test on gq the fragments and accumulators spill)
-  auto head_body = [&](int gq, auto first_tag) {
-    const int h = kvh * ratio + gq;
-    const int lh = lut_head(p.csc, h, p.Hq, p.Hkv);
-    int e0 = 0, e1 = 0;
-    if (cb < p.csc.num_rows)
-      scalar_load2(p.csc.ptr + lh * p.csc.ptr_sh + cb, p.csc.ptr + lh * p.csc.ptr_sh + cb + 1, e0, e1);
-    if (p.seg.entries)  // (every wave has written the same values)
-      e0 = __builtin_amdgcn_readfirstlane(part[0]), e1 = __builtin_amdgcn_readfirstlane(part[1]);
-    else if (p.trim)
-      e1 = entry_lower_bound<EW>(p.csc.idx + lh * p.csc.idx_sh, e0, e1, (sq.past + sq.q_len + 63) / 64);
-    const int nstep = 2 * (e1 - e0);  // two steps of 32 q rows per listed block
-    const int32_t *rows = p.csc.idx + lh * p.csc.idx_sh + e0 * EW;
-    const T *qbase = (const T *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh;
-    const T *dobase = (const T *)p.dout.ptr + sq.b * p.dout.sb + h * p.dout.sh;
-    const float *lsebase = p.lse.ptr + sq.b * p.lse.sb + h * p.lse.sh;
-    const float *deltabase = p.delta + ((int64_t)sq.b * p.Hq + h) * p.seqs.max_q_len;
+  // The q heads of the column form one stream of steps: behind a head's last entry the requests go on with the next
+  // head's first one, so that a head costs no start-up of its own.  gq: head of the next request; [ent, ent_end): its
+  // entries still to come.
+  int gq = gq_first - 1, ent = 0, ent_end = 0;
+  const int32_t *rows = nullptr;
+  const char *qbase = nullptr, *dobase = nullptr;
+  const float *lsebase = nullptr, *deltabase = nullptr;
+  auto have_entry = [&]() __attribute__((always_inline)) -> bool {
+    while (ent >= ent_end) {
+      if (++gq >= gq_end) return false;
+      const auto *a = late_arguments<BwdParams>();
+      const int h = kvh * ratio + gq;
+      const int tables = a->csc.num_heads, lh = tables == 1 ? 0 : tables == a->Hq ? h : kvh;
+      rows = a->csc.idx + lh * a->csc.idx_sh;
+      if (a->seg.entries) {  // (every wave has written the same values)
+        const int first = __builtin_amdgcn_readfirstlane(part[0]), len = __builtin_amdgcn_readfirstlane(part[1]);
+        const int before = (gq - gq_base) * len;  // entries of the heads before this one
+        ent = first + max(__builtin_amdgcn_readfirstlane(part[2]) - before, 0);
+        ent_end = first + min(__builtin_amdgcn_readfirstlane(part[3]) - before, len);
+      } else {
+        const int32_t *ptr = a->csc.ptr + lh * a->csc.ptr_sh + cb;
+        if (cb < a->csc.num_rows) scalar_load2(ptr, ptr + 1, ent, ent_end);
+        if (a->trim) ent_end = entry_lower_bound<EW>(rows, ent, ent_end, (sq.past + sq.q_len + 63) / 64);
+      }
+      qbase = reinterpret_cast<const char *>((const T *)a->q.ptr + sq.b * a->q.sb + h * a->q.sh);
+      dobase = reinterpret_cast<const char *>((const T *)a->dout.ptr + sq.b * a->dout.sb + h * a->dout.sh);
+      lsebase = a->lse.ptr + sq.b * a->lse.sb + h * a->lse.sh;
+      deltabase = a->delta + ((int64_t)sq.b * a->Hq + h) * a->seqs.max_q_len;
+    }
+    return true;
+  };
 
-    // asynchronous copy of half `half` of q block rbq: Q and dO tiles and the 32 lse / 32 delta
-    // values of its rows (lanes 0..31 copy lse, lanes 32..63 delta; every wave copies the same
-    // values, so that every wave issues the same number of load instructions).  Returns false
-    // when rows had to be zero-filled, i.e. when the per-wave load count is not LPT.
-    auto issue = [&](int rbq, int half, int qstage, int dostage) -> bool {
-      const int qi0 = rbq * 64 + half * 32 - sq.past;  // query index of the tile's first row
-      const int row = lane & 31;
-      const bool is_delta = lane >= 32;
-      char *dst = smem + S::kVec + qstage * 256;
-      // main path: a listed block whose 32 rows all are queries (one scalar compare: a padding
-      // entry, rbq < 0, gives a negative qi0)
-      if (D <= 128 && (uint32_t)qi0 < full_span) {
-        qload.issue_full(row_address(reinterpret_cast<const char *>(qbase), qi0, q_row_bytes),
-                         smem + S::kQ + qstage * S::kTile);
-        doload.issue_full(row_address(reinterpret_cast<const char *>(dobase), qi0, do_row_bytes),
-                          smem + S::kDo + dostage * S::kTile);
-        const float *src = is_delta ? deltabase + qi0 + row : lsebase + (int64_t)(qi0 + row) * p.lse.st;
-        lds_dma4_lane(src, lds_address(dst));
-        return true;
-      }
-      // rows before the first query (qi < 0, when k is longer than q) and beyond the last are zero-filled
-      const int lo = rbq < 0 ? S::kRows : -qi0, hi = sq.q_len - qi0;
-      const bool full = qload.issue(reinterpret_cast<const char *>(qbase + (int64_t)qi0 * p.q.st), lo, hi,
-                                    smem + S::kQ + qstage * S::kTile);
-      doload.issue(reinterpret_cast<const char *>(dobase + (int64_t)qi0 * p.dout.st), lo, hi,
-                   smem + S::kDo + dostage * S::kTile);
-      if (full) {
-        const float *src = is_delta ? deltabase + qi0 + row : lsebase + (int64_t)(qi0 + row) * p.lse.st;
-        lds_dma4_lane(src, lds_address(dst));
-      } else if (wave == 0) {
-        // rows outside the sequence: lse = +inf makes their probabilities 0
-        const int qi = qi0 + row;
-        float x = is_delta ? 0.f : INFINITY;
-        if (row >= lo && row < hi) x = is_delta ? deltabase[qi] : lsebase[(int64_t)qi * p.lse.st];
-        reinterpret_cast<float *>(dst)[lane] = x;
-      }
-      return full;
-    };
+  // asynchronous copy of half `half` of q block rbq: Q and dO tiles and the 32 lse / 32 delta
+  // values of its rows (lanes 0..31 copy lse, lanes 32..63 delta; every wave copies the same
+  // values, so that every wave issues the same number of load instructions).  Returns false
+  // when rows had to be zero-filled, i.e. when the per-wave load count is not LPT.
+  auto issue = [&](int rbq, int half, int qstage, int dostage) __attribute__((always_inline)) -> bool {
+    const int qi0 = rbq * 64 + half * 32 - sq.past;  // query index of the tile's first row
+    const int row = lane & 31;
+    const bool is_delta = lane >= 32;
+    char *dst = smem + S::kVec + qstage * 256;
+    // main path: a listed block whose 32 rows all are queries (one scalar compare: a padding
+    // entry, rbq < 0, gives a negative qi0)
+    if (D <= 128 && (uint32_t)qi0 < full_span) {
+      qload.issue_full(row_address(qbase, qi0, q_row_bytes),
+                       smem + S::kQ + qstage * S::kTile);
+      doload.issue_full(row_address(dobase, qi0, do_row_bytes),
+                        smem + S::kDo + dostage * S::kTile);
+      const float *src = is_delta ? deltabase + qi0 + row : lsebase + (int64_t)(qi0 + row) * p.lse.st;
+      lds_dma4_lane(src, lds_address(dst));
+      return true;
+    }
+    // rows before the first query (qi < 0, when k is longer than q) and beyond the last are zero-filled
+    const int lo = rbq < 0 ? S::kRows : -qi0, hi = sq.q_len - qi0;
+    const bool full = qload.issue(qbase + (int64_t)qi0 * q_row_bytes, lo, hi,
+                                  smem + S::kQ + qstage * S::kTile);
+    doload.issue(dobase + (int64_t)qi0 * do_row_bytes, lo, hi,
+                 smem + S::kDo + dostage * S::kTile);
+    if (full) {
+      const float *src = is_delta ? deltabase + qi0 + row : lsebase + (int64_t)(qi0 + row) * p.lse.st;
+      lds_dma4_lane(src, lds_address(dst));
+    } else if (wave == 0) {
+      // rows outside the sequence: lse = +inf makes their probabilities 0
+      const int qi = qi0 + row;
+      float x = is_delta ? 0.f : INFINITY;
+      if (row >= lo && row < hi) x = is_delta ? deltabase[qi] : lsebase[(int64_t)qi * p.lse.st];
+      reinterpret_cast<float *>(dst)[lane] = x;
+    }
+    return full;
+  };
 
-    // second half of the dP wave's work on step u (whose P the S wave published before the
-    // last barrier): dS = P (dP - delta), dK^T += Q^T dS
-    auto finish_dk = [&](int u, int qstage, const floatx16 &dp) {
-      const char *qs_ = smem + S::kQ + qstage * S::kTile;
-      const float *delta_s = reinterpret_cast<const float *>(smem + S::kVec + qstage * 256) + 32;
-      const float *x = xbuf + (u & 1) * 1024;
-      float ds[16];
+  // second half of the dP wave's work on step u (whose P the S wave published before the
+  // last barrier): dS = P (dP - delta), dK^T += Q^T dS
+  auto finish_dk = [&](int u, int qstage, const floatx16 &dp) {
+    const char *qs_ = smem + S::kQ + qstage * S::kTile;
+    const float *delta_s = reinterpret_cast<const float *>(smem + S::kVec + qstage * 256) + 32;
+    const float *x = xbuf + (u & 1) * 1024;
+    float ds[16];
 #pragma unroll
-      for (int r4 = 0; r4 < 4; ++r4) {
-        const float4 p4 = *reinterpret_cast<const float4 *>(x + (r4 * 64 + lane) * 4);
-        const float4 d4 = *reinterpret_cast<const float4 *>(delta_s + r4 * 8 + g * 4);
-        ds[r4 * 4 + 0] = p4.x * (dp[r4 * 4 + 0] - d4.x);  // without sm_scale
-        ds[r4 * 4 + 1] = p4.y * (dp[r4 * 4 + 1] - d4.y);
-        ds[r4 * 4 + 2] = p4.z * (dp[r4 * 4 + 2] - d4.z);
-        ds[r4 * 4 + 3] = p4.w * (dp[r4 * 4 + 3] - d4.w);
-      }
+    for (int r4 = 0; r4 < 4; ++r4) {
+      const float4 p4 = *reinterpret_cast<const float4 *>(x + (r4 * 64 + lane) * 4);
+      const float4 d4 = *reinterpret_cast<const float4 *>(delta_s + r4 * 8 + g * 4);
+      ds[r4 * 4 + 0] = p4.x * (dp[r4 * 4 + 0] - d4.x);  // without sm_scale
+      ds[r4 * 4 + 1] = p4.y * (dp[r4 * 4 + 1] - d4.y);
+      ds[r4 * 4 + 2] = p4.z * (dp[r4 * 4 + 2] - d4.z);
+      ds[r4 * 4 + 3] = p4.w * (dp[r4 * 4 + 3] - d4.w);
+    }
 #pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
-        const vec8 dsb = M::pack(ds + t2 * 8);
-        const int rowoff = t2 * 16 * TL::kRowBytes;
-        vec8 qt[DT];
+    for (int t2 = 0; t2 < 2; ++t2) {
+      const vec8 dsb = M::pack(ds + t2 * 8);
+      const int rowoff = t2 * 16 * TL::kRowBytes;
+      vec8 qt[DT];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) qt[dt] = lds_read_tr8<vec8>(qs_ + rowoff + tr[dt][0], qs_ + rowoff + tr[dt][1]);
+      for (int dt = 0; dt < DT; ++dt) qt[dt] = lds_read_tr8<vec8>(qs_ + rowoff + tr[dt][0], qs_ + rowoff + tr[dt][1]);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[dt] = M::mma(qt[dt], dsb, acc[dt]);
-      }
-    };
+      for (int dt = 0; dt < DT; ++dt) acc[dt] = M::mma(qt[dt], dsb, acc[dt]);
+    }
+  };
 
-    // The loop is instantiated once per role (not branched inside), so that the accumulators
-    // are not merged through a join every iteration.
-    auto run_head = [&](auto role_tag) {
-    constexpr bool kDp = decltype(role_tag)::value;
-    int issued = 0, iq = 0, ido = 0;  // next step to request and its ring positions
-    bool exact = true;                // every wave has issued exactly LPT load instructions per outstanding step
-    static_assert(S::kAhead == 2, "two steps in flight ahead of the one that is worked on");
-    int rb_next = 0;                  // q block of the next step to request (steps 2k and 2k + 1 share block k)
-    // SUB: the steps are the 32-row halves of the listed tiles that attend anything.  ent: next entry to
-    // read; left: halves of block rb_next still to come; s0, s1: the steps that the loop works on next,
-    // each as 32-row tile << 8 | the masks of its two quadrants, 4 bits each.
-    int ent = 0, left = 0, bits_next = 0, s0 = 0, s1 = 0;
-    auto request_next = [&](int &s) -> bool {  // SUB: requests the next such step; false behind the last one
-      while (left == 0 && ent < e1 - e0) {
+  // The loop is instantiated once per role (not branched inside), so that the accumulators
+  // are not merged through a join every iteration.
+  auto run_column = [&](auto role_tag) __attribute__((always_inline)) {
+  constexpr bool kDp = decltype(role_tag)::value;
+  int issued = 0, iq = 0, ido = 0;  // next step to request and its ring positions
+  bool exact = true;                // every wave has issued exactly LPT load instructions per outstanding step
+  static_assert(S::kAhead == 2, "two steps in flight ahead of the one that is worked on");
+  int rb_next = 0;                  // q block of the step that was requested last (steps 2k and 2k + 1 share a block)
+  // SUB: the steps are the 32-row halves of the listed tiles that attend anything.  left: halves of block
+  // rb_next still to come; s0, s1: the steps that the loop works on next, each as 32-row tile << 8 | the masks
+  // of its two quadrants, 4 bits each.
+  int left = 0, bits_next = 0, s0 = 0, s1 = 0;
+  auto request_next = [&](int &s) __attribute__((always_inline)) {  // requests the next step, if there is one
+    int half = issued & 1;
+    if constexpr (SUB) {
+      while (left == 0 && have_entry()) {
         scalar_load2(rows + ent * EW, rows + ent * EW + 1, rb_next, bits_next);
         ++ent;
         bits_next = tile_quadrants(bits_next, p.csc.sub_block);
         left = ((bits_next & 255) != 0 ? 1 : 0) | ((bits_next >> 8) != 0 ? 2 : 0);
       }
-      if (left == 0) return false;
-      const int half = left & 1 ? 0 : 1;
+      if (left == 0) return;
+      half = left & 1 ? 0 : 1;
       left &= left - 1;
       s = (rb_next * 2 + half) << 8 | (bits_next >> (8 * half) & 255);
-      exact = issue(rb_next, half, iq, ido) && exact;
-      iq = iq + 1 == S::kQStages ? 0 : iq + 1;
-      ido = ido + 1 == S::kDoStages ? 0 : ido + 1;
-      ++issued;
-      return true;
-    };
-    if constexpr (SUB) {
-      if (request_next(s0)) request_next(s1);
-    } else if (nstep > 0) {
-      rb_next = scalar_load(rows);
-      for (int i = 0; i < S::kAhead; ++i, ++issued) {
-        exact = issue(rb_next, i, iq, ido) && exact;
-        iq = iq + 1 == S::kQStages ? 0 : iq + 1;
-        ido = ido + 1 == S::kDoStages ? 0 : ido + 1;
-      }
+    } else if (half == 0) {
+      if (!have_entry()) return;
+      rb_next = scalar_load(rows + ent);
+      ++ent;
     }
-    if constexpr (kKvTiles) {
-      if constexpr (decltype(first_tag)::value) {
-        // the K / V tiles are older than the requests above: everything has landed behind this wait
-        wait_tile_loads();
-        __syncthreads();
-        const char *src = dp_wave ? v_tile : k_tile;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) kvf[ks] = lds_read8<vec8>(src + TL::off(nh * 32 + n, 2 * ks + g));
-        // (the loop's first barrier comes before anything is copied over the two tiles: step 2's Q
-        // tile is requested behind it, and the S waves write P behind it)
-      }
-    }
-    floatx16 dp_prev;
-    int cq = 0, cdo = 0, pq = 0;  // ring positions of step t (Q, dO) and of step t - 1 (Q)
-    int rbq = 0;                  // S wave: q block (SUB: 32-row tile) of the current step
-    int quad = 15, quad_prev = 15;  // SUB: masks of this wave's quadrant of steps t and t - 1 (0: both waves of the pair idle)
-    for (int t = 0; SUB ? t < issued : t < nstep; ++t) {
-      const int half = t & 1;
-      wait_tiles_ahead<LPT>(exact ? issued - t - 1 : 0);
-      __syncthreads();  // step t is visible, so is P of step t - 1; the stages of step t - 2 are free
-      if constexpr (SUB) {
-        rbq = s0 >> 8;
-        quad = (s0 >> (4 * nh)) & 15;
-        s0 = s1;
-        request_next(s1);
-      } else if (issued < nstep) {
-        if ((issued & 1) == 0) rb_next = scalar_load(rows + (issued >> 1) * EW);
-        exact = issue(rb_next, issued & 1, iq, ido) && exact;
-        iq = iq + 1 == S::kQStages ? 0 : iq + 1;
-        ido = ido + 1 == S::kDoStages ? 0 : ido + 1;
-        ++issued;
-      }
-      const char *qs_ = smem + S::kQ + cq * S::kTile, *dos_ = smem + S::kDo + cdo * S::kTile;
-      if constexpr (!kDp) {
-        if constexpr (!SUB) {
-          if (half == 0) rbq = scalar_load(rows + (t >> 1));
-        }
-        if (!kIdle || quad != 0) {
-          const int pos0 = SUB ? rbq * 32 : rbq * 64 + half * 32;  // first q position of this step
-          const float *lse_s = reinterpret_cast<const float *>(smem + S::kVec + cq * 256);
-          // S = Q K^T : rows = 32 q positions, cols = 32 keys
-          floatx16 sc;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) sc[r] = 0.f;
-          {
-            vec8 qa[KS];
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) qa[ks] = lds_read8<vec8>(qs_ + rd[ks]);
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) sc = M::mma(qa[ks], kvf[ks], sc);
-          }
-          // first dO^T operands do not depend on P
-          vec8 dot[DT];
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) dot[dt] = lds_read_tr8<vec8>(dos_ + tr[dt][0], dos_ + tr[dt][1]);
-          // P = exp2(S scale - lse log2e).  Rows outside the sequence arrive with lse = +inf
-          // (P = 0).  A row that saw no key has lse = -inf, but then every one of its entries
-          // here is masked by causality and the select below discards the infinite value, so no
-          // conversion is needed.  Masks are applied only in steps that need them (the diagonal
-          // block and the last, partial column block): wave-uniform choice between two loops.
-          const bool edge = (p.causal && (cb * 64 + nh * 32 + 31 > pos0)) || cb * 64 + 63 >= sq.k_len;
-          // last visible q-row offset test: key is visible to row pos iff key <= pos
-          const int kcmp = key_ok ? (p.causal ? key - pos0 : INT_MIN) : INT_MAX;  // masked iff kcmp > row offset
-          float *x = xbuf + (t & 1) * 1024;
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) {
-            // registers 4*r4 .. +3 are q rows 8*r4 + 4g + {0..3} of the step
-            const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + r4 * 8 + g * 4);
-            const float lr[4] = {l4.x, l4.y, l4.z, l4.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              sc[r4 * 4 + i] = fast_exp2(fmaf(sc[r4 * 4 + i], p.scale_log2, -lr[i] * kLog2e));
-          }
-          if (edge) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sc[r] = kcmp > (r >> 2) * 8 + g * 4 + (r & 3) ? 0.f : sc[r];
-          }
-          if constexpr (SUB) {
-            if (quad != 15) {  // wave-uniform: blocks of 16, the quadrant is not attended as a whole
-              const int key_bits = quad >> (n >> 4);
-#pragma unroll
-              for (int r = 0; r < 16; ++r) sc[r] = ((key_bits >> (2 * (r >> 3))) & 1) ? sc[r] : 0.f;
-            }
-          }
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4)
-            *reinterpret_cast<float4 *>(x + (r4 * 64 + lane) * 4) =
-                make_float4(sc[r4 * 4], sc[r4 * 4 + 1], sc[r4 * 4 + 2], sc[r4 * 4 + 3]);
-          // dV^T += dO^T P
-#pragma unroll
-          for (int t2 = 0; t2 < 2; ++t2) {
-            float pf[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) pf[i] = sc[t2 * 8 + i];
-            const vec8 pb = M::pack(pf);
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-              acc[dt] = M::mma(dot[dt], pb, acc[dt]);
-              if (t2 == 0) {
-                const int rowoff = 16 * TL::kRowBytes;
-                dot[dt] = lds_read_tr8<vec8>(dos_ + rowoff + tr[dt][0], dos_ + rowoff + tr[dt][1]);
-              }
-            }
-          }
-        }
-      } else {
-        // second half of step t - 1 first: it frees dp_prev for this step's dP
-        if (t > 0 && (!kIdle || quad_prev != 0)) finish_dk(t - 1, pq, dp_prev);
-        // dP = dO V^T
-#pragma unroll
-        for (int r = 0; r < 16; ++r) dp_prev[r] = 0.f;
-        if (!kIdle || quad != 0) {
-          vec8 da[KS];
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks) da[ks] = lds_read8<vec8>(dos_ + rd[ks]);
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks) dp_prev = M::mma(da[ks], kvf[ks], dp_prev);
-        }
-      }
-      if constexpr (SUB) quad_prev = quad;
-      pq = cq;
-      cq = cq + 1 == S::kQStages ? 0 : cq + 1;
-      cdo = cdo + 1 == S::kDoStages ? 0 : cdo + 1;
-    }
-    __syncthreads();  // P of the last step is visible
-    if constexpr (kDp) {
-      if constexpr (SUB) {
-        if (issued > 0 && (!kIdle || quad_prev != 0)) finish_dk(issued - 1, pq, dp_prev);
-      } else {
-        if (nstep > 0) finish_dk(nstep - 1, pq, dp_prev);
-      }
-    }
-    };
-    if (dp_wave)
-      run_head(BoolConst<true>{});
-    else
-      run_head(BoolConst<false>{});
-    if (gq + 1 < gq_end) __syncthreads();  // every wave is done with every stage before the next head reuses them
+    exact = issue(rb_next, half, iq, ido) && exact;
+    iq = iq + 1 == S::kQStages ? 0 : iq + 1;
+    ido = ido + 1 == S::kDoStages ? 0 : ido + 1;
+    ++issued;
   };
-  head_body(gq_first, BoolConst<true>{});
-  for (int gq = gq_first + 1; gq < gq_end; ++gq) head_body(gq, BoolConst<false>{});
+  for (int i = 0; i < S::kAhead; ++i) {
+    s0 = s1;
+    request_next(s1);
+  }
+  if constexpr (kKvTiles) {
+    // the K / V tiles are older than the requests above: everything has landed behind this wait
+    wait_tile_loads();
+    __syncthreads();
+    const char *src = dp_wave ? v_tile : k_tile;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) kvf[ks] = lds_read8<vec8>(src + TL::off(nh * 32 + n, 2 * ks + g));
+    // (the loop's first barrier comes before anything is copied over the two tiles: step 2's Q
+    // tile is requested behind it, and the S waves write P behind it)
+  }
+  floatx16 dp_prev;
+  int cq = 0, cdo = 0, pq = 0;  // ring positions of step t (Q, dO) and of step t - 1 (Q)
+  int rbq = 0;                  // S wave: q block (SUB: 32-row tile) of the current step
+  int quad = 15, quad_prev = 15;  // SUB: masks of this wave's quadrant of steps t and t - 1 (0: both waves of the pair idle)
+  for (int t = 0; t < issued; ++t) {
+    const int half = t & 1;
+    wait_tiles_ahead<LPT>(exact ? issued - t - 1 : 0);
+    __syncthreads();  // step t is visible, so is P of step t - 1; the stages of step t - 2 are free
+    if constexpr (SUB) {
+      rbq = s0 >> 8;
+      quad = (s0 >> (4 * nh)) & 15;
+      s0 = s1;
+    } else {
+      if (half == 0) rbq = rb_next;  // (both steps of the block have been requested, nothing behind it)
+    }
+    request_next(s1);
+    const char *qs_ = smem + S::kQ + cq * S::kTile, *dos_ = smem + S::kDo + cdo * S::kTile;
+    if constexpr (!kDp) {
+      if (!kIdle || quad != 0) {
+        const int pos0 = SUB ? rbq * 32 : rbq * 64 + half * 32;  // first q position of this step
+        const float *lse_s = reinterpret_cast<const float *>(smem + S::kVec + cq * 256);
+        // S = Q K^T : rows = 32 q positions, cols = 32 keys
+        floatx16 sc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+        {
+          vec8 qa[KS];
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) qa[ks] = lds_read8<vec8>(qs_ + rd[ks]);
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) sc = M::mma(qa[ks], kvf[ks], sc);
+        }
+        // first dO^T operands do not depend on P
+        vec8 dot[DT];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) dot[dt] = lds_read_tr8<vec8>(dos_ + tr[dt][0], dos_ + tr[dt][1]);
+        // P = exp2(S scale - lse log2e).  Rows outside the sequence arrive with lse = +inf
+        // (P = 0).  A row that saw no key has lse = -inf, but then every one of its entries
+        // here is masked by causality and the select below discards the infinite value, so no
+        // conversion is needed.  Masks are applied only in steps that need them (the diagonal
+        // block and the last, partial column block): wave-uniform choice between two loops.
+        const bool edge = (p.causal && (cb * 64 + nh * 32 + 31 > pos0)) || cb * 64 + 63 >= sq.k_len;
+        // last visible q-row offset test: key is visible to row pos iff key <= pos
+        const int kcmp = key_ok ? (p.causal ? key - pos0 : INT_MIN) : INT_MAX;  // masked iff kcmp > row offset
+        float *x = xbuf + (t & 1) * 1024;
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          // registers 4*r4 .. +3 are q rows 8*r4 + 4g + {0..3} of the step
+          const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + r4 * 8 + g * 4);
+          const float lr[4] = {l4.x, l4.y, l4.z, l4.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            sc[r4 * 4 + i] = fast_exp2(fmaf(sc[r4 * 4 + i], p.scale_log2, -lr[i] * kLog2e));
+        }
+        if (edge) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sc[r] = kcmp > (r >> 2) * 8 + g * 4 + (r & 3) ? 0.f : sc[r];
+        }
+        if constexpr (SUB) {
+          if (quad != 15) {  // wave-uniform: blocks of 16, the quadrant is not attended as a whole
+            const int key_bits = quad >> (n >> 4);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[r] = ((key_bits >> (2 * (r >> 3))) & 1) ? sc[r] : 0.f;
+          }
+        }
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+          *reinterpret_cast<float4 *>(x + (r4 * 64 + lane) * 4) =
+              make_float4(sc[r4 * 4], sc[r4 * 4 + 1], sc[r4 * 4 + 2], sc[r4 * 4 + 3]);
+        // dV^T += dO^T P
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2) {
+          float pf[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) pf[i] = sc[t2 * 8 + i];
+          const vec8 pb = M::pack(pf);
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            acc[dt] = M::mma(dot[dt], pb, acc[dt]);
+            if (t2 == 0) {
+              const int rowoff = 16 * TL::kRowBytes;
+              dot[dt] = lds_read_tr8<vec8>(dos_ + rowoff + tr[dt][0], dos_ + rowoff + tr[dt][1]);
+            }
+          }
+        }
+      }
+    } else {
+      // second half of step t - 1 first: it frees dp_prev for this step's dP
+      if (t > 0 && (!kIdle || quad_prev != 0)) finish_dk(t - 1, pq, dp_prev);
+      // dP = dO V^T
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dp_prev[r] = 0.f;
+      if (!kIdle || quad != 0) {
+        vec8 da[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) da[ks] = lds_read8<vec8>(dos_ + rd[ks]);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) dp_prev = M::mma(da[ks], kvf[ks], dp_prev);
+      }
+    }
+    if constexpr (SUB) quad_prev = quad;
+    pq = cq;
+    cq = cq + 1 == S::kQStages ? 0 : cq + 1;
+    cdo = cdo + 1 == S::kDoStages ? 0 : cdo + 1;
+  }
+  __syncthreads();  // P of the last step is visible
+  if constexpr (kDp) {
+    if (issued > 0 && (!kIdle || quad_prev != 0)) finish_dk(issued - 1, pq, dp_prev);
+  }
+  };
+  if (dp_wave)
+    run_column(BoolConst<true>{});
+  else
+    run_column(BoolConst<false>{});
 
   // every wave holds the finished dV^T (S wave) or dK^T (dP wave) of its 32 keys
-  const float out_scale = dp_wave ? p.sm_scale : 1.f;
-  const TensorView &outv = dp_wave ? p.dk : p.dv;
-  const int slot = p.seg.entries ? __builtin_amdgcn_readfirstlane(part[2]) : -1;
+  const auto *a = late_arguments<BwdParams>();
+  const auto &outv = dp_wave ? a->dk : a->dv;
+  const float out_scale = dp_wave ? a->sm_scale : 1.f;
+  const int slot = a->seg.entries ? __builtin_amdgcn_readfirstlane(part[4]) : -1;
   if (head_split || slot >= 0) {  // fp32 partial of this q head, or of this segment
     if (!key_ok) return;
     float *outp;
     if (slot >= 0)
-      outp = p.seg.partial + ((((int64_t)sq.b * gridDim.x + out_head) * p.seg.slots + slot) * 128 + (dp_wave ? 0 : 64) + nh * 32 + n) * p.D;
+      outp = a->seg.partial + ((((int64_t)sq.b * gridDim.x + out_head) * a->seg.slots + slot) * 128 + (dp_wave ? 0 : 64) + nh * 32 + n) * p.D;
     else
       outp = (float *)outv.ptr + sq.b * outv.sb + out_head * outv.sh + (int64_t)key * outv.st;
 #pragma unroll
@@ -1243,7 +1244,7 @@ template <typename TO>
 __global__ __launch_bounds__(256) void segment_sum_kernel(const LutView lut, const SegView seg, SegRows what, TensorView a, TensorView b,
                                                           int Hq, int Hkv, int ratio, int D, float scale, int tokens,
                                                           int past, int trim_rows, int entry_width) {
-  const int place = blockIdx.x / kSumParts, share = blockIdx.x % kSumParts, head = blockIdx.y;
+  const int place = blockIdx.x / kSumParts, share = blockIdx.x % kSumParts, head = blockIdx.y;  // ratio: q heads per `head`
   const int h = head * ratio;  // a q head that the table head of this row serves
   const int lh = lut_head(lut, h, Hq, Hkv);
   const bool pairs = what == SegRows::kQueryPairs, queries = what != SegRows::kKeys;
@@ -1274,7 +1275,7 @@ __global__ __launch_bounds__(256) void segment_sum_kernel(const LutView lut, con
       }
       e1 = lo;
     }
-    len = e1 - e0;
+    len = (e1 - e0) * ratio;  // (1 for queries)
   }
   const int segments = planned_segments(seg, place, len);
   if (segments < 2) return;
@@ -1352,11 +1353,11 @@ size_t bwd_group_bytes(const BwdParams &p) {
   return need <= ((size_t)4 << 30) ? need : 0;
 }
 
-static BwdScratch mfma_bwd_scratch(const BwdParams &p) {
+static BwdScratch mfma_bwd_scratch(const BwdParams &p, bool walk) {
   const int width = mfma_tile_width(p.D), per_cu = width == 64 ? 3 : width == 128 ? 2 : 1;
-  return plan_bwd_scratch(p, bwd_group_bytes(p), width == 256 ? 0 : 256 * per_cu, true, 256 * per_cu);
+  return plan_bwd_scratch(p, bwd_group_bytes(p), width == 256 ? 0 : 256 * per_cu, true, 256 * per_cu, walk ? kWalkFrom : -1);
 }
-size_t mfma_bwd_workspace_bytes(const BwdParams &p) { return mfma_bwd_scratch(p).bytes; }
+size_t mfma_bwd_workspace_bytes(const BwdParams &p) { return mfma_bwd_scratch(p, true).bytes; }
 
 bool mfma_bwd_supported(const BwdParams &p, int dtype) {
   return (dtype == DK_BF16 || dtype == DK_F16) && mfma_head_dim_ok(p.D) && p.csr.block_rows == 64 &&
@@ -1378,7 +1379,7 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
   DK_REQUIRE(tiles <= 65535 && cdiv(s.max_k_len, 64) <= 65535 && p.csc.num_rows <= 65535 &&
                  (!(p.csr.order || p.csr.pair_order) || p.csr.num_rows <= 65535),
              "sequence too long for one launch");
-  const BwdScratch scratch = usable_bwd_scratch(mfma_bwd_scratch(p), workspace, workspace_bytes);
+  const BwdScratch scratch = usable_bwd_scratch([&](bool walk) { return mfma_bwd_scratch(p, walk); }, workspace, workspace_bytes);
   // dQ first: it also writes delta, which the dK/dV pass reads
   if constexpr (D <= 128) {  // two table rows per workgroup
     int pairs = (((past + s.max_q_len - 1) / 64) >> 1) - ((past / 64) >> 1) + 1;
@@ -1404,10 +1405,10 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
     hipLaunchKernelGGL((mfma_dq_kernel<T, D, PAD, SUB>), dim3(p.Hq, rows, s.batch), dim3(256), smem_dq, stream, pq, rows);
   }
   DK_HIP_CHECK(hipGetLastError());
-  // With several q heads per kv head a workgroup per kv head walks all of them, and the longest
-  // column (a vertical one near the start: every later q block, times the group size) alone
-  // outlasts the average CU's share of the whole pass.  Given scratch, the pass runs one
-  // workgroup per q head into per-head partials and a bandwidth-bound kernel sums each group.
+  // With several q heads per kv head a workgroup walks a column for all of them, long columns in segments, or, where
+  // walk_groups() says so, the pass runs one workgroup per q head into per-head partials and a bandwidth-bound kernel sums
+  // each group.  (Without lengths to cut by, the longest column - a vertical one near the start: every later q block, times
+  // the group's size - alone would outlast the average CU's share of the whole pass.)
   const bool per_q_head = scratch.group > 0;
   // The table's longest-first order is taken unless the heads along grid.x are a multiple of the
   // 32 (XCD, shader engine) queues that the hardware deals workgroups to in turn: then every queue

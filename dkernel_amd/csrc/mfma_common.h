@@ -256,6 +256,14 @@ __device__ __forceinline__ void scalar_load2(const int32_t *p0, const int32_t *p
                : "s"(uniform_address(p0)), "s"(uniform_address(p1))
                : "memory");
 }
+// The kernel's first argument as it lies in memory, for code that runs once or rarely: read from the argument itself,
+// the values are fetched at the kernel's start and held in scalar registers through its loop, which spills them.
+template <typename P>
+__device__ __forceinline__ const __attribute__((address_space(4))) P *late_arguments() {
+  auto a = (const __attribute__((address_space(4))) P *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));  // (opaque: nothing is moved ahead of this place)
+  return a;
+}
 // First of the sorted table entries [e0, e1) whose row / column is not below `limit` (wave-uniform).
 template <int EW>
 __device__ __forceinline__ int entry_lower_bound(const int32_t *idx, int e0, int e1, int limit) {
@@ -268,17 +276,21 @@ __device__ __forceinline__ int entry_lower_bound(const int32_t *idx, int e0, int
   }
   return e0;
 }
-// dK/dV pass with columns cut into segments: the entries [e0, e1) of segment `seg` of column cb and how many
-// segments the column has.
+// dK/dV pass with columns cut into segments: a workgroup's column holds the entries [e0, e0 + len) for each of `heads`
+// q heads, one head after the other; segment `seg` is [lo, hi) of these heads * len.  Returns how many segments the
+// column has.
 template <int EW>
-__device__ __forceinline__ int column_part(const BwdParams &p, int lh, int cb, int place, int seg, const SeqInfo &sq, int &e0, int &e1) {
-  e0 = e1 = 0;
+__device__ __forceinline__ int column_part(const BwdParams &p, int lh, int cb, int place, int seg, int heads, const SeqInfo &sq,
+                                           int &e0, int &len, int &lo, int &hi) {
+  int e1 = 0;
+  e0 = 0;
   if (cb < p.csc.num_rows)
     scalar_load2(p.csc.ptr + lh * p.csc.ptr_sh + cb, p.csc.ptr + lh * p.csc.ptr_sh + cb + 1, e0, e1);
   if (p.trim) e1 = entry_lower_bound<EW>(p.csc.idx + lh * p.csc.idx_sh, e0, e1, (sq.past + sq.q_len + 63) / 64);
-  const int len = e1 - e0, segments = planned_segments(p.seg, place, len);
-  e1 = e0 + __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
-  e0 += __builtin_amdgcn_readfirstlane(len * seg / segments);
+  len = e1 - e0;
+  const int total = len * heads, segments = planned_segments(p.seg, place, total);
+  lo = __builtin_amdgcn_readfirstlane(total * seg / segments);
+  hi = __builtin_amdgcn_readfirstlane(total * (seg + 1) / segments);
   return segments;
 }
 // base + rows * row_bytes for a wave-uniform, non-negative row count: one 32 x 32 -> 64 bit

@@ -539,20 +539,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   const int ratio = __builtin_amdgcn_readfirstlane(p.Hq / p.Hkv);
   const int out_head = grid_head(p.csc);
   const int kvh = head_split ? __builtin_amdgcn_readfirstlane(out_head / ratio) : out_head;
-  const int gq_first = head_split ? out_head - kvh * ratio : 0, gq_end = head_split ? gq_first + 1 : ratio;
+  const int gq_base = head_split ? out_head - kvh * ratio : 0, heads = head_split ? 1 : ratio;
   // longest columns first when the table gives the order, long ones in segments (as in the 16-bit pass)
   int place, seg;
   find_segment(p.seg, blockIdx.y, place, seg);
   int cb = place;
   if (p.csc.order)
-    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv) * p.csc.order_sh + place);
+    cb = scalar_load(p.csc.order + lut_head(p.csc, kvh * ratio + gq_base, p.Hq, p.Hkv) * p.csc.order_sh + place);
   if (cb * 64 >= sq.k_len) return;
-  __shared__ int part[3];  // of a cut column: this workgroup's entries and the place of its sums (-1: not cut)
+  // of a cut column: the entries of each q head, the part of all heads' entries that is this workgroup's, and the
+  // place of its sums (-1: not cut)
+  __shared__ int part[5];
   if (p.seg.entries) {
-    int e0, e1;
-    const int segments = column_part<1>(p, lut_head(p.csc, kvh * ratio + gq_first, p.Hq, p.Hkv), cb, place, seg, sq, e0, e1);
+    int e0, len, lo, hi;
+    const int segments = column_part<1>(p, lut_head(p.csc, kvh * ratio + gq_base, p.Hq, p.Hkv), cb, place, seg, heads, sq, e0, len, lo, hi);
     if (seg >= segments) return;
-    part[0] = e0, part[1] = e1, part[2] = segments > 1 ? seg * p.seg.n[1] + place : -1;
+    part[0] = e0, part[1] = len, part[2] = lo, part[3] = hi, part[4] = segments > 1 ? seg * p.seg.n[1] + place : -1;
   }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -574,15 +576,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   qload.init(tid, 2 * p.q.st, 2 * p.D);
   doload.init(tid, 2 * p.dout.st, 2 * p.D);
 
-  for (int gq = gq_first; gq < gq_end; ++gq) {
+  // (the end is worked out again on every turn: one scalar less to keep)
+  for (int gq = gq_base; gq < (head_split ? gq_base + 1 : p.Hq / p.Hkv); ++gq) {
     const int h = kvh * ratio + gq;
     const int lh = lut_head(p.csc, h, p.Hq, p.Hkv);
     int e0 = 0, e1 = 0;
     if (cb < p.csc.num_rows)
       scalar_load2(p.csc.ptr + lh * p.csc.ptr_sh + cb, p.csc.ptr + lh * p.csc.ptr_sh + cb + 1, e0, e1);
     const int32_t *rows = p.csc.idx + lh * p.csc.idx_sh;
-    if (p.seg.entries)  // (every wave has written the same values)
-      e0 = __builtin_amdgcn_readfirstlane(part[0]), e1 = __builtin_amdgcn_readfirstlane(part[1]);
+    if (p.seg.entries) {  // (every wave has written the same values)
+      const int first = __builtin_amdgcn_readfirstlane(part[0]), len = __builtin_amdgcn_readfirstlane(part[1]);
+      const int before = (gq - gq_base) * len;  // entries of the heads before this one
+      e0 = first + max(__builtin_amdgcn_readfirstlane(part[2]) - before, 0);
+      e1 = first + min(__builtin_amdgcn_readfirstlane(part[3]) - before, len);
+    }
     const float *qbase = (const float *)p.q.ptr + sq.b * p.q.sb + h * p.q.sh;
     const float *dobase = (const float *)p.dout.ptr + sq.b * p.dout.sb + h * p.dout.sh;
     const float *lsebase = p.lse.ptr + sq.b * p.lse.sb + h * p.lse.sh;
@@ -656,7 +663,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   __syncthreads();
   float *dkp = (float *)p.dk.ptr + sq.b * p.dk.sb + out_head * p.dk.sh + (int64_t)key * p.dk.st;
   float *dvp = (float *)p.dv.ptr + sq.b * p.dv.sb + out_head * p.dv.sh + (int64_t)key * p.dv.st;
-  const int slot = p.seg.entries ? __builtin_amdgcn_readfirstlane(part[2]) : -1;
+  const int slot = p.seg.entries ? __builtin_amdgcn_readfirstlane(part[4]) : -1;
   if (slot >= 0) {
     dkp = p.seg.partial + ((((int64_t)sq.b * gridDim.x + out_head) * p.seg.slots + slot) * 128 + nh * 32 + n) * p.D;
     dvp = dkp + 64 * p.D;
@@ -735,13 +742,16 @@ int launch_mfma_f32_fwd(const FwdParams &p, hipStream_t stream) {
   return DK_BY_HEAD_DIM(launch_fwd, p.D, pr, tiles, stream);
 }
 
-// Scratch of the dK/dV pass by q heads (wide head dims only: up to 64 the pass of a whole group is
-// short enough that the sum would cost what the balance gains)
-static BwdScratch mfma_f32_bwd_scratch(const BwdParams &p) {
+// Scratch of the backward.  Head dims up to 64: a workgroup of the dK/dV pass walks whole groups of q heads, long columns
+// cut into segments (16 / 4 heads of 64, 2000 tokens, training: 904 us uncut, 407 cut; 4000 tokens 1833 / 821; 3 x 1000,
+// 24 / 8 753 / 565).  Above, one workgroup per q head into partials that are summed is the faster one at every size (a
+// step takes four times the 16-bit kernel's time, the partials as long as there: 4 x 2000, 32 / 8 heads of 128, 5064 us against
+// 5684; 2 x 2000, 24 / 8 of 96, 1599 / 1662), unless the partials would not fit.
+static BwdScratch mfma_f32_bwd_scratch(const BwdParams &p, bool walk) {
   const int slots = 256 * (p.D <= 64 ? 2 : 1);
-  return plan_bwd_scratch(p, p.D > 64 && p.D % 8 == 0 ? bwd_group_bytes(p) : 0, slots, false, slots);
+  return plan_bwd_scratch(p, p.D > 64 && p.D % 8 == 0 ? bwd_group_bytes(p) : 0, slots, false, slots, walk ? INFINITY : -1);
 }
-size_t mfma_f32_bwd_workspace_bytes(const BwdParams &p) { return mfma_f32_bwd_scratch(p).bytes; }
+size_t mfma_f32_bwd_workspace_bytes(const BwdParams &p) { return mfma_f32_bwd_scratch(p, true).bytes; }
 
 int launch_mfma_f32_bwd(const BwdParams &p, void *workspace, size_t workspace_bytes, hipStream_t stream) {
   const SeqView &s = p.seqs;
@@ -756,7 +766,7 @@ int launch_mfma_f32_bwd(const BwdParams &p, void *workspace, size_t workspace_by
     hipLaunchKernelGGL(f32::delta_kernel<32>, dim3(cdiv(s.max_q_len, 8), p.Hq, s.batch), dim3(256), 0, stream, p);
   DK_HIP_CHECK(hipGetLastError());
   DK_REQUIRE(!p.csr.order || p.csr.num_rows <= 65535, "sequence too long for one launch");
-  const BwdScratch scratch = usable_bwd_scratch(mfma_f32_bwd_scratch(p), workspace, workspace_bytes);
+  const BwdScratch scratch = usable_bwd_scratch([&](bool walk) { return mfma_f32_bwd_scratch(p, walk); }, workspace, workspace_bytes);
   BwdParams pq = p;
   if (p.csr.order && segment_items(scratch.dq, p.csr.num_rows) <= 65535) pq.seg = scratch.dq;
   // handed out in the table's order: all of them

@@ -1,0 +1,83 @@
+"""dK / dV passes whose workgroups walk a column for all q heads of a kv head: as one stream of steps against the oracle,
+and cut into segments, as larger launches are, against the pass by q heads."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from dkernel_amd import LocalStrideSparseAttention, SparseAttention, ops
+from helpers import F32_TOL, TOL, assert_close, make_qkv, oracle_fwd
+from oracle import layout as OL
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _run(mod, q, k, v, do, sm):
+    qd, kd, vd = (x.detach().to(DEV).requires_grad_() for x in (q, k, v))
+    mod(qd, kd, vd, sm).backward(do.to(DEV))
+    return [qd.grad, kd.grad, vd.grad], ops.last_bwd_kernels.decode()
+
+
+# without a workspace every launch walks whole groups; fp32 with up to 64 head dims always does
+@pytest.mark.parametrize("B,Hq,Hkv,L,Lk,D,bs,dtype,own_tables", [
+    (1, 4, 2, 200, 200, 128, 64, torch.bfloat16, False),
+    (2, 6, 2, 333, 333, 64, 64, torch.float16, False),
+    (1, 4, 1, 250, 400, 96, 64, torch.bfloat16, False),   # keys before the queries
+    (1, 4, 2, 300, 300, 128, 64, torch.bfloat16, True),   # every q head has a table of its own, some columns empty
+    (1, 4, 2, 320, 320, 64, 16, torch.bfloat16, True),
+    (1, 8, 2, 300, 300, 128, 32, torch.bfloat16, False),
+    (1, 4, 2, 300, 300, 192, 64, torch.bfloat16, False),
+    (1, 4, 2, 300, 300, 64, 64, torch.float32, True),
+    (1, 4, 2, 300, 300, 80, 64, torch.float32, False)])
+def test_stream_of_heads(B, Hq, Hkv, L, Lk, D, bs, dtype, own_tables, monkeypatch):
+    print(f"case B={B} Hq={Hq} Hkv={Hkv} L={L} Lk={Lk} D={D} bs={bs} {dtype} own_tables={own_tables}", flush=True)
+    sm = 1 / math.sqrt(D)
+    n = -(-Lk // bs)
+    if own_tables:
+        rng = np.random.default_rng(3)
+        bm = rng.random((Hq, n, n)) < 0.3
+        bm[1, :, 1] = bm[2, :, 0] = False  # a head without entries in a column, between or before others
+        bm &= np.tril(np.ones((n, n), dtype=bool))[None]
+        bm[:, np.arange(2, n), np.arange(2, n)] = True
+        bm[:, :2, 0] = True
+        mod = SparseAttention(bs, torch.from_numpy(bm)).to(DEV)
+    else:
+        bm = OL.block_mask(Hq, n * bs, bs, 2, 3, num_kv_heads=Hkv)
+        mod = LocalStrideSparseAttention(Hq, n * bs, bs, 2, 3, num_kv_heads=Hkv).to(DEV)
+    q, k, v, do = make_qkv(B, L, Lk, Hq, Hkv, D, dtype, with_do=True)
+    monkeypatch.setattr(ops, "_bwd_workspace", False)
+    got, ran = _run(mod, q, k, v, do, sm)
+    assert "per q head" not in ran and "group_sum" not in ran and "generic" not in ran, ran
+    qo, ko, vo = (x.clone().float().requires_grad_() for x in (q, k, v))
+    ro, _ = oracle_fwd(qo, ko, vo, bm, bs, sm, causal=True)
+    ro.backward(do.float())
+    for name, a, want in zip(("dQ", "dK", "dV"), got, (qo.grad, ko.grad, vo.grad)):
+        assert_close(name, a, want, **(F32_TOL if dtype == torch.float32 else TOL))
+
+
+# launches from some hundred steps per resident workgroup on (fp32 up to 64 dims: any size)
+@pytest.mark.parametrize("B,Hq,Hkv,L,table,D,bs,dtype,cut", [
+    (2, 32, 8, 4000, 4000, 128, 64, torch.bfloat16, True),
+    (4, 32, 8, 2048, 3000, 128, 64, torch.float16, False),   # longest column below the average; a table for longer sequences
+    (1, 32, 8, 6007, 7000, 96, 64, torch.bfloat16, True),
+    (3, 24, 8, 4001, 4001, 64, 64, torch.bfloat16, True),
+    (1, 32, 8, 3600, 3600, 160, 64, torch.bfloat16, True),
+    (2, 32, 8, 4000, 4000, 128, 32, torch.bfloat16, True),
+    (2, 4, 2, 1400, 2000, 64, 64, torch.float32, True),
+    (1, 8, 2, 1401, 1401, 48, 64, torch.float32, True)])
+def test_segments_of_groups(B, Hq, Hkv, L, table, D, bs, dtype, cut, monkeypatch):
+    print(f"case B={B} Hq={Hq} Hkv={Hkv} L={L} table={table} D={D} bs={bs} {dtype}", flush=True)
+    mod = LocalStrideSparseAttention(Hq, table, bs, 16 * 64 // bs, 8, num_kv_heads=Hkv).to(DEV)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q, k, v, do = (torch.randn(B, L, h, D, generator=g, device=DEV).to(dtype) for h in (Hq, Hkv, Hkv, Hq))
+    got, ran = _run(mod, q, k, v, do, D ** -0.5)
+    assert "per q head" not in ran and "group_sum" not in ran and ran.count("segment_sum_kernel") >= int(cut), ran
+    monkeypatch.setitem(mod.kwargs, "row_lengths", ())
+    whole, ran = _run(mod, q, k, v, do, D ** -0.5)
+    assert "segment_sum_kernel" not in ran and ("group_sum" in ran or dtype == torch.float32), ran
+    # (each side rounds its fp32 sums once: an ulp of the type apart; the sums themselves in fp32)
+    ulp = {torch.float32: 2e-5, torch.float16: 1e-3, torch.bfloat16: 8e-3}[dtype]
+    for name, a, b in zip(("dQ", "dK", "dV"), got, whole):
+        assert_close(name, a, b, atol=ulp * float(b.float().abs().max()) / 8, rtol=ulp)
