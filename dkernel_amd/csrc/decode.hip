@@ -133,11 +133,48 @@ __device__ __forceinline__ uint4 fp8x8_to(uint2 w) {
                     pack2_exact<T>(d[0], d[1]));
 }
 
+// Sequence that the workgroups of grid.z = place take when the sequences are handed out by length: the `first` longest
+// ones in ascending order, then the others in descending order (lengths to within a 64th of the longest there can be;
+// equal ones in the batch's order).  At most kRankedSequences sequences, all lanes active.  Every lane loads the geometry
+// of its sequences, so the lengths cost no round trip beyond the workgroup's own; the length at a rank is found bit by bit
+// from the lanes' votes (64 keys to a block: six votes, 0.3 us of a step).
+constexpr int kRankedSequences = 128;
+__device__ __forceinline__ SeqInfo sequence_by_length(const SeqView &s, int place, int first, int causal) {
+  const int rank = place < first ? first - 1 - place : place;
+  const int lane = threadIdx.x & 63;
+  const bool two = s.batch > 64;  // sequences a lane
+  const int drop = max(0, 26 - __clz(s.max_k_len | 1));  // length bits that are left out: six remain
+  auto key = [&](const SeqInfo &t, int i) { return i < s.batch ? (t.q_len > 0 ? t.k_len >> drop : 0) : -1; };
+  const SeqInfo lo = load_seq_lane(s, min(lane, s.batch - 1), causal);
+  SeqInfo hi = lo;
+  if (two) hi = load_seq_lane(s, min(lane + 64, s.batch - 1), causal);
+  const int key_lo = key(lo, lane), key_hi = key(hi, lane + 64);
+  auto votes = [&](int at) { return __popcll(__ballot(key_lo >= at)) + (two ? __popcll(__ballot(key_hi >= at)) : 0); };
+  int len = 0;  // largest length that more than `rank` sequences reach
+  for (int at = 32; at > 0; at >>= 1)
+    if (votes(len + at) > rank) len += at;
+  int n = rank - votes(len + 1);  // among those of that length
+  const unsigned long long same_lo = __ballot(key_lo == len), same_hi = __ballot(key_hi == len);
+  const bool upper = n >= __popcll(same_lo);
+  if (upper) n -= __popcll(same_lo);
+  const unsigned long long same = upper ? same_hi : same_lo, below = (1ull << lane) - 1;
+  const int owner = __ffsll(__ballot(((same >> lane) & 1) && __popcll(same & below) == n)) - 1;
+  auto from_owner = [&](int a, int b) { return __builtin_amdgcn_readlane(upper ? b : a, owner); };
+  SeqInfo r;
+  r.b = owner + (upper ? 64 : 0);
+  r.q_start = from_owner(lo.q_start, hi.q_start), r.q_len = from_owner(lo.q_len, hi.q_len);
+  r.k_start = from_owner(lo.k_start, hi.k_start), r.k_len = from_owner(lo.k_len, hi.k_len);
+  r.past = from_owner(lo.past, hi.past);
+  return r;
+}
+
 // KV8 (with PAGED): the K/V pools hold fp8 bytes, converted to T on the way into LDS.
 // W waves per workgroup = W consecutive units of one row.
-template <typename T, int D, bool PAD, bool SUB, bool PAGED, bool KV8, int W>
+// BY_LENGTH: sequences handed out by length (decode_first_by_length); an instantiation of its own, as the code alone, jumped
+// over, cost the smallest steps 0.15 of 8 us.
+template <typename T, int D, bool PAD, bool SUB, bool PAGED, bool KV8, int W, bool BY_LENGTH>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2, D == 256 ? 1 : 2))) void decode_partial_kernel(
-    const FwdParams p, float *ws, int unit_halves, int max_groups, slot_t launch) {
+    const FwdParams p, float *ws, int unit_halves, int max_groups, slot_t launch, int first_by_length) {
   using M = Mma<T>;
   using vec8 = typename M::vec8;
   using S = DecSmem<D>;
@@ -146,8 +183,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D == 256
   constexpr int EW = SUB ? 2 : 1;  // ints per table entry
   extern __shared__ __align__(16) char smem_all[];
 
-  const int kvh = blockIdx.y, b = blockIdx.z;
-  const SeqInfo sq = load_seq(p.seqs, b, p.causal);
+  const int kvh = blockIdx.y;
+  SeqInfo sq;
+  if constexpr (BY_LENGTH)
+    sq = sequence_by_length(p.seqs, blockIdx.z, first_by_length, p.causal);
+  else
+    sq = load_seq(p.seqs, blockIdx.z, p.causal);
+  const int b = sq.b;
   if (sq.q_len <= 0) return;
   const int ratio = __builtin_amdgcn_readfirstlane(p.Hq / p.Hkv);  // integer division runs on the VALU
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -560,16 +602,44 @@ size_t decode_workspace_bytes(const FwdParams &p) {
   return (size_t)p.seqs.batch * p.Hq * places * (mfma_tile_width(p.D) + 2) * sizeof(float);
 }
 
+// Sequences whose workgroups go to empty compute units when the sequences are handed out by length, 0: they are handed out
+// in the batch's order (nothing to gain while every workgroup has a compute unit of its own).  Beyond 256 workgroups
+// the first compute units get a second one, and the chip's rate is only reached while all of them stream: the first round takes
+// the longest sequences, shortest of them first, so that the second one, longest first, adds the most to the units that
+// have the least.  Order of the batch / by length, us: 8 kv heads of 128, 48 sequences of 256 - 6000 tokens, paged 54.1 / 47.1;
+// 36 of up to 11000 34.9 / 31.0, 62 of 2900 31.7 / 29.8, 41 of 330 11.1 / 11.0; 12 kv heads, 28 of 5900 42.7 / 33.2; 16 of
+// 256, 23 of 1850 75.9 / 64.8.  Beyond four rounds the queue evens the sequences out and every round pays for the votes: 936
+// workgroups 57.3 / 56.1, 1104 133.0 / 133.3, 1856 195.9 / 197.1, 3040 of 256 dims 204.7 / 209.9.  fp8 pools are bound by the
+// conversions of a wave rather than by the memory, and few second workgroups gain nothing: 288 workgroups 26.3 / 27.0 and 22.5 / 22.6,
+// 328 19.0 / 19.4, 352 32.4 / 29.2, 408 25.3 / 24.3, 480 44.5 / 41.8.
+static int decode_first_by_length(const FwdParams &p, int groups) {
+  constexpr int kUnits = 256;
+  const int per_sequence = p.Hkv * groups;
+  const bool ranked = (p.seqs.given & 12) && p.seqs.batch > 1 && p.seqs.batch <= kRankedSequences;
+  const int64_t workgroups = (int64_t)per_sequence * p.seqs.batch;
+  const int64_t from = p.paged.table && p.paged.kv_fp8 ? kUnits + 80 : kUnits;
+  if (!ranked || workgroups <= from || workgroups > 4 * kUnits) return 0;
+  return std::min(p.seqs.batch, std::max(1, kUnits / per_sequence));
+}
+
 template <typename T, int D, bool PAD, bool SUB, bool PAGED, bool KV8 = false>
 static int launch_decode_td(const FwdParams &p, float *ws, hipStream_t stream) {
   constexpr int W = kDecodeWaves;
   const int smem = W * DecSmem<D>::wave_bytes(p.Hq / p.Hkv);
   const int groups = std::max(1, decode_max_groups(p));
   DK_REQUIRE(smem <= 160 * 1024, "decode workgroup needs %d bytes of LDS", smem);
-  DK_ALLOW_DYNAMIC_LDS((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W>), smem);
+  const dim3 grid(groups, p.Hkv, p.seqs.batch), block(64 * W);
+  const int first = decode_first_by_length(p, groups);
   DK_NOTE_KERNEL("decode_partial_kernel");
-  hipLaunchKernelGGL((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W>), dim3(groups, p.Hkv, p.seqs.batch),
-                     dim3(64 * W), smem, stream, p, ws, decode_unit_halves(p), groups, next_launch_number());
+  if (first > 0) {
+    DK_ALLOW_DYNAMIC_LDS((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W, true>), smem);
+    hipLaunchKernelGGL((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W, true>), grid, block, smem, stream, p, ws,
+                       decode_unit_halves(p), groups, next_launch_number(), first);
+  } else {
+    DK_ALLOW_DYNAMIC_LDS((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W, false>), smem);
+    hipLaunchKernelGGL((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W, false>), grid, block, smem, stream, p, ws,
+                       decode_unit_halves(p), groups, next_launch_number(), 0);
+  }
   DK_HIP_CHECK(hipGetLastError());
   return DK_OK;
 }
