@@ -171,6 +171,7 @@ struct SeqView {
   // no query of their sequence, so that the caller need not clear the outputs first; packed inputs:
   // the rows of lse before the first sequence and behind the last one (-inf)
   int32_t zero_outside = 0;
+  int32_t items_in_z = 0;  // set per launch: grid of (heads, batch, items) in place of (heads, items, batch)
 };
 
 // Paged K/V (decode only): k / v point at page pools, token t of sequence b lives in page

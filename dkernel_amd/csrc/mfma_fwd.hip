@@ -55,6 +55,8 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   static_assert(!RP || G == 2, "row pairs: two wave pairs, one q tile each");
   // SUB: table entries are (column, bit mask over the pattern blocks inside the 64 x 64 tile)
   constexpr int EW = SUB ? 2 : 1;  // ints per table entry
+  // grid: (heads, items, batch), padded inputs (heads, batch, items)
+  const int item_y = p.seqs.items_in_z ? blockIdx.z : blockIdx.y, item_z = p.seqs.items_in_z ? blockIdx.y : blockIdx.z;
   SeqInfo sq;
   int tile;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -65,46 +67,46 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
     // workgroup = table rows 2u and 2u + 1 of one head (one per wave pair); tiles_y counts pairs
     int u;
     if (p.seqs.packed) {
-      if (p.seqs.zero_outside && blockIdx.y == 0) lse_outside_packed(p.seqs, p.lse, grid_head(p.csr), 1, tid, NT);
+      if (p.seqs.zero_outside && item_y == 0) lse_outside_packed(p.seqs, p.lse, grid_head(p.csr), 1, tid, NT);
       // the sequences share one token dimension: row pairs are counted through all of them (last
       // pair first: within a sequence the longest rows start first, as for unpacked inputs)
       int idx;
       if (!find_packed_sequence(
-              p.seqs, p.causal, tiles_y - 1 - (int)blockIdx.y, [](const SeqInfo &t) { return seq_row_pairs(t); }, sq, idx))
+              p.seqs, p.causal, tiles_y - 1 - item_y, [](const SeqInfo &t) { return seq_row_pairs(t); }, sq, idx))
         return;
       first_rb = sq.past / 64, last_rb = (sq.past + sq.q_len - 1) / 64;
       u = (first_rb >> 1) + idx;
     } else {
-      sq = load_seq(p.seqs, blockIdx.z, p.causal);
+      sq = load_seq(p.seqs, item_z, p.causal);
       first_rb = sq.past / 64, last_rb = (sq.past + sq.q_len - 1) / 64;
       if (p.csr.pair_order)  // the table's own order, longest pairs first (the grid then covers every pair of it)
-        u = scalar_load(p.csr.pair_order + lut_head(p.csr, grid_head(p.csr), p.Hq, p.Hkv) * p.csr.order_sh + blockIdx.y);
+        u = scalar_load(p.csr.pair_order + lut_head(p.csr, grid_head(p.csr), p.Hq, p.Hkv) * p.csr.order_sh + item_y);
       else
-        u = (first_rb >> 1) + tiles_y - 1 - (int)blockIdx.y;
+        u = (first_rb >> 1) + tiles_y - 1 - item_y;
       if (sq.q_len <= 0 || u > (last_rb >> 1) || u < (first_rb >> 1)) {  // no rows here: only the share of the padding rows, if asked
         if (p.seqs.zero_outside)
-          zero_rows_outside<T>(p.seqs, sq, blockIdx.y, tiles_y, p.o, p.lse, grid_head(p.csr), 1, p.D, p.vec_ok, tid, NT);
+          zero_rows_outside<T>(p.seqs, sq, item_y, tiles_y, p.o, p.lse, grid_head(p.csr), 1, p.D, p.vec_ok, tid, NT);
         return;
       }
     }
     rb = 2 * u + (wave >> 1);
     tile = rb - first_rb;  // outside [0, last_rb - first_rb]: this wave pair has no rows (row_ok false everywhere)
   } else {
-    const int ty = tiles_y - 1 - (int)blockIdx.y;  // longest rows first (of a causal pattern)
+    const int ty = tiles_y - 1 - item_y;  // longest rows first (of a causal pattern)
     bool has_rows;
     if (p.csr.order && !p.seqs.packed) {  // the table's own order, longest rows first (the grid then covers every row of it)
-      sq = load_seq(p.seqs, blockIdx.z, p.causal);
-      tile = scalar_load(p.csr.order + lut_head(p.csr, grid_head(p.csr) * G, p.Hq, p.Hkv) * p.csr.order_sh + blockIdx.y) -
+      sq = load_seq(p.seqs, item_z, p.causal);
+      tile = scalar_load(p.csr.order + lut_head(p.csr, grid_head(p.csr) * G, p.Hq, p.Hkv) * p.csr.order_sh + item_y) -
              sq.past / 64;
       has_rows = tile >= 0 && tile < seq_row_blocks(sq, 64);
     } else {
-      if (p.seqs.packed && p.seqs.zero_outside && blockIdx.y == 0)
+      if (p.seqs.packed && p.seqs.zero_outside && item_y == 0)
         lse_outside_packed(p.seqs, p.lse, grid_head(p.csr) * G, G, tid, NT);
-      has_rows = resolve_tile(p.seqs, p.causal, 64, 1, ty, blockIdx.z, sq, tile);
+      has_rows = resolve_tile(p.seqs, p.causal, 64, 1, ty, item_z, sq, tile);
     }
     if (!has_rows) {
       if (p.seqs.zero_outside && !p.seqs.packed)  // (with packed inputs sq is not set here)
-        zero_rows_outside<T>(p.seqs, sq, blockIdx.y, tiles_y, p.o, p.lse, grid_head(p.csr) * G, G, p.D, p.vec_ok, tid, NT);
+        zero_rows_outside<T>(p.seqs, sq, item_y, tiles_y, p.o, p.lse, grid_head(p.csr) * G, G, p.D, p.vec_ok, tid, NT);
       return;
     }
     rb = sq.past / 64 + tile;
@@ -459,7 +461,7 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   // padded inputs: this workgroup's share of the rows that hold no query, behind its own work (at
   // the start the stores of every workgroup would go out together, ahead of all multiplies)
   if (p.seqs.zero_outside && !p.seqs.packed)
-    zero_rows_outside<T>(p.seqs, sq, blockIdx.y, tiles_y, p.o, p.lse, RP ? hx : hx * G, RP ? 1 : G, p.D,
+    zero_rows_outside<T>(p.seqs, sq, item_y, tiles_y, p.o, p.lse, RP ? hx : hx * G, RP ? 1 : G, p.D,
                          p.vec_ok, tid, NT);
   if (!row_ok) return;
   if (p.lse.ptr && g == 0) {
@@ -563,6 +565,21 @@ static FwdParams for_grid(FwdParams p, int gx, int gy) {
   return p;
 }
 
+// ... and the grid.  Padded inputs: the rows of all sequences side by side, longest first, instead of one sequence behind
+// the other, so that a launch of a few rounds does not end on the long rows of the last sequence.  Sequence behind
+// sequence / side by side, us: 6 prompts of 200 - 2000 tokens, 32 heads of 96, 77.7 / 72.7; 6 x 7800, 8 heads 179.1 / 171.5; 11 x
+// 1400, 16 / 4 heads of 256 115.8 / 98.5; 3 x 1150, 32 / 8 of 96 22.0 / 20.1; 6 x 1850, 8 heads 20.2 / 19.0.  Long launches stay: there
+// the K/V tiles that neighbouring rows share no longer fit the L2s (14080 workgroups, 8 x 7000, 32 heads 1082 / 1203; 3936
+// workgroups 218.1 / 217.7), as do sequences of few rows, which are all alike (4 row pairs 21.0 / 21.2, 7 of them 19.1 /
+// 18.3).  Tables with uneven heads keep their rotation over neighbouring rows.
+static FwdParams for_rows(FwdParams p, int gx, int gy, dim3 &grid) {
+  p = for_grid(p, gx, gy);
+  const int batch = p.seqs.packed ? 1 : p.seqs.batch;
+  p.seqs.items_in_z = p.seqs.given && batch > 1 && !p.csr.rot && gy >= 6 && (int64_t)gx * gy * batch <= 4096;
+  grid = p.seqs.items_in_z ? dim3(gx, batch, gy) : dim3(gx, gy, batch);
+  return p;
+}
+
 // q tiles of `rows` tokens along grid.y (packed inputs: through all sequences), an upper bound
 static int tile_count(const SeqView &s, int causal, int rows) {
   if (s.packed)
@@ -609,9 +626,8 @@ static int launch_tdg(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
   constexpr int smem = 2 * FwdSmem<D>::kStage;
   if (split_pays<D>(p)) return launch_split<T, D, PAD, false, KD>(p, stream);
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, G, PAD, false, false, KD>), smem);
-  grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
-  const FwdParams pr = for_grid(p, grid.x, grid.y);
+  const FwdParams pr = for_rows(p, p.Hq / G, tiles_y, grid);
   DK_NOTE_KERNEL(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
   hipLaunchKernelGGL((mfma_fwd_kernel<T, D, G, PAD, false, false, KD>), grid, dim3(128 * G), smem, stream,
                      pr, tiles_y);
@@ -642,10 +658,10 @@ static int launch_row_pairs_as(const FwdParams &p, hipStream_t stream, const cha
   if (p.csr.pair_order && !s.packed) pairs = (p.csr.num_rows + 1) / 2;  // handed out in the table's order: all of them
   DK_REQUIRE(pairs <= 65535, "too many q tiles for one launch (%d)", pairs);
   if (int rc = launch_item_offsets(p, true, stream)) return rc;
-  const FwdParams pr = for_grid(p, p.Hq, pairs);
+  dim3 grid;
+  const FwdParams pr = for_rows(p, p.Hq, pairs, grid);
   note_kernel(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel", signature);
-  hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 2, PAD, true, SUB, KD>), dim3(p.Hq, pairs, s.packed ? 1 : s.batch), dim3(256), smem,
-                     stream, pr, pairs);
+  hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 2, PAD, true, SUB, KD>), grid, dim3(256), smem, stream, pr, pairs);
   DK_HIP_CHECK(hipGetLastError());
   return DK_OK;
 }
@@ -677,9 +693,8 @@ static int launch_sub_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t 
   constexpr int smem = 2 * FwdSmem<D>::kStage;
   if (split_pays<D>(p)) return launch_split<T, D, PAD, true, KD>(p, stream);
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, G, PAD, false, true, KD>), smem);
-  grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
-  const FwdParams pr = for_grid(p, grid.x, grid.y);
+  const FwdParams pr = for_rows(p, p.Hq / G, tiles_y, grid);
   DK_NOTE_KERNEL(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
   hipLaunchKernelGGL((mfma_fwd_kernel<T, D, G, PAD, false, true, KD>), grid, dim3(128 * G), smem, stream,
                      pr, tiles_y);
@@ -717,9 +732,8 @@ static int launch_256_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t 
   constexpr int smem = 2 * FwdSmem<256>::kStage;
   if (split_pays<256>(p)) return launch_split<T, 256, true, SUB>(p, stream);
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, 256, G, true, false, SUB>), smem);
-  grid.x = p.Hq / G;
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
-  const FwdParams pr = for_grid(p, grid.x, grid.y);
+  const FwdParams pr = for_rows(p, p.Hq / G, tiles_y, grid);
   DK_NOTE_KERNEL(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
   hipLaunchKernelGGL((mfma_fwd_kernel<T, 256, G, true, false, SUB>), grid, dim3(128 * G), smem, stream,
                      pr, tiles_y);
