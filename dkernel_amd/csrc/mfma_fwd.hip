@@ -18,7 +18,8 @@
 //
 // Grid: x = head group (fastest, so that the 8 XCDs, which receive
 // workgroups round-robin, each keep a fixed set of kv heads in their L2),
-// y = q tile with the longest rows first, z = batch.
+// y = q tile with the longest rows first, z = batch (y and z change places for shorter
+// launches of padded inputs, for_rows).
 #include "common.h"
 #include "device_common.h"
 #include "fwd_split.h"
