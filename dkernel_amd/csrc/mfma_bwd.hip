@@ -408,16 +408,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
     if (ra + 1 > last_rb) e1 = emid;
   }
   const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
-  // this workgroup's entries of the two rows, and the place of its partial sum (-1: it takes both rows whole); kept
-  // in LDS until they are used (every wave writes and reads the same values)
-  __shared__ int part[5];
-  part[0] = e0, part[1] = emid, part[2] = emid, part[3] = e1, part[4] = -1;
+  // this workgroup's entries [a0, a1) and [b0, b1) of the two rows, and the place of its partial sum (-1: it takes both rows
+  // whole)
+  int a0 = e0, a1 = emid, b0 = emid, b1 = e1, slot = -1;
   if (p.seg.entries && place < p.seg.n[1]) {
     const int segments = planned_segments(p.seg, place, (e1 - e0 + 1) / 2);
     if (seg >= segments) return;
     if (segments > 1) {
-      part[4] = seg * p.seg.n[1] + place;
-      // columns [lo, hi): an even share of the longer row's entries, and what the other row lists between them
+      slot = seg * p.seg.n[1] + place;
+      // an even share of the longer row's entries, and what the other row lists between their columns
       const bool first_longer = emid - e0 >= e1 - emid;
       const int l0 = first_longer ? e0 : emid, len = first_longer ? emid - e0 : e1 - emid;
       const int s0 = __builtin_amdgcn_readfirstlane(len * seg / segments), s1 = __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
@@ -425,10 +424,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
       int p0 = o0, p1 = o1;
       if (seg > 0) p0 = entry_lower_bound<EW>(cols, o0, o1, scalar_load(cols + (l0 + s0) * EW));
       if (seg + 1 < segments) p1 = entry_lower_bound<EW>(cols, p0, o1, scalar_load(cols + (l0 + s1) * EW));
-      part[0] = first_longer ? l0 + s0 : p0, part[1] = first_longer ? l0 + s1 : p1;
-      part[2] = first_longer ? p0 : l0 + s0, part[3] = first_longer ? p1 : l0 + s1;
+      a0 = first_longer ? l0 + s0 : p0, a1 = first_longer ? l0 + s1 : p1;
+      b0 = first_longer ? p0 : l0 + s0, b1 = first_longer ? p1 : l0 + s1;
     }
   }
+  // Kept in LDS until they are used.  No barrier stands between a wave's store and its reads: that is sound only as
+  // long as every wave stores each place once and all waves the same value.
+  __shared__ int part[5];
+  part[0] = a0, part[1] = a1, part[2] = b0, part[3] = b1, part[4] = slot;
 
   if (PAD && p.D < KD) {  // the slots of the head dims beyond p.D stay zero for the whole kernel
     zero_tiles<NT>(smem, 2 * STAGE, tid);
