@@ -61,7 +61,8 @@ inline BwdScratch plan_bwd_scratch(const BwdParams &p, size_t group, int dq_slot
     kv = plan_segments(p.csc.row_lengths, p.csc.num_rows, 1, copies, kv_slots, kv_limit, share);
   const size_t at = (s.group + 255) / 256 * 256;
   const int64_t dq_slots_all = dq.slots * copies, kv_slots_all = kv.slots * (walk ? copies / (p.Hq / p.Hkv) : copies);
-  const size_t need = at + (size_t)std::max(dq_slots_all, kv_slots_all) * 128 * p.D * sizeof(float);
+  const double partials = (double)std::max(dq_slots_all, kv_slots_all) * 128 * p.D * sizeof(float);  // (no number of slots overflows)
+  const size_t need = partials > (double)kMost ? kMost + 1 : at + (size_t)partials;
   if (walk && need > kMost && group) return plan_bwd_scratch(p, group, dq_slots, dq_pairs, kv_slots, -1);
   if (need > at && need <= kMost && p.D % 4 == 0) s.dq = dq, s.kv = kv, s.bytes = need;
   return s;

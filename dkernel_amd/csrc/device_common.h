@@ -65,11 +65,12 @@ struct LutView {
 // workgroups: each leaves an fp32 partial sum in memory and a second kernel adds a row's partials in order
 // (segment_sum_kernel, mfma_bwd.hip).  Work item y of the launch is segment 1 of the first n[1] rows of the
 // table's order, then segment 2 of the first n[2], ..., at last segment 0 of all of them: the order is by
-// descending length, so the rows that have a segment s come first in it.
+// descending length, so the rows that have a segment s come first in it (or, where lengths say otherwise, lie among the
+// first n[s]: work items without a segment exit at once).
 constexpr int kMaxSegments = 16;
 struct SegView {
   int32_t entries = 0;  // entries per segment, 0: no row is cut
-  int32_t n[kMaxSegments] = {};  // rows that have a segment s in any head (n[0]: unused)
+  int32_t n[kMaxSegments] = {};  // rows of the order up to the last one with a segment s in any head (n[0]: unused), never ascending
   float *partial = nullptr;  // [batch][heads][slots] partial sums, slot = segment * n[1] + place in the order
   int32_t slots = 0;
 };
@@ -104,9 +105,15 @@ __host__ __device__ inline int row_segments(int len, int entries) {
 }
 // Steps that every slot of a launch has to do on average (arguments as below); a workgroup costs its steps and kStartSteps more.
 constexpr int kStartSteps = 5;
+// Steps of a row of `len` entries (of whatever a caller says is its length).
+inline int row_steps(int32_t len, int per_step, int heads) {
+  constexpr int64_t kMost = 1 << 28;
+  const int64_t steps = ((int64_t)(len > 0 ? len : 0) + per_step - 1) / per_step * heads;
+  return (int)(steps < kMost ? steps : kMost);
+}
 inline double average_steps(const int32_t *lengths, int rows, int per_step, int64_t copies, int slots, int heads) {
   int64_t total = 0;
-  for (int i = 0; i < rows; ++i) total += (lengths[i] + per_step - 1) / per_step * heads + kStartSteps;
+  for (int i = 0; i < rows; ++i) total += row_steps(lengths[i], per_step, heads) + kStartSteps;
   return (double)total * (double)copies / slots;
 }
 // Whether and how a launch cuts its long rows.  lengths: entries of the rows in the table's order, `per_step` of them a
@@ -115,15 +122,18 @@ inline double average_steps(const int32_t *lengths, int rows, int per_step, int6
 // `limit` times what every slot has to do on average (below that the hand-out by descending length evens it out), into
 // segments of `share` times the average and of at least eight steps: shorter ones cost more in start-up and
 // partial sums than they even out.  Below kWorth steps the kernel that adds the sums takes what the cut gains.
+// The lengths come from a caller and may be any numbers: a place of the order may have as many segments as the rows from it
+// on need at most (n[] never ascends), and the slots are counted for the place that has the most.
 inline SegView plan_segments(const int32_t *lengths, int rows, int per_step, int64_t copies, int slots, double limit, double share,
                              int heads = 1) {
   constexpr int kLeast = 8;
   const int kWorth = heads > 1 ? 40 : 20;
   SegView s;
   if (!lengths || rows < 1) return s;
-  auto steps = [&](int i) { return (lengths[i] + per_step - 1) / per_step * heads; };
+  auto steps = [&](int i) { return row_steps(lengths[i], per_step, heads); };
   const double average = average_steps(lengths, rows, per_step, copies, slots, heads);
-  const int longest = steps(0);
+  int longest = 0;
+  for (int i = 0; i < rows; ++i) longest = steps(i) > longest ? steps(i) : longest;
   if (longest < kWorth || longest + kStartSteps <= limit * average) return s;
   int entries = average * share > kLeast ? (int)(average * share) : kLeast;
   const int least = (longest + kMaxSegments - 2) / (kMaxSegments - 1);
@@ -132,8 +142,7 @@ inline SegView plan_segments(const int32_t *lengths, int rows, int per_step, int
   if (most < 2) return s;
   s.entries = entries;
   for (int i = 0; i < rows; ++i)
-    for (int j = row_segments(steps(i), entries) - 1; j > 0; --j)
-      if (j < kMaxSegments) ++s.n[j];
+    for (int j = row_segments(steps(i), entries) - 1; j > 0; --j) s.n[j] = i + 1;
   s.slots = most * s.n[1];
   return s;
 }
