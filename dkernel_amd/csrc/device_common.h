@@ -216,7 +216,7 @@ struct BwdParams {
   float sm_scale, scale_log2;
   int32_t vec_ok;
   SegView seg;       // set per launch
-  int32_t trim = 0;  // the column table lists rows beyond the queries (it was built for longer sequences)
+  int32_t trim = 0;  // the column table, in ascending order, lists rows beyond the queries (it was built for longer sequences)
 };
 
 // Which LUT head serves q head h (h is the same for every lane of a wave).

@@ -1419,7 +1419,7 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
   // neighbouring columns - which share most of their Q / dO tiles - together in time (1.7 %
   // faster on the 32-head benchmark; with 8 or 16 heads the order is worth 20 - 40 %).
   BwdParams po = p;
-  po.trim = p.csr.num_rows > tiles + past / 64;
+  po.trim = p.csc.row_lengths && p.csr.num_rows > tiles + past / 64;  // (tables with lengths list their entries in order)
   if (p.csc.order && segment_items(scratch.kv, p.csc.num_rows) <= 65535) po.seg = scratch.kv;
   if (((per_q_head ? p.Hq : p.Hkv) % 32) == 0 && !po.seg.entries) po.csc.order = nullptr;
   // with a hand-out order the grid covers every column of the table (those beyond the keys exit at once)

@@ -783,7 +783,7 @@ int launch_mfma_f32_bwd(const BwdParams &p, void *workspace, size_t workspace_by
   const bool per_q_head = scratch.group > 0;
   const int heads = per_q_head ? p.Hq : p.Hkv;
   BwdParams po = p;  // the order only where heads do not line up with the hardware's 32 workgroup queues
-  po.trim = p.csr.num_rows > tiles + past / 64;
+  po.trim = p.csc.row_lengths && p.csr.num_rows > tiles + past / 64;  // (as in the 16-bit pass)
   if (p.csc.order && segment_items(scratch.kv, p.csc.num_rows) <= 65535) po.seg = scratch.kv;
   if (heads % 32 == 0 && !po.seg.entries) po.csc.order = nullptr;
   DK_REQUIRE(p.csc.num_rows <= 65535, "sequence too long for one launch");

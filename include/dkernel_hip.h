@@ -285,7 +285,8 @@ size_t dk_bwd_workspace_bytes(const dk_bwd_args *args);
 /* Lengths of a backward call's tables in HOST memory, read during the call only: entries of the i-th row in the
  * table's row_order (csr_rows, csc_rows: num_rows values) or of the i-th pair in its pair_order (csr_pairs:
  * (num_rows + 1) / 2 values), the most over the heads.  Any may be NULL, and those of a table without that
- * order are not read.  Wrong lengths cost time, never correctness. */
+ * order are not read.  Wrong lengths cost time, never correctness.  The entries of every row of a table
+ * whose lengths are given ascend (as those of dk_csr_fill do); without lengths they come in any order. */
 typedef struct dk_row_lengths {
   const int32_t *csr_rows, *csr_pairs, *csc_rows;
 } dk_row_lengths;

@@ -129,3 +129,27 @@ def test_scratch_too_small_for_the_segments(monkeypatch):
     assert "segment_sum_kernel" not in ran and "per q head" in ran, ran
     for a, b in zip(got, small):
         assert_close("grad", a, b, atol=1e-3 * float(b.float().abs().max()), rtol=8e-3)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,bs,dtype", [(2, 2, 128, 64, torch.bfloat16), (4, 2, 64, 64, torch.bfloat16),
+                                               (2, 2, 64, 32, torch.bfloat16), (2, 2, 64, 64, torch.float32)])
+def test_columns_in_any_order_without_lengths(Hq, Hkv, D, bs, dtype, monkeypatch):
+    """dk_bwd without the lengths takes the entries of a column in any order, also of a table for longer sequences."""
+    L, table = 700, 1500
+    mod = LocalStrideSparseAttention(Hq, table, bs, 128 // bs, 3, num_kv_heads=Hkv).to(DEV)
+    monkeypatch.setitem(mod.kwargs, "row_lengths", ())
+    name = "masked_csc" if bs < 64 else "layout_csc"
+    ptr, rows = getattr(mod, name + "_ccol").cpu(), getattr(mod, name + "_row")
+    mixed = rows.cpu().clone()
+    g = torch.Generator().manual_seed(1)
+    for h in range(ptr.size(0)):
+        for a, b in zip(ptr[h].tolist(), ptr[h].tolist()[1:]):
+            mixed[h, a:b] = mixed[h, a:b][torch.randperm(b - a, generator=g)]
+    q, k, v, do = make_qkv(1, L, L, Hq, Hkv, D, dtype, with_do=True)
+    want, _ = _run(mod, q, k, v, do, 0.1)
+    monkeypatch.setitem(mod._buffers, name + "_row", mixed.to(DEV))
+    got, ran = _run(mod, q, k, v, do, 0.1)
+    assert "generic" not in ran, ran
+    tol = F32_TOL if dtype == torch.float32 else TOL
+    for what, a, b in zip(("dQ", "dK", "dV"), got, want):
+        assert_close(what, a, b, **tol)
