@@ -94,6 +94,7 @@ SYMBOLS = {
     "dk_fwd_paged": (C.c_int, [C.POINTER(FwdArgs), C.POINTER(PagedKV)]),
     "dk_bwd": (C.c_int, [C.POINTER(BwdArgs)]),
     "dk_bwd_workspace_bytes": (C.c_size_t, [C.POINTER(BwdArgs)]),
+    "dk_call_row_lengths": (C.c_int, [vp, vp, vp, i32, i32, i64, i32, i32, i32, vp]),
     "dk_bwd_balanced": (C.c_int, [C.POINTER(BwdArgs), C.POINTER(RowLengths)]),
     "dk_bwd_balanced_workspace_bytes": (C.c_size_t, [C.POINTER(BwdArgs), C.POINTER(RowLengths)]),
     "dk_combine": (C.c_int, [C.POINTER(CombineArgs)]),

@@ -57,7 +57,7 @@ struct LutView {
   int32_t uneven = 0;  // the heads hold clearly different numbers of entries
   int32_t fixed_walk = 0;  // a row's entries are taken in one order, whatever the size of the launch
   int32_t rot = 0;     // set per launch (head_rotation): 0, or 1 + shift of grid_head()
-  // optional, host memory: entries of the i-th row (pair of rows) of the order, the most in any head
+  // optional, host memory: entries of the i-th row (pair of rows) of the order inside the call, the most in any head
   const int32_t *row_lengths = nullptr, *pair_lengths = nullptr;
 };
 
@@ -113,7 +113,8 @@ inline int row_steps(int32_t len, int per_step, int heads) {
 }
 inline double average_steps(const int32_t *lengths, int rows, int per_step, int64_t copies, int slots, int heads) {
   int64_t total = 0;
-  for (int i = 0; i < rows; ++i) total += row_steps(lengths[i], per_step, heads) + kStartSteps;
+  for (int i = 0; i < rows; ++i)
+    if (lengths[i] >= 0) total += row_steps(lengths[i], per_step, heads) + kStartSteps;  // (else no row of the call)
   return (double)total * (double)copies / slots;
 }
 // Whether and how a launch cuts its long rows.  lengths: entries of the rows in the table's order, `per_step` of them a

@@ -2,6 +2,7 @@
 // CSR / CSC look-up tables with -1 padding, kernel-tile merge / split, and the
 // KV-cache-efficiency check.  Integer work on the CPU, one pass per table; it
 // replaces the per-head Python loops of dkernel/utils.py.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
@@ -262,6 +263,29 @@ int dk_kv_cache_efficient(const uint8_t *pattern, int32_t H, int32_t M, int32_t 
       }
   }
   return 1;
+}
+
+// What dk_bwd_balanced asks for.  A pair of rows counts as its kernel does: rows outside [first, last] hold nothing.
+int dk_call_row_lengths(const int32_t *ptr, const int32_t *idx, const int32_t *order, int32_t heads, int32_t rows, int64_t idx_stride,
+                        int32_t first, int32_t last, int32_t limit, int32_t *out) {
+  dk::clear_error();
+  DK_REQUIRE(ptr && order && out && (idx || rows == 0), "NULL argument");
+  DK_REQUIRE(heads >= 1 && rows >= 0, "bad shape (%d, %d)", heads, rows);
+  const int pairs = (rows + 1) / 2;
+  std::fill(out, out + rows + pairs, -1);
+  std::vector<int32_t> lens((size_t)rows + 1);
+  for (int h = 0; h < heads; ++h) {
+    const int32_t *p = ptr + (size_t)h * (rows + 1), *o = order + (size_t)h * (rows + pairs), *e = idx + h * idx_stride;
+    lens[rows] = -1;  // (an odd table's last pair has one row)
+    for (int r = 0; r < rows; ++r)
+      lens[r] = r < first || r > last ? -1 : (int32_t)(std::lower_bound(e + p[r], e + p[r + 1], limit) - (e + p[r]));
+    for (int i = 0; i < rows; ++i) out[i] = std::max(out[i], lens[o[i]]);
+    for (int i = 0; i < pairs; ++i) {
+      const int32_t a = lens[2 * o[rows + i]], b = lens[2 * o[rows + i] + 1];
+      out[rows + i] = std::max(out[rows + i], a < 0 ? b : b < 0 ? a : a + b);
+    }
+  }
+  return DK_OK;
 }
 
 }  // extern "C"

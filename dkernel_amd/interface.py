@@ -5,7 +5,6 @@ that a model written against `dkernel` runs unchanged.
 """
 from __future__ import annotations
 
-import array
 import copy
 import math
 import warnings
@@ -62,17 +61,6 @@ def _unsorted_rows(pattern: Tensor) -> bool:
         return False
     later = torch.flip(torch.cummax(torch.flip(lens, (1,)), dim=1).values, (1,))[:, 1:]  # longest later row
     return bool((4 * lens[:, :-1] > 5 * later + 8).any())
-
-
-def _row_lengths(ptr: Tensor) -> array.array:
-    """Entries of a table's rows by descending length, the most over the heads at every place, followed by
-    those of the pairs of rows (2u, 2u + 1): what the backward's launches are planned by (host memory)."""
-    ptr = ptr if ptr.dim() == 2 else ptr[None]
-    if ptr.stride(0) == 0:
-        ptr = ptr[:1]
-    lens = (ptr[:, 1:] - ptr[:, :-1]).to("cpu", torch.int32)
-    pairs = torch.nn.functional.pad(lens, (0, lens.size(1) % 2)).view(lens.size(0), -1, 2).sum(2, dtype=torch.int32)
-    return array.array("i", torch.cat([torch.sort(x, dim=1, descending=True).values.amax(0) for x in (lens, pairs)]).tolist())
 
 
 class SparseAttention(torch.nn.Module):
@@ -281,11 +269,19 @@ class SparseAttention(torch.nn.Module):
             self.register_buffer("masked_csc_row", m_csc[1].to(torch.int32), persistent=False)
 
         self._kernel_tables = self._table_names()
-        # lengths of the rows and columns of the tables that the backward reads
-        csr, csc = self._backward_tables()
-        self.kwargs["row_lengths"] = tuple(
-            tuple(_row_lengths(getattr(self, name)) for name in names)
-            for names in [(csr, csc)] + ([("masked_csr_crow", "masked_csc_ccol")] if self.mask_tile is not None else []))
+        self.kwargs["row_lengths"] = self._row_lengths()
+
+    def _row_lengths(self) -> Tuple:
+        """Host copies of the tables that the backward reads: it plans its launches by how much of their rows
+        and columns a call works on."""
+        names = [self._backward_tables()] + ([("masked_csr_crow", "masked_csc_ccol")] if self.mask_tile is not None else [])
+
+        def table(ptr, idx):
+            return ops.TableLengths(self._buffers[ptr], self._buffers[ptr.rpartition("_")[0] + "_" + idx], self.lut_group)
+
+        # (rows are cut where the launches take them in the table's own order)
+        return tuple(ops.BackwardLengths(table(csr, "col") if self.kwargs["unsorted_rows"] else None, table(csc, "row"))
+                     for csr, csc in names)
 
     def _backward_tables(self) -> Tuple[str, str]:
         if self.kernel_tile is not None:
@@ -312,6 +308,8 @@ class SparseAttention(torch.nn.Module):
         self.__dict__.setdefault("mask_lut_max_row", 0)
         self.__dict__.setdefault("_kernel_tables", self._table_names())
         self.kwargs.setdefault("fixed_walk", self.kwargs.get("unsorted_rows", False))
+        if not all(isinstance(x, ops.BackwardLengths) for x in self.kwargs.get("row_lengths", [None])):
+            self.kwargs["row_lengths"] = self._row_lengths()
 
     def forward(self,
                 q: Tensor,

@@ -11,6 +11,7 @@ synchronises with the host.
 """
 from __future__ import annotations
 
+import array
 import ctypes as C
 import os
 import math
@@ -104,20 +105,90 @@ def _lut(layout: Tuple[Tensor, Tensor, int, int], device, group: int = 1, max_ro
         lut.uneven_heads, lut.fixed_walk = int(bool(uneven)), int(bool(fixed_walk))
         order = None
         if longest_first:
-            # rows of every head by descending length (stable: equal lengths stay in index order),
-            # computed on the device once per table: the dK/dV pass hands its columns out in this
-            # order, the forward and dQ kernels the rows of a pattern whose long rows are not its last
-            ptr = layout[0] if layout[0].dim() == 2 else layout[0][None]
-            lens = ptr[:, 1:] - ptr[:, :-1]
-            rows = lens.size(1)
-            # ... followed by the pairs of rows (2u, 2u + 1) by descending length of the pair
-            pair_lens = torch.nn.functional.pad(lens, (0, rows % 2)).view(lens.size(0), -1, 2).sum(2)
-            order = torch.cat([torch.argsort(x, dim=1, descending=True, stable=True) for x in (lens, pair_lens)],
-                              dim=1).to(torch.int32).contiguous()
+            # once per table, on the device: the dK/dV pass hands its columns out in this order, the
+            # forward and dQ kernels the rows of a pattern whose long rows are not its last
+            order = _longest_first(layout[0] if layout[0].dim() == 2 else layout[0][None])
+            rows = layout[0].size(-1) - 1
             lut.row_order, lut.row_order_stride_h = order.data_ptr(), order.stride(0)
             lut.pair_order = order.data_ptr() + 4 * rows
         hit = _LUT_CACHE[key] = (lut, layout[0], layout[1], order)
     return _lib.Lut.from_buffer_copy(hit[0])
+
+
+class TableLengths:
+    """Host copy of a table (`every`: its heads come in runs of so many identical ones): the lengths of its rows in the order
+    of _lut(longest_first=True), as far as a call works on them."""
+
+    def __init__(self, ptr: Tensor, idx: Tensor, every: int = 1):
+        if ptr.dim() == 1:
+            ptr, idx = ptr[None], idx[None]
+        every = ptr.size(0) if ptr.stride(0) == 0 else every if ptr.size(0) % every == 0 else 1
+        self.ptr = ptr[::every].to("cpu", torch.int32).contiguous()
+        idx = idx if idx.dim() == 2 else idx[:, :, 0]  # (column, mask) entries
+        self.idx = idx[::every].to("cpu", torch.int32).contiguous()
+        self.order = _longest_first(self.ptr)
+        self.rows = self.ptr.size(1) - 1
+
+    def of_call(self, first: int, last: int, limit: int) -> array.array:
+        """Lengths of the rows first .. last, counting entries below `limit` (-1 at places of other rows), followed by those of
+        their pairs."""
+        out = array.array("i", bytes(4 * (self.rows + (self.rows + 1) // 2)))
+        _lib.check(_lib.lib().dk_call_row_lengths(self.ptr.data_ptr(), self.idx.data_ptr(), self.order.data_ptr(), self.ptr.size(0),
+                                                  self.rows, self.idx.stride(0), first, last, limit, out.buffer_info()[0]))
+        return out
+
+    def __eq__(self, other):
+        return isinstance(other, TableLengths) and torch.equal(self.ptr, other.ptr) and torch.equal(self.idx, other.idx)
+
+    __hash__ = None
+
+
+class BackwardLengths:
+    """Lengths of the row table (None: its rows are not taken in an order of their own) and the column table of 64 x 64 tiles
+    that a backward reads.  They are worked out once per shape of a call (the blocks of its first and last query and of its
+    last key; some ten microseconds for long tables) and handed to the library as they are from then on."""
+
+    def __init__(self, csr: Optional[TableLengths], csc: TableLengths):
+        self.csr, self.csc = csr, csc
+        self._calls = {}
+
+    def of_call(self, past: int, q_len: int, k_len: int) -> Tuple:
+        key = (past // 64, (past + q_len - 1) // 64, (k_len - 1) // 64)
+        hit = self._calls.get(key)
+        if hit is None:
+            first, last, last_k = key
+            columns = self.csc.of_call(0, last_k, last + 1)
+            rows = self.csr.of_call(first, last, 2**31 - 1) if self.csr is not None else None
+            at = rows.buffer_info()[0] if rows is not None else None
+            lengths = _lib.RowLengths(at, at + 4 * self.csr.rows if at else None, columns.buffer_info()[0])
+            if len(self._calls) >= 64:
+                self._calls.clear()
+            hit = self._calls[key] = (lengths, rows, columns)
+        return hit  # (with the arrays that the lengths lie in)
+
+    def fits(self, layout_csr, layout_csc) -> bool:
+        return (layout_csr[2] == 64 and layout_csc[2] == 64 and layout_csc[0].size(-1) == self.csc.rows + 1 and
+                (self.csr is None or layout_csr[0].size(-1) == self.csr.rows + 1))
+
+    def __eq__(self, other):
+        return isinstance(other, BackwardLengths) and self.csr == other.csr and self.csc == other.csc
+
+    __hash__ = None
+
+    def __getstate__(self):
+        return {**self.__dict__, "_calls": {}}
+
+
+_NO_LENGTHS = _lib.RowLengths()
+
+
+def _longest_first(ptr: Tensor) -> Tensor:
+    """Rows of every head by descending length (stable: equal lengths stay in index order), followed by the pairs of
+    rows (2u, 2u + 1) by descending length of the pair."""
+    lens = ptr[:, 1:] - ptr[:, :-1]
+    pair_lens = torch.nn.functional.pad(lens, (0, lens.size(1) % 2)).view(lens.size(0), -1, 2).sum(2)
+    return torch.cat([torch.argsort(x, dim=1, descending=True, stable=True) for x in (lens, pair_lens)],
+                     dim=1).to(torch.int32).contiguous()
 
 
 def _make_lut(layout: Tuple[Tensor, Tensor, int, int], device, group: int = 1, max_row: int = 0) -> _lib.Lut:
@@ -290,9 +361,9 @@ def _backward(ctx, do: Tensor, dlse: Optional[Tensor],
     masked = getattr(ctx, "masked_layouts", None)
     if masked is not None and _matrix_core_applies(q, k, v, o, do, dq, dk, dv):
         layout_csr, layout_csc = masked[0], masked[1]
-        lengths = ctx.row_lengths[1:]
+        tables = ctx.row_lengths[1] if len(ctx.row_lengths) > 1 else None
     else:
-        lengths = ctx.row_lengths[:1]
+        tables = ctx.row_lengths[0] if ctx.row_lengths else None
     uneven = getattr(ctx, "uneven_heads", False)
     args.csr = _lut(layout_csr, q.device, ctx.lut_group, uneven=uneven,
                     longest_first=getattr(ctx, "unsorted_rows", False))
@@ -302,12 +373,12 @@ def _backward(ctx, do: Tensor, dlse: Optional[Tensor],
     args.dtype, args.causal, args.impl = _DTYPES[q.dtype], int(bool(ctx.causal)), _impl
     args.sm_scale = float(ctx.sm_scale)
     args.stream = _stream()
-    rows = _lib.RowLengths()
-    for (csr_lengths, csc_lengths) in lengths:
-        n, m = args.csr.num_rows, args.csc.num_rows
-        assert len(csr_lengths) == n + (n + 1) // 2 and len(csc_lengths) == m + (m + 1) // 2
-        csr, csc = csr_lengths.buffer_info()[0], csc_lengths.buffer_info()[0]
-        rows = _lib.RowLengths(csr, csr + 4 * n, csc)
+    rows = _NO_LENGTHS
+    if tables is not None and tables.fits(layout_csr, layout_csc):
+        # what this call works on of tables that may be built for longer sequences (`held`: until the call is made)
+        Lk = k.size(seq_dim)
+        held = tables.of_call(Lk - Lq if ctx.causal else 0, Lq, Lk)
+        rows = held[0]
     lib = _lib.lib()
     need = lib.dk_bwd_balanced_workspace_bytes(C.byref(args), C.byref(rows)) if _bwd_workspace else 0
     if need:  # dK/dV partials per q head (several q heads per kv head), partial sums of long rows and columns

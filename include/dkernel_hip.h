@@ -284,12 +284,21 @@ size_t dk_bwd_workspace_bytes(const dk_bwd_args *args);
 
 /* Lengths of a backward call's tables in HOST memory, read during the call only: entries of the i-th row in the
  * table's row_order (csr_rows, csc_rows: num_rows values) or of the i-th pair in its pair_order (csr_pairs:
- * (num_rows + 1) / 2 values), the most over the heads.  Any may be NULL, and those of a table without that
+ * (num_rows + 1) / 2 values), the most over the heads; negative where no head has a row of the call.  Only what the call
+ * works on counts (dk_call_row_lengths).  Any may be NULL, and those of a table without that
  * order are not read.  Wrong lengths cost time, never correctness.  The entries of every row of a table
  * whose lengths are given ascend (as those of dk_csr_fill do); without lengths they come in any order. */
 typedef struct dk_row_lengths {
   const int32_t *csr_rows, *csr_pairs, *csc_rows;
 } dk_row_lengths;
+
+/* Such lengths of a call from a table in HOST memory (a table may be built for longer sequences than a call has, and launches
+ * planned by all of it suit none): rows first .. last, and of each its entries below `limit`.  Row table of a call: the blocks of
+ * its first and last query position, limit INT32_MAX.  Column table: 0 .. block of the last key, limit 1 + block of the last
+ * query position.  ptr: (heads, rows + 1); idx: one int per entry, idx_stride ints a head, ascending in each row; order: (heads, rows +
+ * (rows + 1) / 2), the row order followed by the pair order.  out: rows values for the rows, (rows + 1) / 2 for the pairs. */
+int dk_call_row_lengths(const int32_t *ptr, const int32_t *idx, const int32_t *order, int32_t heads, int32_t rows, int64_t idx_stride,
+                        int32_t first, int32_t last, int32_t limit, int32_t *out);
 
 /* dk_bwd that knows how long the rows of its tables are: rows and columns that would outlast the rest of the launch
  * (global rows, vertical columns with few heads) are cut into segments of their own workgroups, whose fp32 sums

@@ -81,3 +81,20 @@ def test_segments_of_groups(B, Hq, Hkv, L, table, D, bs, dtype, cut, monkeypatch
     ulp = {torch.float32: 2e-5, torch.float16: 1e-3, torch.bfloat16: 8e-3}[dtype]
     for name, a, b in zip(("dQ", "dK", "dV"), got, whole):
         assert_close(name, a, b, atol=ulp * float(b.float().abs().max()) / 8, rtol=ulp)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,table,bs,walks", [
+    (1, 32, 8, 1000, 8192, 64, False), (1, 32, 8, 2048, 32768, 64, False), (2, 24, 8, 700, 4096, 32, False),
+    (4, 32, 8, 2048, 8192, 64, True)])
+def test_short_call_of_a_module_for_long_sequences(B, Hq, Hkv, L, table, bs, walks):
+    """The launches are planned by the call: the kernels, and (nothing being cut) the bits, of a module for that length."""
+    g = torch.Generator(device=DEV).manual_seed(2)
+    q, k, v, do = (torch.randn(B, L, h, 128, generator=g, device=DEV).to(torch.bfloat16) for h in (Hq, Hkv, Hkv, Hq))
+    (got, ran), (want, ran_tight) = (
+        _run(LocalStrideSparseAttention(Hq, n, bs, 16 * 64 // bs, 8, num_kv_heads=Hkv).to(DEV), q, k, v, do, 0.1) for n in (table, L))
+    assert ran == ran_tight and ("per q head" not in ran) == walks, (ran, ran_tight)
+    for name, a, b in zip(("dQ", "dK", "dV"), got, want):
+        if "segment_sum" in ran:
+            assert_close(name, a, b, atol=1e-3 * float(b.float().abs().max()), rtol=8e-3)
+        else:
+            assert torch.equal(a, b), name
