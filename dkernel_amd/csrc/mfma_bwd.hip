@@ -363,7 +363,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 // the L2 into LDS (what the one-tile kernel spent a quarter of its time on) is halved; a wave
 // skips the blocks its own row does not hold.  Every wave owns the finished dQ of its rows:
 // nothing is summed across waves at the end.
-template <typename T, int D, bool PAD, bool SUB, int KD = D>
+// CUT: launches that cut long pairs into segments; an instantiation of its own, as its prologue, jumped over, and the fifty
+// scalars it spills took launches that cut nothing 4 - 8 % longer (16 heads of 128, 2 x 3108 tokens 76.3 / 79.6 us, 32 heads, 2 x 1932
+// 58.4 / 63.2).
+template <typename T, int D, bool PAD, bool SUB, bool CUT, int KD = D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 ? 3 : 2))) void mfma_dq_pair_kernel(const BwdParams p,
                                                                                                       int pairs_y) {
   using M = Mma<T>;
@@ -380,8 +383,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   const int first_rb = sq.past / 64, last_rb = (sq.past + sq.q_len - 1) / 64;
   const int h = grid_head(p.csr);
   int u = (first_rb >> 1) + pairs_y - 1 - (int)blockIdx.y;  // longest rows first (of a causal pattern)
-  int place, seg;  // (long pairs cut into segments: with the table's own order only)
-  find_segment(p.seg, blockIdx.y, place, seg);
+  int place = blockIdx.y, seg = 0;  // (long pairs cut into segments: with the table's own order only)
+  if constexpr (CUT) find_segment(p.seg, blockIdx.y, place, seg);
   if (p.csr.pair_order)  // the table's own order, longest pairs first (the grid then covers every pair of it)
     u = scalar_load(p.csr.pair_order + lut_head(p.csr, h, p.Hq, p.Hkv) * p.csr.order_sh + place);
   if (u > (last_rb >> 1) || u < (first_rb >> 1)) return;
@@ -397,41 +400,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   const bool row_ok = qi >= 0 && qi < sq.q_len;  // (a table row without queries of this sequence: false everywhere)
   // the two table rows: entries [e0, emid) are row 2u, [emid, e1) row 2u + 1 (consecutive rows
   // follow each other in the table); a row without queries of this sequence contributes nothing
-  const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
-  int e0 = 0, emid = 0, e1 = 0;
-  {
+  auto table_rows = [&](int lh, int &e0, int &emid, int &e1) __attribute__((always_inline)) {
     const int32_t *rp = p.csr.ptr + lh * p.csr.ptr_sh;
     if (ra < p.csr.num_rows) scalar_load2(rp + ra, rp + ra + 1, e0, emid);
     e1 = emid;
     if (ra + 1 < p.csr.num_rows) e1 = scalar_load(rp + ra + 2);
     if (ra < first_rb) e0 = emid;
     if (ra + 1 > last_rb) e1 = emid;
-  }
-  const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
-  // this workgroup's entries [a0, a1) and [b0, b1) of the two rows, and the place of its partial sum (-1: it takes both rows
-  // whole)
-  int a0 = e0, a1 = emid, b0 = emid, b1 = e1, slot = -1;
-  if (p.seg.entries && place < p.seg.n[1]) {
-    const int segments = planned_segments(p.seg, place, (e1 - e0 + 1) / 2);
-    if (seg >= segments) return;
-    if (segments > 1) {
-      slot = seg * p.seg.n[1] + place;
-      // an even share of the longer row's entries, and what the other row lists between their columns
-      const bool first_longer = emid - e0 >= e1 - emid;
-      const int l0 = first_longer ? e0 : emid, len = first_longer ? emid - e0 : e1 - emid;
-      const int s0 = __builtin_amdgcn_readfirstlane(len * seg / segments), s1 = __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
-      const int o0 = first_longer ? emid : e0, o1 = first_longer ? e1 : emid;
-      int p0 = o0, p1 = o1;
-      if (seg > 0) p0 = entry_lower_bound<EW>(cols, o0, o1, scalar_load(cols + (l0 + s0) * EW));
-      if (seg + 1 < segments) p1 = entry_lower_bound<EW>(cols, p0, o1, scalar_load(cols + (l0 + s1) * EW));
-      a0 = first_longer ? l0 + s0 : p0, a1 = first_longer ? l0 + s1 : p1;
-      b0 = first_longer ? p0 : l0 + s0, b1 = first_longer ? p1 : l0 + s1;
-    }
-  }
-  // Kept in LDS until they are used.  No barrier stands between a wave's store and its reads: that is sound only as
-  // long as every wave stores each place once and all waves the same value.
+  };
+  // CUT: this workgroup's entries [part[0], part[1]) and [part[2], part[3]) of the two rows, and the place of its partial sum
+  // (part[4], -1: it takes both rows whole), kept in LDS until they are used.  No barrier stands between a wave's store and
+  // its reads: that is sound only as long as every wave stores each place once and all waves the same value.
   __shared__ int part[5];
-  part[0] = a0, part[1] = a1, part[2] = b0, part[3] = b1, part[4] = slot;
+  if constexpr (CUT) {
+    const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
+    int e0 = 0, emid = 0, e1 = 0;
+    table_rows(lh, e0, emid, e1);
+    const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
+    int a0 = e0, a1 = emid, b0 = emid, b1 = e1, slot = -1;
+    if (place < p.seg.n[1]) {
+      const int segments = planned_segments(p.seg, place, (e1 - e0 + 1) / 2);
+      if (seg >= segments) return;
+      if (segments > 1) {
+        slot = seg * p.seg.n[1] + place;
+        // an even share of the longer row's entries, and what the other row lists between their columns
+        const bool first_longer = emid - e0 >= e1 - emid;
+        const int l0 = first_longer ? e0 : emid, len = first_longer ? emid - e0 : e1 - emid;
+        const int s0 = __builtin_amdgcn_readfirstlane(len * seg / segments), s1 = __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
+        const int o0 = first_longer ? emid : e0, o1 = first_longer ? e1 : emid;
+        int p0 = o0, p1 = o1;
+        if (seg > 0) p0 = entry_lower_bound<EW>(cols, o0, o1, scalar_load(cols + (l0 + s0) * EW));
+        if (seg + 1 < segments) p1 = entry_lower_bound<EW>(cols, p0, o1, scalar_load(cols + (l0 + s1) * EW));
+        a0 = first_longer ? l0 + s0 : p0, a1 = first_longer ? l0 + s1 : p1;
+        b0 = first_longer ? p0 : l0 + s0, b1 = first_longer ? p1 : l0 + s1;
+      }
+    }
+    part[0] = a0, part[1] = a1, part[2] = b0, part[3] = b1, part[4] = slot;
+  }
 
   if (PAD && p.D < KD) {  // the slots of the head dims beyond p.D stay zero for the whole kernel
     zero_tiles<NT>(smem, 2 * STAGE, tid);
@@ -474,6 +479,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
     }
   }
 
+  const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
+  int e0 = 0, emid = 0, e1 = 0;
+  if constexpr (!CUT) table_rows(lh, e0, emid, e1);
+  const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
   const T *kbase = (const T *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh;
   const T *vbase = (const T *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh;
 
@@ -518,8 +527,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   // (scalar), pend_a / pend_b the entries after them (vector loads, first used behind a tile
   // wait, so that no table read stalls the loop); flg_cur says which rows hold the current column.
   constexpr int kEnd = 0x7fffffff;
-  int a_pos = __builtin_amdgcn_readfirstlane(part[0]), b_pos = __builtin_amdgcn_readfirstlane(part[2]);
-  const int a_end = __builtin_amdgcn_readfirstlane(part[1]), b_end = __builtin_amdgcn_readfirstlane(part[3]);
+  int a_pos = e0, b_pos = emid, a_end = emid, b_end = e1;
+  if constexpr (CUT) {
+    a_pos = __builtin_amdgcn_readfirstlane(part[0]), b_pos = __builtin_amdgcn_readfirstlane(part[2]);
+    a_end = __builtin_amdgcn_readfirstlane(part[1]), b_end = __builtin_amdgcn_readfirstlane(part[3]);
+  }
   int head_a = kEnd, head_b = kEnd, pend_a = 0, pend_b = 0;
   int hbits_a = 0, hbits_b = 0, pbits_a = 0, pbits_b = 0;  // SUB: the entries' masks, carried like the columns
   if (a_pos < a_end) head_a = scalar_load(cols + a_pos * EW);
@@ -561,7 +573,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   if (row_ok) {
     lse2 = lse_raw == -INFINITY ? INFINITY : lse_raw * kLog2e;
     delta = delta_rows[ts * 64 + rh * 32 + m] - dlse_raw;
-    if (g == 0 && part[4] < p.seg.n[1]) p.delta[((int64_t)sq.b * p.Hq + h) * p.seqs.max_q_len + qi] = delta;
+    if (g == 0 && (!CUT || part[4] < p.seg.n[1])) p.delta[((int64_t)sq.b * p.Hq + h) * p.seqs.max_q_len + qi] = delta;
   }
 
   auto block_step = [&](auto stage_tag) {
@@ -675,8 +687,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
     block_step(IntConst<1>{});
   }
 
-  const int slot_end = p.seg.entries ? __builtin_amdgcn_readfirstlane(part[4]) : -1;
-  if (slot_end >= 0) {  // fp32 partial sum, unscaled
+  int slot_end = -1;
+  if constexpr (CUT) slot_end = __builtin_amdgcn_readfirstlane(part[4]);
+  if (CUT && slot_end >= 0) {  // fp32 partial sum, unscaled
     int late = lane;  // (opaque: the addresses are computed here, not kept through the loop)
     asm volatile("" : "+v"(late));
     float *outp = p.seg.partial + ((((int64_t)sq.b * p.Hq + h) * p.seg.slots + slot_end) * 128 + wave * 32 + (late & 31)) * p.D + (late >> 5) * 4;
@@ -1164,26 +1177,46 @@ template __global__ void mfma_dkdv_kernel<bf16_t, 256, true, false>(const BwdPar
 template __global__ void mfma_dkdv_kernel<bf16_t, 256, true, true>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 256, true, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<f16_t, 256, true, true>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 128, false, false>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, false>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, false, 96>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 128, false, true>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, true>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, true, 96>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 64, false, false>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 64, true, false>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 64, false, true>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<bf16_t, 64, true, true>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 128, false, false>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, false>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, false, 96>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 128, false, true>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, true>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, true, 96>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 64, false, false>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 64, true, false>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 64, false, true>(const BwdParams, int);
-template __global__ void mfma_dq_pair_kernel<f16_t, 64, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, false, false, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, false, false, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, false, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, false, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, false, false, 96>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, false, true, 96>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, false, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, false, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, true, false, 96>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 128, true, true, true, 96>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 64, false, false, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 64, false, false, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 64, true, false, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 64, true, false, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 64, false, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 64, false, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 64, true, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<bf16_t, 64, true, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, false, false, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, false, false, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, false, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, false, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, false, false, 96>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, false, true, 96>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, false, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, false, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, true, false, 96>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 128, true, true, true, 96>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 64, false, false, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 64, false, false, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 64, true, false, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 64, true, false, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 64, false, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 64, false, true, true>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 64, true, true, false>(const BwdParams, int);
+template __global__ void mfma_dq_pair_kernel<f16_t, 64, true, true, true>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 128, false, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 128, true, false>(const BwdParams, int);
 template __global__ void mfma_dkdv_kernel<bf16_t, 128, true, false, 96>(const BwdParams, int);
@@ -1386,14 +1419,19 @@ static int launch_bwd_td(const BwdParams &p, void *workspace, size_t workspace_b
   // dQ first: it also writes delta, which the dK/dV pass reads
   if constexpr (D <= 128) {  // two table rows per workgroup
     int pairs = (((past + s.max_q_len - 1) / 64) >> 1) - ((past / 64) >> 1) + 1;
-    DK_ALLOW_DYNAMIC_LDS((mfma_dq_pair_kernel<T, D, PAD, SUB, KD>), smem_dq);
     if (p.csr.pair_order) pairs = (p.csr.num_rows + 1) / 2;  // handed out in the table's order: all of them
     BwdParams pq = p;
     if (p.csr.pair_order && segment_items(scratch.dq, pairs) <= 65535) pq.seg = scratch.dq;
     const int items = (int)segment_items(pq.seg, pairs);
     pq.csr.rot = head_rotation(p.csr, p.Hq, items);  // (uneven heads: dealt to the queues in rotation)
     DK_NOTE_KERNEL(pq.csr.rot ? "mfma_dq_pair_kernel, heads in rotation" : "mfma_dq_pair_kernel");
-    hipLaunchKernelGGL((mfma_dq_pair_kernel<T, D, PAD, SUB, KD>), dim3(p.Hq, items, s.batch), dim3(256), smem_dq, stream, pq, pairs);
+    if (pq.seg.entries) {
+      DK_ALLOW_DYNAMIC_LDS((mfma_dq_pair_kernel<T, D, PAD, SUB, true, KD>), smem_dq);
+      hipLaunchKernelGGL((mfma_dq_pair_kernel<T, D, PAD, SUB, true, KD>), dim3(p.Hq, items, s.batch), dim3(256), smem_dq, stream, pq, pairs);
+    } else {
+      DK_ALLOW_DYNAMIC_LDS((mfma_dq_pair_kernel<T, D, PAD, SUB, false, KD>), smem_dq);
+      hipLaunchKernelGGL((mfma_dq_pair_kernel<T, D, PAD, SUB, false, KD>), dim3(p.Hq, items, s.batch), dim3(256), smem_dq, stream, pq, pairs);
+    }
     DK_HIP_CHECK(hipGetLastError());
     if (pq.seg.entries) {
       const int dtype = std::is_same<T, bf16_t>::value ? DK_BF16 : DK_F16;
