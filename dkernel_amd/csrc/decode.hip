@@ -134,7 +134,7 @@ __device__ __forceinline__ uint4 fp8x8_to(uint2 w) {
 }
 
 // Sequence that the workgroups of grid.z = place take when the sequences are handed out by length: the `first` longest
-// ones in ascending order, then the others in descending order (lengths to within a 64th of the longest there can be;
+// ones in ascending order, then the others in descending order (lengths to within a 32nd of the longest one or finer;
 // equal ones in the batch's order).  At most kRankedSequences sequences, all lanes active.  Every lane loads the geometry
 // of its sequences, so the lengths cost no round trip beyond the workgroup's own; the length at a rank is found bit by bit
 // from the lanes' votes (64 keys to a block: six votes, 0.3 us of a step).
@@ -143,11 +143,13 @@ __device__ __forceinline__ SeqInfo sequence_by_length(const SeqView &s, int plac
   const int rank = place < first ? first - 1 - place : place;
   const int lane = threadIdx.x & 63;
   const bool two = s.batch > 64;  // sequences a lane
-  const int drop = max(0, 26 - __clz(s.max_k_len | 1));  // length bits that are left out: six remain
-  auto key = [&](const SeqInfo &t, int i) { return i < s.batch ? (t.q_len > 0 ? t.k_len >> drop : 0) : -1; };
   const SeqInfo lo = load_seq_lane(s, min(lane, s.batch - 1), causal);
   SeqInfo hi = lo;
   if (two) hi = load_seq_lane(s, min(lane + 64, s.batch - 1), causal);
+  // length bits that are left out: six remain (of the longest sequence that is there: the extent of the key dimension is the
+  // capacity of a cache or block table, or the tokens of all packed sequences together)
+  const int drop = max(0, 26 - __clz(wave_max(max(lo.k_len, hi.k_len)) | 1));
+  auto key = [&](const SeqInfo &t, int i) { return i < s.batch ? (t.q_len > 0 ? t.k_len >> drop : 0) : -1; };
   const int key_lo = key(lo, lane), key_hi = key(hi, lane + 64);
   auto votes = [&](int at) { return __popcll(__ballot(key_lo >= at)) + (two ? __popcll(__ballot(key_hi >= at)) : 0); };
   int len = 0;  // largest length that more than `rank` sequences reach
@@ -630,7 +632,7 @@ static int launch_decode_td(const FwdParams &p, float *ws, hipStream_t stream) {
   DK_REQUIRE(smem <= 160 * 1024, "decode workgroup needs %d bytes of LDS", smem);
   const dim3 grid(groups, p.Hkv, p.seqs.batch), block(64 * W);
   const int first = decode_first_by_length(p, groups);
-  DK_NOTE_KERNEL("decode_partial_kernel");
+  DK_NOTE_KERNEL(first > 0 ? "decode_partial_kernel, sequences by length" : "decode_partial_kernel");
   if (first > 0) {
     DK_ALLOW_DYNAMIC_LDS((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W, true>), smem);
     hipLaunchKernelGGL((decode_partial_kernel<T, D, PAD, SUB, PAGED, KV8, W, true>), grid, block, smem, stream, p, ws,

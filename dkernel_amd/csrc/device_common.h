@@ -324,6 +324,17 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
   return v;
 }
 
+// Largest v over the lanes of a wave (all of them active, v >= 0), the same way.
+__device__ __forceinline__ int wave_max(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 template <typename Count>
 __device__ __forceinline__ bool find_packed_sequence(const SeqView &s, int causal, int item, Count count, SeqInfo &info,
                                                      int &index_in_seq) {
