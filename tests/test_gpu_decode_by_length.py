@@ -8,7 +8,7 @@ import random
 import pytest
 import torch
 
-from dkernel_amd import LocalStrideSparseAttention
+from dkernel_amd import LocalStrideSparseAttention, _lib
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -33,7 +33,7 @@ def test_every_sequence_as_in_the_order_of_the_batch(batch, kind, padding):
     g = torch.Generator(device=DEV).manual_seed(batch)
     q, k, v = (torch.randn(batch, n, h, D, generator=g, device=DEV, dtype=torch.bfloat16)
                for n, h in ((1, HQ), (LMAX, HKV), (LMAX, HKV)))
-    mod = LocalStrideSparseAttention(HQ, LMAX, 64, 4, 4, num_kv_heads=HKV).to(DEV)
+    mod = LocalStrideSparseAttention(HQ, LMAX, 64, 16, 4, num_kv_heads=HKV).to(DEV)  # (rows that grow with their sequences)
 
     def step(rows):
         n = torch.tensor([lens[i] for i in rows], dtype=torch.int32, device=DEV)
@@ -46,6 +46,7 @@ def test_every_sequence_as_in_the_order_of_the_batch(batch, kind, padding):
         return mod(q[at], k[at], v[at], D ** -0.5, return_lse=True, **lengths)
 
     out, lse = step(list(range(batch)))
+    assert (b"sequences by length" in _lib.lib().dk_last_kernels()) == (batch <= 128)
     for i in range(0, batch, PLAIN):
         rows = [min(j, batch - 1) for j in range(i, i + PLAIN)]
         ref_out, ref_lse = step(rows)

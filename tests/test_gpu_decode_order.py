@@ -1,4 +1,4 @@
-"""Decode steps that hand their sequences out by length (sequence_by_length, decode.hip): that the order, by the
+"""Which decode steps hand their sequences out by length (decode_first_by_length, decode.hip), and that the order, by the
 longest sequence present, does not show in the results: caches, block tables and packed keys far larger than their sequences."""
 from __future__ import annotations
 
@@ -53,3 +53,23 @@ def test_capacity_beyond_the_sequences(form, batch, longest):
         ref = step([min(j, batch - 1) for j in range(i, i + PLAIN)])
         assert not _by_length()
         assert torch.equal(out[i:i + PLAIN], ref[:min(PLAIN, batch - i)])
+
+
+@pytest.mark.parametrize("batch,length,local,vert,D,ranked", [
+    (48, 1216, 16, 64, 64, True),    # 19 blocks, rows of 17: they grow with their sequences, 17 x 64 = 1088
+    (48, 1216, 8, 64, 64, False),    # rows of 9: a window and a column
+    (40, 200, 2, 8, 256, True),      # 256 dims: always
+    (48, 384, 16, 8, 64, True),      # 6 blocks of 64 dims: 384
+    (48, 320, 16, 8, 64, False),     # 5: 320
+    (48, 4096, 13, 8, 64, True),     # rows of 20: 1280
+    (48, 4096, 12, 8, 64, False),    # of 19
+    (16, 1024, 16, 8, 128, False),   # growing rows of 16, 256 workgroups
+    (20, 1024, 16, 8, 128, True),    # 320, two a row: 1024 each
+    (10, 1536, 16, 3, 128, False),   # four a row of 19: 608
+    (128, 4096, 16, 8, 128, True),   # 1024 workgroups
+    (129, 4096, 16, 8, 128, False)])
+def test_which_steps_take_it(batch, length, local, vert, D, ranked):
+    mod = LocalStrideSparseAttention(16, length, 64, local, vert, num_kv_heads=HKV).to(DEV)
+    q, k, v = (torch.randn(batch, n, h, D, device=DEV, dtype=torch.bfloat16) for n, h in ((1, 16), (length, HKV), (length, HKV)))
+    mod(q, k, v, 0.1, seqlens=torch.full((batch,), length, dtype=torch.int32, device=DEV))
+    assert _by_length() == ranked, mod.lut_max_row
