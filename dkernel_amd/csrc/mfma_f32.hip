@@ -420,8 +420,9 @@ __global__ __launch_bounds__(256) void delta_kernel(const BwdParams p) {
 
 // dQ: workgroup = 64 q rows of one head; wave = 32 rows x 32 keys of every listed block: S^T = K Q^T,
 // dP^T = V dO^T (lane = q row: lse and delta are per-lane scalars), dS^T = P^T (dP^T - delta),
-// dQ^T += K^T dS^T; the two key halves are added at the end.
-template <int KD, bool PAD>
+// dQ^T += K^T dS^T; the two key halves are added at the end.  CUT: launches that cut long rows into segments, as in the 16-bit
+// pass (in one instantiation with them launches that cut nothing spilled forty scalars more).
+template <int KD, bool PAD, bool CUT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2 : 1, KD <= 64 ? 2 : 1))) void dq_kernel(
     const BwdParams p, int tiles_y) {
   using S = Shape<KD, PAD>;
@@ -429,22 +430,27 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   const SeqInfo sq = load_seq(p.seqs, blockIdx.z, p.causal);
   const int h = grid_head(p.csr), kvh = __builtin_amdgcn_readfirstlane(h / (p.Hq / p.Hkv));
   int tile = tiles_y - 1 - (int)blockIdx.y;
-  int place, seg, segments = 1;  // (long rows are cut into segments: with the table's own order only)
-  find_segment(p.seg, blockIdx.y, place, seg);
+  int place = blockIdx.y, seg = 0, segments = 1;  // (long rows are cut into segments: with the table's own order only)
+  if constexpr (CUT) find_segment(p.seg, blockIdx.y, place, seg);
   if (p.csr.order)
     tile = scalar_load(p.csr.order + lut_head(p.csr, h, p.Hq, p.Hkv) * p.csr.order_sh + place) - sq.past / 64;
   if (tile < 0 || tile >= seq_row_blocks(sq, 64)) return;
   const int rb = sq.past / 64 + tile;
   const int lh = lut_head(p.csr, h, p.Hq, p.Hkv);
   int e0 = 0, e1 = 0;
-  if (rb < p.csr.num_rows)
-    scalar_load2(p.csr.ptr + lh * p.csr.ptr_sh + rb, p.csr.ptr + lh * p.csr.ptr_sh + rb + 1, e0, e1);
-  if (p.seg.entries && place < p.seg.n[1]) {
-    const int len = e1 - e0;
-    segments = planned_segments(p.seg, place, len);
-    if (seg >= segments) return;
-    e1 = e0 + __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
-    e0 += __builtin_amdgcn_readfirstlane(len * seg / segments);
+  auto table_row = [&]() __attribute__((always_inline)) {
+    if (rb < p.csr.num_rows)
+      scalar_load2(p.csr.ptr + lh * p.csr.ptr_sh + rb, p.csr.ptr + lh * p.csr.ptr_sh + rb + 1, e0, e1);
+  };
+  if constexpr (CUT) {
+    table_row();
+    if (place < p.seg.n[1]) {
+      const int len = e1 - e0;
+      segments = planned_segments(p.seg, place, len);
+      if (seg >= segments) return;
+      e1 = e0 + __builtin_amdgcn_readfirstlane(len * (seg + 1) / segments);
+      e0 += __builtin_amdgcn_readfirstlane(len * seg / segments);
+    }
   }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -458,6 +464,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
     __syncthreads();
   }
 
+  if constexpr (!CUT) table_row();
   const int32_t *cols = p.csr.idx + lh * p.csr.idx_sh;
   const float *kbase = (const float *)p.k.ptr + sq.b * p.k.sb + kvh * p.k.sh;
   const float *vbase = (const float *)p.v.ptr + sq.b * p.v.sb + kvh * p.v.sh;
@@ -518,9 +525,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(KD <= 64 ? 2
   give_half<S::DT>(acc, kh == 1, buf, lane);
   __syncthreads();
   float *row = (float *)p.dq.ptr + sq.b * p.dq.sb + h * p.dq.sh + (int64_t)qi * p.dq.st;
-  if (segments > 1)
+  if (CUT && segments > 1)
     row = p.seg.partial + ((((int64_t)sq.b * p.Hq + h) * p.seg.slots + seg * p.seg.n[1] + place) * 128 + rh * 32 + m) * p.D;
-  const float scale = segments > 1 ? 1.f : p.sm_scale;
+  const float scale = CUT && segments > 1 ? 1.f : p.sm_scale;
   take_half_and_store<S::DT>(acc, kh == 1, buf, lane, scale, scale, row, row_ok, p.D);
 }
 
@@ -691,8 +698,13 @@ static int launch_fwd(const FwdParams &p, int tiles, hipStream_t stream) {
 template <int KD, bool PAD>
 static int launch_dq(const BwdParams &p, int rows, hipStream_t stream) {
   constexpr int smem = Shape<KD, PAD>::kSmem;
-  DK_ALLOW_DYNAMIC_LDS((dq_kernel<KD, PAD>), smem);
-  hipLaunchKernelGGL((dq_kernel<KD, PAD>), dim3(p.Hq, rows, p.seqs.batch), dim3(NT), smem, stream, p, rows);
+  if (p.seg.entries) {
+    DK_ALLOW_DYNAMIC_LDS((dq_kernel<KD, PAD, true>), smem);
+    hipLaunchKernelGGL((dq_kernel<KD, PAD, true>), dim3(p.Hq, rows, p.seqs.batch), dim3(NT), smem, stream, p, rows);
+  } else {
+    DK_ALLOW_DYNAMIC_LDS((dq_kernel<KD, PAD, false>), smem);
+    hipLaunchKernelGGL((dq_kernel<KD, PAD, false>), dim3(p.Hq, rows, p.seqs.batch), dim3(NT), smem, stream, p, rows);
+  }
   DK_HIP_CHECK(hipGetLastError());
   return DK_OK;
 }

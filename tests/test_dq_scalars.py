@@ -45,3 +45,11 @@ def test_launches_that_cut_nothing_spill_few_scalars(tmp_path):
     uncut = {k: v for k, v in kernels.items() if re.search(r"Lb[01]ELb[01]ELb0ELi\d+EEEv", k)}
     assert len(kernels) == 40 and len(uncut) == 20, list(kernels)
     assert max(uncut.values()) <= 22, uncut
+
+
+@pytest.mark.skipif(shutil.which(READELF) is None, reason="llvm-readelf not installed")
+def test_fp32_launches_that_cut_nothing_spill_few_scalars(tmp_path):
+    kernels = {k: v for k, v in _kernels(str(tmp_path)).items() if "f329dq_kernel" in k}
+    uncut = {k: v for k, v in kernels.items() if re.search(r"Lb[01]ELb0EEEv", k)}  # <head dims, PAD, CUT>
+    assert len(kernels) == 10 and len(uncut) == 5, list(kernels)
+    assert max(uncut.values()) <= 8, uncut
