@@ -25,6 +25,14 @@ struct BwdScratch {
 // (110) 661 / 610, 3 x 3000 (138) 808 / 742, 8000 (171) 937 / 872, 10000 (236) 1261 / 1186, 10000, local 8, vertical 16 (128)
 // 773 / 684; blocks of 32, 3 x 3000 (110) 675 / 614; 24 / 8 heads of 64, 6 x 2000 (85) 444 / 416.
 constexpr double kWalkFrom = 105;
+
+// What cutting the columns of a 16-bit call with one head a workgroup must gain, in steps: the kernel that adds the sums takes 5 us and
+// more, and the longest column, once it is left alone on its compute unit, runs faster than the average one.  Fit over 70 training
+// calls of 64 - 256 dims (backward, us of 128 dims): 1.1 a step, - 0.022 a partial sum, - 2.  Below the line, not cut / cut: 16
+// heads, 2 x 1831 121 / 129, 8 heads of 256 dims, 2 x 1826 165 / 178, 32 heads, 1 x 1377 85 / 90, 8 heads, 2 x 1464 80 / 84; just above it 16
+// / 4 heads, 3 x 1358 106 / 93, 12 heads, 2 x 2057 127 / 136, 16 heads of 64, 3 x 2006 106 / 93.  Not for global columns, which stand
+// out of short ones (8 heads, 4 x 2553, longest column 1.04 times the average: 206 / 184), nor for masked tiles, whose average is overestimated.
+constexpr double kLeastGain = 3.5;
 inline bool walk_groups(const BwdParams &p, size_t group, int kv_slots, double from) {
   const int ratio = p.Hq / p.Hkv;
   const bool one_table = p.csc.num_heads != p.Hq || p.csc.group % ratio == 0;  // for all q heads of a kv head
@@ -34,8 +42,10 @@ inline bool walk_groups(const BwdParams &p, size_t group, int kv_slots, double f
 
 // group: bytes of the per-q-head partials if the pass uses them; dq_slots, kv_slots: workgroups of the two passes that the
 // chip holds at once (0: its rows are not cut); dq_pairs: the dQ pass takes pairs of rows; walk_from: steps per resident
-// workgroup from which on the dK/dV pass walks whole groups although it could use partials (< 0: it does not walk them).
-inline BwdScratch plan_bwd_scratch(const BwdParams &p, size_t group, int dq_slots, bool dq_pairs, int kv_slots, double walk_from) {
+// workgroup from which on the dK/dV pass walks whole groups although it could use partials (< 0: it does not walk them);
+// kv_gain: steps that cutting columns of one head must gain (plan_segments), where they fall off gradually.
+inline BwdScratch plan_bwd_scratch(const BwdParams &p, size_t group, int dq_slots, bool dq_pairs, int kv_slots, double walk_from,
+                                   double kv_gain) {
   constexpr size_t kMost = (size_t)4 << 30;
   const bool walk = walk_from >= 0 && walk_groups(p, group, kv_slots, walk_from);
   BwdScratch s;
@@ -58,12 +68,13 @@ inline BwdScratch plan_bwd_scratch(const BwdParams &p, size_t group, int dq_slot
   if (walk)
     kv = plan_segments(p.csc.row_lengths, p.csc.num_rows, 1, (int64_t)p.seqs.batch * p.Hkv, kv_slots, limit, 0.4, p.Hq / p.Hkv);
   else if (kv_slots && (p.Hq == p.Hkv || s.group))
-    kv = plan_segments(p.csc.row_lengths, p.csc.num_rows, 1, copies, kv_slots, kv_limit, share);
+    kv = plan_segments(p.csc.row_lengths, p.csc.num_rows, 1, copies, kv_slots, kv_limit, share, 1,
+                       p.csr.order || p.csr.sub_block ? -1 : kv_gain);
   const size_t at = (s.group + 255) / 256 * 256;
   const int64_t dq_slots_all = dq.slots * copies, kv_slots_all = kv.slots * (walk ? copies / (p.Hq / p.Hkv) : copies);
   const double partials = (double)std::max(dq_slots_all, kv_slots_all) * 128 * p.D * sizeof(float);  // (no number of slots overflows)
   const size_t need = partials > (double)kMost ? kMost + 1 : at + (size_t)partials;
-  if (walk && need > kMost && group) return plan_bwd_scratch(p, group, dq_slots, dq_pairs, kv_slots, -1);
+  if (walk && need > kMost && group) return plan_bwd_scratch(p, group, dq_slots, dq_pairs, kv_slots, -1, kv_gain);
   if (need > at && need <= kMost && p.D % 4 == 0) s.dq = dq, s.kv = kv, s.bytes = need;
   return s;
 }

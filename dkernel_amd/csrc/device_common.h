@@ -125,8 +125,9 @@ inline double average_steps(const int32_t *lengths, int rows, int per_step, int6
 // partial sums than they even out.  Below kWorth steps the kernel that adds the sums takes what the cut gains.
 // The lengths come from a caller and may be any numbers: a place of the order may have as many segments as the rows from it
 // on need at most (n[] never ascends), and the slots are counted for the place that has the most.
+// least_gain: steps that the longest row must come down by, a fiftieth of a step for each partial sum taken off, or nothing is cut.
 inline SegView plan_segments(const int32_t *lengths, int rows, int per_step, int64_t copies, int slots, double limit, double share,
-                             int heads = 1) {
+                             int heads = 1, double least_gain = -1) {
   constexpr int kLeast = 8;
   const int kWorth = heads > 1 ? 40 : 20;
   SegView s;
@@ -141,6 +142,12 @@ inline SegView plan_segments(const int32_t *lengths, int rows, int per_step, int
   if (entries < least) entries = least;
   const int most = row_segments(longest, entries);
   if (most < 2) return s;
+  if (least_gain > 0) {
+    int64_t partials = 0;
+    for (int i = 0; i < rows; ++i) partials += row_segments(steps(i), entries) > 1 ? row_segments(steps(i), entries) : 0;
+    const double left = 1.5 * entries + kStartSteps;  // (the longest segment)
+    if (longest + kStartSteps - (left > average ? left : average) - (double)partials * (double)copies / 50 < least_gain) return s;
+  }
   s.entries = entries;
   for (int i = 0; i < rows; ++i)
     for (int j = row_segments(steps(i), entries) - 1; j > 0; --j) s.n[j] = i + 1;

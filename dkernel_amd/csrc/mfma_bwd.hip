@@ -1391,7 +1391,7 @@ size_t bwd_group_bytes(const BwdParams &p) {
 
 static BwdScratch mfma_bwd_scratch(const BwdParams &p, bool walk) {
   const int width = mfma_tile_width(p.D), per_cu = width == 64 ? 3 : width == 128 ? 2 : 1;
-  return plan_bwd_scratch(p, bwd_group_bytes(p), width == 256 ? 0 : 256 * per_cu, true, 256 * per_cu, walk ? kWalkFrom : -1);
+  return plan_bwd_scratch(p, bwd_group_bytes(p), width == 256 ? 0 : 256 * per_cu, true, 256 * per_cu, walk ? kWalkFrom : -1, kLeastGain);
 }
 size_t mfma_bwd_workspace_bytes(const BwdParams &p) { return mfma_bwd_scratch(p, true).bytes; }
 

@@ -761,7 +761,7 @@ int launch_mfma_f32_fwd(const FwdParams &p, hipStream_t stream) {
 // 5684; 2 x 2000, 24 / 8 of 96, 1599 / 1662), unless the partials would not fit.
 static BwdScratch mfma_f32_bwd_scratch(const BwdParams &p, bool walk) {
   const int slots = 256 * (p.D <= 64 ? 2 : 1);
-  return plan_bwd_scratch(p, p.D > 64 && p.D % 8 == 0 ? bwd_group_bytes(p) : 0, slots, false, slots, walk ? INFINITY : -1);
+  return plan_bwd_scratch(p, p.D > 64 && p.D % 8 == 0 ? bwd_group_bytes(p) : 0, slots, false, slots, walk ? INFINITY : -1, -1);
 }
 size_t mfma_f32_bwd_workspace_bytes(const BwdParams &p) { return mfma_f32_bwd_scratch(p, true).bytes; }
 

@@ -40,7 +40,7 @@ extern "C" void scratch(int batch, int Hq, int Hkv, int D, int queries, int keys
   p.csc = LutView{nullptr, nullptr, 0, 0, 1, 1, cols, 64, 64, Hq, 0, 0};
   p.csr.pair_lengths = pair_lengths, p.csc.row_lengths = col_lengths;
   const size_t group = Hq == Hkv ? 0 : 2 * (size_t)batch * Hq * keys * D * 4;
-  const BwdScratch s = plan_bwd_scratch(p, group, 512, true, 512, kWalkFrom);
+  const BwdScratch s = plan_bwd_scratch(p, group, 512, true, 512, kWalkFrom, kLeastGain);
   out[0] = s.group > 0, out[1] = s.dq.entries, out[2] = s.kv.entries;
 }
 """
@@ -202,3 +202,13 @@ def test_modules_saved_with_other_lengths_get_the_present_ones(saved):
     else:
         old.kwargs["row_lengths"] = saved
     assert pickle.loads(pickle.dumps(old)).kwargs == mod.kwargs
+
+
+@pytest.mark.parametrize("batch,heads,L,local,vert,cut", [
+    (2, 16, 1831, 16, 8, False), (1, 32, 1377, 16, 8, False), (2, 16, 1333, 8, 4, False),   # the longest column hardly stands out
+    (2, 8, 1464, 16, 8, False),                                                              # or too much is cut with it
+    (1, 8, 3181, 4, 16, True), (2, 12, 2776, 4, 16, True), (1, 16, 8546, 16, 8, True), (1, 12, 4872, 8, 8, True)])
+def test_columns_are_cut_where_it_gains(plan, batch, heads, L, local, vert, cut):
+    mod = LocalStrideSparseAttention(heads, L, 64, local, vert)
+    how, _ = _plan_of(plan, mod, batch, heads, heads, 128, L)
+    assert (how[2] > 0) == cut, how
