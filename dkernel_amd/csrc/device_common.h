@@ -98,6 +98,20 @@ __device__ __forceinline__ int grid_head(const LutView &l) {
   return __builtin_amdgcn_readfirstlane((int)x);
 }
 
+// Grid of (heads, batch, items): sequence of the workgroups at (y, z).  With y = sequence the items of a sequence lie heads x
+// batch apart in the linear ids, which keeps it on a few of the 32 queues where that is a multiple of a power of two above the number of
+// heads (4 sequences and 8 heads: each on one shader engine of every die, the longest one on a quarter of the chip).  The
+// sequences then move on by one whenever the queues have come round, after 32 / gcd(32, heads x batch) items.  Elsewhere they
+// stay (31), which keeps a head of a sequence on its dies: 5 sequences, 12 heads 466 / 503 us.
+inline int padded_shift(int heads, int batch) {
+  int shift = 5;
+  for (int64_t step = (int64_t)heads * batch; shift > 0 && step % 2 == 0; step /= 2) --shift;
+  return 32 >> shift > heads ? shift : 31;
+}
+__host__ __device__ inline int padded_sequence(int y, int z, int batch, int shift) {
+  return (int)(((unsigned)y + ((unsigned)z >> shift)) % (unsigned)batch);
+}
+
 // Segments of a row of `len` entries: len / entries, rounded.
 __host__ __device__ inline int row_segments(int len, int entries) {
   const int n = (2 * len + entries) / (2 * entries);
@@ -188,7 +202,7 @@ struct SeqView {
   // no query of their sequence, so that the caller need not clear the outputs first; packed inputs:
   // the rows of lse before the first sequence and behind the last one (-inf)
   int32_t zero_outside = 0;
-  int32_t items_in_z = 0;  // set per launch: grid of (heads, batch, items) in place of (heads, items, batch)
+  int32_t items_in_z = 0;  // set per launch: grid of (heads, batch, items) in place of (heads, items, batch), 1 + shift of padded_sequence()
 };
 
 // Paged K/V (decode only): k / v point at page pools, token t of sequence b lives in page

@@ -57,7 +57,11 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   // SUB: table entries are (column, bit mask over the pattern blocks inside the 64 x 64 tile)
   constexpr int EW = SUB ? 2 : 1;  // ints per table entry
   // grid: (heads, items, batch), padded inputs (heads, batch, items)
-  const int item_y = p.seqs.items_in_z ? blockIdx.z : blockIdx.y, item_z = p.seqs.items_in_z ? blockIdx.y : blockIdx.z;
+  int item_y = blockIdx.y, item_z = blockIdx.z;
+  if (p.seqs.items_in_z) {
+    item_z = __builtin_amdgcn_readfirstlane(padded_sequence(blockIdx.y, blockIdx.z, gridDim.y, p.seqs.items_in_z - 1));
+    item_y = blockIdx.z;
+  }
   SeqInfo sq;
   int tile;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -572,13 +576,19 @@ static FwdParams for_grid(FwdParams p, int gx, int gy) {
 // 1400, 16 / 4 heads of 256 115.8 / 98.5; 3 x 1150, 32 / 8 of 96 22.0 / 20.1; 6 x 1850, 8 heads 20.2 / 19.0.  Long launches stay: there
 // the K/V tiles that neighbouring rows share no longer fit the L2s (14080 workgroups, 8 x 7000, 32 heads 1082 / 1203; 3936
 // workgroups 218.1 / 217.7), as do sequences of few rows, which are all alike (4 row pairs 21.0 / 21.2, 7 of them 19.1 /
-// 18.3).  Tables with uneven heads keep their rotation over neighbouring rows.
+// 18.3), and two sequences (46 launches 0.91 - 1.22, 1.00 on average; 3 - 16 sequences, 194 launches 0.92 - 1.32, 1.05).
+// Tables with uneven heads keep their rotation over neighbouring rows.
 static FwdParams for_rows(FwdParams p, int gx, int gy, dim3 &grid) {
   p = for_grid(p, gx, gy);
   const int batch = p.seqs.packed ? 1 : p.seqs.batch;
-  p.seqs.items_in_z = p.seqs.given && batch > 1 && !p.csr.rot && gy >= 6 && (int64_t)gx * gy * batch <= 4096;
+  const bool side_by_side = p.seqs.given && batch > 2 && !p.csr.rot && gy >= 6 && (int64_t)gx * gy * batch <= 4096;
+  p.seqs.items_in_z = side_by_side ? 1 + padded_shift(gx, batch) : 0;
   grid = p.seqs.items_in_z ? dim3(gx, batch, gy) : dim3(gx, gy, batch);
   return p;
+}
+
+static const char *fwd_kernel_name(const FwdParams &p) {
+  return p.csr.rot ? "mfma_fwd_kernel, heads in rotation" : p.seqs.items_in_z ? "mfma_fwd_kernel, sequences side by side" : "mfma_fwd_kernel";
 }
 
 // q tiles of `rows` tokens along grid.y (packed inputs: through all sequences), an upper bound
@@ -629,7 +639,7 @@ static int launch_tdg(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t st
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, G, PAD, false, false, KD>), smem);
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
   const FwdParams pr = for_rows(p, p.Hq / G, tiles_y, grid);
-  DK_NOTE_KERNEL(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+  DK_NOTE_KERNEL(fwd_kernel_name(pr));
   hipLaunchKernelGGL((mfma_fwd_kernel<T, D, G, PAD, false, false, KD>), grid, dim3(128 * G), smem, stream,
                      pr, tiles_y);
   DK_HIP_CHECK(hipGetLastError());
@@ -661,7 +671,7 @@ static int launch_row_pairs_as(const FwdParams &p, hipStream_t stream, const cha
   if (int rc = launch_item_offsets(p, true, stream)) return rc;
   dim3 grid;
   const FwdParams pr = for_rows(p, p.Hq, pairs, grid);
-  note_kernel(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel", signature);
+  note_kernel(fwd_kernel_name(pr), signature);
   hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 2, PAD, true, SUB, KD>), grid, dim3(256), smem, stream, pr, pairs);
   DK_HIP_CHECK(hipGetLastError());
   return DK_OK;
@@ -696,7 +706,7 @@ static int launch_sub_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t 
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, D, G, PAD, false, true, KD>), smem);
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
   const FwdParams pr = for_rows(p, p.Hq / G, tiles_y, grid);
-  DK_NOTE_KERNEL(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+  DK_NOTE_KERNEL(fwd_kernel_name(pr));
   hipLaunchKernelGGL((mfma_fwd_kernel<T, D, G, PAD, false, true, KD>), grid, dim3(128 * G), smem, stream,
                      pr, tiles_y);
   DK_HIP_CHECK(hipGetLastError());
@@ -735,7 +745,7 @@ static int launch_256_g(const FwdParams &p, dim3 grid, int tiles_y, hipStream_t 
   DK_ALLOW_DYNAMIC_LDS((mfma_fwd_kernel<T, 256, G, true, false, SUB>), smem);
   if (int rc = launch_item_offsets(p, false, stream)) return rc;
   const FwdParams pr = for_rows(p, p.Hq / G, tiles_y, grid);
-  DK_NOTE_KERNEL(pr.csr.rot ? "mfma_fwd_kernel, heads in rotation" : "mfma_fwd_kernel");
+  DK_NOTE_KERNEL(fwd_kernel_name(pr));
   hipLaunchKernelGGL((mfma_fwd_kernel<T, 256, G, true, false, SUB>), grid, dim3(128 * G), smem, stream,
                      pr, tiles_y);
   DK_HIP_CHECK(hipGetLastError());
