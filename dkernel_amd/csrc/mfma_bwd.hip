@@ -12,7 +12,7 @@
 //              memory for the dK/dV pass, which therefore runs second.
 //   dK/dV pass (CSC columns) workgroup = 64 keys x one kv head (the q heads of
 //              a GQA group are looped inside), 4 waves, two workgroups per
-//              CU.  A listed q block is worked on in two steps of 32 q rows;
+//              CU (three at 64 head dims).  A listed q block is worked on in two steps of 32 q rows;
 //              each 32 x 32 quadrant (q rows of the step x key half) has an S
 //              wave (S = Q K^T, P, dV^T += dO^T P; K fragments in registers)
 //              and a dP wave (dP = dO V^T, dS = P (dP - delta), dK^T += Q^T dS;
@@ -715,7 +715,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
 // ---------------------------------------------------------------------------
 // dK / dV pass
 // ---------------------------------------------------------------------------
-// One workgroup = one 64-key column block of one kv head, 4 waves, two workgroups per CU (the
+// One workgroup = one 64-key column block of one kv head, 4 waves, two workgroups per CU (three at 64 head dims; the
 // start-up and close-down of one column then overlap with the other workgroup's loop, and the
 // two workgroups' barriers are independent).  A listed q block is worked on in two steps of 32
 // q rows; in each step the two 32 x 32 (q rows x keys) quadrants are each shared by a pair of
@@ -742,7 +742,7 @@ struct DkdvSmem {
 };
 
 // At the 64-wide tile a step is eight multiplies per wave against the same barrier, waits and scalar work as at the
-// 128-wide one, so a third workgroup per CU (45 KB of LDS and 142 registers each) fills what two leave idle: training,
+// 128-wide one, so a third workgroup per CU (45 KB of LDS and 136 - 141 registers each) fills what two leave idle: training,
 // 64 dims, two / three workgroups, us: 32 heads x 8192 tokens 558 / 523, 4 x 3000 tokens of 12 heads with global blocks of
 // 32 334 / 310.
 template <typename T, int D, bool PAD, bool SUB, int KD = D>
