@@ -615,11 +615,11 @@ size_t decode_workspace_bytes(const FwdParams &p) {
 // conversions of a wave rather than by the memory, and few second workgroups gain nothing: 288 workgroups 26.3 / 27.0 and 22.5 / 22.6,
 // 328 19.0 / 19.4, 352 32.4 / 29.2, 408 25.3 / 24.3, 480 44.5 / 41.8.
 // The votes and a longest sequence that starts later than in the batch's order cost half a microsecond to two, which steps of
-// little work get back only if the work of their sequences differs: rows that grow with the sequence (at least three quarters
+// little work get back only if the work of their sequences differs: rows that grow with the sequence (at least half
 // as many blocks as the longest one has) do, rows that end in a window and few columns are all alike.  Sweep of 337
 // steps of 10 - 180 us, order of the batch / by length, on average: 256 dims (one workgroup per compute unit) 1.09; from 320 KB of K/V
-// for a workgroup of the longest row (blocks x dims >= 1280) 1.08; growing rows from 96 KB, up to three workgroups a row, 1.05 (four, 10
-// sequences of 1286, 96 dims: 20.8 / 23.2 us); the others 0.996, between 0.86 (22 sequences of 4495, 96 dims, 16.1 / 18.6) and 1.2.
+// for a workgroup of the longest row (blocks x dims >= 1280) 1.08; growing rows from 96 KB, up to three workgroups a row, 1.04 (four, 10
+// sequences of 1286, 96 dims: 20.8 / 23.2 us); the others 0.99, between 0.86 (22 sequences of 4495, 96 dims, 16.1 / 18.6) and 1.11.
 static int decode_first_by_length(const FwdParams &p, int groups) {
   constexpr int kUnits = 256;
   const int per_sequence = p.Hkv * groups;
@@ -629,7 +629,7 @@ static int decode_first_by_length(const FwdParams &p, int groups) {
   if (!ranked || workgroups <= from || workgroups > 4 * kUnits) return 0;
   const int entries = decode_max_row_entries(p);
   const int64_t work = (int64_t)entries * p.D / groups;
-  const bool growing = (int64_t)4 * entries >= (int64_t)3 * std::min(cdiv(p.seqs.max_k_len, 64), p.csr.num_rows);
+  const bool growing = (int64_t)2 * entries >= std::min(cdiv(p.seqs.max_k_len, 64), p.csr.num_rows);
   if (mfma_tile_width(p.D) < 256 && work < (growing && groups <= 3 ? 384 : 1280)) return 0;
   return std::min(p.seqs.batch, std::max(1, kUnits / per_sequence));
 }

@@ -58,6 +58,7 @@ def test_capacity_beyond_the_sequences(form, batch, longest):
 @pytest.mark.parametrize("batch,length,local,vert,D,ranked", [
     (48, 1216, 16, 64, 64, True),    # 19 blocks, rows of 17: they grow with their sequences, 17 x 64 = 1088
     (48, 1216, 8, 64, 64, False),    # rows of 9: a window and a column
+    (48, 1152, 8, 64, 64, True),     # of 18 blocks
     (40, 200, 2, 8, 256, True),      # 256 dims: always
     (48, 384, 16, 8, 64, True),      # 6 blocks of 64 dims: 384
     (48, 320, 16, 8, 64, False),     # 5: 320
