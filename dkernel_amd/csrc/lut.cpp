@@ -279,6 +279,8 @@ int dk_call_row_lengths(const int32_t *ptr, const int32_t *idx, const int32_t *o
     lens[rows] = -1;  // (an odd table's last pair has one row)
     for (int r = 0; r < rows; ++r)
       lens[r] = r < first || r > last ? -1 : (int32_t)(std::lower_bound(e + p[r], e + p[r + 1], limit) - (e + p[r]));
+    for (int i = 0; i < rows + pairs; ++i)
+      DK_REQUIRE(o[i] >= 0 && o[i] < (i < rows ? rows : pairs), "order of head %d is no permutation", h);
     for (int i = 0; i < rows; ++i) out[i] = std::max(out[i], lens[o[i]]);
     for (int i = 0; i < pairs; ++i) {
       const int32_t a = lens[2 * o[rows + i]], b = lens[2 * o[rows + i] + 1];

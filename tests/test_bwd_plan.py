@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 import torch
 
-from dkernel_amd import LocalStrideSparseAttention, SparseAttention
+from dkernel_amd import LocalStrideSparseAttention, SparseAttention, _lib
 from test_kernel_resources import CSRC, HIPCC
 
 pytestmark = pytest.mark.skipif(shutil.which(HIPCC) is None, reason="hipcc not installed")
@@ -161,6 +161,18 @@ def test_lengths_of_a_call(heads, n, causal, block):
             limit = min(call[2], rows)
             assert got[:rows] == _lengths(mask_t[::step], call[0], call[1], limit, order[:, :rows], False)
             assert got[rows:] == _lengths(mask_t[::step], call[0], call[1], limit, order[:, rows:], True)
+
+
+def test_lengths_refuse_what_they_cannot_read():
+    ptr, idx, out = (C.c_int32 * 4)(0, 1, 2, 3), (C.c_int32 * 3)(0, 1, 2), (C.c_int32 * 5)()
+
+    def call(order, at=ptr, heads=1):
+        return _lib.lib().dk_call_row_lengths(at, idx, (C.c_int32 * 5)(*order), heads, 3, 3, 0, 2, 2, out)
+
+    assert call((2, 1, 0, 1, 0)) == 0 and list(out) == [0, 1, 1, 0, 2]
+    for bad in ((3, 1, 0, 1, 0), (-1, 1, 0, 1, 0), (2, 1, 0, 2, 0)):
+        assert call(bad) != 0
+    assert call((2, 1, 0, 1, 0), at=None) != 0 and call((2, 1, 0, 1, 0), heads=0) != 0
 
 
 def _plan_of(plan, mod, batch, Hq, Hkv, D, L):
