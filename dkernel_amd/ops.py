@@ -15,6 +15,7 @@ import array
 import ctypes as C
 import os
 import math
+from functools import cached_property
 from typing import Dict, Optional, Tuple, Union
 
 import torch
@@ -123,18 +124,31 @@ class TableLengths:
         if ptr.dim() == 1:
             ptr, idx = ptr[None], idx[None]
         every = ptr.size(0) if ptr.stride(0) == 0 else every if ptr.size(0) % every == 0 else 1
-        self.ptr = ptr[::every].to("cpu", torch.int32).contiguous()
         idx = idx if idx.dim() == 2 else idx[:, :, 0]  # (column, mask) entries
-        self.idx = idx[::every].to("cpu", torch.int32).contiguous()
-        self.order = _longest_first(self.ptr)
-        self.rows = self.ptr.size(1) - 1
+        # (a module is built on the host as a rule: views of its tables, copied and sorted at the first backward)
+        self._tables = ptr[::every].to("cpu", torch.int32), idx[::every].to("cpu", torch.int32)
+        self.rows = ptr.size(1) - 1
+
+    @property
+    def ptr(self) -> Tensor:
+        return self._tables[0]
+
+    @property
+    def idx(self) -> Tensor:
+        return self._tables[1]
+
+    @cached_property
+    def order(self) -> Tensor:
+        self._tables = tuple(x.contiguous() for x in self._tables)
+        return _longest_first(self.ptr)
 
     def of_call(self, first: int, last: int, limit: int) -> array.array:
         """Lengths of the rows first .. last, counting entries below `limit` (-1 at places of other rows), followed by those of
         their pairs."""
-        out = array.array("i", bytes(4 * (self.rows + (self.rows + 1) // 2)))
-        _lib.check(_lib.lib().dk_call_row_lengths(self.ptr.data_ptr(), self.idx.data_ptr(), self.order.data_ptr(), self.ptr.size(0),
-                                                  self.rows, self.idx.stride(0), first, last, limit, out.buffer_info()[0]))
+        out, order = array.array("i", bytes(4 * (self.rows + (self.rows + 1) // 2))), self.order
+        ptr, idx = self._tables
+        _lib.check(_lib.lib().dk_call_row_lengths(ptr.data_ptr(), idx.data_ptr(), order.data_ptr(), ptr.size(0), self.rows,
+                                                  idx.stride(0), first, last, limit, out.buffer_info()[0]))
         return out
 
     def __eq__(self, other):
