@@ -728,6 +728,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
 // barrier has published P), so one barrier per step is enough: Q tiles and the lse / delta
 // vectors live one iteration longer than dO tiles (rings of 4 and 3 stages of 32-row tiles), and
 // tile loads run two steps ahead.
+//
+// Two in-order waves per SIMD: what a wave issues between its multiplies is what the pass waits for, more than LDS or HBM.
+// Hence the loop takes a block's two steps in one iteration (P buffers and the second half's Q places are immediates),
+// operand addresses are moved on in place, everything that only the change of heads or a partial tile needs is computed
+// there from opaque copies, and the multiplies of one step stand next to the exponentials of the next: the S wave leaves
+// the second half of dV to the following step, the dP wave forms dP of its step before dS of the one before.  Scalar
+// instructions per step and wave 113 -> 60, vector 85 -> 70.  Training, us: 32 heads of 128 x 8192 tokens 927 -> 892
+// (this pass 473 -> 421), 4 x 2048, 32 / 8 heads 597 -> 572, 4 x 3000 tokens of 12 heads of 64 with global blocks of 32
+// 249 -> 241, 3000 tokens of 256 dims 287 -> 276.
 template <int D>
 struct DkdvSmem {
   using TL = Tile<D>;
@@ -847,11 +856,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
 
-  int rd[KS], tr[DT][2];
+  // operand read addresses inside a 32-row tile at offset 0; the Q stage is a compile-time constant of the loop body, so
+  // that stage and row offsets are instruction immediates
+  using OA = OperandAddress<D>;
+  typename OA::type rd[KS], tr[DT][2];
+  {
+    int tro[DT][2];
+    transposed_offsets<D>(lane, tro);
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) rd[ks] = TL::off(n, 2 * ks + g);
-  transposed_offsets<D>(lane, tr);
-  float *xbuf = reinterpret_cast<float *>(smem + S::kX) + nh * 2 * 1024;  // this pair's two P buffers
+    for (int ks = 0; ks < KS; ++ks) rd[ks] = OA::make(smem, TL::off(n, 2 * ks + g));
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) tr[dt][0] = OA::make(smem, tro[dt][0]), tr[dt][1] = OA::make(smem, tro[dt][1]);
+  }
+  const uint32_t xbuf = opaque_lds_address(lds_address(smem) + S::kX + nh * 8192 + lane * 16);  // this pair's two P buffers
+  const uint32_t vecs = opaque_lds_address(lds_address(smem) + S::kVec + g * 16);               // lse and delta of a Q stage
 
   // tiles whose first query index lies in [0, full_span) hold 32 queries
   const uint32_t full_span = sq.q_len >= S::kRows ? (uint32_t)(sq.q_len - S::kRows) + 1u : 0u;
@@ -862,10 +880,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   int gq = gq_first - 1, ent = 0, ent_end = 0;
   const int32_t *rows = nullptr;
   const char *qbase = nullptr, *dobase = nullptr;
-  const float *lsebase = nullptr, *deltabase = nullptr;
-  auto have_entry = [&]() __attribute__((always_inline)) -> bool {
-    while (ent >= ent_end) {
-      if (++gq >= gq_end) return false;
+  // lanes 0 .. 31: lse of the first 32 queries, lanes 32 .. 63: their delta; bytes from one query to the next
+  const char *vec = nullptr;
+  const int64_t vec_step = lane >= 32 ? (int64_t)sizeof(float) : p.lse.st * (int64_t)sizeof(float);
+  auto next_head = [&]() __attribute__((always_inline)) {  // on to the next head that has entries, if there is one
+    while (ent >= ent_end && gq + 1 < gq_end) {
+      ++gq;
       const auto *a = late_arguments<BwdParams>();
       const int h = kvh * ratio + gq;
       const int tables = a->csc.num_heads, lh = tables == 1 ? 0 : tables == a->Hq ? h : kvh;
@@ -882,62 +902,62 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       }
       qbase = reinterpret_cast<const char *>((const T *)a->q.ptr + sq.b * a->q.sb + h * a->q.sh);
       dobase = reinterpret_cast<const char *>((const T *)a->dout.ptr + sq.b * a->dout.sb + h * a->dout.sh);
-      lsebase = a->lse.ptr + sq.b * a->lse.sb + h * a->lse.sh;
-      deltabase = a->delta + ((int64_t)sq.b * a->Hq + h) * a->seqs.max_q_len;
+      const float *lsebase = a->lse.ptr + sq.b * a->lse.sb + h * a->lse.sh;
+      const float *deltabase = a->delta + ((int64_t)sq.b * a->Hq + h) * a->seqs.max_q_len;
+      vec = reinterpret_cast<const char *>(lane >= 32 ? deltabase : lsebase) + (lane & 31) * vec_step;
     }
-    return true;
   };
 
-  // asynchronous copy of half `half` of q block rbq: Q and dO tiles and the 32 lse / 32 delta
-  // values of its rows (lanes 0..31 copy lse, lanes 32..63 delta; every wave copies the same
+  // asynchronous copy of 32-row q tile `tile`: Q and dO rows and the 32 lse / 32 delta
+  // values (lanes 0..31 copy lse, lanes 32..63 delta; every wave copies the same
   // values, so that every wave issues the same number of load instructions).  Returns false
   // when rows had to be zero-filled, i.e. when the per-wave load count is not LPT.
-  auto issue = [&](int rbq, int half, int qstage, int dostage) __attribute__((always_inline)) -> bool {
-    const int qi0 = rbq * 64 + half * 32 - sq.past;  // query index of the tile's first row
-    const int row = lane & 31;
-    const bool is_delta = lane >= 32;
-    char *dst = smem + S::kVec + qstage * 256;
+  const uint32_t lds0 = lds_address(smem);
+  auto issue = [&](int tile, int q_at, int do_at) __attribute__((always_inline)) -> bool {
+    const int qi0 = tile * 32 - sq.past;  // query index of the tile's first row
     // main path: a listed block whose 32 rows all are queries (one scalar compare: a padding
-    // entry, rbq < 0, gives a negative qi0)
-    if (D <= 128 && (uint32_t)qi0 < full_span) {
-      qload.issue_full(row_address(qbase, qi0, q_row_bytes),
-                       smem + S::kQ + qstage * S::kTile);
-      doload.issue_full(row_address(dobase, qi0, do_row_bytes),
-                        smem + S::kDo + dostage * S::kTile);
-      const float *src = is_delta ? deltabase + qi0 + row : lsebase + (int64_t)(qi0 + row) * p.lse.st;
-      lds_dma4_lane(src, lds_address(dst));
+    // entry, tile < 0, gives a negative qi0)
+    if ((uint32_t)qi0 < full_span) {
+      qload.issue_full_at(row_address(qbase, qi0, q_row_bytes), lds0 + q_at);
+      doload.issue_full_at(row_address(dobase, qi0, do_row_bytes), lds0 + do_at);
+      lds_dma4_lane(vec + (uint64_t)(uint32_t)qi0 * (uint64_t)vec_step, lds0 + S::kVec + q_at / (S::kTile / 256));
       return true;
     }
-    // rows before the first query (qi < 0, when k is longer than q) and beyond the last are zero-filled
-    const int lo = rbq < 0 ? S::kRows : -qi0, hi = sq.q_len - qi0;
-    const bool full = qload.issue(qbase + (int64_t)qi0 * q_row_bytes, lo, hi,
-                                  smem + S::kQ + qstage * S::kTile);
-    doload.issue(dobase + (int64_t)qi0 * do_row_bytes, lo, hi,
-                 smem + S::kDo + dostage * S::kTile);
+    char *const q_dst = smem + q_at, *const do_dst = smem + do_at, *const dst = smem + S::kVec + q_at / (S::kTile / 256);
+    // Rows before the first query (qi < 0, when k is longer than q) and beyond the last are zero-filled.  Rare: everything
+    // is computed here from opaque copies, or it would be held in registers through the loop, for each of its steps.
+    int late = tid;
+    asm volatile("" : "+v"(late));
+    const auto *a = late_arguments<BwdParams>();
+    Loader ql, dol;
+    ql.init(late, a->q.st, a->D);
+    dol.init(late, a->dout.st, a->D);
+    const int lo = tile < 0 ? S::kRows : -qi0, hi = sq.q_len - qi0;
+    const bool full = ql.issue(qbase + (int64_t)qi0 * q_row_bytes, lo, hi, q_dst);
+    dol.issue(dobase + (int64_t)qi0 * do_row_bytes, lo, hi, do_dst);
+    const char *src = vec + (int64_t)qi0 * vec_step;
     if (full) {
-      const float *src = is_delta ? deltabase + qi0 + row : lsebase + (int64_t)(qi0 + row) * p.lse.st;
       lds_dma4_lane(src, lds_address(dst));
     } else if (wave == 0) {
       // rows outside the sequence: lse = +inf makes their probabilities 0
-      const int qi = qi0 + row;
-      float x = is_delta ? 0.f : INFINITY;
-      if (row >= lo && row < hi) x = is_delta ? deltabase[qi] : lsebase[(int64_t)qi * p.lse.st];
-      reinterpret_cast<float *>(dst)[lane] = x;
+      const int row = late & 31;
+      float x = late & 32 ? 0.f : INFINITY;
+      if (row >= lo && row < hi) x = *reinterpret_cast<const float *>(src);
+      reinterpret_cast<float *>(dst)[late & 63] = x;
     }
     return full;
   };
 
-  // second half of the dP wave's work on step u (whose P the S wave published before the
+  // second half of the dP wave's work on a step (whose P the S wave published before the
   // last barrier): dS = P (dP - delta), dK^T += Q^T dS
-  auto finish_dk = [&](int u, int qstage, const floatx16 &dp) {
-    const char *qs_ = smem + S::kQ + qstage * S::kTile;
-    const float *delta_s = reinterpret_cast<const float *>(smem + S::kVec + qstage * 256) + 32;
-    const float *x = xbuf + (u & 1) * 1024;
+  // (ta: operand addresses of its Q tile)
+  auto finish_dk = [&](const auto &ta, int row_off, int qs_, int x_, const floatx16 &dp) __attribute__((always_inline)) {
+    const uint32_t x = xbuf + x_, delta_s = vecs + qs_ / (S::kTile / 256) + 128;
     float ds[16];
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4) {
-      const float4 p4 = *reinterpret_cast<const float4 *>(x + (r4 * 64 + lane) * 4);
-      const float4 d4 = *reinterpret_cast<const float4 *>(delta_s + r4 * 8 + g * 4);
+      const floatx4 p4 = lds_read8_at<floatx4>(x + r4 * 1024);
+      const floatx4 d4 = lds_read8_at<floatx4>(delta_s + r4 * 32);
       ds[r4 * 4 + 0] = p4.x * (dp[r4 * 4 + 0] - d4.x);  // without sm_scale
       ds[r4 * 4 + 1] = p4.y * (dp[r4 * 4 + 1] - d4.y);
       ds[r4 * 4 + 2] = p4.z * (dp[r4 * 4 + 2] - d4.z);
@@ -949,7 +969,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
       const int rowoff = t2 * 16 * TL::kRowBytes;
       vec8 qt[DT];
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) qt[dt] = lds_read_tr8<vec8>(qs_ + rowoff + tr[dt][0], qs_ + rowoff + tr[dt][1]);
+      for (int dt = 0; dt < DT; ++dt) qt[dt] = lds_operand_tr<vec8>(ta[dt][0] + (row_off + rowoff), ta[dt][1] + (row_off + rowoff));
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) acc[dt] = M::mma(qt[dt], dsb, acc[dt]);
     }
@@ -959,41 +979,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // are not merged through a join every iteration.
   auto run_column = [&](auto role_tag) __attribute__((always_inline)) {
   constexpr bool kDp = decltype(role_tag)::value;
-  int issued = 0, iq = 0, ido = 0;  // next step to request and its ring positions
-  bool exact = true;                // every wave has issued exactly LPT load instructions per outstanding step
-  static_assert(S::kAhead == 2, "two steps in flight ahead of the one that is worked on");
-  int rb_next = 0;                  // q block of the step that was requested last (steps 2k and 2k + 1 share a block)
-  // SUB: the steps are the 32-row halves of the listed tiles that attend anything.  left: halves of block
-  // rb_next still to come; s0, s1: the steps that the loop works on next, each as 32-row tile << 8 | the masks
-  // of its two quadrants, 4 bits each.
-  int left = 0, bits_next = 0, s0 = 0, s1 = 0;
-  auto request_next = [&](int &s) __attribute__((always_inline)) {  // requests the next step, if there is one
-    int half = issued & 1;
+  // A step is the number of its 32-row q tile; SUB: << 8 | the masks of its two quadrants, 4 bits each (steps
+  // without an attended block are left out).  Without SUB steps come in pairs, the halves of a listed block.
+  constexpr int kNone = INT_MAX;
+  bool exact = true;  // every wave has issued exactly LPT load instructions per outstanding step
+  static_assert(S::kAhead == 2 && S::kQStages == 4 && S::kDoStages == 3, "two steps in flight ahead of the one that is worked on");
+  int left = 0, bits_next = 0, rb_next = 0;  // SUB: halves of block rb_next still to come
+  // Requests the next step into place q_dst of the Q ring and do_dst of the dO ring (HALF 1: the second half of the block
+  // whose first half, `before`, was requested last).
+  auto request = [&](auto half_tag, int before, int q_dst, int do_dst) __attribute__((always_inline)) -> int {
+    constexpr int kHalf = decltype(half_tag)::value;
+    int step = kNone;
     if constexpr (SUB) {
-      while (left == 0 && have_entry()) {
-        scalar_load2(rows + ent * EW, rows + ent * EW + 1, rb_next, bits_next);
-        ++ent;
-        bits_next = tile_quadrants(bits_next, p.csc.sub_block);
-        left = ((bits_next & 255) != 0 ? 1 : 0) | ((bits_next >> 8) != 0 ? 2 : 0);
+      if (left == 0) {
+        if (__builtin_expect(ent >= ent_end, 0)) next_head();
+        if (ent < ent_end) {
+          scalar_load2(rows + ent * EW, rows + ent * EW + 1, rb_next, bits_next);
+          ++ent;
+          bits_next = tile_quadrants(bits_next, p.csc.sub_block);
+          left = ((bits_next & 255) != 0 ? 1 : 0) | ((bits_next >> 8) != 0 ? 2 : 0);
+          if (left == 0) left = 1;  // (a listed tile without an attended block: one step that adds nothing)
+        }
       }
-      if (left == 0) return;
-      half = left & 1 ? 0 : 1;
-      left &= left - 1;
-      s = (rb_next * 2 + half) << 8 | (bits_next >> (8 * half) & 255);
-    } else if (half == 0) {
-      if (!have_entry()) return;
-      rb_next = scalar_load(rows + ent);
-      ++ent;
+      if (left != 0) {
+        const int half = left & 1 ? 0 : 1;
+        left &= left - 1;
+        step = (rb_next * 2 + half) << 8 | (bits_next >> (8 * half) & 255);
+      }
+    } else if constexpr (kHalf == 0) {
+      if (__builtin_expect(ent >= ent_end, 0)) next_head();
+      if (ent < ent_end) {
+        step = scalar_load(rows + ent) * 2;
+        ++ent;
+      }
+    } else {
+      if (before != kNone) step = before + 1;
     }
-    exact = issue(rb_next, half, iq, ido) && exact;
-    iq = iq + 1 == S::kQStages ? 0 : iq + 1;
-    ido = ido + 1 == S::kDoStages ? 0 : ido + 1;
-    ++issued;
+    if (step != kNone)
+      exact = issue(SUB ? step >> 8 : step, q_dst, do_dst) && exact;
+    return step;
   };
-  for (int i = 0; i < S::kAhead; ++i) {
-    s0 = s1;
-    request_next(s1);
-  }
+  static_assert(S::kQ == 0, "Q ring places are offsets");
+  int do_0 = S::kDo, do_1 = S::kDo + S::kTile, do_2 = S::kDo + 2 * S::kTile;  // dO ring places of this step and the next two
+  next_head();
+  int cur = request(IntConst<0>{}, kNone, 0, do_0);
+  int nxt = request(IntConst<1>{}, cur, S::kTile, do_1);
   if constexpr (kKvTiles) {
     // the K / V tiles are older than the requests above: everything has landed behind this wait
     wait_tile_loads();
@@ -1005,26 +1035,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     // tile is requested behind it, and the S waves write P behind it)
   }
   floatx16 dp_prev;
-  int cq = 0, cdo = 0, pq = 0;  // ring positions of step t (Q, dO) and of step t - 1 (Q)
-  int rbq = 0;                  // S wave: q block (SUB: 32-row tile) of the current step
   int quad = 15, quad_prev = 15;  // SUB: masks of this wave's quadrant of steps t and t - 1 (0: both waves of the pair idle)
-  for (int t = 0; t < issued; ++t) {
-    const int half = t & 1;
-    wait_tiles_ahead<LPT>(exact ? issued - t - 1 : 0);
-    __syncthreads();  // step t is visible, so is P of step t - 1; the stages of step t - 2 are free
-    if constexpr (SUB) {
-      rbq = s0 >> 8;
-      quad = (s0 >> (4 * nh)) & 15;
-      s0 = s1;
-    } else {
-      if (half == 0) rbq = rb_next;  // (both steps of the block have been requested, nothing behind it)
-    }
-    request_next(s1);
-    const char *qs_ = smem + S::kQ + cq * S::kTile, *dos_ = smem + S::kDo + cdo * S::kTile;
+  int q_ring = 0;                 // Q ring place of this step (without SUB: of the block's first one)
+  int x_ring = 0;                 // SUB: the P buffer of this step
+  bool first = true;              // no step before this one
+  // Operand addresses of the tiles that are read now, moved on with the rings.  S wave: rows of Q, columns of dO; dP wave:
+  // rows of dO, columns of Q of the step before.  (Without SUB those of Q move once a block, its halves are immediates.)
+  typename OA::type ra[KS], ta[DT][2];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) ra[ks] = rd[ks] + (kDp ? (int)S::kDo : 0);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) ta[dt][j] = tr[dt][j] + (kDp ? SUB ? 3 * S::kTile : 2 * S::kTile : (int)S::kDo);
+  auto move_rows = [&](int by) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) ra[ks] += by;
+  };
+  auto move_cols = [&](int by) __attribute__((always_inline)) {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) ta[dt][0] += by, ta[dt][1] += by;
+  };
+  // (not where steps are left out: the guards cost registers, 64 dims then lose their third workgroup, 241 -> 265 us)
+  constexpr bool kLag = !kDp && !kIdle;
+  constexpr bool kAhead = !kIdle;
+  vec8 lag_dot[DT], lag_pb;  // dO^T and P of the second half of the step before
+  if constexpr (kLag) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) lag_pb[i] = 0;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) lag_dot[dt] = lag_pb;
+  }
+  auto finish_dv = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) acc[dt] = M::mma(lag_dot[dt], lag_pb, acc[dt]);
+  };
+  auto work = [&](auto half_tag) __attribute__((always_inline)) {
+    constexpr int kHalf = decltype(half_tag)::value;  // (SUB: 0)
+    if (nxt != kNone && exact)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPT) : "memory");
+    else
+      wait_tile_loads();
+    __syncthreads();  // this step is visible, so is P of the step before; the stages of the step before that are free
+    const int step = cur, cdo = do_0;
+    const int qs_ = q_ring + kHalf * S::kTile, x_ = SUB ? x_ring : kHalf * 4096;
+    // the Q place of the step before, and its P buffer
+    const int pq = SUB ? (q_ring - S::kTile) & (3 * S::kTile) : kHalf ? q_ring : (q_ring ^ 2 * S::kTile) + S::kTile;
+    cur = nxt;
+    nxt = request(half_tag, cur, SUB || kHalf == 0 ? qs_ ^ 2 * S::kTile : (q_ring ^ 2 * S::kTile) + S::kTile, do_2);
+    do_0 = do_1, do_1 = do_2, do_2 = cdo;
+    if constexpr (SUB) quad = (step >> (4 * nh)) & 15;
     if constexpr (!kDp) {
       if (!kIdle || quad != 0) {
-        const int pos0 = SUB ? rbq * 32 : rbq * 64 + half * 32;  // first q position of this step
-        const float *lse_s = reinterpret_cast<const float *>(smem + S::kVec + cq * 256);
+        const int pos0 = (SUB ? step >> 8 : step) * 32;  // first q position of this step
         // S = Q K^T : rows = 32 q positions, cols = 32 keys
         floatx16 sc;
 #pragma unroll
@@ -1032,14 +1095,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         {
           vec8 qa[KS];
 #pragma unroll
-          for (int ks = 0; ks < KS; ++ks) qa[ks] = lds_read8<vec8>(qs_ + rd[ks]);
+          for (int ks = 0; ks < KS; ++ks) qa[ks] = lds_operand<vec8>(ra[ks] + kHalf * S::kTile);
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) sc = M::mma(qa[ks], kvf[ks], sc);
         }
+        if constexpr (kLag) finish_dv();
         // first dO^T operands do not depend on P
         vec8 dot[DT];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) dot[dt] = lds_read_tr8<vec8>(dos_ + tr[dt][0], dos_ + tr[dt][1]);
+        for (int dt = 0; dt < DT; ++dt) dot[dt] = lds_operand_tr<vec8>(ta[dt][0], ta[dt][1]);
         // P = exp2(S scale - lse log2e).  Rows outside the sequence arrive with lse = +inf
         // (P = 0).  A row that saw no key has lse = -inf, but then every one of its entries
         // here is masked by causality and the select below discards the infinite value, so no
@@ -1048,11 +1112,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         const bool edge = (p.causal && (cb * 64 + nh * 32 + 31 > pos0)) || cb * 64 + 63 >= sq.k_len;
         // last visible q-row offset test: key is visible to row pos iff key <= pos
         const int kcmp = key_ok ? (p.causal ? key - pos0 : INT_MIN) : INT_MAX;  // masked iff kcmp > row offset
-        float *x = xbuf + (t & 1) * 1024;
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
           // registers 4*r4 .. +3 are q rows 8*r4 + 4g + {0..3} of the step
-          const float4 l4 = *reinterpret_cast<const float4 *>(lse_s + r4 * 8 + g * 4);
+          const floatx4 l4 = lds_read8_at<floatx4>(vecs + qs_ / (S::kTile / 256) + r4 * 32);
           const float lr[4] = {l4.x, l4.y, l4.z, l4.w};
 #pragma unroll
           for (int i = 0; i < 4; ++i)
@@ -1071,8 +1134,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         }
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4)
-          *reinterpret_cast<float4 *>(x + (r4 * 64 + lane) * 4) =
-              make_float4(sc[r4 * 4], sc[r4 * 4 + 1], sc[r4 * 4 + 2], sc[r4 * 4 + 3]);
+          lds_write16_at(xbuf + x_ + r4 * 1024, floatx4{sc[r4 * 4], sc[r4 * 4 + 1], sc[r4 * 4 + 2], sc[r4 * 4 + 3]});
         // dV^T += dO^T P
 #pragma unroll
         for (int t2 = 0; t2 < 2; ++t2) {
@@ -1080,38 +1142,66 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 #pragma unroll
           for (int i = 0; i < 8; ++i) pf[i] = sc[t2 * 8 + i];
           const vec8 pb = M::pack(pf);
+          if (t2 == 1 && kLag) {
+            lag_pb = pb;
+            continue;
+          }
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) {
             acc[dt] = M::mma(dot[dt], pb, acc[dt]);
             if (t2 == 0) {
               const int rowoff = 16 * TL::kRowBytes;
-              dot[dt] = lds_read_tr8<vec8>(dos_ + rowoff + tr[dt][0], dos_ + rowoff + tr[dt][1]);
+              (kLag ? lag_dot[dt] : dot[dt]) = lds_operand_tr<vec8>(ta[dt][0] + rowoff, ta[dt][1] + rowoff);
             }
           }
         }
       }
     } else {
-      // second half of step t - 1 first: it frees dp_prev for this step's dP
-      if (t > 0 && (!kIdle || quad_prev != 0)) finish_dk(t - 1, pq, dp_prev);
-      // dP = dO V^T
+      auto product = [&](floatx16 &dp) __attribute__((always_inline)) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) dp_prev[r] = 0.f;
-      if (!kIdle || quad != 0) {
-        vec8 da[KS];
+        for (int r = 0; r < 16; ++r) dp[r] = 0.f;
+        if (!kIdle || quad != 0) {
+          vec8 da[KS];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) da[ks] = lds_read8<vec8>(dos_ + rd[ks]);
+          for (int ks = 0; ks < KS; ++ks) da[ks] = lds_operand<vec8>(ra[ks]);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) dp_prev = M::mma(da[ks], kvf[ks], dp_prev);
-      }
+          for (int ks = 0; ks < KS; ++ks) dp = M::mma(da[ks], kvf[ks], dp);
+        }
+      };
+      floatx16 dp;
+      if constexpr (kAhead) product(dp);
+      if (!first && (!kIdle || quad_prev != 0)) finish_dk(ta, SUB || kHalf ? 0 : S::kTile, pq, x_ ^ 4096, dp_prev);
+      if (SUB || kHalf == 0) move_cols(qs_ - (SUB ? pq : pq - S::kTile));
+      if constexpr (kAhead)
+        dp_prev = dp;
+      else
+        product(dp_prev);
     }
     if constexpr (SUB) quad_prev = quad;
-    pq = cq;
-    cq = cq + 1 == S::kQStages ? 0 : cq + 1;
-    cdo = cdo + 1 == S::kDoStages ? 0 : cdo + 1;
+    first = false;
+    if constexpr (kDp)
+      move_rows(do_0 - cdo);
+    else
+      move_cols(do_0 - cdo);
+  };
+  while (cur != kNone) {
+    work(IntConst<0>{});
+    if constexpr (SUB) {
+      const int next = (q_ring + S::kTile) & (3 * S::kTile);
+      if constexpr (!kDp) move_rows(next - q_ring);
+      q_ring = next, x_ring ^= 4096;
+    } else {
+      work(IntConst<1>{});
+      const int next = q_ring ^ 2 * S::kTile;
+      if constexpr (!kDp) move_rows(next - q_ring);
+      q_ring = next;
+    }
   }
   __syncthreads();  // P of the last step is visible
+  if constexpr (kLag) finish_dv();
   if constexpr (kDp) {
-    if (issued > 0 && (!kIdle || quad_prev != 0)) finish_dk(issued - 1, pq, dp_prev);
+    const int pq = SUB ? (q_ring - S::kTile) & (3 * S::kTile) : (q_ring ^ 2 * S::kTile) + S::kTile;
+    if (!first && (!kIdle || quad_prev != 0)) finish_dk(ta, SUB ? 0 : S::kTile, pq, SUB ? x_ring ^ 4096 : 4096, dp_prev);
   }
   };
   if (dp_wave)

@@ -129,6 +129,12 @@ __device__ __forceinline__ V lds_read8_at(uint32_t addr) {
   return __builtin_bit_cast(V, *(lds_ptr)(uintptr_t)addr);
 }
 template <typename V>
+__device__ __forceinline__ void lds_write16_at(uint32_t addr, V v) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  typedef u32x4 __attribute__((address_space(3))) * lds_ptr;
+  *(lds_ptr)(uintptr_t)addr = __builtin_bit_cast(u32x4, v);
+}
+template <typename V>
 __device__ __forceinline__ V lds_read_tr8_at(uint32_t a0, uint32_t a1) {
   typedef shortx4 __attribute__((address_space(3))) * lds_ptr;
   shortx4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(uintptr_t)a0);
@@ -365,8 +371,10 @@ struct TileLoader {
   // Callers test for this case with scalar arithmetic and take it on the main path: the general
   // `issue` below costs some thirty scalar instructions per tile in range tests and selects,
   // which all waves of a CU execute behind the same barrier.
-  __device__ __forceinline__ void issue_full(const char *gblk, char *tile) const {
-    const uint32_t base = lds_address(tile) + row0 * Tile<D>::kRowBytes;
+  __device__ __forceinline__ void issue_full(const char *gblk, char *tile) const { issue_full_at(gblk, lds_address(tile)); }
+  // (tile: 32-bit LDS address.  Of a generic pointer at a run-time offset the compiler checks for null in front of every copy.)
+  __device__ __forceinline__ void issue_full_at(const char *gblk, uint32_t tile) const {
+    const uint32_t base = tile + row0 * Tile<D>::kRowBytes;
 #pragma unroll
     for (int c = 0; c < kChunks; ++c)
       if (!PAD || ((inside >> c) & 1)) lds_dma16(gblk, goff[c], base + c * (NT / kCPR) * Tile<D>::kRowBytes);
