@@ -583,22 +583,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
     const int bits = bits_cur;
     wait_tile_loads();
     __syncthreads();  // the tile is visible; every wave is done with the other stage
+    // All four values that may be needed are read ahead of the requests for the ones after them: read behind such a
+    // request the compiler waits for it (vmcnt(0): a round trip to the L2 in every block, ahead of the next tile's request).
+    const int next_a = __builtin_amdgcn_readfirstlane(pend_a), next_b = __builtin_amdgcn_readfirstlane(pend_b);
+    int nbits_a = 0, nbits_b = 0;
+    if constexpr (SUB) nbits_a = __builtin_amdgcn_readfirstlane(pbits_a), nbits_b = __builtin_amdgcn_readfirstlane(pbits_b);
     if (flg & 1) {
       ++a_pos;
-      head_a = a_pos < a_end ? __builtin_amdgcn_readfirstlane(pend_a) : kEnd;
-      if (a_pos + 1 < a_end) pend_a = cols[(a_pos + 1) * EW];
-      if constexpr (SUB) {
-        hbits_a = __builtin_amdgcn_readfirstlane(pbits_a);
-        if (a_pos + 1 < a_end) pbits_a = cols[(a_pos + 1) * EW + 1];
+      head_a = a_pos < a_end ? next_a : kEnd;
+      hbits_a = nbits_a;
+      if (a_pos + 1 < a_end) {
+        pend_a = cols[(a_pos + 1) * EW];
+        if constexpr (SUB) pbits_a = cols[(a_pos + 1) * EW + 1];
       }
     }
     if (flg & 2) {
       ++b_pos;
-      head_b = b_pos < b_end ? __builtin_amdgcn_readfirstlane(pend_b) : kEnd;
-      if (b_pos + 1 < b_end) pend_b = cols[(b_pos + 1) * EW];
-      if constexpr (SUB) {
-        hbits_b = __builtin_amdgcn_readfirstlane(pbits_b);
-        if (b_pos + 1 < b_end) pbits_b = cols[(b_pos + 1) * EW + 1];
+      head_b = b_pos < b_end ? next_b : kEnd;
+      hbits_b = nbits_b;
+      if (b_pos + 1 < b_end) {
+        pend_b = cols[(b_pos + 1) * EW];
+        if constexpr (SUB) pbits_b = cols[(b_pos + 1) * EW + 1];
       }
     }
     const int col_next = min(head_a, head_b);

@@ -250,22 +250,27 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
     __syncthreads();  // tile e is visible; every wave is done with the other stage
     if constexpr (RP) {
       const int flg = flg_cur;
+      // All four values that may be needed are read ahead of the requests for the ones after them: read behind such a
+      // request the compiler waits for it (vmcnt(0): a round trip to the L2 in every block, ahead of the next tile's request).
+      const int next_a = __builtin_amdgcn_readfirstlane(pend_a), next_b = __builtin_amdgcn_readfirstlane(pend_b);
+      int nbits_a = 0, nbits_b = 0;
+      if constexpr (SUB) nbits_a = __builtin_amdgcn_readfirstlane(pbits_a), nbits_b = __builtin_amdgcn_readfirstlane(pbits_b);
       if (flg & 1) {
         ++a_pos;
-        head_a = a_pos < emid ? __builtin_amdgcn_readfirstlane(pend_a) : kEnd;
-        if (a_pos + 1 < emid) pend_a = cols[(a_pos + 1) * EW];
-        if constexpr (SUB) {
-          hbits_a = __builtin_amdgcn_readfirstlane(pbits_a);
-          if (a_pos + 1 < emid) pbits_a = cols[(a_pos + 1) * EW + 1];
+        head_a = a_pos < emid ? next_a : kEnd;
+        hbits_a = nbits_a;
+        if (a_pos + 1 < emid) {
+          pend_a = cols[(a_pos + 1) * EW];
+          if constexpr (SUB) pbits_a = cols[(a_pos + 1) * EW + 1];
         }
       }
       if (flg & 2) {
         ++b_pos;
-        head_b = b_pos < e1 ? __builtin_amdgcn_readfirstlane(pend_b) : kEnd;
-        if (b_pos + 1 < e1) pend_b = cols[(b_pos + 1) * EW];
-        if constexpr (SUB) {
-          hbits_b = __builtin_amdgcn_readfirstlane(pbits_b);
-          if (b_pos + 1 < e1) pbits_b = cols[(b_pos + 1) * EW + 1];
+        head_b = b_pos < e1 ? next_b : kEnd;
+        hbits_b = nbits_b;
+        if (b_pos + 1 < e1) {
+          pend_b = cols[(b_pos + 1) * EW];
+          if constexpr (SUB) pbits_b = cols[(b_pos + 1) * EW + 1];
         }
       }
       const int col_next = min(head_a, head_b);
