@@ -402,9 +402,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   // follow each other in the table); a row without queries of this sequence contributes nothing
   auto table_rows = [&](int lh, int &e0, int &emid, int &e1) __attribute__((always_inline)) {
     const int32_t *rp = p.csr.ptr + lh * p.csr.ptr_sh;
-    if (ra < p.csr.num_rows) scalar_load2(rp + ra, rp + ra + 1, e0, emid);
-    e1 = emid;
-    if (ra + 1 < p.csr.num_rows) e1 = scalar_load(rp + ra + 2);
+    if (ra < p.csr.num_rows) scalar_load_row_pair(rp, ra, p.csr.num_rows, e0, emid, e1);
     if (ra < first_rb) e0 = emid;
     if (ra + 1 > last_rb) e1 = emid;
   };
@@ -534,13 +532,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
   }
   int head_a = kEnd, head_b = kEnd, pend_a = 0, pend_b = 0;
   int hbits_a = 0, hbits_b = 0, pbits_a = 0, pbits_b = 0;  // SUB: the entries' masks, carried like the columns
-  if (a_pos < a_end) head_a = scalar_load(cols + a_pos * EW);
-  if (b_pos < b_end) head_b = scalar_load(cols + b_pos * EW);
+  scalar_load_heads<EW>(cols, a_pos, a_end, b_pos, b_end, head_a, head_b, hbits_a, hbits_b);
   if (a_pos + 1 < a_end) pend_a = cols[(a_pos + 1) * EW];
   if (b_pos + 1 < b_end) pend_b = cols[(b_pos + 1) * EW];
   if constexpr (SUB) {
-    if (a_pos < a_end) hbits_a = scalar_load(cols + a_pos * EW + 1);
-    if (b_pos < b_end) hbits_b = scalar_load(cols + b_pos * EW + 1);
     if (a_pos + 1 < a_end) pbits_a = cols[(a_pos + 1) * EW + 1];
     if (b_pos + 1 < b_end) pbits_b = cols[(b_pos + 1) * EW + 1];
   }

@@ -262,6 +262,37 @@ __device__ __forceinline__ void scalar_load2(const int32_t *p0, const int32_t *p
                : "s"(uniform_address(p0)), "s"(uniform_address(p1))
                : "memory");
 }
+// Table rows ra and ra + 1 (ra < num_rows) of num_rows + 1 row pointers: entries [e0, emid) and [emid, e1), the second
+// row empty if it lies beyond the table.  One round trip.
+__device__ __forceinline__ void scalar_load_row_pair(const int32_t *ptr, int ra, int num_rows, int &e0, int &emid, int &e1) {
+  asm volatile("s_load_dword %0, %3, 0x0\n\ts_load_dword %1, %3, 0x4\n\ts_load_dword %2, %4, 0x0\n\ts_waitcnt lgkmcnt(0)"
+               : "=&s"(e0), "=&s"(emid), "=&s"(e1)
+               : "s"(uniform_address(ptr + ra)), "s"(uniform_address(ptr + min(ra + 2, num_rows)))
+               : "memory");
+}
+// First entries of two table rows, [a, a_end) and [b, b_end): column and, where an entry is two ints wide, mask (the
+// caller's values stay where a row is empty).  One round trip.
+template <int EW>
+__device__ __forceinline__ void scalar_load_heads(const int32_t *cols, int a, int a_end, int b, int b_end, int &head_a, int &head_b,
+                                                  int &bits_a, int &bits_b) {
+  const bool has_a = a < a_end, has_b = b < b_end;
+  if (!has_a && !has_b) return;
+  const uint64_t pa = uniform_address(cols + (int64_t)(has_a ? a : b) * EW), pb = uniform_address(cols + (int64_t)(has_b ? b : a) * EW);
+  int ca, cb, ma = 0, mb = 0;
+  if constexpr (EW == 2)
+    asm volatile("s_load_dword %0, %4, 0x0\n\ts_load_dword %1, %4, 0x4\n\ts_load_dword %2, %5, 0x0\n\ts_load_dword %3, %5, 0x4\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&s"(ca), "=&s"(ma), "=&s"(cb), "=&s"(mb)
+                 : "s"(pa), "s"(pb)
+                 : "memory");
+  else
+    asm volatile("s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(ca), "=&s"(cb)
+                 : "s"(pa), "s"(pb)
+                 : "memory");
+  if (has_a) head_a = ca, bits_a = ma;
+  if (has_b) head_b = cb, bits_b = mb;
+}
 // The kernel's first argument as it lies in memory, for code that runs once or rarely: read from the argument itself,
 // the values are fetched at the kernel's start and held in scalar registers through its loop, which spills them.
 template <typename P>

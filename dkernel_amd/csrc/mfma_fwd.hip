@@ -147,9 +147,7 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   if constexpr (RP) {
     const int32_t *rp = p.csr.ptr + lh * p.csr.ptr_sh;
     const int ra = rb & ~1;
-    if (ra < p.csr.num_rows) scalar_load2(rp + ra, rp + ra + 1, e0, emid);
-    e1 = emid;
-    if (ra + 1 < p.csr.num_rows) e1 = scalar_load(rp + ra + 2);
+    if (ra < p.csr.num_rows) scalar_load_row_pair(rp, ra, p.csr.num_rows, e0, emid, e1);
     if (ra < first_rb) e0 = emid;     // a row without queries of this sequence contributes nothing
     if (ra + 1 > last_rb) e1 = emid;
   } else if (rb < p.csr.num_rows) {  // table reads go through the scalar unit (no vector-memory wait)
@@ -219,13 +217,10 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
   int hbits_a = 0, hbits_b = 0, pbits_a = 0, pbits_b = 0;  // RP with SUB: the masks of those entries
   const bool second_row = RP && (wave >> 1) != 0;          // RP: this wave's table row is 2u + 1
   if constexpr (RP) {
-    if (a_pos < emid) head_a = scalar_load(cols + a_pos * EW);
-    if (b_pos < e1) head_b = scalar_load(cols + b_pos * EW);
+    scalar_load_heads<EW>(cols, a_pos, emid, b_pos, e1, head_a, head_b, hbits_a, hbits_b);
     if (a_pos + 1 < emid) pend_a = cols[(a_pos + 1) * EW];
     if (b_pos + 1 < e1) pend_b = cols[(b_pos + 1) * EW];
     if constexpr (SUB) {
-      if (a_pos < emid) hbits_a = scalar_load(cols + a_pos * EW + 1);
-      if (b_pos < e1) hbits_b = scalar_load(cols + b_pos * EW + 1);
       if (a_pos + 1 < emid) pbits_a = cols[(a_pos + 1) * EW + 1];
       if (b_pos + 1 < e1) pbits_b = cols[(b_pos + 1) * EW + 1];
       bits_cur = second_row ? hbits_b : hbits_a;
