@@ -159,9 +159,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = key0 + (r >> 2) * 8 + g * 4 + (r & 3) > lim ? -INFINITY : s[r];
     }
-    float mx = max2(s[0], s[1]);
-#pragma unroll
-    for (int r = 2; r < 16; r += 2) mx = max3(mx, s[r], s[r + 1]);
+    float mx = max_of(s);
     mx = max_with_other_half(mx) * p.scale_log2;  // scale > 0: max commutes with it
     const float m_new = fmaxf(m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;

@@ -532,6 +532,25 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
   return d;
 }
+// Maximum of the 16 or 32 scores of accumulators s and t; the multiplies that made t (or s alone) may have been issued just
+// ahead.  A multiply's result can be read some wait states after its issue, which the compiler keeps for the instructions
+// it knows: it does not look inside the asm statements above.  All of them therefore follow from one value that
+// it reads itself (the canonicalisation is one v_max_f32).  Four chains side by side: in a single one every instruction
+// waits for the one before it, with an s_nop between: prefill of 2 x 8192 tokens 392.6 -> 389.5 us.
+__device__ __forceinline__ float max_of(const floatx16 &s) {
+  const float x = __builtin_canonicalizef(s[0]);
+  float a = max3(x, s[1], s[2]), b = max3(x, s[3], s[4]), c = max3(x, s[5], s[6]), d = max3(x, s[7], s[8]);
+  a = max3(a, s[9], s[10]), b = max3(b, s[11], s[12]), c = max3(c, s[13], s[14]), d = max2(d, s[15]);
+  return max3(a, b, max2(c, d));
+}
+__device__ __forceinline__ float max_of(const floatx16 &s, const floatx16 &t) {
+  const float x = __builtin_canonicalizef(t[0]);
+  float a = max3(x, s[0], s[1]), b = max3(x, s[2], s[3]), c = max3(x, s[4], s[5]), d = max3(x, s[6], s[7]);
+  a = max3(a, s[8], s[9]), b = max3(b, s[10], s[11]), c = max3(c, s[12], s[13]), d = max3(d, s[14], s[15]);
+  a = max3(a, t[1], t[2]), b = max3(b, t[3], t[4]), c = max3(c, t[5], t[6]), d = max3(d, t[7], t[8]);
+  a = max3(a, t[9], t[10]), b = max3(b, t[11], t[12]), c = max3(c, t[13], t[14]), d = max2(d, t[15]);
+  return max3(a, b, max2(c, d));
+}
 // Maximum of a lane's value and the one of the lane 32 away (one VALU exchange, no LDS round
 // trip: v_permlane32_swap of (x, x) leaves the lower half's values in one result and the upper
 // half's in the other).

@@ -368,15 +368,10 @@ __global__ __launch_bounds__(128 * G) __attribute__((amdgpu_waves_per_eu(G == 1 
           }
       }
       float mx;
-      if constexpr (N1 - N0 == 2) {
-        mx = max2(sacc[0][0], sacc[1][0]);
-#pragma unroll
-        for (int r = 1; r < 16; ++r) mx = max3(mx, sacc[0][r], sacc[1][r]);
-      } else {
-        mx = max2(sacc[N0][0], sacc[N0][1]);
-#pragma unroll
-        for (int r = 2; r < 16; r += 2) mx = max3(mx, sacc[N0][r], sacc[N0][r + 1]);
-      }
+      if constexpr (N1 - N0 == 2)
+        mx = max_of(sacc[0], sacc[1]);
+      else
+        mx = max_of(sacc[N0]);
       mx = max_with_other_half(mx) * p.scale_log2;  // scale > 0: max commutes with it
       if (__builtin_amdgcn_ballot_w64(mx > m_run + 8.f) != 0) {  // wave-uniform: some row needs a new reference
         const float m_new = fmaxf(m_run, mx);
