@@ -638,17 +638,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
         for (int i = 0; i < KS / 2; ++i) va[i] = lds_operand<vec8>(rd[half * (KS / 2) + i] + vs_ + kh * kRow32);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < KS / 2; ++i) dp = M::mma(va[i], dof[half * (KS / 2) + i], dp);
-      }
-      // K^T operands of the dQ product do not depend on dS: fetch them now
-      vec8 kt[DT];
+        for (int i = 0; i < KS / 2; ++i) {
+          dp = M::mma(va[i], dof[half * (KS / 2) + i], dp);
+          // the probabilities only wait for S: their exponentials stand between the multiplies of dP
+          if (half == 1) {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) kt[dt] = lds_operand_tr<vec8>(tr[dt][0] + ks_ + kh * kRow32, tr[dt][1] + ks_ + kh * kRow32);
+            for (int r = i * 32 / KS; r < (i + 1) * 32 / KS; ++r) s[r] = fast_exp2(fmaf(s[r], p.scale_log2, -lse2));
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+      }
+      // K^T operands of the dQ product do not depend on dS: all of them are fetched now, behind the multiplies (with the
+      // exponentials between those: training, 4 x 2048 tokens, 32 / 8 heads 580 -> 576 us)
+      vec8 kt[2][DT];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          kt[t][dt] = lds_operand_tr<vec8>(tr[dt][0] + ks_ + kh * kRow32 + t * 16 * TL::kRowBytes, tr[dt][1] + ks_ + kh * kRow32 + t * 16 * TL::kRowBytes);
 
       const bool need_mask = (key0 + 31 >= sq.k_len) || (p.causal && key0 + 31 > row0);
       const int lim = p.causal ? min(pos, sq.k_len - 1) : sq.k_len - 1;  // last visible key of this row
-#pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = fast_exp2(fmaf(s[r], p.scale_log2, -lse2));
       if (need_mask) {  // wave-uniform: only the diagonal block and the last, partial one pay for masks
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -672,12 +682,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
         for (int i = 0; i < 8; ++i) f[i] = s[t * 8 + i];
         const vec8 dsb = M::pack(f);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          acc[dt] = M::mma(kt[dt], dsb, acc[dt]);
-          if (t == 0)  // refill with the second k-step's operand as soon as the register is free
-            kt[dt] = lds_operand_tr<vec8>(tr[dt][0] + ks_ + kh * kRow32 + 16 * TL::kRowBytes,
-                                          tr[dt][1] + ks_ + kh * kRow32 + 16 * TL::kRowBytes);
-        }
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = M::mma(kt[t][dt], dsb, acc[dt]);
       }
     }
   };
