@@ -120,12 +120,19 @@ def lib():
     return _lib
 
 
-_host = None
+_host = _bound = None
+
+
+def launcher():
+    """host() for training's launches, or None where lib() has been replaced by something else than the library that it
+    launches through (a wrapper that wants to see the calls)."""
+    module = host()
+    return module if lib() is _bound else None
 
 
 def host():
-    """The C++ host path of the inference calls (dkernel_amd/_host.so, loaded on first use)."""
-    global _host
+    """The C++ host path of the inference calls and of training's launches (dkernel_amd/_host.so, loaded on first use)."""
+    global _host, _bound
     if _host is None:
         path = os.path.join(_HERE, "_host.so")
         if not os.path.exists(path):
@@ -133,8 +140,9 @@ def host():
         from . import _host as module
         handle = lib()
         module.bind(*(C.cast(getattr(handle, name), vp).value
-                      for name in ("dk_fwd", "dk_fwd_workspace_bytes", "dk_fwd_paged")))
-        _host = module
+                      for name in ("dk_fwd", "dk_fwd_workspace_bytes", "dk_fwd_paged", "dk_bwd_balanced",
+                                   "dk_bwd_balanced_workspace_bytes")))
+        _host, _bound = module, handle
     return _host
 
 

@@ -1,7 +1,9 @@
 // Host path of the inference calls in C++ (CPython module dkernel_amd._host): what ops.py does for a
 // forward that needs no gradient - checks, outputs, scratch, the argument block of dk_fwd - without
 // the interpreter.  A single-token step or a short prompt keeps the GPU busy for 8 - 15 us; the
-// Python launcher took 15 us of host time per call around the launch itself (2.5 us).
+// Python launcher took 15 us of host time per call around the launch itself (2.5 us).  For the two halves of a training
+// step (train_forward, train_backward) it is the launch alone: which tables, lengths and gradients, and all of autograd, stay
+// in ops.py.
 //
 // The functions take the common case only: tensors as the kernels want them.  They return None,
 // having done nothing, for anything else (tensors on the host, strides to be fixed, lengths of another
@@ -22,6 +24,7 @@
 
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <optional>
 
 #include "../../include/dkernel_hip.h"
@@ -31,6 +34,8 @@ namespace {
 int (*fwd_fn)(const dk_fwd_args *) = nullptr;
 size_t (*fwd_bytes_fn)(const dk_fwd_args *) = nullptr;
 int (*fwd_paged_fn)(const dk_fwd_args *, const dk_paged_kv *) = nullptr;
+int (*bwd_fn)(const dk_bwd_args *, const dk_row_lengths *) = nullptr;
+size_t (*bwd_bytes_fn)(const dk_bwd_args *, const dk_row_lengths *) = nullptr;
 
 PyObject *k_max_seqlen, *k_causal, *k_group, *k_max_row, *k_uneven, *k_unsorted, *k_fixed, *k_out, *k_inference;
 
@@ -337,6 +342,126 @@ PyObject *paged_impl(PyObject *const *args) {
   return result(out, lse, bytes);
 }
 
+// The bytes of a ctypes structure
+template <typename T>
+T structure(PyObject *o) {
+  Py_buffer b;
+  if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) != 0) {
+    PyErr_Clear();
+    throw Unsupported{};
+  }
+  T t;
+  const bool ok = b.len == (Py_ssize_t)sizeof(T);
+  if (ok) std::memcpy(&t, b.buf, sizeof(T));
+  PyBuffer_Release(&b);
+  need(ok);
+  return t;
+}
+
+// A tensor of a training step: on `dev`, of q's type, rows of consecutive elements
+void check_row_tensor(const at::Tensor &t, const at::Tensor &q) {
+  need(t.is_cuda() && t.get_device() == q.get_device() && t.scalar_type() == q.scalar_type() && t.dim() == 4 && t.stride(3) == 1);
+}
+
+// train_forward(q, k, v, csr, sm_scale, seq_dim, causal, impl, want_lse, use_workspace) -> (out, lse or None, scratch bytes) or None
+PyObject *train_forward_impl(PyObject *const *args) {
+  const at::Tensor &q = tensor(args[0]), &k = tensor(args[1]), &v = tensor(args[2]);
+  check_row_tensor(q, q), check_row_tensor(k, q), check_row_tensor(v, q);
+  need(q.get_device() == c10::hip::current_device());
+  dk_fwd_args a{};
+  a.csr = structure<dk_lut>(args[3]);
+  const double scale = PyFloat_AsDouble(args[4]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    throw Unsupported{};
+  }
+  const int64_t seq_dim = integer(args[5]);
+  need(seq_dim == 1 || seq_dim == 2);
+  const int s = (int)seq_dim, h = 3 - s;
+  const int64_t B = q.size(0), Lq = q.size(s), Lk = k.size(s), Hq = q.size(h), Hkv = k.size(h), D = q.size(3);
+  need(B > 0 && Lq > 0 && Lk > 0 && D > 0 && k.sizes() == v.sizes() && k.size(0) == B && k.size(3) == D);
+  check_heads(a.csr, Hq, Hkv);
+  a.dtype = dtype_code(q.scalar_type());
+  a.causal = truth(args[6]), a.impl = (int32_t)integer(args[7]), a.head_dim = (int32_t)D, a.sm_scale = (float)scale;
+  const bool want_lse = truth(args[8]), use_workspace = truth(args[9]);
+  a.seqs.batch = (int32_t)B, a.seqs.max_q_len = (int32_t)Lq, a.seqs.max_k_len = (int32_t)Lk;
+  a.num_q_heads = (int32_t)Hq, a.num_kv_heads = (int32_t)Hkv;
+  at::Tensor out, lse;
+  std::optional<Unlocked> unlocked;
+  unlocked.emplace();
+  out = at::empty(q.sizes(), q.options());
+  if (want_lse) {
+    lse = at::empty({B, Hq, Lq}, q.options().dtype(at::kFloat));
+    a.lse = dk_rowvec{static_cast<float *>(lse.data_ptr()), Hq * Lq, Lq, 1};
+  }
+  a.q = view(q, 0, h, s), a.k = view(k, 0, h, s), a.v = view(v, 0, h, s), a.o = view(out, 0, h, s);
+  const size_t bytes = launch(a, q, use_workspace);
+  unlocked.reset();
+  return result(out, lse, bytes);
+}
+
+// train_backward(q, k, v, o, dout, lse, dlse or None, dq or None, dk or None, dv or None, csr, csc, lengths, sm_scale, seq_dim,
+//                causal, impl, use_workspace) -> (dq, dk, dv) or None
+PyObject *train_backward_impl(PyObject *const *args) {
+  const at::Tensor &q = tensor(args[0]), &k = tensor(args[1]), &v = tensor(args[2]), &o = tensor(args[3]), &dout = tensor(args[4]);
+  const at::Tensor &lse = tensor(args[5]), *dlse = optional_tensor(args[6]);
+  need(bwd_fn);
+  const at::Tensor *given[3] = {optional_tensor(args[7]), optional_tensor(args[8]), optional_tensor(args[9])}, *like[3] = {&q, &k, &v};
+  for (const at::Tensor *t : {&q, &k, &v, &o, &dout}) check_row_tensor(*t, q);
+  need(q.get_device() == c10::hip::current_device());
+  need(k.sizes() == v.sizes() && o.sizes() == q.sizes() && dout.sizes() == q.sizes() && k.size(0) == q.size(0) && k.size(3) == q.size(3));
+  for (int i = 0; i < 3; ++i)
+    if (given[i]) {
+      check_row_tensor(*given[i], q);
+      need(given[i]->sizes() == like[i]->sizes());
+    }
+  dk_bwd_args a{};
+  a.csr = structure<dk_lut>(args[10]), a.csc = structure<dk_lut>(args[11]);
+  const dk_row_lengths lengths = structure<dk_row_lengths>(args[12]);
+  const double scale = PyFloat_AsDouble(args[13]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    throw Unsupported{};
+  }
+  const int64_t seq_dim = integer(args[14]);
+  need(seq_dim == 1 || seq_dim == 2);
+  const int s = (int)seq_dim, h = 3 - s;
+  const int64_t B = q.size(0), Lq = q.size(s), Lk = k.size(s), Hq = q.size(h), Hkv = k.size(h), D = q.size(3);
+  need(B > 0 && Lq > 0 && Lk > 0 && D > 0);
+  check_heads(a.csr, Hq, Hkv), check_heads(a.csc, Hq, Hkv);
+  auto rows = [&](const at::Tensor &t) {
+    need(t.is_cuda() && t.get_device() == q.get_device() && t.scalar_type() == at::kFloat && t.dim() == 3 && t.size(0) == B && t.size(1) == Hq &&
+         t.size(2) == Lq);
+    return dk_rowvec{static_cast<float *>(t.data_ptr()), t.stride(0), t.stride(1), t.stride(2)};
+  };
+  a.lse = rows(lse);
+  if (dlse) a.dlse = rows(*dlse);
+  a.dtype = dtype_code(q.scalar_type());
+  a.causal = truth(args[15]), a.impl = (int32_t)integer(args[16]), a.head_dim = (int32_t)D, a.sm_scale = (float)scale;
+  const bool use_workspace = truth(args[17]);
+  a.seqs.batch = (int32_t)B, a.seqs.max_q_len = (int32_t)Lq, a.seqs.max_k_len = (int32_t)Lk;
+  a.num_q_heads = (int32_t)Hq, a.num_kv_heads = (int32_t)Hkv;
+  at::Tensor grads[3], delta, ws;
+  std::optional<Unlocked> unlocked;
+  unlocked.emplace();
+  for (int i = 0; i < 3; ++i) grads[i] = given[i] ? *given[i] : at::empty(like[i]->sizes(), like[i]->options());
+  delta = at::empty({B, Hq, Lq}, q.options().dtype(at::kFloat));
+  a.q = view(q, 0, h, s), a.k = view(k, 0, h, s), a.v = view(v, 0, h, s), a.o = view(o, 0, h, s), a.dout = view(dout, 0, h, s);
+  a.dq = view(grads[0], 0, h, s), a.dk = view(grads[1], 0, h, s), a.dv = view(grads[2], 0, h, s);
+  a.delta = static_cast<float *>(delta.data_ptr());
+  a.stream = current_stream();
+  const size_t bytes = use_workspace ? bwd_bytes_fn(&a, &lengths) : 0;
+  if (bytes) {
+    ws = at::empty({(int64_t)bytes}, q.options().dtype(at::kByte));
+    a.workspace = ws.data_ptr(), a.workspace_bytes = bytes;
+  }
+  need(bwd_fn(&a, &lengths) == DK_OK);
+  unlocked.reset();
+  PyObject *t = PyTuple_New(3);
+  for (int i = 0; i < 3; ++i) PyTuple_SET_ITEM(t, i, THPVariable_Wrap(grads[i]));
+  return t;
+}
+
 template <PyObject *(*Impl)(PyObject *const *), int N>
 PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != N || !fwd_fn) {
@@ -359,19 +484,23 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   }
 }
 
-// bind(address of dk_fwd, of dk_fwd_workspace_bytes, of dk_fwd_paged)
+// bind(address of dk_fwd, of dk_fwd_workspace_bytes, of dk_fwd_paged[, of dk_bwd_balanced, of dk_bwd_balanced_workspace_bytes])
 PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
-  if (n != 3) {
-    PyErr_SetString(PyExc_TypeError, "bind takes three addresses");
+  if (n != 3 && n != 5) {
+    PyErr_SetString(PyExc_TypeError, "bind takes three or five addresses");
     return nullptr;
   }
-  void *p[3];
-  for (int i = 0; i < 3; ++i) {
+  void *p[5] = {};
+  for (int i = 0; i < n; ++i) {
     p[i] = PyLong_AsVoidPtr(args[i]);
     if (PyErr_Occurred()) return nullptr;
   }
   fwd_bytes_fn = reinterpret_cast<decltype(fwd_bytes_fn)>(p[1]);
   fwd_paged_fn = reinterpret_cast<decltype(fwd_paged_fn)>(p[2]);
+  if (n == 5) {
+    bwd_bytes_fn = reinterpret_cast<decltype(bwd_bytes_fn)>(p[4]);
+    bwd_fn = reinterpret_cast<decltype(bwd_fn)>(p[3]);
+  }
   fwd_fn = reinterpret_cast<decltype(fwd_fn)>(p[0]);
   Py_RETURN_NONE;
 }
@@ -380,6 +509,8 @@ PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, "Addresses of the C ABI's forward functions."},
     {"forward", (PyCFunction)(void (*)(void))entry<forward_impl, 16>, METH_FASTCALL, "Forward without gradients, or None."},
     {"paged", (PyCFunction)(void (*)(void))entry<paged_impl, 16>, METH_FASTCALL, "Paged decode step, or None."},
+    {"train_forward", (PyCFunction)(void (*)(void))entry<train_forward_impl, 10>, METH_FASTCALL, "Forward of a training step, or None."},
+    {"train_backward", (PyCFunction)(void (*)(void))entry<train_backward_impl, 18>, METH_FASTCALL, "Backward of a training step, or None."},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods};

@@ -311,23 +311,30 @@ def _forward(ctx, q: Tensor, k: Tensor, v: Tensor, sm_scale: float,
 
     q, k, v = _unit_last(q), _unit_last(k), _unit_last(v)
     _check_out(out, q)
-    o = out if out is not None else q.new_empty(q.shape).contiguous()
     if inference is None:
         inference = (not q.requires_grad) and (not k.requires_grad) and (not v.requires_grad)
     need_lse = return_lse or not inference
-    lse = torch.empty((q.size(0), num_heads, qlen), dtype=torch.float32, device=q.device) if need_lse else None
-
-    args = _lib.FwdArgs()
-    args.q, args.k, args.v, args.o = (_tensor4(x, hdim, seq_dim) for x in (q, k, v, o))
-    args.lse = _rowvec(lse)
-    args.csr = _lut(layout_csr, q.device, lut_group, lut_max_row, uneven=uneven_heads,
-                    longest_first=unsorted_rows and qlen > 1, fixed_walk=fixed_walk)
-    args.seqs = _lib.Seqs(q.size(0), qlen, klen, 0, None, None, None, None)
-    args.num_q_heads, args.num_kv_heads, args.head_dim = num_heads, num_kv_heads, q.size(-1)
-    args.dtype, args.causal, args.impl = _DTYPES[q.dtype], int(bool(causal)), _impl
-    args.sm_scale = float(sm_scale)
-    args.stream = _stream()
-    _run_fwd(args, q.device)
+    csr = _lut(layout_csr, q.device, lut_group, lut_max_row, uneven=uneven_heads,
+               longest_first=unsorted_rows and qlen > 1, fixed_walk=fixed_walk)
+    # the outputs, scratch and the launch from C++ (None: not such tensors, or an error to be raised below)
+    host = _lib.launcher() if out is None and not inference else None
+    res = host and host.train_forward(q, k, v, csr, float(sm_scale), seq_dim, causal, _impl, need_lse, _fwd_workspace)
+    if res is not None:
+        global last_fwd_workspace_bytes
+        o, lse, last_fwd_workspace_bytes = res
+    else:
+        o = out if out is not None else q.new_empty(q.shape).contiguous()
+        lse = torch.empty((q.size(0), num_heads, qlen), dtype=torch.float32, device=q.device) if need_lse else None
+        args = _lib.FwdArgs()
+        args.q, args.k, args.v, args.o = (_tensor4(x, hdim, seq_dim) for x in (q, k, v, o))
+        args.lse = _rowvec(lse)
+        args.csr = csr
+        args.seqs = _lib.Seqs(q.size(0), qlen, klen, 0, None, None, None, None)
+        args.num_q_heads, args.num_kv_heads, args.head_dim = num_heads, num_kv_heads, q.size(-1)
+        args.dtype, args.causal, args.impl = _DTYPES[q.dtype], int(bool(causal)), _impl
+        args.sm_scale = float(sm_scale)
+        args.stream = _stream()
+        _run_fwd(args, q.device)
 
     ctx.save_for_backward(q, k, v, o, lse)
     ctx.sm_scale = sm_scale
@@ -350,6 +357,37 @@ def _backward(ctx, do: Tensor, dlse: Optional[Tensor],
     assert lse is not None, "forward ran in inference mode; backward needs the saved log-sum-exp"
     do = _unit_last(do)
 
+    Lq, Lk = q.size(seq_dim), k.size(seq_dim)
+    layout_csr, layout_csc = ctx.layout_csr, ctx.layout_csc
+    masked = getattr(ctx, "masked_layouts", None)
+    if masked is not None and _matrix_core_applies(q, k, v, o, do, *(x for x in (dq, dk, dv) if x is not None)):
+        layout_csr, layout_csc = masked[0], masked[1]
+        tables = ctx.row_lengths[1] if len(ctx.row_lengths) > 1 else None
+    else:
+        tables = ctx.row_lengths[0] if ctx.row_lengths else None
+    uneven = getattr(ctx, "uneven_heads", False)
+    csr = _lut(layout_csr, q.device, ctx.lut_group, uneven=uneven, longest_first=getattr(ctx, "unsorted_rows", False))
+    csc = _lut(layout_csc, q.device, ctx.lut_group, longest_first=True, uneven=uneven)
+    rows = _NO_LENGTHS
+    if tables is not None and tables.fits(layout_csr, layout_csc):
+        # what this call works on of tables that may be built for longer sequences (`held`: until the call is made)
+        held = tables.of_call(Lk - Lq if ctx.causal else 0, Lq, Lk)
+        rows = held[0]
+    lib = _lib.lib()
+    # the gradients, scratch and the launches from C++ (None: not such tensors, or an error to be raised below)
+    host = _lib.launcher()
+    res = host and host.train_backward(q, k, v, o, do, lse, dlse, dq, dk, dv, csr, csc, rows, float(ctx.sm_scale), seq_dim,
+                                       ctx.causal, _impl, _bwd_workspace)
+    if res is None:
+        res = _python_backward(ctx, q, k, v, o, lse, do, dlse, dq, dk, dv, csr, csc, rows)
+    global last_bwd_kernels
+    last_bwd_kernels = lib.dk_last_kernels()  # (backward runs on an autograd thread; the list is per thread)
+    return res
+
+
+def _python_backward(ctx, q, k, v, o, lse, do, dlse, dq, dk, dv, csr, csc, rows) -> Tuple[Tensor, Tensor, Tensor]:
+    hdim, seq_dim = ctx.hdim, ctx.seq_dim
+
     def _check_or_new(x, like):
         if x is not None:
             assert x.shape == like.shape
@@ -371,36 +409,18 @@ def _backward(ctx, do: Tensor, dlse: Optional[Tensor],
     else:
         args.dlse = _rowvec(None)
     args.delta = delta.data_ptr()
-    layout_csr, layout_csc = ctx.layout_csr, ctx.layout_csc
-    masked = getattr(ctx, "masked_layouts", None)
-    if masked is not None and _matrix_core_applies(q, k, v, o, do, dq, dk, dv):
-        layout_csr, layout_csc = masked[0], masked[1]
-        tables = ctx.row_lengths[1] if len(ctx.row_lengths) > 1 else None
-    else:
-        tables = ctx.row_lengths[0] if ctx.row_lengths else None
-    uneven = getattr(ctx, "uneven_heads", False)
-    args.csr = _lut(layout_csr, q.device, ctx.lut_group, uneven=uneven,
-                    longest_first=getattr(ctx, "unsorted_rows", False))
-    args.csc = _lut(layout_csc, q.device, ctx.lut_group, longest_first=True, uneven=uneven)
+    args.csr, args.csc = csr, csc
     args.seqs = _lib.Seqs(B, Lq, k.size(seq_dim), 0, None, None, None, None)
     args.num_q_heads, args.num_kv_heads, args.head_dim = Hq, k.size(hdim), q.size(-1)
     args.dtype, args.causal, args.impl = _DTYPES[q.dtype], int(bool(ctx.causal)), _impl
     args.sm_scale = float(ctx.sm_scale)
     args.stream = _stream()
-    rows = _NO_LENGTHS
-    if tables is not None and tables.fits(layout_csr, layout_csc):
-        # what this call works on of tables that may be built for longer sequences (`held`: until the call is made)
-        Lk = k.size(seq_dim)
-        held = tables.of_call(Lk - Lq if ctx.causal else 0, Lq, Lk)
-        rows = held[0]
     lib = _lib.lib()
     need = lib.dk_bwd_balanced_workspace_bytes(C.byref(args), C.byref(rows)) if _bwd_workspace else 0
     if need:  # dK/dV partials per q head (several q heads per kv head), partial sums of long rows and columns
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
         args.workspace, args.workspace_bytes = ws.data_ptr(), need
     _lib.check(lib.dk_bwd_balanced(C.byref(args), C.byref(rows)))
-    global last_bwd_kernels
-    last_bwd_kernels = lib.dk_last_kernels()  # (backward runs on an autograd thread; the list is per thread)
     return dq, dk, dv
 
 

@@ -164,3 +164,61 @@ def test_user_pattern_and_errors():
     with pytest.raises(TypeError):
         mod(q.double(), k.double(), v.double())
     assert math.isfinite(mod(q[:, :0 + 1], k[:, :1], v[:, :1]).float().sum().item())
+
+
+@pytest.mark.parametrize("dtype,D,bs,seq_dim,Hq,Hkv,fused,lse_grad", [
+    (torch.bfloat16, 128, 64, 1, 8, 2, True, False), (torch.float16, 64, 32, 2, 4, 4, False, True),
+    (torch.float32, 64, 64, 1, 4, 2, False, False), (torch.bfloat16, 96, 128, 2, 6, 2, False, True)])
+def test_training_step(monkeypatch, dtype, D, bs, seq_dim, Hq, Hkv, fused, lse_grad):
+    """Both halves of a training step through train_forward / train_backward and through ops.py: the same bits."""
+    B, L = 2, 500
+    print(f"case {dtype} D={D} bs={bs} seq_dim={seq_dim} fused={fused}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    mod = New(Hq, 512, bs, 2, 3, num_kv_heads=Hkv, seq_dim=seq_dim).to(DEV)
+
+    def rand(h):
+        return torch.randn((B, L, h, D) if seq_dim == 1 else (B, h, L, D), generator=g, device=DEV).to(dtype)
+
+    if fused:
+        xs = (rand(Hq + 2 * Hkv).requires_grad_(),)
+    else:
+        xs = tuple(rand(h).requires_grad_() for h in (Hq, Hkv, Hkv))
+    dout, dlse = rand(Hq), torch.randn(B, Hq, L, generator=g, device=DEV)
+
+    def step():
+        if fused:
+            out, lse = mod(xs[0], return_lse=True, split_qkv=lambda x: (x[:, :, :Hq], x[:, :, Hq:Hq + Hkv], x[:, :, Hq + Hkv:]))
+        else:
+            out, lse = mod(*xs, return_lse=True)
+        return (out, lse) + torch.autograd.grad((out, lse) if lse_grad else out, xs, (dout, dlse) if lse_grad else dout)
+
+    real, taken = _lib.host(), []
+
+    class Spy:
+        train_forward = staticmethod(lambda *a: taken.append(real.train_forward(*a)) or taken[-1])
+        train_backward = staticmethod(lambda *a: taken.append(real.train_backward(*a)) or taken[-1])
+
+    class Never:
+        train_forward = train_backward = staticmethod(lambda *a: None)
+
+    monkeypatch.setattr(_lib, "host", lambda: Spy)
+    fast = step()
+    assert len(taken) == 2 and all(x is not None for x in taken), "the C++ path did not take this step"
+    monkeypatch.setattr(_lib, "host", lambda: Never)
+    slow = step()
+    monkeypatch.undo()
+    same(tuple(x.detach() for x in fast), tuple(x.detach() for x in slow))
+
+
+def test_training_step_left_to_ops():
+    """Steps whose tensors are not as the launch wants them: a gradient expanded from one value, a log-sum-exp gradient
+    of another type, double differentiation asked for (refused, as before)."""
+    mod = New(2, 256, 64, 2, 3).to(DEV)
+    q, k, v = (torch.randn(1, 256, 2, 64, device=DEV, dtype=torch.bfloat16, requires_grad=True) for _ in range(3))
+    out, lse = mod(q, k, v, return_lse=True)
+    a = torch.autograd.grad(out.sum(), (q, k, v), retain_graph=True)
+    b = torch.autograd.grad(out, (q, k, v), torch.ones_like(out), retain_graph=True)
+    same(a, b)
+    c = torch.autograd.grad(lse.double().sum(), (q, k), retain_graph=True)
+    d = torch.autograd.grad(lse, (q, k), torch.ones_like(lse))
+    same(c, d)
