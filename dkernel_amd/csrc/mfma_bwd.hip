@@ -1063,7 +1063,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   };
   // (not where steps are left out: the guards cost registers, 64 dims then lose their third workgroup, 241 -> 265 us)
   constexpr bool kLag = !kDp && !kIdle;
-  constexpr bool kAhead = !kIdle;
+  constexpr bool kProductFirst = !kIdle;  // dP of a step ahead of dS of the one before
   vec8 lag_dot[DT], lag_pb;  // dO^T and P of the second half of the step before
   if constexpr (kLag) {
 #pragma unroll
@@ -1174,10 +1174,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
         }
       };
       floatx16 dp;
-      if constexpr (kAhead) product(dp);
+      if constexpr (kProductFirst) product(dp);
       if (!first && (!kIdle || quad_prev != 0)) finish_dk(ta, SUB || kHalf ? 0 : S::kTile, pq, x_ ^ 4096, dp_prev);
       if (SUB || kHalf == 0) move_cols(qs_ - (SUB ? pq : pq - S::kTile));
-      if constexpr (kAhead)
+      if constexpr (kProductFirst)
         dp_prev = dp;
       else
         product(dp_prev);

@@ -226,7 +226,7 @@ __device__ __forceinline__ void transposed_offsets(int lane, int (&off)[DT][2]) 
 // builtin the compiler places "s_waitcnt vmcnt(0)" in front of every later
 // LDS read (it cannot tell which LDS bytes a copy in flight will write), which
 // serialises a prefetch with the reads of the tile before it.  Here the caller
-// owns the ordering: wait_tile_loads / wait_tiles_ahead, then a barrier,
+// owns the ordering: wait_tile_loads (or an exact vmcnt), then a barrier,
 // before anything reads what was copied.  Vector memory operations complete in
 // order, so the compiler's own vmcnt bookkeeping for ordinary loads stays
 // conservative (it can only wait for more than it asked for).
@@ -498,23 +498,6 @@ __device__ __forceinline__ void zero_tiles(char *lds, int bytes, int tid) {
 
 // All asynchronous tile loads (and any other vector memory loads) of this wave have landed.
 __device__ __forceinline__ void wait_tile_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// Multi-stage pipelines: wait until at most `ahead` later tiles (LPT vector
-// memory instructions per wave each) are still in flight, i.e. until the
-// oldest tile has landed.  Vector memory loads return in order.  `ahead` is
-// wave-uniform and at most 3.
-template <int LPT>
-__device__ __forceinline__ void wait_tiles_ahead(int ahead) {
-  static_assert(3 * LPT <= 63, "vmcnt is a 6-bit counter");
-  if (ahead <= 0)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  else if (ahead == 1)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPT) : "memory");
-  else if (ahead == 2)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPT) : "memory");
-  else
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * LPT) : "memory");
-}
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
