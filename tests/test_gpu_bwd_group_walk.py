@@ -98,3 +98,27 @@ def test_short_call_of_a_module_for_long_sequences(B, Hq, Hkv, L, table, bs, wal
             assert_close(name, a, b, atol=1e-3 * float(b.float().abs().max()), rtol=8e-3)
         else:
             assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("D,bs,dtype", [(128, 64, torch.bfloat16), (64, 64, torch.float16), (256, 64, torch.bfloat16),
+                                        (128, 32, torch.bfloat16), (64, 16, torch.float16)])
+def test_short_columns(D, bs, dtype):
+    """dK / dV of columns with one to five listed blocks, fewer than the steps that are requested ahead and around the
+    lengths of the rings, their last step whole, one row or one row short; the second head lists nothing below the diagonal."""
+    n = 6 * 64 // bs
+    bm = np.zeros((2, n, n), dtype=bool)
+    for c in range(n):
+        bm[0, c:c + 1 + c % 5, c] = True
+    bm[1] = np.eye(n, dtype=bool)
+    mod = SparseAttention(bs, torch.from_numpy(bm)).to(DEV)
+    sm = 1 / math.sqrt(D)
+    for L, Lk in ((1, 1), (31, 31), (32, 32), (33, 33), (65, 65), (97, 97), (320, 320), (353, 353), (384, 384), (40, 300)):
+        print(f"case D={D} bs={bs} {dtype} L={L} Lk={Lk}", flush=True)
+        q, k, v, do = make_qkv(1, L, Lk, 2, 2, D, dtype, with_do=True)
+        got, ran = _run(mod, q, k, v, do, sm)
+        assert "mfma_dkdv" in ran, ran
+        qo, ko, vo = (x.clone().float().requires_grad_() for x in (q, k, v))
+        ro, _ = oracle_fwd(qo, ko, vo, bm, bs, sm, causal=True)
+        ro.backward(do.float())
+        for name, a, want in zip(("dQ", "dK", "dV"), got, (qo.grad, ko.grad, vo.grad)):
+            assert_close(f"{name} L={L} Lk={Lk}", a, want, **TOL)
