@@ -132,7 +132,7 @@ def test_paged(monkeypatch, bs, fp8, dims):
 
 
 def test_launches_run_without_the_interpreter_lock():
-    """PyGILState_Check in the place of dk_fwd and dk_fwd_paged: its 0 for a thread that does not hold the
+    """PyGILState_Check in the place of dk_fwd, dk_fwd_paged and dk_bwd_balanced: its 0 for a thread that does not hold the
     lock reads as DK_OK, its 1 as a refusal, for which the C++ path returns None.  (Nothing is launched.)"""
     def address(f):
         return C.cast(f, C.c_void_p).value
@@ -141,14 +141,20 @@ def test_launches_run_without_the_interpreter_lock():
     q, k, v = (torch.zeros(1, 256, h, 64, device=DEV, dtype=torch.bfloat16) for h in (4, 2, 2))
     n = torch.tensor([0, 256], dtype=torch.int32, device=DEV)
     tail = (mod._buffers, mod._kernel_tables, mod.mask_lut_max_row)
+    csr = ops._lut((mod.layout_csr_crow, mod.layout_csr_col, 64, 64), q.device)
+    csc = ops._lut((mod.layout_csc_ccol, mod.layout_csc_row, 64, 64), q.device)
+    sizes = [address(lib.dk_fwd_workspace_bytes), address(lib.dk_bwd_balanced_workspace_bytes)]
     try:
-        host.bind(check, address(lib.dk_fwd_workspace_bytes), check)
+        host.bind(check, sizes[0], check, check, sizes[1])
         res = [host.forward(q, k, v, 0.1, *tail, mod.kwargs, 1, None, None, None, None, True, ops._impl, True),
                host.forward(q[0], k[0], v[0], 0.1, *tail, mod.kwargs, 1, n, None, None, None, True, ops._impl, True),
                host.paged(q[:, 0], k.view(4, 64, 2, 64), v.view(4, 64, 2, 64), torch.arange(4, dtype=torch.int32, device=DEV)[None],
-                          n[1:], 0.1, *tail, mod.lut_max_row, mod.lut_group, 256, True, 1.0, 1.0, ops._impl)]
+                          n[1:], 0.1, *tail, mod.lut_max_row, mod.lut_group, 256, True, 1.0, 1.0, ops._impl),
+               host.train_forward(q, k, v, csr, 0.1, 1, True, ops._impl, True, True),
+               host.train_backward(q, k, v, q, q, torch.zeros(1, 4, 256, device=DEV), None, None, None, None, csr, csc, ops._NO_LENGTHS, 0.1, 1,
+                                   True, ops._impl, True)]
     finally:
-        host.bind(*(address(f) for f in (lib.dk_fwd, lib.dk_fwd_workspace_bytes, lib.dk_fwd_paged)))
+        host.bind(address(lib.dk_fwd), sizes[0], address(lib.dk_fwd_paged), address(lib.dk_bwd_balanced), sizes[1])
     assert all(r is not None for r in res)
 
 
@@ -210,15 +216,60 @@ def test_training_step(monkeypatch, dtype, D, bs, seq_dim, Hq, Hkv, fused, lse_g
     same(tuple(x.detach() for x in fast), tuple(x.detach() for x in slow))
 
 
-def test_training_step_left_to_ops():
-    """Steps whose tensors are not as the launch wants them: a gradient expanded from one value, a log-sum-exp gradient
-    of another type, double differentiation asked for (refused, as before)."""
+class _Subclass(torch.Tensor):
+    pass
+
+
+def test_training_step_left_to_ops(monkeypatch):
+    """What the C++ halves refuse (None) and the launches of ops.py then do with the same bits: tensors of a subclass, a
+    backward that is to be differentiated, a log-sum-exp gradient of another type; and gradient tensors of the caller's."""
     mod = New(2, 256, 64, 2, 3).to(DEV)
-    q, k, v = (torch.randn(1, 256, 2, 64, device=DEV, dtype=torch.bfloat16, requires_grad=True) for _ in range(3))
-    out, lse = mod(q, k, v, return_lse=True)
-    a = torch.autograd.grad(out.sum(), (q, k, v), retain_graph=True)
-    b = torch.autograd.grad(out, (q, k, v), torch.ones_like(out), retain_graph=True)
+    xs = tuple(torch.randn(1, 256, 2, 64, device=DEV, dtype=torch.bfloat16, requires_grad=True) for _ in range(3))
+    dout, dlse = torch.randn_like(xs[0]), torch.randn(1, 2, 256, device=DEV)
+    real, taken = _lib.host(), []
+
+    class Spy:
+        train_forward = staticmethod(lambda *a: taken.append(real.train_forward(*a)) or taken[-1])
+        train_backward = staticmethod(lambda *a: taken.append(real.train_backward(*a)) or taken[-1])
+
+    def took(*what):  # of the calls since the last time: which ones the C++ halves did
+        done, taken[:] = [x is not None for x in taken], []
+        assert done == list(what), done
+
+    monkeypatch.setattr(_lib, "host", lambda: Spy)
+    out, lse = mod(*xs, return_lse=True)
+    want = torch.autograd.grad((out, lse), xs, (dout, dlse), retain_graph=True)
+    took(True, True)
+
+    sub_out, sub_lse = mod(*(x.detach().as_subclass(_Subclass).requires_grad_() for x in xs), return_lse=True)
+    took(False)
+    assert torch.equal(sub_out, out) and torch.equal(sub_lse, lse)
+
+    got = torch.autograd.grad((out, lse), xs, (dout, dlse), create_graph=True)
+    took(False)
+    same(got, want)
+    assert not any(x.requires_grad for x in got)  # there is no second derivative to be had
+
+    def backward(*a):
+        with torch.no_grad():  # as autograd calls it
+            return ops._backward(out.grad_fn, dout, *a)
+
+    same(backward(dlse.double()), backward(dlse))
+    took(False, True)
+
+    # gradient tensors of the caller's: written in place where their rows are consecutive, refused otherwise
+    given = [torch.zeros(1, 256, 2, 96, device=DEV, dtype=torch.bfloat16)[..., :64] for _ in range(3)]
+    got = backward(dlse, *given)
+    took(True)
+    for a, b, w in zip(got, given, want):
+        assert a.data_ptr() == b.data_ptr() and torch.equal(b, w)
+    with pytest.raises(AssertionError):
+        backward(dlse, torch.zeros(1, 256, 2, 128, device=DEV, dtype=torch.bfloat16)[..., ::2])
+    took(False)
+
+    # a gradient expanded from one value is laid out first, one of another type is cast by autograd: both ordinary steps
+    a = torch.autograd.grad(out.sum(), xs, retain_graph=True)
+    b = torch.autograd.grad(out, xs, torch.ones_like(out), retain_graph=True)
     same(a, b)
-    c = torch.autograd.grad(lse.double().sum(), (q, k), retain_graph=True)
-    d = torch.autograd.grad(lse, (q, k), torch.ones_like(lse))
-    same(c, d)
+    same(torch.autograd.grad(lse.double().sum(), xs[:2], retain_graph=True), torch.autograd.grad(lse, xs[:2], torch.ones_like(lse)))
+    took(True, True, True, True)
