@@ -100,25 +100,56 @@ def test_short_call_of_a_module_for_long_sequences(B, Hq, Hkv, L, table, bs, wal
             assert torch.equal(a, b), name
 
 
-@pytest.mark.parametrize("D,bs,dtype", [(128, 64, torch.bfloat16), (64, 64, torch.float16), (256, 64, torch.bfloat16),
-                                        (128, 32, torch.bfloat16), (64, 16, torch.float16)])
-def test_short_columns(D, bs, dtype):
-    """dK / dV of columns with one to five listed blocks, fewer than the steps that are requested ahead and around the
-    lengths of the rings, their last step whole, one row or one row short; the second head lists nothing below the diagonal."""
-    n = 6 * 64 // bs
-    bm = np.zeros((2, n, n), dtype=bool)
-    for c in range(n):
-        bm[0, c:c + 1 + c % 5, c] = True
-    bm[1] = np.eye(n, dtype=bool)
-    mod = SparseAttention(bs, torch.from_numpy(bm)).to(DEV)
+def _check_against_oracle(mod, bm, bs, D, dtype, heads, lengths):
     sm = 1 / math.sqrt(D)
-    for L, Lk in ((1, 1), (31, 31), (32, 32), (33, 33), (65, 65), (97, 97), (320, 320), (353, 353), (384, 384), (40, 300)):
+    for L, Lk in lengths:
         print(f"case D={D} bs={bs} {dtype} L={L} Lk={Lk}", flush=True)
-        q, k, v, do = make_qkv(1, L, Lk, 2, 2, D, dtype, with_do=True)
+        q, k, v, do = make_qkv(1, L, Lk, *heads, D, dtype, with_do=True)
         got, ran = _run(mod, q, k, v, do, sm)
-        assert "mfma_dkdv" in ran, ran
+        assert "mfma_dkdv" in ran and ("SUB = true" in ran) == (bs < 64) and "per q head" not in ran, ran
         qo, ko, vo = (x.clone().float().requires_grad_() for x in (q, k, v))
         ro, _ = oracle_fwd(qo, ko, vo, bm, bs, sm, causal=True)
         ro.backward(do.float())
         for name, a, want in zip(("dQ", "dK", "dV"), got, (qo.grad, ko.grad, vo.grad)):
             assert_close(f"{name} L={L} Lk={Lk}", a, want, **TOL)
+
+
+SHORT = [(128, 64, torch.bfloat16), (64, 64, torch.float16), (256, 64, torch.bfloat16), (128, 32, torch.bfloat16), (64, 16, torch.float16),
+         (256, 32, torch.bfloat16), (112, 32, torch.float16)]  # (the last two: masked steps of which no wave sits one out)
+
+
+@pytest.mark.parametrize("D,bs,dtype", SHORT)
+def test_short_columns(D, bs, dtype):
+    """dK / dV of columns with one to five listed blocks (and of the call's part of them), fewer than the steps that are
+    requested ahead and around the lengths of the rings, their last step whole, one row or one row short; the second head lists nothing
+    below the diagonal."""
+    n = 10 * 64 // bs
+    bm = np.zeros((2, n, n), dtype=bool)
+    for c in range(n):
+        bm[0, c:c + 1 + c % 5, c] = True
+    bm[1] = np.eye(n, dtype=bool)
+    tiles = bm[0, :, :5].sum(0)
+    assert list(tiles) == [1, 2, 3, 4, 5]
+    mod = SparseAttention(bs, torch.from_numpy(bm)).to(DEV)
+    _check_against_oracle(mod, bm, bs, D, dtype, (2, 2), (
+        (1, 1), (31, 31), (32, 32), (33, 33), (65, 65), (97, 97), (320, 320), (353, 353), (384, 384), (609, 609), (640, 640), (40, 300)))
+
+
+@pytest.mark.parametrize("D,bs,dtype", SHORT)
+def test_short_columns_of_a_group(D, bs, dtype, monkeypatch):
+    """The same where a workgroup goes on from head to head: columns in which the two heads of a group list none, one or two tiles
+    each, in every combination, so that the stream ends, or changes heads, within the steps that
+    are requested ahead."""
+    n, first = 6, (0, 1, 2, 1, 0, 0)  # tiles; what head h lists in column 0
+    tiles = np.zeros((6, n, n), dtype=bool)
+    for h in range(6):
+        for c in range(n):
+            tiles[h, c:c + (c + first[h]) % 3, c] = True
+        tiles[h, 0, 0] = True  # (every row has a key)
+    lists = tiles.sum(1)
+    pairs = {(int(a), int(b)) for h in (0, 2, 4) for a, b in zip(lists[h, 1:-1], lists[h + 1, 1:-1])}
+    assert pairs == {(0, 1), (1, 2), (2, 0), (2, 1), (0, 2), (1, 0), (0, 0), (1, 1), (2, 2)}
+    bm = np.kron(tiles, np.ones((1, 64 // bs, 64 // bs), dtype=bool))
+    mod = SparseAttention(bs, torch.from_numpy(bm)).to(DEV)
+    monkeypatch.setattr(ops, "_bwd_workspace", False)
+    _check_against_oracle(mod, bm, bs, D, dtype, (6, 3), ((33, 33), (321, 321), (353, 353), (384, 384), (100, 350)))
