@@ -47,7 +47,7 @@ using dk::fail;
 
 extern "C" {
 
-int dk_version(void) { return 600; /* 0.6.0 */ }
+int dk_version(void) { return 700; /* 0.7.0 */ }
 const char *dk_last_error(void) { return dk::g_err; }
 const char *dk_last_kernels(void) { return dk::g_kernels; }
 

@@ -739,9 +739,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
 // operand addresses are moved on in place, everything that only the change of heads or a partial tile needs is computed
 // there from opaque copies, and the multiplies of one step stand next to the exponentials of the next: the S wave leaves
 // the second half of dV to the following step, the dP wave forms dP of its step before dS of the one before.  Scalar
-// instructions per step and wave 113 -> 60, vector 85 -> 70.  Training, us: 32 heads of 128 x 8192 tokens 927 -> 892
-// (this pass 473 -> 421), 4 x 2048, 32 / 8 heads 597 -> 572, 4 x 3000 tokens of 12 heads of 64 with global blocks of 32
-// 249 -> 241, 3000 tokens of 256 dims 287 -> 276.
+// instructions per step and wave 113 -> 60, vector ones next to the 16 multiplies 85 -> 77, matrix pipe 40 -> 46 % busy.
+// This pass, us, both sides traced twice on one box: 32 heads of 128 x 8192 tokens 412 / 415 -> 388 / 386, 4 x 2048, 32 / 8 heads
+// 293 / 288 -> 265 / 264, 4 x 3000 tokens of 12 heads of 64 with global blocks of 32 101 / 97 -> 94 / 95, 3000 tokens of
+// 16 heads of 256 122 / 123 -> 113 / 114.
 template <int D>
 struct DkdvSmem {
   using TL = Tile<D>;
@@ -756,7 +757,7 @@ struct DkdvSmem {
 };
 
 // At the 64-wide tile a step is eight multiplies per wave against the same barrier, waits and scalar work as at the
-// 128-wide one, so a third workgroup per CU (45 KB of LDS and 136 - 141 registers each) fills what two leave idle: training,
+// 128-wide one, so a third workgroup per CU (45 KB of LDS and 152 - 154 registers each) fills what two leave idle: training,
 // 64 dims, two / three workgroups, us: 32 heads x 8192 tokens 558 / 523, 4 x 3000 tokens of 12 heads with global blocks of
 // 32 334 / 310.
 template <typename T, int D, bool PAD, bool SUB, int KD = D>
@@ -861,8 +862,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
 
-  // operand read addresses inside a 32-row tile at offset 0; the Q stage is a compile-time constant of the loop body, so
-  // that stage and row offsets are instruction immediates
+  // operand read addresses inside a 32-row tile at offset 0; each role moves its copy of them on with the rings (below), so
+  // that row offsets, and the half of a block, are instruction immediates
   using OA = OperandAddress<D>;
   typename OA::type rd[KS], tr[DT][2];
   {

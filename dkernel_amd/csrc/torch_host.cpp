@@ -1,4 +1,4 @@
-// Host path of the inference calls in C++ (CPython module dkernel_amd._host): what ops.py does for a
+// Host path of inference calls and training steps in C++ (CPython module dkernel_amd._host): what ops.py does for a
 // forward that needs no gradient - checks, outputs, scratch, the argument block of dk_fwd - without
 // the interpreter.  A single-token step or a short prompt keeps the GPU busy for 8 - 15 us; the
 // Python launcher took 15 us of host time per call around the launch itself (2.5 us).  For the two halves of a training
@@ -468,7 +468,9 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
     PyErr_SetString(PyExc_TypeError, "wrong number of arguments, or bind() was not called");
     return nullptr;
   }
-  // training takes the Python path: told without the cost of an exception
+  // Nothing done here is recorded for gradients.  autograd calls both halves of a training step with gradient mode off, unless
+  // the backward is to be differentiated itself; with it on, an input that asks for gradients leaves the call to ops.py: told
+  // without the cost of an exception.
   if (at::GradMode::is_enabled())
     for (int i = 0; i < 3; ++i)
       if (THPVariable_Check(args[i]) && THPVariable_Unpack(args[i]).requires_grad()) Py_RETURN_NONE;
