@@ -62,7 +62,7 @@ def test_sparse_tiles(B, Hq, Hkv, L, D, bs, dtype, causal, density):
     (256, 32, torch.bfloat16, False), (256, 16, torch.float16, True), (112, 32, torch.bfloat16, False), (112, 32, torch.float16, True),
     (128, 16, torch.bfloat16, False), (96, 32, torch.bfloat16, True), (64, 16, torch.float16, False), (64, 32, torch.bfloat16, True)])
 def test_listed_tiles_without_an_attended_block(D, bs, dtype, walk, monkeypatch):
-    """Entries of an empty mask in the column table are passed over, at any place of a column, as a column's only ones and where
+    """Entries of an empty mask in the column table add nothing, at any place of a column, as a column's only ones and where
     one head's entries follow another's: rows that a column meets in such a tile alone may hold anything."""
     print(f"case D={D} bs={bs} {dtype} walk={walk}", flush=True)
     Hq, Hkv, L, n, f = 4, 2, 256, 4, 64 // bs
