@@ -740,7 +740,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, D == 64 
 // there from opaque copies, and the multiplies of one step stand next to the exponentials of the next: the S wave leaves
 // the second half of dV to the following step, the dP wave forms dP of its step before dS of the one before.  Scalar
 // instructions per step and wave 113 -> 60, vector ones next to the 16 multiplies 85 -> 77, matrix pipe 40 -> 46 % busy.
-// This pass, us, both sides traced twice on one box: 32 heads of 128 x 8192 tokens 412 / 415 -> 388 / 386, 4 x 2048, 32 / 8 heads
+// This pass, us, both sides traced twice in turn: 32 heads of 128 x 8192 tokens 412 / 415 -> 388 / 386, 4 x 2048, 32 / 8 heads
 // 293 / 288 -> 265 / 264, 4 x 3000 tokens of 12 heads of 64 with global blocks of 32 101 / 97 -> 94 / 95, 3000 tokens of
 // 16 heads of 256 122 / 123 -> 113 / 114.
 template <int D>
